@@ -284,6 +284,9 @@ void apply_gemm_flags(cubert::GemmParams* p, int flags) {
     p->splits = CUBERT_SPLITS_OF(flags) > 1 ? CUBERT_SPLITS_OF(flags) : 1;
     p->xcd_partition = ((flags >> 16) & 0xf) - 1;
 }
+int result_layout(int flags) {
+    return (flags & CUBERT_Y_SPLIT) ? cubert::kSplit : (flags & CUBERT_Y_PACKED) ? cubert::kPacked : cubert::kRowMajor;
+}
 }  // namespace
 
 int cubert_op_gemm(const void* X, const void* W, const float* bias, void* Y, int M, int N, int K, int ldx, int elt,
@@ -336,12 +339,21 @@ int cubert_op_gemm_qkv(const void* X, const void* W, const float* bias, void* q,
     return cubert::launch_gemm(p, static_cast<hipStream_t>(stream)) ? 0 : 1;
 }
 
+size_t cubert_split_bytes(size_t rows, size_t K) { return cubert::split_bytes(rows, K); }
+int cubert_op_split_operand(const float* src, void* dst, int K, int N, int row0, void* stream) {
+    cubert::set_error("");
+    return cubert::launch_transpose_convert(src, dst, K, N, cubert::kF32Split, false, row0, static_cast<hipStream_t>(stream)) ? 0 : 1;
+}
+
 size_t cubert_packed_bytes(size_t rows, size_t row_bytes) { return cubert::packed_bytes(rows, row_bytes); }
 size_t cubert_packed_offset(int row, int kbyte, int row_bytes) { return cubert::packed_offset(row, kbyte, row_bytes / 64); }
 
 int cubert_op_attention(const void* q, const void* k, const void* vt, const float* maskadd, void* ctx, int B,
                         int heads, int S, float scale, int elt, int flags, void* stream) {
     cubert::set_error("");
+    if (elt == cubert::kF32Split)
+        return cubert::launch_attention_f32(q, k, vt, maskadd, ctx, B, heads, S, cubert::round_up(S > 0 ? S : 1, 32), scale,
+                                            static_cast<hipStream_t>(stream)) ? 0 : 1;
     return cubert::launch_attention(q, k, vt, maskadd, ctx, (flags & CUBERT_Y_PACKED) != 0, B, heads, S,
                                     cubert::round_up(S > 0 ? S : 1, 32), scale, elt,
                                     static_cast<hipStream_t>(stream), nullptr, (flags & CUBERT_V_ROWMAJOR) != 0, false,
@@ -351,8 +363,7 @@ int cubert_op_attention(const void* q, const void* k, const void* vt, const floa
 int cubert_op_add_layernorm(float* x, const void* y, int y_elt, const float* gamma, const float* beta, void* xb,
                             int rows, int hidden, int flags, void* stream) {
     cubert::set_error("");
-    return cubert::launch_add_layernorm(x, y, y_elt, gamma, beta, static_cast<cubert::bf16_t*>(xb),
-                                        (flags & CUBERT_Y_PACKED) != 0, rows, hidden,
+    return cubert::launch_add_layernorm(x, y, y_elt, gamma, beta, xb, result_layout(flags), rows, hidden,
                                         static_cast<hipStream_t>(stream),
                                         CUBERT_SPLITS_OF(flags) > 1 ? CUBERT_SPLITS_OF(flags) : 1,
                                         (flags & CUBERT_LN_NO_RESIDUAL) == 0) ? 0 : 1;
@@ -364,7 +375,7 @@ int cubert_op_embed_layernorm(const int* ids, const int* seg, const int* mask, c
                               void* stream) {
     cubert::set_error("");
     return cubert::launch_embed_layernorm(ids, seg, mask, word, pos, type, gamma, beta, x,
-                                          static_cast<cubert::bf16_t*>(xb), (flags & CUBERT_Y_PACKED) != 0, maskadd, B, S,
+                                          xb, result_layout(flags), maskadd, B, S,
                                           cubert::round_up(S > 0 ? S : 1, 32), hidden, vocab, type_vocab,
                                           static_cast<hipStream_t>(stream)) ? 0 : 1;
 }

@@ -7,7 +7,7 @@
 
 namespace cubert {
 
-enum Precision : int { kF32 = 0, kBF16 = 1 };
+enum Precision : int { kF32 = 0, kBF16 = 1, kF32Split = 2 };   // kF32Split: GEMM operands only, float32 in the split layout below
 
 struct Dims {
     int hidden = 768;
@@ -60,6 +60,36 @@ __host__ __device__ inline size_t packed_offset(int r, int kbyte, int KB) {
            (kbyte & 15);
 }
 
+// ---- split operand layout --------------------------------------------------
+// float32 operands of a GEMM, every element as the exact sum of three bfloat16 numbers (split_bf16x3): plane 0 is the
+// element rounded to bf16, plane 1 what is left rounded to bf16, plane 2 the rest (at most 7 bits, so exact).  Six of the
+// nine products of two such elements give their float32 product: the dropped ones (planes 1 and 2, 2 and 2) are below
+// 2^-24 of it at the worst and 2^-28 typically, less than one rounding of a float32 multiply-add chain.  gfx950 multiplies
+// bf16 sixteen times as fast as float32 on the matrix pipe, so six products take 0.375 of the time of one.
+// Layout: 1 KiB units of 32 rows x 16 k x one plane, in the register layout of the 32x32x16 MFMA operand (lane
+// 32 (k / 8 % 2) + row % 32 owns 16 bytes), unit (row / 32, k / 16, plane) at ((row / 32 * (K / 16) + k / 16) * 3 + plane).
+// Rows are padded to a multiple of 32.
+enum OperandLayout : int { kRowMajor = 0, kPacked = 1, kSplit = 2 };
+__host__ __device__ inline size_t split_bytes(size_t rows, size_t K) { return (rows + 31) / 32 * (K / 16) * 3072; }
+// Byte offset of plane 0 of element (r, k); planes 1 and 2 follow 1024 and 2048 bytes further.
+__host__ __device__ inline size_t split_offset(int r, int k, int K) {
+    return ((size_t)(r >> 5) * (K >> 4) + (k >> 4)) * 3072 + ((k >> 3) & 1) * 512 + (r & 31) * 16 + (k & 7) * 2;
+}
+// float32 Q, K, V of the attention (attention_f32.hip): per (batch, head) and block of 32 positions twelve units (four
+// groups of 16 features x three planes).  V's positions are permuted inside a half unit (half: features 8 half .. + 7 of the
+// 16) so that its transposing LDS reads spread over the banks.
+__host__ __device__ inline int attn_v_slot(int pos, int half, int kk) { return pos ^ (4 * half + 8 * (kk & 1)); }
+#if defined(__HIPCC__)
+// (Within 0.4 % of the largest float the first plane rounds to infinity; infinities and NaNs end as NaN.)
+__device__ __forceinline__ void split_bf16x3(float x, __bf16& p0, __bf16& p1, __bf16& p2) {
+#pragma clang fp contract(off)
+    p0 = (__bf16)x;
+    const float r1 = x - (float)p0;
+    p1 = (__bf16)r1;
+    p2 = (__bf16)(r1 - (float)p1);
+}
+#endif
+
 // ---- LayerNorm statistics -------------------------------------------------
 // Every LayerNorm of the engine (the row kernels and the GEMM epilogue that normalises) forms its
 // row statistics the same way, so that a row gets the same bits whichever kernel handles it.
@@ -87,6 +117,30 @@ __device__ __forceinline__ float ln_dpp_lanes(float v) {
 // compiler's builtin returns the first register twice.)
 __device__ __forceinline__ void half_swap(float& a, float& b) {
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+// Accumulator layout -> split layout.  x: four consecutive values (features or k) of group 2 u and four of group 2 u + 1 of
+// my row, the halves lane / 32 of the two groups of eight; after exchanging with lane ^ 32 a lane holds all eight of group
+// 2 u + lane / 32, i.e. the 16 bytes per plane of a unit that are its own.  Every lane of the wave takes part.
+typedef __attribute__((ext_vector_type(4))) unsigned int split_u32x4_t;
+__device__ __forceinline__ void split_unit_rows(const float (&x)[8], split_u32x4_t (&planes)[3]) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+    float w[3][4];                       // [plane][pairs 0 1, 2 3 of group 2 u; of group 2 u + 1], as bits
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        __bf16 a0, a1, a2, b0, b1, b2;
+        split_bf16x3(x[2 * i], a0, a1, a2);
+        split_bf16x3(x[2 * i + 1], b0, b1, b2);
+        w[0][i] = __builtin_bit_cast(float, bf16x2_t{a0, b0});
+        w[1][i] = __builtin_bit_cast(float, bf16x2_t{a1, b1});
+        w[2][i] = __builtin_bit_cast(float, bf16x2_t{a2, b2});
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        half_swap(w[p][0], w[p][2]);
+        half_swap(w[p][1], w[p][3]);
+        planes[p] = split_u32x4_t{__builtin_bit_cast(unsigned, w[p][0]), __builtin_bit_cast(unsigned, w[p][1]),
+                                  __builtin_bit_cast(unsigned, w[p][2]), __builtin_bit_cast(unsigned, w[p][3])};
+    }
 }
 __device__ __forceinline__ float half_swap_sum(float v) {
     float a = v, b = v;

@@ -101,13 +101,14 @@ bool Model::init(const ModelOptions& opt_in) {
 
     const int elt = opt_.precision;
     const size_t es = elt == kBF16 ? 2 : 4;
+    const size_t os = elt == kBF16 ? 2 : 6;      // bytes per element of a GEMM operand: bf16, or float32 as three bf16 planes
     const size_t H = D.hidden, I = D.inter;
 
     // ---- weight block layout ----
     Arena wa;
     const size_t o_word = wa.take((size_t)D.vocab * H * 4), o_pos = wa.take((size_t)D.max_pos * H * 4),
                  o_type = wa.take((size_t)D.type_vocab * H * 4), o_eg = wa.take(H * 4), o_eb = wa.take(H * 4);
-    auto wbytes = [&](size_t rows, size_t k) { return elt == kBF16 ? packed_bytes(rows, k * 2) : rows * k * es; };
+    auto wbytes = [&](size_t rows, size_t k) { return elt == kBF16 ? packed_bytes(rows, k * 2) : split_bytes(rows, k); };
     struct LayerOff { size_t w_qkv, w_ao, w_in, w_out, b_qkv, b_ao, b_in, b_out, g1, be1, g2, be2; };
     std::vector<LayerOff> lo(D.layers);
     for (auto& l : lo) {
@@ -131,18 +132,16 @@ bool Model::init(const ModelOptions& opt_in) {
     };
     // [in, out] float32 on disk -> [out, in] operand type on device
     float* stage = reinterpret_cast<float*>(wblock_ + o_stage);
-    // bf16 mode keeps GEMM operands in the packed layout (common.h); the pooler
-    // weight stays row-major (its kernel is a plain dot product).
-    const bool packed = elt == kBF16;
+    // GEMM operands are kept in the packed (bf16) or split (float32) layout (common.h); the
+    // pooler weight stays row-major (its kernel is a plain dot product).
     bool pack_this = true;
     // `row0`: first output row of this tensor inside the destination matrix (the
     // Q, K and V kernels are stacked into one [3H, H] operand).
     auto up_t = [&](size_t off, const NpyArray* a, int row0 = 0) -> bool {
         const int K = (int)a->shape[0], N = (int)a->shape[1];
         CUBERT_HIP_OK(hipMemcpyAsync(stage, a->data.data(), a->data.size() * 4, hipMemcpyHostToDevice, stream_));
-        const bool pk = packed && pack_this;
-        unsigned char* dst = wblock_ + off + (pk ? 0 : (size_t)row0 * K * es);
-        if (!launch_transpose_convert(stage, dst, K, N, elt, pk, pk ? row0 : 0, stream_)) return false;
+        if (!launch_transpose_convert(stage, wblock_ + off, K, N, elt == kF32 && pack_this ? (int)kF32Split : elt,
+                                      elt == kBF16 && pack_this, row0, stream_)) return false;
         CUBERT_HIP_OK(hipStreamSynchronize(stream_));      // the staging buffer is reused
         return true;
     };
@@ -190,10 +189,11 @@ bool Model::init(const ModelOptions& opt_in) {
     const size_t Npad = N + 32 * 1024;
     Arena aa;
     const size_t o_x32 = aa.take(N * H * 4);
-    const size_t o_xb = elt == kBF16 ? aa.take(N * H * 2) : 0;
-    const size_t o_q = aa.take((N + 64) * H * es), o_k = aa.take((N + 64) * H * es);
-    const size_t o_vt = aa.take(Npad * H * es), o_ctx = aa.take(N * H * es);
-    const size_t o_h = aa.take(N * I * es), o_y = aa.take((N + kSplitRows) * H * 4);
+    const size_t o_xb = aa.take(N * H * os);
+    // float32 mode: q, k and v in blocks of 32 positions (attention_f32.hip)
+    const size_t o_q = aa.take((elt == kF32 ? Npad : N + 64) * H * os), o_k = aa.take((elt == kF32 ? Npad : N + 64) * H * os);
+    const size_t o_vt = aa.take(Npad * H * os), o_ctx = aa.take(N * H * os);
+    const size_t o_h = aa.take(N * I * os), o_y = aa.take((N + kSplitRows) * H * 4);
     const size_t o_mask = aa.take(Npad * 4), o_pool = aa.take((size_t)1024 * H * 4), o_cls = aa.take(1024 * 8 * 4);
     const size_t o_in = aa.take(3 * N * 4);
     const size_t meta_ints = N + (size_t)kMaxParts * kCuStride;
@@ -201,8 +201,8 @@ bool Model::init(const ModelOptions& opt_in) {
     ln_ws_bytes_ = (gemm_ln_workspace_bytes(N) + 255) / 256 * 256;
     const size_t o_lnws = aa.take(ln_ws_bytes_ * kMaxParts);
     const size_t NC = (size_t)kMaxParts * 1024;       // first-token rows: B <= 1024 per part, parts 1024 rows apart
-    const size_t o_xc = aa.take(NC * H * 4), o_yc = aa.take(NC * H * 4), o_xbc = elt == kBF16 ? aa.take(NC * H * 2) : 0;
-    const size_t o_ctxc = aa.take(NC * H * es), o_hc = aa.take(NC * I * es);
+    const size_t o_xc = aa.take(NC * H * 4), o_yc = aa.take(NC * H * 4), o_xbc = aa.take(NC * H * os);
+    const size_t o_ctxc = aa.take(NC * H * os), o_hc = aa.take(NC * I * os);
     act_bytes_ = aa.off;
     size_t free_b = 0, total_b = 0;
     CUBERT_HIP_OK(hipMemGetInfo(&free_b, &total_b));
@@ -216,7 +216,7 @@ bool Model::init(const ModelOptions& opt_in) {
     // masked out); they must hold finite numbers, so start from all zeros.
     CUBERT_HIP_OK(hipMemsetAsync(ablock_, 0, act_bytes_, stream_));
     x32_ = reinterpret_cast<float*>(ablock_ + o_x32);
-    xb_ = elt == kBF16 ? reinterpret_cast<bf16_t*>(ablock_ + o_xb) : nullptr;
+    xb_ = ablock_ + o_xb;
     q_ = ablock_ + o_q; k_ = ablock_ + o_k; vt_ = ablock_ + o_vt; ctx_ = ablock_ + o_ctx; h_ = ablock_ + o_h;
     y32_ = reinterpret_cast<float*>(ablock_ + o_y);
     maskadd_ = reinterpret_cast<float*>(ablock_ + o_mask);
@@ -228,7 +228,7 @@ bool Model::init(const ModelOptions& opt_in) {
     ln_ws_ = ablock_ + o_lnws;       // all zero from the clearing above, which is what the first launch needs
     xc32_ = reinterpret_cast<float*>(ablock_ + o_xc);
     yc32_ = reinterpret_cast<float*>(ablock_ + o_yc);
-    xbc_ = elt == kBF16 ? reinterpret_cast<bf16_t*>(ablock_ + o_xbc) : nullptr;
+    xbc_ = ablock_ + o_xbc;
     ctxc_ = ablock_ + o_ctxc;
     hc_ = ablock_ + o_hc;
     CUBERT_HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_meta_), meta_ints * 4, hipHostMallocDefault));
@@ -519,7 +519,8 @@ bool Model::enqueue(int B, int S, bool has_mask) {
 bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp) {
     const Dims& D = opt_.dims;
     const int elt = opt_.precision;
-    const size_t es = elt == kBF16 ? 2 : 4;
+    const size_t os = elt == kBF16 ? 2 : 6;      // bytes per element of a GEMM operand and of q, k, v
+    const int gelt = elt == kBF16 ? kBF16 : kF32Split, layout = elt == kBF16 ? kPacked : kSplit;
     // rows of this part: every token, or (unpadded pass) the valid ones only, stored from row r0
     const int H = D.hidden, I = D.inter, N = cp ? cp->rows : B * S, Sp = round_up(S, 32);
     const size_t cap = (size_t)cap_tokens_, t0 = (size_t)b0 * S;
@@ -527,14 +528,14 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     const int *ids = d_in_ + t0, *seg = d_in_ + cap + t0, *mask = has_mask ? d_in_ + 2 * cap + t0 : nullptr;
     float* x32 = x32_ + (cp ? r0 : t0) * H;
     float* y32 = y32_ + r0 * H;
-    bf16_t* xb = xb_ ? xb_ + r0 * H : nullptr;
-    unsigned char* q = static_cast<unsigned char*>(q_) + t0 * H * es;
-    unsigned char* k = static_cast<unsigned char*>(k_) + t0 * H * es;
-    unsigned char* vt = static_cast<unsigned char*>(vt_) + (size_t)b0 * H * Sp * es;
-    unsigned char* ctx = static_cast<unsigned char*>(ctx_) + r0 * H * es;
-    unsigned char* h = static_cast<unsigned char*>(h_) + r0 * I * es;
+    unsigned char* xb = xb_ + r0 * H * os;
+    const size_t qk0 = elt == kF32 ? (size_t)b0 * Sp : t0;      // first position of this part in q and k
+    unsigned char* q = static_cast<unsigned char*>(q_) + qk0 * H * os;
+    unsigned char* k = static_cast<unsigned char*>(k_) + qk0 * H * os;
+    unsigned char* vt = static_cast<unsigned char*>(vt_) + (size_t)b0 * H * Sp * os;
+    unsigned char* ctx = static_cast<unsigned char*>(ctx_) + r0 * H * os;
+    unsigned char* h = static_cast<unsigned char*>(h_) + r0 * I * os;
     float* maskadd = maskadd_ + (size_t)b0 * Sp;
-    const void* xin = elt == kBF16 ? static_cast<const void*>(xb) : static_cast<const void*>(x32);
     const float scale = 1.0f / std::sqrt(64.0f);
 
     // Short batches: the two GEMMs with only `hidden` output features have too few tiles for the
@@ -546,35 +547,42 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             max_splits = 16;
             while (max_splits > 1 && (long)max_splits * N > (long)N + kSplitRows) max_splits /= 2;
         }
-        return gemm_plan(N, H, K, elt, max_splits, true, false);
+        return gemm_plan(N, H, K, gelt, max_splits, true, false);
     };
+    const bool any_order = cur_parts_ == 1 && opt_.split_k;
     const GemmPlan plan_ao = plan_for(H), plan_fo = plan_for(I);
     const int sp_ao = plan_ao.splits, sp_fo = plan_fo.splits;
     // the attn-out / FFN-out GEMMs add the residual stream in their epilogue, so LayerNorm reads one operand
     const bool fuse_res = opt_.fuse_residual;
     // ... and, where the GEMM kernel can, normalise there as well: x32 and its bf16 copy come straight out of
     // the GEMM and the LayerNorm launch disappears.  (Not with split K, whose parts the LayerNorm kernel adds.)
-    const bool ln_ao = fuse_res && opt_.fuse_layernorm && sp_ao == 1 && gemm_ln_supported(N, H, H, elt);
-    const bool ln_fo = fuse_res && opt_.fuse_layernorm && sp_fo == 1 && gemm_ln_supported(N, H, I, elt);
+    const bool ln_ao = fuse_res && opt_.fuse_layernorm && sp_ao == 1 && gemm_ln_supported(N, H, H, gelt);
+    const bool ln_fo = fuse_res && opt_.fuse_layernorm && sp_fo == 1 && gemm_ln_supported(N, H, I, gelt);
     void* ln_ws = ln_ws_ + (size_t)part * ln_ws_bytes_;
     if (ln_ao || ln_fo) ln_used_ = std::max(ln_used_, part + 1);
 
+    auto attention = [&](void* out, bool vrow, bool first_only) {
+        if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only);
+        return launch_attention(q, k, vt, maskadd, out, true, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto);
+    };
+
     if (!mark(kPhEmbed)) return false;
-    const bool pk = elt == kBF16;           // packed GEMM operands (weights were packed at load)
-    if (!launch_embed_layernorm(ids, seg, mask, word_, pos_, type_, emb_g_, emb_b_, x32, xb, pk, maskadd, B, S, Sp,
+    const bool pk = elt == kBF16;           // packed GEMM operands (weights were packed at load); else split ones
+    if (!launch_embed_layernorm(ids, seg, mask, word_, pos_, type_, emb_g_, emb_b_, x32, xb, layout, maskadd, B, S, Sp,
                                 H, D.vocab, D.type_vocab, st, cp))
         return false;
     for (int i = 0; i < D.layers; ++i) {
         const LayerDev& L = layers_[i];
         GemmParams g;
-        g.elt = elt;
+        g.elt = gelt;
         // QKV projection, scattered per head (V transposed, unless the attention kernel that follows
         // transposes on its own LDS reads)
         const bool vrow = opt_.v_rowmajor && elt == kBF16 && S <= 512;
-        g.X = xin; g.ldx = H; g.W = L.w_qkv; g.bias = L.b_qkv; g.M = N; g.N = 3 * H; g.K = H;
+        g.X = xb; g.ldx = H; g.W = L.w_qkv; g.bias = L.b_qkv; g.M = N; g.N = 3 * H; g.K = H;
         g.epilogue = kEpiQKV; g.q = q; g.k = k; g.vt = vt; g.S = S; g.Sp = Sp; g.heads = D.heads;
         g.v_rowmajor = vrow;
         g.rowmap = cp ? cp->rowmap : nullptr;
+        g.any_k_order = any_order;
         g.x_packed = g.w_packed = pk;
         if (!mark(kPhQKV) || !launch_gemm(g, st)) return false;
         // The last layer of a pass whose caller gets no sequence output: keys and values are needed of every token,
@@ -587,58 +595,58 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             const size_t c0 = (size_t)part * 1024;
             float* xc = xc32_ + c0 * H;
             float* yc = yc32_ + c0 * H;
-            bf16_t* xbc = xbc_ ? xbc_ + c0 * H : nullptr;
-            unsigned char* ctxc = static_cast<unsigned char*>(ctxc_) + c0 * H * es;
-            unsigned char* hc = static_cast<unsigned char*>(hc_) + c0 * I * es;
-            const void* xcin = elt == kBF16 ? static_cast<const void*>(xbc) : static_cast<const void*>(xc);
-            if (!launch_attention(q, k, vt, maskadd, ctxc, pk, B, D.heads, S, Sp, scale, elt, st, cu, vrow, true, vrow ? cur_attn_ : kAttnAuto)) return false;
+            unsigned char* xbc = xbc_ + c0 * H * os;
+            unsigned char* ctxc = static_cast<unsigned char*>(ctxc_) + c0 * H * os;
+            unsigned char* hc = static_cast<unsigned char*>(hc_) + c0 * I * os;
+            if (!attention(ctxc, vrow, true)) return false;
             if (!launch_gather_first_rows(x32, cu, xc, B, S, H, st)) return false;
             g = GemmParams();
-            g.elt = elt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
+            g.elt = gelt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
             g.M = B; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk;
             g.residual = fuse_res ? xc : nullptr;
             if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
-            if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, pk, B, H, st, 1, !fuse_res)) return false;
+            if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, layout, B, H, st, 1, !fuse_res)) return false;
             g = GemmParams();
-            g.elt = elt; g.out_elt = elt; g.X = xcin; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
+            g.elt = g.out_elt = gelt; g.X = xbc; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
             g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = pk;
             if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
             g = GemmParams();
-            g.elt = elt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;
+            g.elt = gelt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;
             g.M = B; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk;
             g.residual = fuse_res ? xc : nullptr;
             if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
-            if (!launch_add_layernorm(xc, yc, kF32, L.g2, L.be2, nullptr, false, B, H, st, 1, !fuse_res)) return false;
+            if (!launch_add_layernorm(xc, yc, kF32, L.g2, L.be2, nullptr, kRowMajor, B, H, st, 1, !fuse_res)) return false;
             if (!mark(kPhPooler)) return false;
             return launch_pooler(xc, w_pool_, elt, b_pool_, pooled_ + (size_t)b0 * H, B, 1, H, st, nullptr);
         }
-        if (!launch_attention(q, k, vt, maskadd, ctx, pk, B, D.heads, S, Sp, scale, elt, st, cu, vrow, false, vrow ? cur_attn_ : kAttnAuto)) return false;
+        if (!attention(ctx, vrow, false)) return false;
         // attention output projection -> f32, then residual add + LayerNorm
         g = GemmParams();
-        g.elt = elt; g.out_elt = kF32; g.X = ctx; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = y32;
+        g.elt = gelt; g.out_elt = kF32; g.X = ctx; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = y32;
         g.M = N; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk; g.splits = sp_ao;
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = plan_ao.tile;
         if (ln_ao) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
-        if (!ln_ao && !launch_add_layernorm(x32, y32, kF32, L.g1, L.be1, xb, pk, N, H, st, sp_ao, !fuse_res)) return false;
+        if (!ln_ao && !launch_add_layernorm(x32, y32, kF32, L.g1, L.be1, xb, layout, N, H, st, sp_ao, !fuse_res)) return false;
         // feed-forward
         g = GemmParams();
-        g.elt = elt; g.out_elt = elt; g.X = xin; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = h;
+        g.elt = g.out_elt = gelt; g.X = xb; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = h;
         g.M = N; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = pk;
+        g.any_k_order = any_order;
         if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
         g = GemmParams();
-        g.elt = elt; g.out_elt = kF32; g.X = h; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = y32;
+        g.elt = gelt; g.out_elt = kF32; g.X = h; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = y32;
         g.M = N; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk; g.splits = sp_fo;
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = plan_fo.tile;
         if (ln_fo) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
-        if (!ln_fo && !launch_add_layernorm(x32, y32, kF32, L.g2, L.be2, xb, pk, N, H, st, sp_fo, !fuse_res)) return false;
+        if (!ln_fo && !launch_add_layernorm(x32, y32, kF32, L.g2, L.be2, xb, layout, N, H, st, sp_fo, !fuse_res)) return false;
     }
     // pooler: first-token gather + dense + tanh on the float32 sequence output
     if (!mark(kPhPooler)) return false;

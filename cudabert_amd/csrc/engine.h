@@ -44,7 +44,7 @@ struct ModelOptions {
 };
 
 struct LayerDev {
-    void *w_qkv, *w_ao, *w_in, *w_out;            // [out, in] in the operand type
+    void *w_qkv, *w_ao, *w_in, *w_out;            // [out, in] as GEMM operands: bf16 packed, or float32 split (common.h)
     float *b_qkv, *b_ao, *b_in, *b_out;
     float *g1, *be1, *g2, *be2;
 };
@@ -123,7 +123,7 @@ class Model {
     size_t act_bytes_ = 0;
     long cap_tokens_ = 0;
     float* x32_ = nullptr;       // residual stream / sequence output [N, H] f32
-    bf16_t* xb_ = nullptr;       // bf16 copy of x (bf16 mode only)
+    unsigned char* xb_ = nullptr;   // GEMM-operand copy of x: bf16 packed, or float32 split
     void *q_ = nullptr, *k_ = nullptr, *vt_ = nullptr, *ctx_ = nullptr, *h_ = nullptr;
     float* y32_ = nullptr;       // attn-out / ffn-out GEMM result [N, H] f32
     float* maskadd_ = nullptr;   // [B, Sp]
@@ -146,7 +146,7 @@ class Model {
     std::vector<int> last_lens_;       // lengths of the last unpadded pass
     // Last layer for the first tokens only: [kMaxParts * 1024] rows each (a part's sequences at part * 1024)
     float *xc32_ = nullptr, *yc32_ = nullptr;      // residual stream / GEMM result of those rows
-    bf16_t* xbc_ = nullptr;                        // bf16 copy (bf16 mode)
+    unsigned char* xbc_ = nullptr;                 // GEMM-operand copy
     void *ctxc_ = nullptr, *hc_ = nullptr;         // attention context / FFN activation of those rows
     bool first_only_ = false;                      // the pass being enqueued (and the last one run) is of that kind
     bool last_compact_ = false;

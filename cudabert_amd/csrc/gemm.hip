@@ -40,6 +40,8 @@ bool launch_gemm_bf16_t256(const gemm_detail::GemmDev& d, int out_elt, int epilo
 bool launch_gemm_bf16_t256x128(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
 bool launch_gemm_bf16_t128(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
 bool launch_gemm_bf16_t256x128_deep(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
+bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream);
+bool launch_gemm_split(const gemm_detail::GemmDev& d, int tile, int epilogue, hipStream_t stream);
 int gemm_pick_tile(int M, int N, int K, int elt);
 int gemm_ln_pick_tile(int M, int N, int K, int elt);
 
@@ -419,9 +421,103 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
     }
     return best;
 }
+
+// float32 operands in the split layout.  Estimated time (microseconds) of a launch from that of a workgroup alone on its CU
+// and w = workgroups / 256, with constants measured on MI355X (cold weights: launches that cycle through 24 matrices, 17 to
+// 1600 rows of the linears of BERT-base and BERT-large, and up to 19600 rows for the large tiles):
+//   128 x 128, 256 x 128: (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly
+//     what the first did, and the hand-out is uneven by half a workgroup; the larger tile wins from about 900 tiles on;
+//   the skinny tiles: fixed + per_step * steps * (w > 1 ? w + 0.5 : 1), bound by what a CU fetches (60 - 65 GB/s of operands).
+// At 128 rows (QKV 3072 x 1024 / FFN-in 4096 x 1024 / FFN-out 1024 x 4096): 13.9 / 15.6 / 14.6 us with the skinny tile,
+// 35.2 / 40.7 / 24.0 with the 128 one; at 1600 rows 81 / 102 / 102 against 65 / 79 / 76.
+// any_order: the caller does not need the k order that all tiles but the skinny ones share.
+GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool any_order) {
+    struct Cand { int tile, bm, bn; double fixed, per_step; bool skinny; };
+    static const Cand cands[] = {
+        {128, 128, 128, 6.0, 0.455, false},
+        {kTile256x128, 128, 256, 8.0, 0.98, false},
+        {kTileSkinny12, 64, 32, 4.5, 0.144, true},
+        {kTileSkinny22, 64, 64, 4.5, 0.214, true},
+    };
+    GemmPlan best{128, min_splits};
+    double best_cost = 1e30;
+    for (const Cand& c : cands) {
+        if (c.skinny && (!any_order || N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
+        for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
+            if (sp > min_splits && K / sp < 128) break;
+            if (c.skinny && 4 * sp > K / 16) break;
+            const double w = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * sp / 256.0, g = w > 1.0 ? w + 0.5 : 1.0;
+            const double loop = c.per_step * (K / 16.0 / sp);
+            double cost = c.skinny ? c.fixed + loop * g : (c.fixed + loop) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
+            // every part of a split result is written and read again by the consumer
+            if (sp > 1) cost += 0.6 + (double)M * N * 4.0 * sp / 4.0e6;
+            if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
+        }
+    }
+    return best;
+}
+
+// Launches a GEMM on split operands.
+bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
+    if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.K % 16 != 0 || p.N % 4 != 0) { set_error("gemm: split operands need K to be a multiple of 16 and N of 4"); return false; }
+    if (!p.X || !p.W || !p.bias || ((reinterpret_cast<uintptr_t>(p.X) | reinterpret_cast<uintptr_t>(p.W) | reinterpret_cast<uintptr_t>(p.bias)) & 15)) {
+        set_error("gemm: null or misaligned operand");
+        return false;
+    }
+    if ((size_t)p.K * 6 * 256 >= (1ull << 31)) { set_error("gemm: K too large"); return false; }
+    if (p.ln_gamma || p.compiler_scheduled || (p.tile != 0 && p.tile != 128 && p.tile != kTile256x128 && p.tile != kTileSkinny12 && p.tile != kTileSkinny22)) {
+        set_error("gemm: split operands take the 128, the 256x128 or a skinny tile and no LayerNorm epilogue");
+        return false;
+    }
+    GemmDev d{};
+    d.X = static_cast<const unsigned char*>(p.X);
+    d.W = static_cast<const unsigned char*>(p.W);
+    d.bias = p.bias;
+    d.Y = static_cast<unsigned char*>(p.Y);
+    d.M = p.M; d.N = p.N; d.K = p.K; d.ldx = p.K;
+    d.splits = p.splits > 0 ? p.splits : 1;
+    int epi = p.epilogue;
+    if (epi == kEpiQKV) {
+        if (!p.q || !p.k || !p.vt || p.S <= 0 || p.heads <= 0 || p.N != 3 * p.heads * 64 || (!p.rowmap && p.M % p.S != 0) ||
+            p.Sp < p.S || p.Sp % 32 != 0 || p.residual || d.splits > 1) {
+            set_error("gemm: bad QKV epilogue arguments");
+            return false;
+        }
+        d.q = static_cast<unsigned char*>(p.q);
+        d.k = static_cast<unsigned char*>(p.k);
+        d.vt = static_cast<unsigned char*>(p.vt);
+        d.S = p.S; d.Sp = p.Sp; d.heads = p.heads; d.hidden = p.heads * 64;
+        d.rowmap = p.rowmap;
+        if (p.rowmap) epi = kEpiQKVMap;
+    } else {
+        if (!p.Y || (reinterpret_cast<uintptr_t>(p.Y) & 15)) { set_error("gemm: bad Y"); return false; }
+        if (epi == kEpiBiasGelu ? (p.out_elt != kF32Split || p.N % 32 != 0 || p.residual || d.splits > 1) : (epi != kEpiBias || p.out_elt != kF32)) {
+            set_error("gemm: split operands give float32 results (bias, residual) or split ones (GELU, N a multiple of 32)");
+            return false;
+        }
+        if (p.residual) {
+            if (reinterpret_cast<uintptr_t>(p.residual) & 15) { set_error("gemm: misaligned residual"); return false; }
+            epi = kEpiBiasRes;
+            d.R = p.residual;
+        }
+    }
+    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.any_k_order).tile;
+    const bool skinny = tile == kTileSkinny12 || tile == kTileSkinny22;
+    const int bn = tile == kTile256x128 ? 256 : tile == kTileSkinny12 ? 32 : tile == kTileSkinny22 ? 64 : 128, bm = skinny ? 64 : 128;
+    d.tiles_n = (p.N + bn - 1) / bn;
+    d.tiles_m = (p.M + bm - 1) / bm;
+    d.xn_parts = gemm_pick_partition((double)p.M * p.K * 6, (double)p.N * p.K * 6, d.tiles_n, d.tiles_m, 8);
+    if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
+    if (skinny && (split_bytes(p.M, p.K) >= (1ull << 31) || split_bytes(p.N, p.K) >= (1ull << 31))) {
+        set_error("gemm: operand exceeds the 2 GiB addressable through one buffer descriptor");
+        return false;
+    }
+    return skinny ? launch_gemm_skinny(d, kF32Split, tile, epi, stream) : launch_gemm_split(d, tile, epi, stream);
+}
 }  // namespace
 
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu) {
+    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, max_splits > 1);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {
@@ -438,6 +534,7 @@ GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result
 }
 
 bool launch_gemm(const GemmParams& p, hipStream_t stream) {
+    if (p.elt == kF32Split) return launch_split_operands(p, stream);
     const int es = (p.elt == kBF16) ? 2 : 4;
     const int bk = 128 / es;
     if (p.elt != kBF16 && p.elt != kF32) { set_error("gemm: bad operand type"); return false; }
@@ -549,6 +646,19 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
             return launch_gemm_bf16_t256x128_deep(d, out, epi, stream);
         }
         return launch_gemm_bf16_t256x128(d, out, epi, stream);
+    }
+    if (bt == kTileSkinny12 || bt == kTileSkinny22) {
+        if (p.elt != kBF16 || !p.x_packed || !p.w_packed || p.N % 8 != 0 || (epi != kEpiQKV && epi != kEpiQKVMap && epi != kEpiBiasGelu && out != kF32) ||
+            (epi == kEpiBiasGelu && !p.y_packed) || ((epi == kEpiQKV || epi == kEpiQKVMap) && !p.v_rowmajor)) {
+            set_error("gemm: the skinny tiles need packed bf16 operands and a packed GELU, row-major QKV or float32 result");
+            return false;
+        }
+        const int bn = bt == kTileSkinny12 ? 32 : 64;
+        d.tiles_n = (p.N + bn - 1) / bn;
+        d.tiles_m = (p.M + 63) / 64;
+        d.xn_parts = gemm_pick_partition((double)p.M * p.K * es, (double)p.N * p.K * es, d.tiles_n, d.tiles_m, 8);
+        if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
+        return launch_gemm_skinny(d, kBF16, bt, epi, stream);
     }
     if (bt == kTile128Hand) {
         if (p.elt != kBF16) { set_error("gemm: the hand-scheduled 128 tile is bf16 only"); return false; }

@@ -7,6 +7,11 @@ string) of the bf16 GEMM macro tiles:
     python gen_gemm_asm.py quarter > gemm_bf16_128_loop.inc     # 128 x 128, three per CU (end of file)
     python gen_gemm_asm.py deep > gemm_bf16_256x128_deep_loop.inc  # 256 x 128, one per CU, the 256 x 256 pipeline
 
+and of the float32 GEMM on operands split into three bf16 planes (end of file):
+
+    python gen_gemm_asm.py split128 > gemm_split_128_loop.inc         # 128 x 128
+    python gen_gemm_asm.py split256x128 > gemm_split_256x128_loop.inc # 256 x 128
+
 The rest of this comment describes the 256 x 256 loop.
 
 Why hand-scheduled: with 256 accumulator registers per lane a SIMD holds one
@@ -428,6 +433,140 @@ def main_skewed(c):
         print('"%s\\n"' % ln)
 
 
+# ---------------------------------------------------------------------------
+# float32 operands, each split into three bf16 planes (common.h, split layout):
+#     python gen_gemm_asm.py split128     > gemm_split_128_loop.inc
+#     python gen_gemm_asm.py split256x128 > gemm_split_256x128_loop.inc
+#
+# A step covers 16 k, one MFMA k-slice.  Its tile holds, per block of 32 rows, three 1 KiB units (one per plane) that
+# are exactly the MFMA operand (lane l's 16 bytes at 16 l), so a global->LDS load moves one unit and a fragment read
+# is linear in the lane.  A wave multiplies nwb x 2 blocks with the six plane products that reach float32 precision:
+# 12 nwb MFMAs on 3 (nwb + 2) fragments, i.e. a quarter to a half of a fragment read per MFMA, where the bf16 loops
+# need three quarters to one.  With two or three waves per SIMD the matrix pipe always has another wave's work while one
+# waits for its first fragments, so nothing is read ahead of the barrier.
+#   s92  stage offset of the tile being multiplied   s93  of the tile being fetched   s94  M0 base (LDS base + wave * 3072)
+#   s95  M0 base of the tile being fetched   s96  K byte offset (the same for both operands)   s97  counter
+class Split:
+    def __init__(self, name, nwb, nstage, frag):
+        self.name, self.nwb, self.nxb, self.nstage = name, nwb, 2, nstage
+        self.w = frag                                # W fragment (plane p, block i): w + 4 (p nwb + i)
+        self.x = frag + 12 * nwb
+        self.base = self.x + 12 * self.nxb           # W, X fragment addresses in stage 0, then of the current stage
+        self.voff = self.base + 4                    # lane offsets of my loads
+        self.x_lds = 2 * nwb * 3072                  # the X tile follows the W tile
+        self.stage = self.x_lds + 4 * 3072
+        self.n = 3 * (nwb // 2) + 3                  # global->LDS loads per step and wave
+        self.last = self.voff + self.n - 1
+
+
+SPLIT128 = Split("split128", 2, 3, 40)
+SPLIT256 = Split("split256x128", 4, 2, 36)
+# (W plane, X plane), the operand pairs whose product counts in float32
+PLANE_PRODUCTS = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)]
+
+
+def main_split(c):
+    e = Emitter()
+    wf = lambda p, i: c.w + 4 * (p * c.nwb + i)
+    xf = lambda p, j: c.x + 4 * (p * c.nxb + j)
+    e.emit("; ======== setup ========")
+    e.emit("v_mov_b32 v%d, %%[wb]" % c.base)
+    e.emit("v_mov_b32 v%d, %%[xb]" % (c.base + 1))
+    # my loads: the three units of W row blocks wave, wave + 4, ... and of X row block wave
+    e.emit("v_mov_b32 v%d, %%[wv0]" % c.voff)
+    for k in range(1, c.n - 3):
+        if k % 3:
+            e.emit("v_add_u32 v%d, 0x400, v%d" % (c.voff + k, c.voff + k - 1))
+        else:
+            e.emit("v_add_u32 v%d, %%[rb4], v%d" % (c.voff + k, c.voff + k - 3))
+    e.emit("v_mov_b32 v%d, %%[xv0]" % (c.voff + c.n - 3))
+    for k in range(c.n - 2, c.n):
+        e.emit("v_add_u32 v%d, 0x400, v%d" % (c.voff + k, c.voff + k - 1))
+    for r in range(4):
+        e.emit("v_mov_b32 v%d, 0" % (c.w + r))
+    e.emit("s_nop 7")      # VALU result -> MFMA source operand
+    for i in range(c.nwb):
+        for j in range(c.nxb):
+            e.emit("v_mfma_f32_32x32x16_bf16 %%[c%d%d], %s, %s, 0" % (i, j, vreg4(c.w), vreg4(c.w)))
+    e.emit("s_mov_b32 s94, %[m0b]")
+    e.emit("s_mov_b32 s92, 0")
+    e.emit("s_mov_b32 s93, 0")
+    e.emit("s_mov_b32 s96, %[k0]")
+
+    lds_off = [(k // 3) * 4 * 3072 + (k % 3) * 1024 for k in range(c.n - 3)] + [c.x_lds + k * 1024 for k in range(3)]
+
+    def dma(k):
+        m0 = "s_add_u32 m0, s95, 0x%x" % lds_off[k]
+        return m0, "buffer_load_dwordx4 v%d, %%[%s], s96 offen lds" % (c.voff + k, "xres" if k >= c.n - 3 else "wres")
+
+    def rotate(reg):
+        e.emit("s_add_u32 s%d, s%d, 0x%x" % (reg, reg, c.stage))
+        e.emit("s_cmp_eq_u32 s%d, 0x%x" % (reg, c.nstage * c.stage))
+        e.emit("s_cselect_b32 s%d, 0, s%d" % (reg, reg))
+
+    def advance():
+        # loads past the end of K fetch the last tile again and are never used
+        e.emit("s_add_u32 s96, s96, 0xc00")
+        e.emit("s_min_u32 s96, s96, %[kmax]")
+
+    e.emit("; ======== prologue ========")
+    for t in range(c.nstage - 1):
+        e.emit("s_add_u32 s95, s94, s93")
+        for k in range(c.n):
+            m0, ld = dma(k)
+            e.emit(m0)
+            e.emit("s_nop 0")
+            e.emit(ld)
+        rotate(93)
+        advance()
+    ahead = c.n * (c.nstage - 2)
+    e.emit("s_waitcnt vmcnt(%d)" % ahead)
+    e.emit("s_barrier")
+    e.emit("s_mov_b32 s97, 0")
+    e.emit("L_loop_%=:")
+    e.forget_bound()
+    e.emit("v_add_u32 v%d, s92, v%d" % (c.base + 2, c.base))
+    e.emit("v_add_u32 v%d, s92, v%d" % (c.base + 3, c.base + 1))
+    e.emit("s_add_u32 s95, s94, s93")
+    for p in range(3):
+        order = [("w", 0)] + [("x", b) for b in range(c.nxb)] + [("w", b) for b in range(1, c.nwb)]
+        for kind, b in order:
+            if kind == "w":
+                e.read(wf(p, b), c.base + 2, b * 3072 + p * 1024)
+            else:
+                e.read(xf(p, b), c.base + 3, c.x_lds + b * 3072 + p * 1024)
+    total = len(PLANE_PRODUCTS) * c.nwb * c.nxb
+    every = max(1, (total - 4) // c.n)
+    m = d = 0
+    for wp, xp in PLANE_PRODUCTS:
+        for i in range(c.nwb):
+            for j in range(c.nxb):
+                e.need(wf(wp, i), xf(xp, j))
+                load = m % every == 0 and d < c.n
+                if load:
+                    e.emit(dma(d)[0])
+                e.emit("v_mfma_f32_32x32x16_bf16 %%[c%d%d], %s, %s, %%[c%d%d]" % (i, j, vreg4(wf(wp, i)), vreg4(xf(xp, j)), i, j))
+                if load:
+                    e.emit(dma(d)[1])
+                    d += 1
+                m += 1
+    assert d == c.n
+    rotate(92)
+    rotate(93)
+    advance()
+    # the next tile has landed; my reads of this one were done before its last MFMAs
+    e.emit("s_waitcnt vmcnt(%d)" % ahead)
+    e.emit("s_barrier")
+    e.emit("s_add_u32 s97, s97, 1")
+    e.emit("s_cmp_lt_u32 s97, %[steps]")
+    e.emit("s_cbranch_scc1 L_loop_%=")
+    e.emit("s_waitcnt vmcnt(0)")
+    e.emit("s_barrier")
+    print("// Generated by gen_gemm_asm.py %s -- do not edit." % c.name)
+    for ln in e.lines:
+        print('"%s\\n"' % ln)
+
+
 if __name__ == "__main__":
     import sys
     if len(sys.argv) > 1 and sys.argv[1] == "half":
@@ -440,5 +579,8 @@ if __name__ == "__main__":
         if len(sys.argv) > 2:
             QUARTER.nstage = int(sys.argv[2])
         main_skewed(QUARTER)
+    elif len(sys.argv) > 1 and sys.argv[1] in ("split128", "split256x128"):
+        c = SPLIT128 if sys.argv[1] == "split128" else SPLIT256
+        main_split(c)
     else:
         main()

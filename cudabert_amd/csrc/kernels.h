@@ -40,6 +40,9 @@ constexpr int kTile256x128 = 384;     // GemmParams::tile value of the 256 featu
 constexpr int kTile256x128Deep = 385; // ... of the 256 x 128 kernel with one workgroup per CU and the deeper pipeline (K % 128 == 0)
 constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 kernel (bf16, three workgroups per CU, splits K)
 
+constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
+constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: packed bf16 or split float32 operands, any K split for float32 results)
+
 struct GemmParams {
     const void* X = nullptr;
     const void* W = nullptr;
@@ -47,7 +50,7 @@ struct GemmParams {
     void* Y = nullptr;        // [M, N] row-major, type out_elt (unused for kEpiQKV)
     int M = 0, N = 0, K = 0;
     int ldx = 0;              // row stride of X in elements (>= K)
-    int elt = kBF16;          // operand type of X and W
+    int elt = kBF16;          // operand type of X and W (a Precision)
     int out_elt = kBF16;      // type of Y
     int epilogue = kEpiBias;
     // kEpiQKV: N == 3*hidden.  Feature n -> (which = n / hidden, head, dd).
@@ -80,12 +83,17 @@ struct GemmParams {
     // writes its partial result to Y + z * M * N; the bias goes into partial 0.  The consumer adds
     // them up (launch_add_layernorm's y_parts).  Y must hold splits * M * N floats.
     int splits = 1;
+    // A kernel may be chosen that groups the sums over k its own way (the skinny tiles do, as split K does): the result then
+    // depends, in its last bits, on which kernel the row count asks for.
+    bool any_k_order = false;
     bool compiler_scheduled = false;   // 256 tile: use the generic kernel, not the hand-scheduled one
     // Packed operand layout (common.h): X / W read from it, Y (bf16, plain epilogues) written in it.
     bool x_packed = false, w_packed = false, y_packed = false;
     int xcd_partition = -1;   // how the eight XCDs divide the tile grid (see tile_of_block): -1 = estimate and choose, 0 = contiguous
                               // runs of the tile sequence, 2 / 4 = 4 x 2 / 2 x 4 cells (for measurements)
 };
+// elt == kF32Split: X and W in the split layout (common.h), K a multiple of 16; Y is float32 row-major, or, with the GELU
+// epilogue, split as well (out_elt kF32Split, N a multiple of 32); tile 0, 128, kTile256x128 or a skinny one.
 bool launch_gemm(const GemmParams& p, hipStream_t stream);
 // The tile (a GemmParams::tile value, never 0) and split count launch_gemm's cost model prefers for a problem.
 // max_splits > 1: the caller can take a float32 result as up to that many partial sums (a power of two is chosen).
@@ -122,17 +130,22 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
 // first_only: only the context of every sequence's first token is produced, as row b of ctx [B, heads*64] (same bits
 // as row b * S of the full result).
 
+// float32 attention on split operands: q, k, v as the QKV GEMM with elt == kF32Split writes them, [B, heads, Sp / 32] blocks
+// of twelve 1 KiB units each (attention_f32.hip); ctx in the split layout.  Other arguments as above.
+bool launch_attention_f32(const void* q, const void* k, const void* v, const float* maskadd, void* ctx, int B, int heads,
+                          int S, int Sp, float scale, hipStream_t stream, const int* cu = nullptr, bool first_only = false);
+
 // ----------------------------------------------------------- LayerNorm -----
 // x <- LayerNorm(x + y) * gamma + beta   over rows of length H, in place on the
-// float32 residual stream x; when xb != nullptr a bf16 copy of the result is
-// written as the next GEMM's operand.  y has type y_elt (may be nullptr: plain
+// float32 residual stream x; when xb != nullptr a copy of the result is written
+// as the next GEMM's operand (bf16, or float32 in the split layout).  y has type y_elt (may be nullptr: plain
 // LayerNorm).  eps = 1e-12 inside the square root, biased variance
 // (cuda_bert/ops/layernorm.cu:136-182; modeling.py:168-172).
-// xb_packed: write the copy in the packed GEMM-operand layout (common.h).
+// xb_layout: an OperandLayout (common.h).
 // add_x = false: x <- LayerNorm(y): y is already the sum with the residual stream (a GEMM with
 // GemmParams::residual produced it) and x is only written.
 bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma,
-                          const float* beta, bf16_t* xb, bool xb_packed, int rows, int H,
+                          const float* beta, void* xb, int xb_layout, int rows, int H,
                           hipStream_t stream, int y_parts = 1, bool add_x = true);
 
 // --------------------------------------------------- embedding + LN --------
@@ -142,7 +155,7 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
 // (cuda_bert/ops/embedding.cu:3-58; utils/bert.cu:94-97 for the positions.)
 bool launch_embed_layernorm(const int* ids, const int* seg, const int* mask, const float* word,
                             const float* pos, const float* type, const float* gamma,
-                            const float* beta, float* x, bf16_t* xb, bool xb_packed, float* maskadd,
+                            const float* beta, float* x, void* xb, int xb_layout, float* maskadd,
                             int B, int S, int Sp, int H, int vocab, int type_vocab, hipStream_t stream,
                             const Compact* compact = nullptr);
 
@@ -176,7 +189,7 @@ bool launch_unpad_rows(const float* xc, const int* cu, float* out, int B, int S,
 
 // ------------------------------------------------------ load helpers -------
 // dst[n, k] = convert(src[k, n])  : on-disk [in,out] float32 -> [out,in] operand type,
-// row-major or (bf16) packed; in the packed case dst is the whole operand and the
+// row-major, (bf16) packed or (kF32Split) split; in the latter cases dst is the whole operand and the
 // tensor's rows land at row0 .. row0 + N - 1 of it.
 bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt, bool packed, int row0,
                               hipStream_t stream);

@@ -71,28 +71,39 @@ __device__ __forceinline__ void ln_chunk_stats(const float (&v)[4], int c, int H
     *m2_hi = upper ? q : q_other;
 }
 
+// LAYOUT: the OperandLayout of the GEMM-operand copy xb; a run-time switch here costs the bf16 row kernels 1 % of a short pass.
 // Normalises features i .. i + 3 of a row (mean, rstd known) and writes them to x (f32) and optionally to the bf16
-// copy xb: row-major when xb_packed == 0, else in the packed GEMM-operand layout (common.h).
+// GEMM-operand copy xb: bf16 row-major or packed, or float32 in the split layout (OperandLayout, common.h).
+template <int LAYOUT>
 __device__ __forceinline__ void ln_store4(const float (&v)[4], float mean, float rstd, const f32x4_t& g4, const f32x4_t& b4,
-                                          float* xrow, bf16_t* xb, int row, int i, int H, int xb_packed) {
+                                          float* xrow, void* xb, int row, int i, int H) {
     f32x4_t o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = ln_apply(v[e], mean, rstd, g4[e], b4[e]);
     __builtin_nontemporal_store(o, reinterpret_cast<f32x4_t*>(xrow + i));
-    if (xb) {
+    unsigned char* dst = static_cast<unsigned char*>(xb);
+    if (!xb) return;
+    if constexpr (LAYOUT == kSplit) {
+        __bf16 s[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split_bf16x3(o[e], s[0][e], s[1][e], s[2][e]);
+        dst += split_offset(row, i, H);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x4_t*>(dst + p * 1024) = bf16x4_t{s[p][0], s[p][1], s[p][2], s[p][3]};
+    } else {
         bf16x4_t ob = {(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
-        unsigned char* dst = reinterpret_cast<unsigned char*>(xb);
-        const size_t off = xb_packed ? packed_offset(row, i * 2, H * 2 / 64) : ((size_t)row * H + i) * 2;
+        const size_t off = LAYOUT == kPacked ? packed_offset(row, i * 2, H * 2 / 64) : ((size_t)row * H + i) * 2;
         *reinterpret_cast<bf16x4_t*>(dst + off) = ob;
     }
 }
 
 // Normalises the row held in v[][] (lane owns elements c*256 + lane*4 + e) and
-// writes it to x (f32) and optionally xb (bf16).
+// writes it to x (f32) and optionally xb (ln_store4).
+template <int LAYOUT>
 __device__ __forceinline__ void normalise_store(float (&v)[kMaxChunks][4], int H, int lane,
                                                 const float* __restrict__ gamma,
                                                 const float* __restrict__ beta, float* xrow,
-                                                bf16_t* xb, int row, int xb_packed) {
+                                                void* xb, int row) {
     float ssum[2 * kMaxChunks], sm2[2 * kMaxChunks];
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c)
@@ -105,18 +116,18 @@ __device__ __forceinline__ void normalise_store(float (&v)[kMaxChunks][4], int H
         if (i < H) {
             const f32x4_t g4 = *reinterpret_cast<const f32x4_t*>(gamma + i);
             const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(beta + i);
-            ln_store4(v[c], mean, rstd, g4, b4, xrow, xb, row, i, H, xb_packed);
+            ln_store4<LAYOUT>(v[c], mean, rstd, g4, b4, xrow, xb, row, i, H);
         }
     }
 }
 
-template <int YELT>   // -1: no addend
+template <int YELT, int LAYOUT>   // YELT -1: no addend
 __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ x,
                                                             const unsigned char* __restrict__ y,
                                                             const float* __restrict__ gamma,
                                                             const float* __restrict__ beta,
-                                                            bf16_t* __restrict__ xb, int rows, int H,
-                                                            int xb_packed, int y_parts, int add_x) {
+                                                            void* __restrict__ xb, int rows, int H,
+                                                            int y_parts, int add_x) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -144,7 +155,7 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
             for (int e = 0; e < 4; ++e) v[c][e] = a[e];
         }
     }
-    normalise_store(v, H, lane, gamma, beta, xrow, xb, row, xb_packed);
+    normalise_store<LAYOUT>(v, H, lane, gamma, beta, xrow, xb, row);
 }
 
 // The same operation for a short batch whose addend comes as the partial sums of a split-K GEMM
@@ -154,11 +165,12 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
 // parts of features 256 w .. 256 w + 255 and forms the statistics of its two slots; the waves exchange
 // those through the LDS, every wave combines them (the same arithmetic in the same order as
 // add_layernorm_kernel, hence the same bits) and normalises its own features.
+template <int LAYOUT>
 __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restrict__ x, const float* __restrict__ y,
                                                                   const float* __restrict__ gamma,
                                                                   const float* __restrict__ beta,
-                                                                  bf16_t* __restrict__ xb, int rows, int H,
-                                                                  int xb_packed, int y_parts, int add_x) {
+                                                                  void* __restrict__ xb, int rows, int H,
+                                                                  int y_parts, int add_x) {
     __shared__ float stats[kMaxChunks][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = blockIdx.x;
@@ -201,15 +213,16 @@ __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restr
     }
     float mean, rstd;
     ln_combine_slots(ssum, sm2, H, &mean, &rstd);
-    if (in) ln_store4(v, mean, rstd, g4, b4, xrow, xb, row, i, H, xb_packed);
+    if (in) ln_store4<LAYOUT>(v, mean, rstd, g4, b4, xrow, xb, row, i, H);
 }
 
+template <int LAYOUT>
 __global__ __launch_bounds__(256) void embed_layernorm_kernel(
     const int* __restrict__ ids, const int* __restrict__ seg, const int* __restrict__ mask,
     const float* __restrict__ word, const float* __restrict__ pos, const float* __restrict__ type,
     const float* __restrict__ gamma, const float* __restrict__ beta, float* __restrict__ x,
-    bf16_t* __restrict__ xb, float* __restrict__ maskadd, int B, int S, int Sp, int H, int vocab,
-    int type_vocab, int xb_packed, const int* __restrict__ rowmap, const int* __restrict__ cu, int nrows) {
+    void* __restrict__ xb, float* __restrict__ maskadd, int B, int S, int Sp, int H, int vocab,
+    int type_vocab, const int* __restrict__ rowmap, const int* __restrict__ cu, int nrows) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);        // output row
     if (row >= nrows) return;
@@ -247,7 +260,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
             for (int e = 0; e < 4; ++e) v[c][e] = (a[e] + p4[e]) + t4[e];
         }
     }
-    normalise_store(v, H, lane, gamma, beta, x + (size_t)row * H, xb, row, xb_packed);
+    normalise_store<LAYOUT>(v, H, lane, gamma, beta, x + (size_t)row * H, xb, row);
 }
 
 // One wave per score row of length S <= 512 (8 elements per lane, strided by
@@ -479,7 +492,10 @@ __global__ __launch_bounds__(256) void transpose_convert_kernel(const float* __r
         const int nn = n0 + r, kk = k0 + tx;
         if (nn < N && kk < K) {
             const float val = tile[tx][r];
-            if constexpr (ELT == kBF16) {
+            if constexpr (ELT == kF32Split) {
+                __bf16* d = reinterpret_cast<__bf16*>(dst + split_offset(row0 + nn, kk, K));
+                split_bf16x3(val, d[0], d[512], d[1024]);
+            } else if constexpr (ELT == kBF16) {
                 const size_t off = packed ? packed_offset(row0 + nn, kk * 2, K * 2 / 64) : ((size_t)nn * K + kk) * 2;
                 *reinterpret_cast<__bf16*>(dst + off) = (__bf16)val;
             } else {
@@ -579,11 +595,10 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 
 bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma, const float* beta,
-                          bf16_t* xb, bool xb_packed, int rows, int H, hipStream_t stream, int y_parts, bool add_x) {
+                          void* xb, int xb_layout, int rows, int H, hipStream_t stream, int y_parts, bool add_x) {
     if (!add_x && !y) { set_error("layernorm: without the residual stream an addend is required"); return false; }
     if (y_parts < 1 || (y_parts > 1 && (!y || y_elt != kF32))) { set_error("layernorm: partial addends must be float32"); return false; }
-    if (xb && xb_packed && H % 32 != 0) { set_error("layernorm: a packed copy needs H to be a multiple of 32"); return false; }
-    const int xp = xb_packed ? 1 : 0;
+    if (xb && xb_layout != kRowMajor && H % 32 != 0) { set_error("layernorm: a packed copy needs H to be a multiple of 32"); return false; }
     if (rows <= 0 || H <= 0 || H % 4 != 0 || H > kMaxChunks * 256) {
         set_error("layernorm: H must be a multiple of 4 and at most 1024");
         return false;
@@ -595,24 +610,31 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
     }
     dim3 grid((rows + 3) / 4), block(256);
     const unsigned char* yc = static_cast<const unsigned char*>(y);
-    if (!y) hipLaunchKernelGGL(add_layernorm_kernel<-1>, grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, xp, y_parts, add_x ? 1 : 0);
-    else if (y_elt == kF32 && y_parts > 1) hipLaunchKernelGGL(add_layernorm_parts_kernel, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, xp, y_parts, add_x ? 1 : 0);
-    else if (y_elt == kF32) hipLaunchKernelGGL(add_layernorm_kernel<kF32>, grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, xp, y_parts, add_x ? 1 : 0);
-    else if (y_elt == kBF16) hipLaunchKernelGGL(add_layernorm_kernel<kBF16>, grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, xp, y_parts, add_x ? 1 : 0);
-    else { set_error("layernorm: bad addend type"); return false; }
+    auto go = [&](auto layout) {
+        constexpr int L = decltype(layout)::value;
+        const int ax = add_x ? 1 : 0;
+        if (!y) hipLaunchKernelGGL((add_layernorm_kernel<-1, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
+        else if (y_elt == kF32 && y_parts > 1) hipLaunchKernelGGL(add_layernorm_parts_kernel<L>, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, y_parts, ax);
+        else if (y_elt == kF32) hipLaunchKernelGGL((add_layernorm_kernel<kF32, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
+        else hipLaunchKernelGGL((add_layernorm_kernel<kBF16, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
+    };
+    if (y && y_elt != kF32 && y_elt != kBF16) { set_error("layernorm: bad addend type"); return false; }
+    if (xb_layout == kSplit) go(std::integral_constant<int, kSplit>());
+    else if (xb_layout == kPacked) go(std::integral_constant<int, kPacked>());
+    else go(std::integral_constant<int, kRowMajor>());
     CUBERT_HIP_OK(hipGetLastError());
     return true;
 }
 
 bool launch_embed_layernorm(const int* ids, const int* seg, const int* mask, const float* word,
                             const float* pos, const float* type, const float* gamma, const float* beta,
-                            float* x, bf16_t* xb, bool xb_packed, float* maskadd, int B, int S, int Sp, int H,
+                            float* x, void* xb, int xb_layout, float* maskadd, int B, int S, int Sp, int H,
                             int vocab, int type_vocab, hipStream_t stream, const Compact* compact) {
     if (compact && (!compact->rowmap || !compact->cu || compact->rows <= 0 || compact->rows > (long)B * S)) {
         set_error("embedding: bad compact-row description");
         return false;
     }
-    if (xb && xb_packed && H % 32 != 0) { set_error("embedding: a packed copy needs H to be a multiple of 32"); return false; }
+    if (xb && xb_layout != kRowMajor && H % 32 != 0) { set_error("embedding: a packed copy needs H to be a multiple of 32"); return false; }
     if (B <= 0 || S <= 0 || H <= 0 || H % 4 != 0 || H > kMaxChunks * 256) {
         set_error("embedding: H must be a multiple of 4 and at most 1024");
         return false;
@@ -629,8 +651,9 @@ bool launch_embed_layernorm(const int* ids, const int* seg, const int* mask, con
     }
     const long rows = compact ? compact->rows : (long)B * S;
     dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    hipLaunchKernelGGL(embed_layernorm_kernel, grid, block, 0, stream, ids, seg, mask, word, pos, type, gamma,
-                       beta, x, xb, maskadd, B, S, Sp, H, vocab, type_vocab, xb_packed ? 1 : 0,
+    auto kernel = xb_layout == kSplit ? embed_layernorm_kernel<kSplit> : xb_layout == kPacked ? embed_layernorm_kernel<kPacked> : embed_layernorm_kernel<kRowMajor>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, ids, seg, mask, word, pos, type, gamma,
+                       beta, x, xb, maskadd, B, S, Sp, H, vocab, type_vocab,
                        compact ? compact->rowmap : nullptr, compact ? compact->cu : nullptr, (int)rows);
     CUBERT_HIP_OK(hipGetLastError());
     return true;
@@ -734,7 +757,9 @@ bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt
     const int pk = packed ? 1 : 0;
     dim3 grid((N + 31) / 32, (K + 31) / 32), block(256);
     unsigned char* d = static_cast<unsigned char*>(dst);
-    if (elt == kBF16) hipLaunchKernelGGL(transpose_convert_kernel<kBF16>, grid, block, 0, stream, src, d, K, N, pk, row0);
+    if (elt == kF32Split && K % 16 != 0) { set_error("transpose: the split layout needs K to be a multiple of 16"); return false; }
+    if (elt == kF32Split) hipLaunchKernelGGL(transpose_convert_kernel<kF32Split>, grid, block, 0, stream, src, d, K, N, pk, row0);
+    else if (elt == kBF16) hipLaunchKernelGGL(transpose_convert_kernel<kBF16>, grid, block, 0, stream, src, d, K, N, pk, row0);
     else if (elt == kF32) hipLaunchKernelGGL(transpose_convert_kernel<kF32>, grid, block, 0, stream, src, d, K, N, pk, row0);
     else { set_error("transpose: bad element type"); return false; }
     CUBERT_HIP_OK(hipGetLastError());

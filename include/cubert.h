@@ -194,6 +194,11 @@ long cubert_capacity_tokens(void* model);
 #define CUBERT_LN_NO_RESIDUAL 16    /* cubert_op_add_layernorm: y already contains the residual stream */
 #define CUBERT_V_ROWMAJOR 32        /* cubert_op_gemm_qkv / cubert_op_attention (bf16, S <= 512): the `vt` argument holds V as
                                        [B, heads, S, 64] like k instead of transposed */
+#define CUBERT_Y_SPLIT 64           /* float32 context / copy in the split layout (cubert_op_attention, _add_layernorm, _embed_layernorm) */
+/* elt = 2 (cubert_op_gemm, _gemm_residual, _gemm_qkv): float32 operands in the split layout, every element as the exact sum
+ * of three bfloat16 numbers; the product is formed from six bf16 matrix products and has float32 accuracy.  K must be a
+ * multiple of 16; Y is float32 row-major, or (GELU epilogue) split, out_elt 2.  fp32 mode runs on this. */
+#define CUBERT_F32_SPLIT 2
 /* cubert_op_attention with CUBERT_V_ROWMAJOR: which kernel.  0 (no flag) = by batch size; 1 = one workgroup per
  * (batch, head); 2 = one workgroup per (batch, head, 32 queries) whose four waves share the keys (short batches). */
 #define CUBERT_ATTN_VARIANT(n) (((n) & 3) << 20)
@@ -208,6 +213,11 @@ long cubert_capacity_tokens(void* model);
 #define CUBERT_SPLITS_OF(flags) (((flags) >> 8) & 0xff)
 size_t cubert_packed_bytes(size_t rows, size_t row_bytes);
 size_t cubert_packed_offset(int row, int byte_in_row, int row_bytes);
+
+/* Size of a [rows, K] operand in the split layout, and the conversion into it of the transpose of src [K, N] (float32
+ * row-major, like the Linear kernels on disk): src's column n becomes row row0 + n of the operand. */
+size_t cubert_split_bytes(size_t rows, size_t K);
+int cubert_op_split_operand(const float* src, void* dst, int K, int N, int row0, void* stream);
 
 /* Y[M,N] = epilogue(X[M,K] (row stride ldx) * W[N,K]^T + bias[N]);
  * epilogue 0 bias, 1 bias+GELU(erf), 2 bias+tanh.  tile 0 = automatic.
