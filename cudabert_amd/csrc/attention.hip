@@ -30,11 +30,15 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
 typedef __attribute__((ext_vector_type(8))) short s16x8_t;
 
+__device__ __forceinline__ size_t operand_offset(int layout, int r, int kbyte, int KB) {
+    return layout == kUnits ? units_offset(r, kbyte, KB) : packed_offset(r, kbyte, KB);
+}
+
 template <int ELT>
 __global__ __launch_bounds__(256) void attention_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
     const unsigned char* __restrict__ vt, const float* __restrict__ maskadd,
-    unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale, int ctx_packed,
+    unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale, int ctx_layout,
     const int* __restrict__ cu, int first_only) {
     constexpr int ES = (ELT == kBF16) ? 2 : 4;
     constexpr int ROWB = 64 * ES;            // bytes per Q/K row
@@ -180,8 +184,8 @@ __global__ __launch_bounds__(256) void attention_kernel(
             if constexpr (ELT == kBF16) {
                 bf16x4_t w = {(__bf16)(o[db][4 * j] * inv), (__bf16)(o[db][4 * j + 1] * inv),
                               (__bf16)(o[db][4 * j + 2] * inv), (__bf16)(o[db][4 * j + 3] * inv)};
-                if (ctx_packed)
-                    *reinterpret_cast<bf16x4_t*>(ctx + packed_offset((int)row_base + qi, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
+                if (ctx_layout != kRowMajor)
+                    *reinterpret_cast<bf16x4_t*>(ctx + operand_offset(ctx_layout, (int)row_base + qi, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
                 else
                     *reinterpret_cast<bf16x4_t*>(orow + d * 2) = w;
             } else {
@@ -220,7 +224,7 @@ template <bool VROW>
 __global__ __launch_bounds__(1024) void attention_lds_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
     const unsigned char* __restrict__ vt, const float* __restrict__ maskadd,
-    unsigned char* __restrict__ ctx, int heads, int S, int Sp, int vstride, float scale_log2e, int ctx_packed,
+    unsigned char* __restrict__ ctx, int heads, int S, int Sp, int vstride, float scale_log2e, int ctx_layout,
     const int* __restrict__ cu, int first_only) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* sK = smem;
@@ -448,8 +452,8 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
             const int d = 32 * db + 8 * j + 4 * g;
             bf16x4_t w = {(__bf16)(o[db][4 * j] * inv), (__bf16)(o[db][4 * j + 1] * inv),
                           (__bf16)(o[db][4 * j + 2] * inv), (__bf16)(o[db][4 * j + 3] * inv)};
-            if (ctx_packed)
-                *reinterpret_cast<bf16x4_t*>(ctx + packed_offset((int)row_base + qi, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
+            if (ctx_layout != kRowMajor)
+                *reinterpret_cast<bf16x4_t*>(ctx + operand_offset(ctx_layout, (int)row_base + qi, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
             else
                 *reinterpret_cast<bf16x4_t*>(orow + d * 2) = w;
         }
@@ -472,7 +476,7 @@ template <int NW>
 __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
     const unsigned char* __restrict__ v, const float* __restrict__ maskadd,
-    unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale_log2e, int ctx_packed,
+    unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale_log2e, int ctx_layout,
     const int* __restrict__ cu, int first_only) {
     constexpr int OSTRIDE = 68;                          // floats per query row of a partial context
     constexpr int OBYTES = 32 * OSTRIDE * 4;             // two V blocks (8 KiB) first, the partial context later
@@ -653,7 +657,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const size_t hidden = (size_t)heads * 64;
     const size_t row = first_only ? (size_t)b : (cu ? (size_t)cu[b] : (size_t)b * S) + qrow;
     const int kbyte = (h * 64 + fg * FPT) * 2;
-    unsigned char* dst = ctx_packed ? ctx + packed_offset((int)row, kbyte, (int)hidden * 2 / 64) : ctx + row * hidden * 2 + kbyte;
+    unsigned char* dst = ctx_layout != kRowMajor ? ctx + operand_offset(ctx_layout, (int)row, kbyte, (int)hidden * 2 / 64) : ctx + row * hidden * 2 + kbyte;
 #pragma unroll
     for (int e = 0; e < FPT; e += 4) {
         const bf16x4_t w4 = {(__bf16)(acc[e] * inv), (__bf16)(acc[e + 1] * inv), (__bf16)(acc[e + 2] * inv), (__bf16)(acc[e + 3] * inv)};
@@ -664,15 +668,15 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
 }  // namespace
 
 bool launch_attention(const void* q, const void* k, const void* vt, const float* maskadd, void* ctx,
-                      bool ctx_packed, int B, int heads, int S, int Sp, float scale, int elt, hipStream_t stream,
+                      int ctx_layout, int B, int heads, int S, int Sp, float scale, int elt, hipStream_t stream,
                       const int* cu, bool v_rowmajor, bool first_only, int variant) {
     const int fo = first_only ? 1 : 0;
     if (variant < kAttnAuto || variant > kAttnSplitKeys || (variant > kAttnPerHead && !(v_rowmajor && elt == kBF16 && S <= 512))) {
         set_error("attention: the key-split variants need bf16 operands, S <= 512 and V as [B, heads, S, 64]");
         return false;
     }
-    if (ctx_packed && elt != kBF16) { set_error("attention: only a bf16 context can be packed"); return false; }
-    const int cp = ctx_packed ? 1 : 0;
+    if (ctx_layout != kRowMajor && (elt != kBF16 || ctx_layout == kSplit)) { set_error("attention: only a bf16 context can be packed"); return false; }
+    const int cp = ctx_layout;
     if (elt != kBF16 && elt != kF32) { set_error("attention: bad operand type"); return false; }
     if (B <= 0 || heads <= 0 || S <= 0) { set_error("attention: empty problem"); return false; }
     if (!(scale > 0.0f)) { set_error("attention: scale must be positive"); return false; }

@@ -280,12 +280,15 @@ void apply_gemm_flags(cubert::GemmParams* p, int flags) {
     p->x_packed = (flags & CUBERT_X_PACKED) != 0;
     p->w_packed = (flags & CUBERT_W_PACKED) != 0;
     p->y_packed = (flags & CUBERT_Y_PACKED) != 0;
+    p->x_units = (flags & CUBERT_X_UNITS) != 0;
+    p->w_units = (flags & CUBERT_W_UNITS) != 0;
+    p->y_units = (flags & CUBERT_Y_UNITS) != 0;
     p->compiler_scheduled = (flags & CUBERT_COMPILER_SCHEDULED) != 0;
     p->splits = CUBERT_SPLITS_OF(flags) > 1 ? CUBERT_SPLITS_OF(flags) : 1;
     p->xcd_partition = ((flags >> 16) & 0xf) - 1;
 }
 int result_layout(int flags) {
-    return (flags & CUBERT_Y_SPLIT) ? cubert::kSplit : (flags & CUBERT_Y_PACKED) ? cubert::kPacked : cubert::kRowMajor;
+    return (flags & CUBERT_Y_SPLIT) ? cubert::kSplit : (flags & CUBERT_Y_UNITS) ? cubert::kUnits : (flags & CUBERT_Y_PACKED) ? cubert::kPacked : cubert::kRowMajor;
 }
 }  // namespace
 
@@ -323,7 +326,7 @@ int cubert_op_gemm_residual_layernorm(const void* X, const void* W, const float*
     p.out_elt = cubert::kF32; p.epilogue = cubert::kEpiBias; p.tile = tile; p.residual = R;
     p.ln_gamma = gamma; p.ln_beta = beta; p.ln_xb = xb; p.ln_xb_packed = (flags & CUBERT_Y_PACKED) != 0; p.ln_ws = workspace;
     apply_gemm_flags(&p, flags);
-    p.y_packed = false;                 // CUBERT_Y_PACKED describes the bf16 copy here; Y itself is float32 row-major
+    p.y_packed = p.y_units = false;     // CUBERT_Y_PACKED describes the bf16 copy here; Y itself is float32 row-major
     return cubert::launch_gemm(p, static_cast<hipStream_t>(stream)) ? 0 : 1;
 }
 
@@ -339,6 +342,7 @@ int cubert_op_gemm_qkv(const void* X, const void* W, const float* bias, void* q,
     return cubert::launch_gemm(p, static_cast<hipStream_t>(stream)) ? 0 : 1;
 }
 
+size_t cubert_units_offset(int row, int kbyte, int row_bytes) { return cubert::units_offset(row, kbyte, row_bytes / 64); }
 size_t cubert_split_bytes(size_t rows, size_t K) { return cubert::split_bytes(rows, K); }
 int cubert_op_split_operand(const float* src, void* dst, int K, int N, int row0, void* stream) {
     cubert::set_error("");
@@ -354,7 +358,7 @@ int cubert_op_attention(const void* q, const void* k, const void* vt, const floa
     if (elt == cubert::kF32Split)
         return cubert::launch_attention_f32(q, k, vt, maskadd, ctx, B, heads, S, cubert::round_up(S > 0 ? S : 1, 32), scale,
                                             static_cast<hipStream_t>(stream)) ? 0 : 1;
-    return cubert::launch_attention(q, k, vt, maskadd, ctx, (flags & CUBERT_Y_PACKED) != 0, B, heads, S,
+    return cubert::launch_attention(q, k, vt, maskadd, ctx, result_layout(flags & ~CUBERT_Y_SPLIT), B, heads, S,
                                     cubert::round_up(S > 0 ? S : 1, 32), scale, elt,
                                     static_cast<hipStream_t>(stream), nullptr, (flags & CUBERT_V_ROWMAJOR) != 0, false,
                                     (flags >> 20) & 3) ? 0 : 1;

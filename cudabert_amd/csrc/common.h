@@ -44,6 +44,12 @@ inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 // ds_read_b128 fragment reads (lane = row, 64-byte row pitch) run at the full
 // 256 bytes per clock of the LDS; measured alternatives: none 85, xor of
 // (r>>1)^(r>>3) 158 bytes per clock.
+//
+// The "units" layout (bf16) has the same 16 KiB blocks of 256 rows x 32 k, but inside a block 1 KiB units of 32 rows x 16 k in
+// the register layout of the 32x32x16 MFMA operand (lane 32 (k / 8 % 2) + row % 32 owns 16 bytes): unit (r / 32 % 8, k / 16
+// % 2).  A GEMM epilogue writes it straight from the accumulators, a kernel without an LDS-staged loop loads its operands from
+// it as they are, and LDS fragment reads are linear in the lane; writers that hold whole rows (LayerNorm) prefer the
+// packed layout, whose pieces of a row are 64 bytes instead of 16.
 // Attention kernels (launch_attention's `variant`).
 constexpr int kAttnAuto = 0, kAttnPerHead = 1, kAttnSplitKeys = 2;
 constexpr int kAttnSplitMaxWorkgroups = 768; // B * heads * ceil(S / 32) up to which kAttnAuto takes the key-split kernel
@@ -60,6 +66,10 @@ __host__ __device__ inline size_t packed_offset(int r, int kbyte, int KB) {
            (kbyte & 15);
 }
 
+__host__ __device__ inline size_t units_offset(int r, int kbyte, int KB) {
+    return ((size_t)(r >> 8) * KB + (kbyte >> 6)) * 16384 + ((r >> 5) & 7) * 2048 + ((kbyte >> 4) & 3) * 512 + (r & 31) * 16 + (kbyte & 15);
+}
+
 // ---- split operand layout --------------------------------------------------
 // float32 operands of a GEMM, every element as the exact sum of three bfloat16 numbers (split_bf16x3): plane 0 is the
 // element rounded to bf16, plane 1 what is left rounded to bf16, plane 2 the rest (at most 7 bits, so exact).  Six of the
@@ -69,7 +79,7 @@ __host__ __device__ inline size_t packed_offset(int r, int kbyte, int KB) {
 // Layout: 1 KiB units of 32 rows x 16 k x one plane, in the register layout of the 32x32x16 MFMA operand (lane
 // 32 (k / 8 % 2) + row % 32 owns 16 bytes), unit (row / 32, k / 16, plane) at ((row / 32 * (K / 16) + k / 16) * 3 + plane).
 // Rows are padded to a multiple of 32.
-enum OperandLayout : int { kRowMajor = 0, kPacked = 1, kSplit = 2 };
+enum OperandLayout : int { kRowMajor = 0, kPacked = 1, kSplit = 2, kUnits = 3 };
 __host__ __device__ inline size_t split_bytes(size_t rows, size_t K) { return (rows + 31) / 32 * (K / 16) * 3072; }
 // Byte offset of plane 0 of element (r, k); planes 1 and 2 follow 1024 and 2048 bytes further.
 __host__ __device__ inline size_t split_offset(int r, int k, int K) {

@@ -141,7 +141,7 @@ bool Model::init(const ModelOptions& opt_in) {
         const int K = (int)a->shape[0], N = (int)a->shape[1];
         CUBERT_HIP_OK(hipMemcpyAsync(stage, a->data.data(), a->data.size() * 4, hipMemcpyHostToDevice, stream_));
         if (!launch_transpose_convert(stage, wblock_ + off, K, N, elt == kF32 && pack_this ? (int)kF32Split : elt,
-                                      elt == kBF16 && pack_this, row0, stream_)) return false;
+                                      elt == kBF16 && pack_this ? (int)kUnits : 0, row0, stream_)) return false;
         CUBERT_HIP_OK(hipStreamSynchronize(stream_));      // the staging buffer is reused
         return true;
     };
@@ -563,7 +563,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
 
     auto attention = [&](void* out, bool vrow, bool first_only) {
         if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only);
-        return launch_attention(q, k, vt, maskadd, out, true, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto);
+        return launch_attention(q, k, vt, maskadd, out, kUnits, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto);
     };
 
     if (!mark(kPhEmbed)) return false;
@@ -583,7 +583,8 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         g.v_rowmajor = vrow;
         g.rowmap = cp ? cp->rowmap : nullptr;
         g.any_k_order = any_order;
-        g.x_packed = g.w_packed = pk;
+        g.x_packed = g.w_packed = g.w_units = pk;
+        g.x_units = layout == kUnits;
         if (!mark(kPhQKV) || !launch_gemm(g, st)) return false;
         // The last layer of a pass whose caller gets no sequence output: keys and values are needed of every token,
         // everything after them only of the first token of each sequence, which is all the pooler reads.  Its B rows
@@ -602,18 +603,19 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             if (!launch_gather_first_rows(x32, cu, xc, B, S, H, st)) return false;
             g = GemmParams();
             g.elt = gelt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
-            g.M = B; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk;
+            g.M = B; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
             if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
             if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, layout, B, H, st, 1, !fuse_res)) return false;
             g = GemmParams();
             g.elt = g.out_elt = gelt; g.X = xbc; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
-            g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = pk;
+            g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
+        g.x_units = layout == kUnits;
             if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
             g = GemmParams();
             g.elt = gelt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;
-            g.M = B; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk;
+            g.M = B; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
             if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
@@ -625,7 +627,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         // attention output projection -> f32, then residual add + LayerNorm
         g = GemmParams();
         g.elt = gelt; g.out_elt = kF32; g.X = ctx; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = y32;
-        g.M = N; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk; g.splits = sp_ao;
+        g.M = N; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk; g.splits = sp_ao;
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = plan_ao.tile;
         if (ln_ao) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
@@ -635,12 +637,13 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         // feed-forward
         g = GemmParams();
         g.elt = g.out_elt = gelt; g.X = xb; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = h;
-        g.M = N; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = pk;
+        g.M = N; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
+        g.x_units = layout == kUnits;
         g.any_k_order = any_order;
         if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
         g = GemmParams();
         g.elt = gelt; g.out_elt = kF32; g.X = h; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = y32;
-        g.M = N; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = pk; g.splits = sp_fo;
+        g.M = N; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk; g.splits = sp_fo;
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = plan_fo.tile;
         if (ln_fo) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }

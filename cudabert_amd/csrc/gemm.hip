@@ -70,10 +70,10 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmDev p) {
     // Separate LDS objects (not one array indexed by stage): the compiler
     // then knows that the asynchronous global->LDS loads filling one buffer
     // cannot alias the fragment reads of another and does not serialise them.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds0[2 * TILE_BYTES];   // W tile, then X tile
-    __shared__ __attribute__((aligned(1024))) unsigned char lds1[2 * TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds2[NS == 4 ? 2 * TILE_BYTES : 16];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds3[NS == 4 ? 2 * TILE_BYTES : 16];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds0[2 * TILE_BYTES];   // W tile, then X tile
+    __shared__ __attribute__((aligned(2048))) unsigned char lds1[2 * TILE_BYTES];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds2[NS == 4 ? 2 * TILE_BYTES : 16];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds3[NS == 4 ? 2 * TILE_BYTES : 16];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -139,10 +139,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmDev p) {
     // Lane (row l32, group g) of 32x32 block i reads chunk 2*(kk&1) + g of row
     // base + 32 i + l32 in sub-block kk >> 1.  swz(row) only depends on l32 (the
     // quadrant base and 32 i do not reach the bits it uses), so the byte offset is
-    //   (off0 ^ ((kk & 1) << 5)) + (kk >> 1) * SUB + i * 2048.
-    const int sw = packed_swizzle(l32);
-    const int woff0 = (wn * (BT / 2) + l32) * 64 + ((g ^ sw) << 4);
-    const int xoff0 = TILE_BYTES + (wm * (BT / 2) + l32) * 64 + ((g ^ sw) << 4);
+    //   (off0 ^ (kk & 1 ? kphase : 0)) + (kk >> 1) * SUB + i * 2048.
+    const int woff0 = frag_base(wn * (BT / 2), p.w_units, l32, g), wkp = frag_kphase(p.w_units);
+    const int xoff0 = TILE_BYTES + frag_base(wm * (BT / 2), p.x_units, l32, g), xkp = frag_kphase(p.x_units);
 
     f32x16_t acc[NB][NB];
 #pragma unroll
@@ -164,15 +163,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmDev p) {
             const int cur = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)(BUF);           \
             _Pragma("unroll") for (int i = 0; i < NB; ++i)                                                  \
                 asm volatile("ds_read_b128 %0, %1" : "=v"(WF[i])                                            \
-                             : "v"(cur + (wb ^ (((kk) & 1) << 5)) + ((kk) >> 1) * SUB + i * 2048));         \
+                             : "v"(cur + (wb ^ (((kk) & 1) ? wkp : 0)) + ((kk) >> 1) * SUB + i * 2048));         \
             _Pragma("unroll") for (int j = 0; j < NB; ++j)                                                  \
                 asm volatile("ds_read_b128 %0, %1" : "=v"(XF[j])                                            \
-                             : "v"(cur + (xb ^ (((kk) & 1) << 5)) + ((kk) >> 1) * SUB + j * 2048));         \
+                             : "v"(cur + (xb ^ (((kk) & 1) ? xkp : 0)) + ((kk) >> 1) * SUB + j * 2048));         \
         } else {                                                                                            \
             _Pragma("unroll") for (int i = 0; i < NB; ++i)                                                  \
-                WF[i] = *reinterpret_cast<const u32x4_t*>((BUF) + (wb ^ (((kk) & 1) << 5)) + ((kk) >> 1) * SUB + i * 2048); \
+                WF[i] = *reinterpret_cast<const u32x4_t*>((BUF) + (wb ^ (((kk) & 1) ? wkp : 0)) + ((kk) >> 1) * SUB + i * 2048); \
             _Pragma("unroll") for (int j = 0; j < NB; ++j)                                                  \
-                XF[j] = *reinterpret_cast<const u32x4_t*>((BUF) + (xb ^ (((kk) & 1) << 5)) + ((kk) >> 1) * SUB + j * 2048); \
+                XF[j] = *reinterpret_cast<const u32x4_t*>((BUF) + (xb ^ (((kk) & 1) ? xkp : 0)) + ((kk) >> 1) * SUB + j * 2048); \
         }                                                                                                   \
     } while (0)
 #define CUBERT_FENCE_FRAGS(WF, XF)                                                                          \
@@ -294,6 +293,9 @@ bool launch_epi(const GemmDev& d, int epi, int bt, hipStream_t stream) {
     switch (epi) {
         case kEpiBias: return launch_tile<ELT, OUT, kEpiBias>(d, bt, stream);
         case kEpiBiasGelu: return launch_tile<ELT, OUT, kEpiBiasGelu>(d, bt, stream);
+        case kEpiBiasGeluUnits:
+            if constexpr (OUT == kBF16) return launch_tile<ELT, OUT, kEpiBiasGeluUnits>(d, bt, stream);
+            break;
         case kEpiBiasTanh: return launch_tile<ELT, OUT, kEpiBiasTanh>(d, bt, stream);
         case kEpiQKV: return launch_tile<ELT, OUT, kEpiQKV>(d, bt, stream);
         case kEpiQKVMap: return launch_tile<ELT, OUT, kEpiQKVMap>(d, bt, stream);
@@ -563,9 +565,14 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     d.Y = static_cast<unsigned char*>(p.Y);
     d.M = p.M; d.N = p.N; d.K = p.K; d.ldx = p.ldx;
     d.x_packed = p.x_packed; d.w_packed = p.w_packed; d.y_packed = p.y_packed;
+    d.x_units = p.x_units; d.w_units = p.w_units; d.y_units = p.y_units;
+    if ((p.x_units && !p.x_packed) || (p.w_units && !p.w_packed) || (p.y_units && !p.y_packed) || ((p.x_units || p.w_units) && p.elt != kBF16)) {
+        set_error("gemm: the units layout is a packed layout of bf16 operands");
+        return false;
+    }
     int out = p.out_elt;
     int epi = (p.epilogue == kEpiQKV && p.rowmap) ? (int)kEpiQKVMap : p.epilogue;
-    if (p.epilogue == kEpiQKVMap || p.epilogue == kEpiBiasRes || p.epilogue == kEpiBiasResLN) { set_error("gemm: unknown epilogue"); return false; }
+    if (p.epilogue == kEpiQKVMap || p.epilogue == kEpiBiasRes || p.epilogue == kEpiBiasResLN || p.epilogue == kEpiBiasGeluUnits) { set_error("gemm: unknown epilogue"); return false; }
     if (p.residual) {
         if (p.epilogue != kEpiBias || out != kF32 || p.y_packed || p.N % 4 != 0 ||
             (reinterpret_cast<uintptr_t>(p.residual) & 15)) {
@@ -607,12 +614,13 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
         d.v_rowmajor = p.v_rowmajor ? 1 : 0;
         d.S = p.S; d.Sp = p.Sp; d.heads = p.heads; d.hidden = p.heads * 64;
         d.rowmap = p.rowmap;
-        d.y_packed = 0;
+        d.y_packed = d.y_units = 0;
         out = p.elt;
     } else {
         if (!p.Y || (reinterpret_cast<uintptr_t>(p.Y) & 15)) { set_error("gemm: bad Y"); return false; }
         if (out != kBF16 && out != kF32) { set_error("gemm: bad output type"); return false; }
-        if (p.y_packed && (out != kBF16 || p.N % 32 != 0)) {
+        if (p.y_units && epi == kEpiBiasGelu) epi = kEpiBiasGeluUnits;
+        if (p.y_packed && (out != kBF16 || p.N % 32 != 0 || (p.y_units && epi != kEpiBiasGeluUnits))) {
             set_error("gemm: a packed Y must be bf16 with N a multiple of 32");
             return false;
         }
@@ -628,7 +636,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     if (!bt) {
         // the caller has settled on the split count; the tile follows
         if (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0)
-            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, epi == kEpiBiasGelu).tile;
+            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu).tile;
         else
             bt = gemm_pick_tile(p.M, p.N, p.K, p.elt);
     }
@@ -648,9 +656,8 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
         return launch_gemm_bf16_t256x128(d, out, epi, stream);
     }
     if (bt == kTileSkinny12 || bt == kTileSkinny22) {
-        if (p.elt != kBF16 || !p.x_packed || !p.w_packed || p.N % 8 != 0 || (epi != kEpiQKV && epi != kEpiQKVMap && epi != kEpiBiasGelu && out != kF32) ||
-            (epi == kEpiBiasGelu && !p.y_packed) || ((epi == kEpiQKV || epi == kEpiQKVMap) && !p.v_rowmajor)) {
-            set_error("gemm: the skinny tiles need packed bf16 operands and a packed GELU, row-major QKV or float32 result");
+        if (p.elt != kBF16 || !p.x_units || !p.w_units || p.N % 8 != 0 || (epi != kEpiQKV && epi != kEpiQKVMap && epi != kEpiBiasGeluUnits && out != kF32) || ((epi == kEpiQKV || epi == kEpiQKVMap) && !p.v_rowmajor)) {
+            set_error("gemm: the skinny tiles need bf16 operands in the units layout and a GELU result in it, row-major QKV or float32 result");
             return false;
         }
         const int bn = bt == kTileSkinny12 ? 32 : 64;
@@ -658,7 +665,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
         d.tiles_m = (p.M + 63) / 64;
         d.xn_parts = gemm_pick_partition((double)p.M * p.K * es, (double)p.N * p.K * es, d.tiles_n, d.tiles_m, 8);
         if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
-        return launch_gemm_skinny(d, kBF16, bt, epi, stream);
+        return launch_gemm_skinny(d, kBF16, bt, epi == kEpiBiasGeluUnits ? (int)kEpiBiasGelu : epi, stream);
     }
     if (bt == kTile128Hand) {
         if (p.elt != kBF16) { set_error("gemm: the hand-scheduled 128 tile is bf16 only"); return false; }

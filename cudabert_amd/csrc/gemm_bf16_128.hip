@@ -20,7 +20,7 @@ using namespace gemm_detail;
 template <int OUT, int EPI>
 __global__ __launch_bounds__(256, 3) void gemm_bf16_t128_kernel(const GemmDev p) {
     // Three stages of 16 KiB: W tile (128 rows x 64 B) at +0, X tile (128 rows x 64 B) at +0x2000.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * 16384];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[3 * 16384];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -52,9 +52,8 @@ __global__ __launch_bounds__(256, 3) void gemm_bf16_t128_kernel(const GemmDev p)
     const int w64 = p.w_packed ? 4096 : 64 * w_rowb, x64 = p.x_packed ? 4096 : 64 * x_rowb;
     const int wkstep = p.w_packed ? 16384 : 64, xkstep = p.x_packed ? 16384 : 64;
     const int lds_base = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    const int sw = packed_swizzle(l32);
-    const int wb = lds_base + (wn * 64 + l32) * 64 + ((g ^ sw) << 4);
-    const int xb = lds_base + (wm * 64 + l32) * 64 + ((g ^ sw) << 4);       // + 0x2000 is in the read offsets
+    const int wb = lds_base + frag_base(wn * 64, p.w_units, l32, g), wx = frag_kphase(p.w_units);
+    const int xb = lds_base + frag_base(wm * 64, p.x_units, l32, g), xx = frag_kphase(p.x_units);       // + 0x2000 is in the read offsets
     const int m0b = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
     // half-steps of this workgroup: all of K, or (split K) the blockIdx.y-th share of it
     const int hs = p.K / 32;
@@ -67,7 +66,7 @@ __global__ __launch_bounds__(256, 3) void gemm_bf16_t128_kernel(const GemmDev p)
     asm volatile(
 #include "gemm_bf16_128_loop.inc"
         : CUBERT_ACC_OPERANDS_Q
-        : [wb] "v"(wb), [xb] "v"(xb), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
+        : [wb] "v"(wb), [xb] "v"(xb), [wx] "s"(wx), [xx] "s"(xx), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
           [w64] "s"(w64), [x64] "s"(x64), [ht] "s"(ht), [m0b] "s"(m0b), [wkstep] "s"(wkstep), [xkstep] "s"(xkstep),
           [wkmax] "s"(wkmax), [xkmax] "s"(xkmax), [wk0] "s"(wk0), [xk0] "s"(xk0)
         : "memory", "scc", "m0", "s92", "s93", "s94", "s96", "s97", "s98", "v48", "v49", CUBERT_V10(5), CUBERT_V10(6),
@@ -92,6 +91,12 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiBiasRes:
             if constexpr (OUT == kF32) {
                 hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+                break;
+            }
+            [[fallthrough]];
+        case kEpiBiasGeluUnits:
+            if constexpr (OUT == kBF16) {
+                hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
                 break;
             }
             [[fallthrough]];

@@ -26,7 +26,7 @@ template <int OUT, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
     constexpr int BT = 256;
     // Four stages of 32 KiB: W tile (256 rows x 64 B) then X tile.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * 32768];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[4 * 32768];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -69,9 +69,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
     const int wkstep = p.w_packed ? 16384 : 64, xkstep = p.x_packed ? 16384 : 64;
     // fragment reads: chunk g of my row in the W / X tile of stage 0, k-phase 0
     const int lds_base = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    const int sw = packed_swizzle(l32);
-    const int wb = lds_base + (wn * 128 + l32) * 64 + ((g ^ sw) << 4);
-    const int xb = lds_base + 16384 + (wm * 128 + l32) * 64 + ((g ^ sw) << 4);
+    const int wb = lds_base + frag_base(wn * 128, p.w_units, l32, g), wx = frag_kphase(p.w_units);
+    const int xb = lds_base + 16384 + frag_base(wm * 128, p.x_units, l32, g), xx = frag_kphase(p.x_units);
     const int m0b = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
     const int ht = p.K / 32;          // half-steps; a multiple of 4
 
@@ -82,7 +81,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
     asm volatile(
 #include "gemm_bf16_256_loop.inc"
         : CUBERT_ACC_OPERANDS
-        : [wb] "v"(wb), [xb] "v"(xb), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
+        : [wb] "v"(wb), [xb] "v"(xb), [wx] "s"(wx), [xx] "s"(xx), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
           [w64] "s"(w64), [x64] "s"(x64), [ht] "s"(ht), [m0b] "s"(m0b), [wkstep] "s"(wkstep), [xkstep] "s"(xkstep)
         : "memory", "scc", "m0", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "v96", "v97", "v98", "v99",
           CUBERT_V10(10), CUBERT_V10(11), CUBERT_V10(12), CUBERT_V10(13), CUBERT_V10(14), CUBERT_V10(15), CUBERT_V10(16),
@@ -111,7 +110,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
 template <int OUT, int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_bf16_t256x128_kernel(const GemmDev p) {
     // Three stages of 24 KiB: W tile (256 rows x 64 B) at +0, X tile (128 rows x 64 B) at +0x4000.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[3 * 24576];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[3 * 24576];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -147,9 +146,8 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_t256x128_kernel(const GemmDe
     const int w64 = p.w_packed ? 4096 : 64 * w_rowb, x64 = p.x_packed ? 4096 : 64 * x_rowb;
     const int wkstep = p.w_packed ? 16384 : 64, xkstep = p.x_packed ? 16384 : 64;
     const int lds_base = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    const int sw = packed_swizzle(l32);
-    const int wb = lds_base + (wn * 128 + l32) * 64 + ((g ^ sw) << 4);
-    const int xb = lds_base + (wm * 64 + l32) * 64 + ((g ^ sw) << 4);       // + 0x4000 is in the read offsets
+    const int wb = lds_base + frag_base(wn * 128, p.w_units, l32, g), wx = frag_kphase(p.w_units);
+    const int xb = lds_base + frag_base(wm * 64, p.x_units, l32, g), xx = frag_kphase(p.x_units);       // + 0x4000 is in the read offsets
     const int m0b = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
     const int ht = p.K / 32;
     const int wkmax = (ht - 1) * wkstep, xkmax = (ht - 1) * xkstep;      // K offset of the last tile
@@ -159,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_t256x128_kernel(const GemmDe
     asm volatile(
 #include "gemm_bf16_256x128_loop.inc"
         : CUBERT_ACC_OPERANDS_H
-        : [wb] "v"(wb), [xb] "v"(xb), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
+        : [wb] "v"(wb), [xb] "v"(xb), [wx] "s"(wx), [xx] "s"(xx), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
           [w64] "s"(w64), [x64] "s"(x64), [ht] "s"(ht), [m0b] "s"(m0b), [wkstep] "s"(wkstep), [xkstep] "s"(xkstep),
           [wkmax] "s"(wkmax), [xkmax] "s"(xkmax)
         : "memory", "scc", "m0", "s92", "s93", "s94", "s96", "s97", "s98", "v64", "v65", "v66", "v67", "v68", "v69",
@@ -186,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_t256x128_kernel(const GemmDe
 template <int OUT, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_t256x128_deep_kernel(const GemmDev p) {
     // Four stages of 24 KiB: W tile (256 rows x 64 B) at +0, X tile (128 rows x 64 B) at +0x4000.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * 24576];
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[4 * 24576];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -215,9 +213,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256x128_deep_kernel(const Gemm
     const int w64 = p.w_packed ? 4096 : 64 * w_rowb, x64 = p.x_packed ? 4096 : 64 * x_rowb;
     const int wkstep = p.w_packed ? 16384 : 64, xkstep = p.x_packed ? 16384 : 64;
     const int lds_base = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    const int sw = packed_swizzle(l32);
-    const int wb = lds_base + (wn * 128 + l32) * 64 + ((g ^ sw) << 4);
-    const int xb = lds_base + 0x4000 + (wm * 64 + l32) * 64 + ((g ^ sw) << 4);
+    const int wb = lds_base + frag_base(wn * 128, p.w_units, l32, g), wx = frag_kphase(p.w_units);
+    const int xb = lds_base + 0x4000 + frag_base(wm * 64, p.x_units, l32, g), xx = frag_kphase(p.x_units);
     const int m0b = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
     const int ht = p.K / 32;          // half-steps; a multiple of 4
 
@@ -226,7 +223,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256x128_deep_kernel(const Gemm
     asm volatile(
 #include "gemm_bf16_256x128_deep_loop.inc"
         : CUBERT_ACC_OPERANDS_H
-        : [wb] "v"(wb), [xb] "v"(xb), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
+        : [wb] "v"(wb), [xb] "v"(xb), [wx] "s"(wx), [xx] "s"(xx), [wv0] "v"(w_v0), [xv0] "v"(x_v0), [wres] "s"(wres), [xres] "s"(xres),
           [w64] "s"(w64), [x64] "s"(x64), [ht] "s"(ht), [m0b] "s"(m0b), [wkstep] "s"(wkstep), [xkstep] "s"(xkstep)
         : "memory", "scc", "m0", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "v64", "v65", "v66", "v67", "v68", "v69",
           CUBERT_V10(7), CUBERT_V10(8), CUBERT_V10(9), CUBERT_V10(10), CUBERT_V10(11), "v120", "v121", "v122",
@@ -252,6 +249,12 @@ bool launch_epi_half_deep(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiBiasRes:
             if constexpr (OUT == kF32) {
                 hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+                break;
+            }
+            [[fallthrough]];
+        case kEpiBiasGeluUnits:
+            if constexpr (OUT == kBF16) {
+                hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
                 break;
             }
             [[fallthrough]];
@@ -288,6 +291,12 @@ bool launch_epi_half(const GemmDev& d, int epi, hipStream_t stream) {
                 }
             }
             [[fallthrough]];
+        case kEpiBiasGeluUnits:
+            if constexpr (OUT == kBF16) {
+                hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+                break;
+            }
+            [[fallthrough]];
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());
@@ -315,6 +324,12 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
                     hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasResLN>), ln_grid(d), block, 0, stream, d);
                     break;
                 }
+            }
+            [[fallthrough]];
+        case kEpiBiasGeluUnits:
+            if constexpr (OUT == kBF16) {
+                hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+                break;
             }
             [[fallthrough]];
         default: set_error("gemm: unknown epilogue"); return false;

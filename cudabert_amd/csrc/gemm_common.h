@@ -24,7 +24,8 @@ struct GemmDev {
     int M, N, K, ldx;
     int S, Sp, heads, hidden;
     int tiles_n, tiles_m;
-    int x_packed, w_packed, y_packed;     // operand / result in the packed layout (common.h)
+    int x_packed, w_packed, y_packed;     // operand / result in the packed or units layout (common.h)
+    int x_units, w_units, y_units;        // ... in the units layout
     int xn_parts;                         // how the XCDs divide the tile grid (tile_of_block)
     const int* rowmap;                    // QKV epilogue: row m -> token b * S + s (nullptr: m itself)
     int v_rowmajor;                       // QKV epilogue: V is stored like q / k instead of transposed
@@ -39,6 +40,13 @@ struct GemmDev {
     unsigned long long* ln_stats;         // [row][2 * tiles_n] (sum, M2 about the slot's mean) as two floats in 64 bits
     int ln_bands;
 };
+
+// Where a lane's MFMA fragment (k-phase 0) of rows row0 .. row0 + 31 lies in a tile's LDS image (64 bytes per row), and what
+// leads to k-phase 1 (xor).
+__device__ __forceinline__ int frag_base(int row0, int units, int l32, int g) {
+    return row0 * 64 + (units ? (l32 + 32 * g) * 16 : l32 * 64 + ((g ^ packed_swizzle(l32)) << 4));
+}
+__device__ __forceinline__ int frag_kphase(int units) { return units ? 0x400 : 0x20; }
 
 constexpr int kLnCntFirst = 64;           // first counter word of the workspace (the words before it: flags)
 constexpr int kLnSpinLimit = 1 << 21;     // polls of a band's arrival counter before a workgroup gives up
@@ -84,6 +92,12 @@ __device__ __forceinline__ void mfma_chunk(const u32x4_t& a, const u32x4_t& b, f
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[2], fb[2], acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[3], fb[3], acc, 0, 0, 0);
     }
+}
+
+// Two floats rounded to bf16, in one register.
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+    return __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)a, (__bf16)b});
 }
 
 template <int OUT>
@@ -236,10 +250,51 @@ __device__ __forceinline__ void gemm_epilogue_prefetch(const GemmDev& p, int n_b
     }
 }
 
+// bias + GELU, bf16, in the units layout, straight from the accumulators: a lane holds, of its token, features 8 t + 4 g .. + 3 of
+// every group t of eight; after exchanging halves with lane ^ 32 it holds all eight of group 2 u + g, its 16 bytes of the unit,
+// and a unit leaves as one 1 KiB store.
+template <int NBI, int NBJ>
+__device__ __forceinline__ void gemm_epilogue_units(const GemmDev& p, f32x16_t (&acc)[NBI][NBJ], const f32x4_t (&bias)[4 * NBI],
+                                                    int n_base, int m_base, int l32, int g) {
+    const int KB = p.N * 2 / 64, row_blocks = (p.M + 31) / 32;
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j) {
+        const int rb = (m_base >> 5) + j;
+        if (rb >= row_blocks) continue;                    // wave-uniform, as the next one
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+            if (n_base + 32 * i >= p.N) continue;          // N % 32 == 0
+            unsigned char* dst = p.Y + ((size_t)(rb >> 3) * KB + (n_base >> 5) + i) * 16384 + (rb & 7) * 2048 + (l32 + 32 * g) * 16;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float w[4];                                // pairs 0 1, 2 3 of group 2 u; of group 2 u + 1, as bits
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = gelu_fast(acc[i][j][4 * (2 * u + t) + e] + bias[4 * i + 2 * u + t][e]);
+                    w[2 * t] = __builtin_bit_cast(float, pack_bf16(v[0], v[1]));
+                    w[2 * t + 1] = __builtin_bit_cast(float, pack_bf16(v[2], v[3]));
+                }
+                half_swap(w[0], w[2]);
+                half_swap(w[1], w[3]);
+                const u32x4_t d = {__builtin_bit_cast(unsigned, w[0]), __builtin_bit_cast(unsigned, w[1]),
+                                   __builtin_bit_cast(unsigned, w[2]), __builtin_bit_cast(unsigned, w[3])};
+                *reinterpret_cast<u32x4_t*>(dst + u * 1024) = d;
+            }
+        }
+    }
+}
+
 template <int OUT, int EPI, int NBI, int NBJ, bool SPLITK = false, int RPB = 4, bool RDB = false>
 __device__ __forceinline__ void gemm_epilogue(const GemmDev& p, f32x16_t (&acc)[NBI][NBJ], const f32x4_t (&bias)[4 * NBI],
                                               int n_base, int m_base, int l32, int g, unsigned char* scratch,
                                               const EpiPrefetch<EpiGeometry<OUT, EPI, NBI, SPLITK, RPB>::PB>* pre = nullptr) {
+    if constexpr (EPI == kEpiBiasGeluUnits) {
+        // (a kernel of its own: a branch inside the one that writes rows costs both of them registers)
+        gemm_epilogue_units<NBI, NBJ>(p, acc, bias, n_base, m_base, l32, g);
+        return;
+    }
     constexpr int OES = (OUT == kBF16) ? 2 : 4;
     constexpr int RB = 32 * NBI * OES;      // bytes per token row of the staging block
     constexpr int CH = RB / 16;             // 16-byte chunks per row

@@ -1,4 +1,4 @@
-// GEMM for launches of a few hundred rows (gfx950):  Y = epilogue(X * W^T + bias), bf16 packed or float32 split operands.
+// GEMM for launches of a few hundred rows (gfx950):  Y = epilogue(X * W^T + bias), bf16 (units layout) or float32 (split layout) operands.
 //
 // Such a launch is bound by latency: a workgroup that streams its tile through the LDS spends most of every short K step
 // on the barrier and the round trip of the loads.  Here nothing is staged and the K loop has no barrier: the four waves of a
@@ -25,17 +25,17 @@ struct Operand<kF32Split> {
     static constexpr int kStepBytes = 3072;
     static __device__ int frag_offset(int lane_off, int f) { return lane_off + f * 1024; }
 };
-// bf16 packed: a step is 32 k (one 16 KiB block of 256 rows); per block of 32 rows two fragments, one per k-phase
+// bf16 units: a step is 32 k (one 16 KiB block of 256 rows); per block of 32 rows two fragments, one per k-phase
 template <>
 struct Operand<kBF16> {
     static constexpr int kFrags = 2, kStepK = 32;
     static __host__ __device__ size_t bytes(int rows, int K) { return packed_bytes(rows, (size_t)K * 2); }
     static __device__ int lane_offset(int row0, int K, int l32, int g) {
-        return (row0 >> 8) * (K / 32) * 16384 + ((row0 & 255) + l32) * 64 + ((g ^ packed_swizzle(l32)) << 4);
+        return (row0 >> 8) * (K / 32) * 16384 + (row0 & 255) * 64 + (l32 + 32 * g) * 16;
     }
     static __device__ int block_stride(int) { return 2048; }                 // 32 rows further in the same 256-row block
     static constexpr int kStepBytes = 16384;
-    static __device__ int frag_offset(int lane_off, int f) { return lane_off ^ (f << 5); }
+    static __device__ int frag_offset(int lane_off, int f) { return lane_off + f * 1024; }
 };
 
 template <int ELT, int EPI, int NBI, int NBJ, int DEPTH>
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
         const int idx = tid + it * 256;
-        if constexpr (EPI == kEpiBiasGelu && ELT == kF32Split) {       // units of 32 rows x 16 features
+        if constexpr (EPI == kEpiBiasGelu) {       // units of 32 rows x 16 features
             const int unit = idx >> 6;
             row[it] = 32 * (unit / (2 * NBI)) + l32;
             c8[it] = 2 * (unit % (2 * NBI)) + g;
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
                     dst = base + unit * 1024 + half * 512 + (which == 2 ? attn_v_slot(pos, half, kk) : pos) * 16;
                 }
             } else {
-                dst = p.Y + (ELT == kBF16 ? packed_offset(m, n * 2, p.N * 2 / 64) : split_offset(m, n, p.N));
+                dst = p.Y + (ELT == kBF16 ? units_offset(m, n * 2, p.N * 2 / 64) : split_offset(m, n, p.N));
             }
 #pragma unroll
             for (int q = 0; q < (FR == 3 ? 3 : 1); ++q) *reinterpret_cast<bf16x8_t*>(dst + q * 1024) = pl[q];
@@ -239,7 +239,7 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
 
 }  // namespace
 
-// elt kBF16 (both operands packed; packed, per-head row-major or float32 results) or kF32Split; tile kTileSkinny12 (32
+// elt kBF16 (both operands and a GELU result in the units layout; per-head row-major Q, K, V; float32 results) or kF32Split; tile kTileSkinny12 (32
 // features x 64 tokens) or kTileSkinny22 (64 x 64); d.tiles_n / d.tiles_m for it; d.N % 8 == 0.
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream) {
     const int step = elt == kBF16 ? 32 : 16;

@@ -47,7 +47,10 @@ LDS swizzle: a tile row is 64 bytes = four 16-byte chunks; chunk c of row r sits
 in slot c ^ ((r >> 2) & 3), which spreads the fragment reads of any
 8 or 16 consecutive rows over all banks.  One buffer_load_dwordx4 ... lds moves
 16 rows (64 lanes x 16 B) to M0 + 16 * lane; the swizzle is applied on the
-global side (which chunk a lane fetches).
+global side (which chunk a lane fetches).  An operand in the units layout
+(common.h) arrives as 1 KiB units of 32 rows x 16 k instead; only the lane's
+fragment address (%[wb], %[xb]) and what leads to k-phase 1 (%[wx], %[xx]: 0x20,
+or 0x400 for units) differ, block i is 2048 i bytes further in both.
 """
 def vreg4(base):
     return "v[%d:%d]" % (base, base + 3)
@@ -180,9 +183,9 @@ def main(c=FULL):
     e = Emitter()
     e.emit("; ======== setup ========")
     e.emit("v_mov_b32 v%d, %%[wb]" % (c.addr + 0))
-    e.emit("v_xor_b32 v%d, 0x20, %%[wb]" % (c.addr + 1))
+    e.emit("v_xor_b32 v%d, %%[wx], %%[wb]" % (c.addr + 1))
     e.emit("v_mov_b32 v%d, %%[xb]" % (c.addr + 2))
-    e.emit("v_xor_b32 v%d, 0x20, %%[xb]" % (c.addr + 3))
+    e.emit("v_xor_b32 v%d, %%[xx], %%[xb]" % (c.addr + 3))
     for r in range(4):
         e.emit("v_add_u32 v%d, 0x%x, v%d" % (c.addr + 4 + r, 2 * c.stage, c.addr + r))
     e.emit("v_mov_b32 v%d, %%[wv0]" % c.wvoff)
@@ -296,9 +299,9 @@ def main_skewed(c):
     e = Emitter()
     e.emit("; ======== setup ========")
     e.emit("v_mov_b32 v%d, %%[wb]" % (c.base + 0))
-    e.emit("v_xor_b32 v%d, 0x20, %%[wb]" % (c.base + 1))
+    e.emit("v_xor_b32 v%d, %%[wx], %%[wb]" % (c.base + 1))
     e.emit("v_mov_b32 v%d, %%[xb]" % (c.base + 2))
-    e.emit("v_xor_b32 v%d, 0x20, %%[xb]" % (c.base + 3))
+    e.emit("v_xor_b32 v%d, %%[xx], %%[xb]" % (c.base + 3))
     e.emit("v_mov_b32 v%d, %%[wv0]" % c.wvoff)
     e.emit("v_mov_b32 v%d, %%[xv0]" % c.xvoff)
     for i in range(1, c.nw):

@@ -24,6 +24,7 @@ enum GemmEpilogue : int {
     kEpiQKV = 3,       // scatter into per-head Q, K and transposed V (see below)
     kEpiQKVMap = 4,    // the same on compact rows: row m is token rowmap[m] (chosen by launch_gemm when rowmap is set)
     kEpiBiasRes = 5,   // Y = acc + bias + R, float32 row-major (chosen by launch_gemm when residual is set)
+    kEpiBiasGeluUnits = 7,   // kEpiBiasGelu with a bf16 result in the units layout (chosen by launch_gemm when y_units is set)
     kEpiBiasResLN = 6, // Y = LayerNorm(acc + bias + R) (chosen by launch_gemm when ln_gamma is set)
 };
 
@@ -41,7 +42,7 @@ constexpr int kTile256x128Deep = 385; // ... of the 256 x 128 kernel with one wo
 constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 kernel (bf16, three workgroups per CU, splits K)
 
 constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
-constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: packed bf16 or split float32 operands, any K split for float32 results)
+constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results)
 
 struct GemmParams {
     const void* X = nullptr;
@@ -89,6 +90,7 @@ struct GemmParams {
     bool compiler_scheduled = false;   // 256 tile: use the generic kernel, not the hand-scheduled one
     // Packed operand layout (common.h): X / W read from it, Y (bf16, plain epilogues) written in it.
     bool x_packed = false, w_packed = false, y_packed = false;
+    bool x_units = false, w_units = false, y_units = false;    // ... in its "units" form (bf16; with the flag above set too; Y: GELU only)
     int xcd_partition = -1;   // how the eight XCDs divide the tile grid (see tile_of_block): -1 = estimate and choose, 0 = contiguous
                               // runs of the tile sequence, 2 / 4 = 4 x 2 / 2 x 4 cells (for measurements)
 };
@@ -118,9 +120,9 @@ bool gemm_ln_supported(int M, int N, int K, int elt);
 // Replaces Query_Key / op_SoftMax / Prob_Value of the reference
 // (cuda_bert/ops/batch_matmul.cu:48-83,107-141; ops/softmax.cu:86-143)
 // without materialising the [B,S,heads,S] score tensor.
-// ctx_packed (bf16 only): write ctx in the packed GEMM-operand layout (common.h).
+// ctx_layout: kRowMajor, or (bf16) kPacked / kUnits, the layouts of the GEMM that follows (common.h).
 bool launch_attention(const void* q, const void* k, const void* vt, const float* maskadd,
-                      void* ctx, bool ctx_packed, int B, int heads, int S, int Sp, float scale, int elt,
+                      void* ctx, int ctx_layout, int B, int heads, int S, int Sp, float scale, int elt,
                       hipStream_t stream, const int* cu = nullptr, bool v_rowmajor = false, bool first_only = false,
                       int variant = kAttnAuto);
 // v_rowmajor (bf16, S <= 512 only): `vt` holds V as [B, heads, S, 64] like k.
@@ -189,9 +191,9 @@ bool launch_unpad_rows(const float* xc, const int* cu, float* out, int B, int S,
 
 // ------------------------------------------------------ load helpers -------
 // dst[n, k] = convert(src[k, n])  : on-disk [in,out] float32 -> [out,in] operand type,
-// row-major, (bf16) packed or (kF32Split) split; in the latter cases dst is the whole operand and the
+// row-major, (bf16; packed = kPacked or kUnits) packed or (kF32Split) split; in the latter cases dst is the whole operand and the
 // tensor's rows land at row0 .. row0 + N - 1 of it.
-bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt, bool packed, int row0,
+bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt, int packed, int row0,
                               hipStream_t stream);
 bool launch_fill_f32(float* dst, float value, size_t n, hipStream_t stream);
 

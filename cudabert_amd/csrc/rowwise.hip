@@ -92,7 +92,7 @@ __device__ __forceinline__ void ln_store4(const float (&v)[4], float mean, float
         for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x4_t*>(dst + p * 1024) = bf16x4_t{s[p][0], s[p][1], s[p][2], s[p][3]};
     } else {
         bf16x4_t ob = {(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
-        const size_t off = LAYOUT == kPacked ? packed_offset(row, i * 2, H * 2 / 64) : ((size_t)row * H + i) * 2;
+        const size_t off = LAYOUT == kUnits ? units_offset(row, i * 2, H * 2 / 64) : LAYOUT == kPacked ? packed_offset(row, i * 2, H * 2 / 64) : ((size_t)row * H + i) * 2;
         *reinterpret_cast<bf16x4_t*>(dst + off) = ob;
     }
 }
@@ -496,7 +496,7 @@ __global__ __launch_bounds__(256) void transpose_convert_kernel(const float* __r
                 __bf16* d = reinterpret_cast<__bf16*>(dst + split_offset(row0 + nn, kk, K));
                 split_bf16x3(val, d[0], d[512], d[1024]);
             } else if constexpr (ELT == kBF16) {
-                const size_t off = packed ? packed_offset(row0 + nn, kk * 2, K * 2 / 64) : ((size_t)nn * K + kk) * 2;
+                const size_t off = packed == kUnits ? units_offset(row0 + nn, kk * 2, K * 2 / 64) : packed ? packed_offset(row0 + nn, kk * 2, K * 2 / 64) : ((size_t)nn * K + kk) * 2;
                 *reinterpret_cast<__bf16*>(dst + off) = (__bf16)val;
             } else {
                 reinterpret_cast<float*>(dst)[(size_t)nn * K + kk] = val;
@@ -620,6 +620,7 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
     };
     if (y && y_elt != kF32 && y_elt != kBF16) { set_error("layernorm: bad addend type"); return false; }
     if (xb_layout == kSplit) go(std::integral_constant<int, kSplit>());
+    else if (xb_layout == kUnits) go(std::integral_constant<int, kUnits>());
     else if (xb_layout == kPacked) go(std::integral_constant<int, kPacked>());
     else go(std::integral_constant<int, kRowMajor>());
     CUBERT_HIP_OK(hipGetLastError());
@@ -651,7 +652,7 @@ bool launch_embed_layernorm(const int* ids, const int* seg, const int* mask, con
     }
     const long rows = compact ? compact->rows : (long)B * S;
     dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    auto kernel = xb_layout == kSplit ? embed_layernorm_kernel<kSplit> : xb_layout == kPacked ? embed_layernorm_kernel<kPacked> : embed_layernorm_kernel<kRowMajor>;
+    auto kernel = xb_layout == kSplit ? embed_layernorm_kernel<kSplit> : xb_layout == kUnits ? embed_layernorm_kernel<kUnits> : xb_layout == kPacked ? embed_layernorm_kernel<kPacked> : embed_layernorm_kernel<kRowMajor>;
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, ids, seg, mask, word, pos, type, gamma,
                        beta, x, xb, maskadd, B, S, Sp, H, vocab, type_vocab,
                        compact ? compact->rowmap : nullptr, compact ? compact->cu : nullptr, (int)rows);
@@ -750,11 +751,11 @@ bool launch_unpad_rows(const float* xc, const int* cu, float* out, int B, int S,
     return true;
 }
 
-bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt, bool packed, int row0,
+bool launch_transpose_convert(const float* src, void* dst, int K, int N, int elt, int packed, int row0,
                               hipStream_t stream) {
     if (!src || !dst || K <= 0 || N <= 0) { set_error("transpose: bad arguments"); return false; }
     if (packed && (elt != kBF16 || K % 32 != 0)) { set_error("transpose: packed output is bf16 with K a multiple of 32"); return false; }
-    const int pk = packed ? 1 : 0;
+    const int pk = packed;
     dim3 grid((N + 31) / 32, (K + 31) / 32), block(256);
     unsigned char* d = static_cast<unsigned char*>(dst);
     if (elt == kF32Split && K % 16 != 0) { set_error("transpose: the split layout needs K to be a multiple of 16"); return false; }

@@ -195,6 +195,9 @@ long cubert_capacity_tokens(void* model);
 #define CUBERT_V_ROWMAJOR 32        /* cubert_op_gemm_qkv / cubert_op_attention (bf16, S <= 512): the `vt` argument holds V as
                                        [B, heads, S, 64] like k instead of transposed */
 #define CUBERT_Y_SPLIT 64           /* float32 context / copy in the split layout (cubert_op_attention, _add_layernorm, _embed_layernorm) */
+#define CUBERT_X_UNITS 128          /* with the corresponding _PACKED flag: the units form of the packed layout (bf16): inside */
+#define CUBERT_W_UNITS (1 << 24)    /* a block of 256 rows x 64 bytes, units of 32 rows x 32 bytes in MFMA operand order */
+#define CUBERT_Y_UNITS (1 << 25)
 /* elt = 2 (cubert_op_gemm, _gemm_residual, _gemm_qkv): float32 operands in the split layout, every element as the exact sum
  * of three bfloat16 numbers; the product is formed from six bf16 matrix products and has float32 accuracy.  K must be a
  * multiple of 16; Y is float32 row-major, or (GELU epilogue) split, out_elt 2.  fp32 mode runs on this. */
@@ -213,6 +216,7 @@ long cubert_capacity_tokens(void* model);
 #define CUBERT_SPLITS_OF(flags) (((flags) >> 8) & 0xff)
 size_t cubert_packed_bytes(size_t rows, size_t row_bytes);
 size_t cubert_packed_offset(int row, int byte_in_row, int row_bytes);
+size_t cubert_units_offset(int row, int byte_in_row, int row_bytes);
 
 /* Size of a [rows, K] operand in the split layout, and the conversion into it of the transpose of src [K, N] (float32
  * row-major, like the Linear kernels on disk): src's column n becomes row row0 + n of the operand. */
