@@ -197,8 +197,126 @@ __global__ __launch_bounds__(256) void attention_kernel(
 }
 
 
+// One block of 32 keys for the 32 queries of a wave, out of the LDS.  krow: row l32 of the block (K, 16-byte chunks permuted by
+// ksw = row & 7); vpiece[db]: VROW: my piece of the first transposing read of feature block db, else key 4 g of the block in row
+// 32 db + l32 of V^T; sMk: the block's mask row (times log2 e); is_plain: every key visible, mask terms zero.
+template <bool VROW>
+__device__ __forceinline__ void attend_block(const unsigned char* krow, int ksw, const uint4 (&qf)[4], const float* sMk, bool is_plain,
+                                             const unsigned char* const (&vpiece)[2], float scale_log2e, int g, f32x16_t (&o)[2],
+                                             float& run_max, float& run_sum) {
+    // ---- scores^T: rows = the keys, column = my query ----
+    f32x16_t sc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        const uint4 kf = *reinterpret_cast<const uint4*>(krow + (((2 * kk + g) ^ ksw) << 4));
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf),
+                                                     __builtin_bit_cast(bf16x8_t, qf[kk]), sc, 0, 0, 0);
+    }
+    // Softmax with a lazily moved reference exponent: p = exp2(t - ref), where ref is the row
+    // maximum seen when it was last moved.  It only moves (and the sums are rescaled) when a
+    // block exceeds it by more than 2^20, so that in almost every block there is no rescaling
+    // of the 32 context accumulators and no second exponential; p stays below 2^20 and the
+    // final division by the row sum removes the common factor.  The first processed block
+    // (ref = -inf) always takes the move.
+    float blk_max = -INFINITY;
+    if (is_plain) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) blk_max = fmaxf(blk_max, sc[v]);
+        blk_max *= scale_log2e;                          // scale_log2e > 0
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4_t m4 = *reinterpret_cast<const f32x4_t*>(sMk + 8 * j + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float t = fmaf(sc[4 * j + e], scale_log2e, m4[e]);
+                sc[4 * j + e] = t;
+                blk_max = fmaxf(blk_max, t);
+            }
+        }
+    }
+    blk_max = half_swap_max(blk_max);
+    if (__ballot(blk_max > run_max + 20.0f) != 0ull) {    // finite blk_max: a processed block holds a real key column
+        const float new_max = fmaxf(run_max, blk_max);
+        const float alpha = __builtin_amdgcn_exp2f(run_max - new_max);     // 1 for the lanes that stay
+        run_sum *= alpha;
+        run_max = new_max;
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
+    }
+    float blk_sum = 0.0f;
+    if (is_plain) {
+        const float neg_ref = -run_max;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float pv = __builtin_amdgcn_exp2f(fmaf(sc[v], scale_log2e, neg_ref));
+            sc[v] = pv;
+            blk_sum += pv;
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float pv = __builtin_amdgcn_exp2f(sc[v] - run_max);
+            sc[v] = pv;
+            blk_sum += pv;
+        }
+    }
+    blk_sum = half_swap_sum(blk_sum);
+    run_sum += blk_sum;
+
+    // ---- ctx^T += V^T (rows = head features) x P^T (column = my query) ----
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {        // keys 16 f + {4g..4g+3, 8+4g..8+4g+3}
+        bf16x8_t pf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pf[e] = (__bf16)sc[8 * f + e];
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+            if constexpr (VROW) {
+                // my piece: 4 features of key 16 f + 4 g + (i >> 2) (and of the key 8 further), i = l32 & 15
+                const unsigned char* piece = vpiece[db] + 16 * f * 128;
+                const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>((__attribute__((address_space(3))) unsigned char*)piece));
+                const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>((__attribute__((address_space(3))) unsigned char*)(piece + 8 * 128)));
+                const s16x8_t vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf), pf, o[db], 0, 0, 0);
+            } else {
+                const unsigned char* vrow = vpiece[db] + 32 * f;
+                const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
+                const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 16);
+                const uint4 vf = {lo.x, lo.y, hi.x, hi.y};
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf), pf, o[db], 0, 0, 0);
+            }
+        }
+    }
+}
+
+// ctx of a wave's 32 queries: lane owns query qi, features 32 db + 8 j + 4 g + e of head h, row `row` of the context.
+__device__ __forceinline__ void store_context(unsigned char* ctx, int ctx_layout, size_t row, int heads, int h, int g, const f32x16_t (&o)[2], float run_sum) {
+    const float inv = 1.0f / run_sum;
+    const size_t hidden = (size_t)heads * 64;
+    unsigned char* orow = ctx + (row * hidden + (size_t)h * 64) * 2;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int d = 32 * db + 8 * j + 4 * g;
+            bf16x4_t w = {(__bf16)(o[db][4 * j] * inv), (__bf16)(o[db][4 * j + 1] * inv),
+                          (__bf16)(o[db][4 * j + 2] * inv), (__bf16)(o[db][4 * j + 3] * inv)};
+            if (ctx_layout != kRowMajor)
+                *reinterpret_cast<bf16x4_t*>(ctx + operand_offset(ctx_layout, (int)row, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
+            else
+                *reinterpret_cast<bf16x4_t*>(orow + d * 2) = w;
+        }
+}
+
 // ---------------------------------------------------------------------------
-// bf16, S <= 512: one workgroup per (batch, head) with one wave per block of 32
+// bf16, S <= 512, V transposed: one workgroup per (batch, head) with one wave per block of 32
 // queries.  K [S, 64] and V^T [64, Sp] of the head are brought into LDS once
 // (instead of once per wave through the vector memory path) and every wave
 // takes its MFMA operands from there:
@@ -212,15 +330,6 @@ __global__ __launch_bounds__(256) void attention_kernel(
 // visible key in the row their probabilities are exactly zero in float32
 // (exp2 of less than -14000), so the result is bit-identical to walking them.
 // If no key at all is visible nothing is skipped.
-//
-// VROW: V arrives as [S, 64] rows like K (the QKV GEMM then stores it in whole row segments instead
-// of two bytes at a time).  It sits in the LDS as rows of 128 bytes whose four 32-byte blocks are
-// permuted by (row >> 1) & 3, and the transposition the second MFMA needs happens in the read:
-// ds_read_b64_tr_b16 hands lane i of a group of 16 the i-th 16-bit element of each of the four
-// 32-byte pieces that lanes 4r .. 4r+3 (r = 0..3) point at, so with piece r = 16 features of key
-// kb + r a lane receives its feature for four consecutive keys.  The block permutation puts the
-// four pieces of a group into four different bank ranges.
-template <bool VROW>
 __global__ __launch_bounds__(1024) void attention_lds_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
     const unsigned char* __restrict__ vt, const float* __restrict__ maskadd,
@@ -229,7 +338,7 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* sK = smem;
     unsigned char* sV = smem + (size_t)Sp * 128;
-    float* sM = reinterpret_cast<float*>(sV + (VROW ? (size_t)Sp * 128 : 64 * (size_t)vstride));
+    float* sM = reinterpret_cast<float*>(sV + 64 * (size_t)vstride);
     int* sLive = reinterpret_cast<int*>(sM + Sp);
 
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -240,7 +349,7 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
     const size_t bh = (size_t)b * heads + h;
     const unsigned char* qb = q + bh * S * 128;
     const unsigned char* kb = k + bh * S * 128;
-    const unsigned char* vb = vt + (VROW ? bh * S * 128 : bh * 64 * (size_t)Sp * 2);
+    const unsigned char* vb = vt + bh * 64 * (size_t)Sp * 2;
 
     // Q fragments ("B" operand: column = query), kept for the whole key loop.  Requested first, together with the
     // K / V loads below: a short batch's launch is one chain of round trips, and this one is then not a link of it.
@@ -271,16 +380,9 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = tid + i * nthr;
-        if constexpr (VROW) {
-            vrow_i[i] = c >> 3;
-            vch_i[i] = c & 7;
-            vd[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (vrow_i[i] < S) vd[i] = *reinterpret_cast<const uint4*>(vb + (size_t)c * 16);
-        } else {
-            vrow_i[i] = c / vchunks;
-            vch_i[i] = c - vrow_i[i] * vchunks;
-            vd[i] = *reinterpret_cast<const uint4*>(vb + ((size_t)vrow_i[i] * Sp + vch_i[i] * 8) * 2);
-        }
+        vrow_i[i] = c / vchunks;
+        vch_i[i] = c - vrow_i[i] * vchunks;
+        vd[i] = *reinterpret_cast<const uint4*>(vb + ((size_t)vrow_i[i] * Sp + vch_i[i] * 8) * 2);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -290,14 +392,9 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        if constexpr (VROW) {
-            const int row = vrow_i[i], ch = vch_i[i];
-            *reinterpret_cast<uint4*>(sV + row * 128 + ((((ch >> 1) ^ ((row >> 1) & 3)) << 5) | ((ch & 1) << 4))) = vd[i];
-        } else {
-            uint2* dst = reinterpret_cast<uint2*>(sV + (size_t)vrow_i[i] * vstride + vch_i[i] * 16);     // rows are 8-byte aligned
-            dst[0] = make_uint2(vd[i].x, vd[i].y);
-            dst[1] = make_uint2(vd[i].z, vd[i].w);
-        }
+        uint2* dst = reinterpret_cast<uint2*>(sV + (size_t)vrow_i[i] * vstride + vch_i[i] * 16);     // rows are 8-byte aligned
+        dst[0] = make_uint2(vd[i].x, vd[i].y);
+        dst[1] = make_uint2(vd[i].z, vd[i].w);
     }
     {
         // wave w looks at mask block w
@@ -331,132 +428,141 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
         for (int v = 0; v < 16; ++v) o[db][v] = 0.0f;
     float run_max = -INFINITY, run_sum = 0.0f;
     const int ksw = l32 & 7;
-    // VROW: where my 8-byte piece of a transposing read lies for key block 0, f = 0, per feature block db.
-    // Row 4 g + (i >> 2), i = l32 & 15; logical 32-byte block 2 db + (l32 >> 4), permuted by (row >> 1) & 3,
-    // which the multiples of 8 that k0, f and the second read add to the row do not change.
-    const unsigned char* vpiece[2];
-    {
-        const int i16 = l32 & 15, prow = 4 * g + (i16 >> 2), psw = (prow >> 1) & 3;
-#pragma unroll
-        for (int db = 0; db < 2; ++db)
-            vpiece[db] = sV + prow * 128 + (((2 * db + (l32 >> 4)) ^ psw) << 5) + (i16 & 3) * 8;
-    }
+    // key 4 g of key block 0 in my two rows of V^T
+    const unsigned char* const vrow[2] = {sV + (size_t)l32 * vstride + 4 * g * 2, sV + (size_t)(32 + l32) * vstride + 4 * g * 2};
 
     for (int kblk = 0; kblk < nblk; ++kblk) {
         if (!((live >> kblk) & 1u)) continue;
         const int k0 = kblk * 32;
-        // ---- scores^T block: rows = keys k0..k0+31, column = my query ----
-        f32x16_t sc;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
-        const unsigned char* krow = sK + (k0 + l32) * 128;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const uint4 kf = *reinterpret_cast<const uint4*>(krow + (((2 * kk + g) ^ ksw) << 4));
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf),
-                                                         __builtin_bit_cast(bf16x8_t, qf[kk]), sc, 0, 0, 0);
-        }
-        // Softmax with a lazily moved reference exponent: p = exp2(t - ref), where ref is the row
-        // maximum seen when it was last moved.  It only moves (and the sums are rescaled) when a
-        // block exceeds it by more than 2^20, so that in almost every block there is no rescaling
-        // of the 32 context accumulators and no second exponential; p stays below 2^20 and the
-        // final division by the row sum removes the common factor.  The first processed block
-        // (ref = -inf) always takes the move.
-        const bool is_plain = (plain >> kblk) & 1u;           // every key visible, mask term zero
-        float blk_max = -INFINITY;
-        if (is_plain) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) blk_max = fmaxf(blk_max, sc[v]);
-            blk_max *= scale_log2e;                          // scale_log2e > 0
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const f32x4_t m4 = *reinterpret_cast<const f32x4_t*>(sM + k0 + 8 * j + 4 * g);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float t = fmaf(sc[4 * j + e], scale_log2e, m4[e]);
-                    sc[4 * j + e] = t;
-                    blk_max = fmaxf(blk_max, t);
-                }
-            }
-        }
-        blk_max = half_swap_max(blk_max);
-        if (__ballot(blk_max > run_max + 20.0f) != 0ull) {    // finite blk_max: a processed block holds a real key column
-            const float new_max = fmaxf(run_max, blk_max);
-            const float alpha = __builtin_amdgcn_exp2f(run_max - new_max);     // 1 for the lanes that stay
-            run_sum *= alpha;
-            run_max = new_max;
-#pragma unroll
-            for (int db = 0; db < 2; ++db)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
-        }
-        float blk_sum = 0.0f;
-        if (is_plain) {
-            const float neg_ref = -run_max;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float pv = __builtin_amdgcn_exp2f(fmaf(sc[v], scale_log2e, neg_ref));
-                sc[v] = pv;
-                blk_sum += pv;
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float pv = __builtin_amdgcn_exp2f(sc[v] - run_max);
-                sc[v] = pv;
-                blk_sum += pv;
-            }
-        }
-        blk_sum = half_swap_sum(blk_sum);
-        run_sum += blk_sum;
-
-        // ---- ctx^T += V^T (rows = head features) x P^T (column = my query) ----
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {        // keys k0 + 16 f + {4g..4g+3, 8+4g..8+4g+3}
-            bf16x8_t pf;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pf[e] = (__bf16)sc[8 * f + e];
-#pragma unroll
-            for (int db = 0; db < 2; ++db) {
-                if constexpr (VROW) {
-                    // my piece: 4 features of key k0 + 16 f + 4 g + (i >> 2) (and of the key 8 further), i = l32 & 15
-                    const unsigned char* piece = vpiece[db] + (k0 + 16 * f) * 128;
-                    const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>((__attribute__((address_space(3))) unsigned char*)piece));
-                    const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>((__attribute__((address_space(3))) unsigned char*)(piece + 8 * 128)));
-                    const s16x8_t vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf), pf, o[db], 0, 0, 0);
-                } else {
-                    const unsigned char* vrow = sV + (size_t)(32 * db + l32) * vstride + (k0 + 16 * f + 4 * g) * 2;
-                    const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
-                    const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 16);
-                    const uint4 vf = {lo.x, lo.y, hi.x, hi.y};
-                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf), pf, o[db], 0, 0, 0);
-                }
-            }
-        }
+        const unsigned char* const vp[2] = {vrow[0] + k0 * 2, vrow[1] + k0 * 2};
+        attend_block<false>(sK + (k0 + l32) * 128, ksw, qf, sM + k0, (plain >> kblk) & 1u, vp, scale_log2e, g, o, run_max, run_sum);
     }
 
-    // ---- normalise and store: lane owns query q0 + l32, features 32 db + 8 j + 4 g + e ----
     const int qi = q0 + l32;
     if (qi >= qlen || (first_only && qi != 0)) return;
-    const float inv = 1.0f / run_sum;
-    const size_t hidden = (size_t)heads * 64;
-    unsigned char* orow = ctx + ((row_base + qi) * hidden + (size_t)h * 64) * 2;
+    store_context(ctx, ctx_layout, row_base + qi, heads, h, g, o, run_sum);
+}
+
+
+// ---------------------------------------------------------------------------
+// bf16, S <= 512, V as [B, heads, S, 64] rows like K (the QKV GEMM then stores whole row segments): a workgroup of NW waves
+// owns 32 NW queries of one (batch, head) and walks the keys in chunks of 32 NW, which it brings into the LDS one after the
+// other (memory-to-LDS loads).  K rows lie there as in attention_lds_kernel; V rows of 128 bytes have their four 32-byte blocks
+// permuted by (row >> 1) & 3, and the transposition the second MFMA needs happens in the read: ds_read_b64_tr_b16 hands lane i
+// of a group of 16 the i-th 16-bit element of each of the four 32-byte pieces that lanes 4r .. 4r+3 (r = 0 .. 3) point at, so
+// with piece r = 16 features of key kb + r a lane receives its feature for four consecutive keys.  The block permutation puts
+// the four pieces of a group into four different bank ranges.
+//
+// Bound: the vector ALU's softmax work, and what is resident to hide the loads behind it.  A chunk of 128 keys is 34 KiB of
+// LDS, so a CU holds four workgroups whatever S is (a whole head of S = 512 is 130 KiB: one workgroup, whose waves past a short
+// sequence's end idle while they hold it), and the query blocks of a long sequence spread over CUs.  K and V are read again for
+// every 128 queries, out of the L2.  Measured against one workgroup per (batch, head) with all of K and V staged, 16 heads,
+// microseconds: B=64 S=512 114 -> 107, B=128 S=300 110 -> 92, B=128 S=200 50.8 -> 48.5, B=128 S=128 31.1 -> 25.9, B=23 S=77
+// 7.4 -> 6.7, B=1 S=512 22.5 -> 12.5; 64 lines of 32 to 512 valid tokens in compact rows (a pass of BERT-large) 9.2 -> 8.5 ms.
+// Up to 64 keys four waves would idle (S = 33: 8.5 -> 9.5), hence NW = ceil(S / 32) there.
+// The same key blocks in the same order with the same arithmetic per wave as attention_lds_kernel, hence the same bits.
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 4) void attention_chunk_kernel(
+    const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
+    const float* __restrict__ maskadd, unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale_log2e, int ctx_layout,
+    const int* __restrict__ cu, int first_only) {
+    __shared__ __attribute__((aligned(1024))) unsigned char sK[NW * 4096];
+    __shared__ __attribute__((aligned(1024))) unsigned char sV[NW * 4096];
+    __shared__ __attribute__((aligned(16))) float sM[NW == 4 ? 512 : NW * 32];
+    __shared__ int sLive[NW == 4 ? 16 : NW];
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, g = lane >> 5;
+    // the queries of the longest sequences first: their workgroups take longest
+    const int h = blockIdx.x, b = blockIdx.y, qc0 = (gridDim.z - 1 - blockIdx.z) * (32 * NW), q0 = qc0 + wave * 32;
+    const int qlen = cu ? cu[b + 1] - cu[b] : S;
+    if (qc0 >= qlen) return;                             // the whole workgroup: no barrier has been met
+    const int nblk = Sp >> 5;                            // at most 16, or NW < 4
+    const size_t bh = (size_t)b * heads + h;
+    const unsigned char* qb = q + bh * S * 128;
+    // rows S .. Sp - 1 lie outside the descriptors and arrive as zeros
+    const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(k + bh * S * 128), 0, S * 128, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(v + bh * S * 128), 0, S * 128, 0x00020000);
+    // One load moves eight rows: lane l fills slot l & 7 of row l >> 3, which holds chunk slot ^ (row & 7) of K and, of V, the
+    // chunk whose 32-byte block is the slot's, permuted by (row >> 1) & 3.  Wave w loads the rows of block w of the chunk.
+    const int lrow = lane >> 3, slot = lane & 7;
+    const int k_lane = lrow * 128 + ((slot ^ lrow) << 4);
+    const int v_lane = lrow * 128 + (((((slot >> 1) ^ ((lrow >> 1) & 3)) << 1) | (slot & 1)) << 4);
+    auto stage = [&](int blk0) {
+        if (blk0 + wave >= nblk) return;
+        const int row0 = (blk0 + wave) * 32;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(kres, (lds_ptr_t)(sK + wave * 4096 + i * 1024), 16, (row0 + 8 * i) * 128 + k_lane, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(vres, (lds_ptr_t)(sV + wave * 4096 + i * 1024), 16, (row0 + 8 * i) * 128 + v_lane, 0, 0, 0);
+        }
+    };
+    stage(0);
+    uint4 qf[4];
+    {
+        int qrow = q0 + l32;
+        qrow = qrow < qlen ? qrow : qlen - 1;            // qlen >= 1; a wave past the end only helps with the loads
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            qf[kk] = *reinterpret_cast<const uint4*>(qb + (size_t)qrow * 128 + (2 * kk + g) * 16);
+    }
+    for (int blk = wave; blk < nblk; blk += NW) {
+        const float m = lane < 32 ? maskadd[(size_t)b * Sp + blk * 32 + lane] : -INFINITY;
+        if (lane < 32) sM[blk * 32 + lane] = m * 1.4426950408889634f;
+        const unsigned long long vis = __ballot(m > -5000.0f);
+        const unsigned long long zero = __ballot(lane < 32 && m == 0.0f);
+        // bit 0: some key of the block is visible; bit 1: all 32 are, with a zero mask term
+        if (lane == 0) sLive[blk] = (vis != 0ull ? 1 : 0) | (zero == 0xffffffffull ? 2 : 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the compiler does not count the memory-to-LDS loads for the transposing reads
+    __syncthreads();
+    unsigned live = 0, plain = 0;
+    for (int i = 0; i < nblk; ++i) {
+        const int f = sLive[i];
+        live |= (f & 1) ? (1u << i) : 0u;
+        plain |= (f & 2) ? (1u << i) : 0u;
+    }
+    if (live == 0) live = 0xffffu >> (16 - nblk);
+    live = __builtin_amdgcn_readfirstlane(live);
+    plain = __builtin_amdgcn_readfirstlane(plain);
+
+    const bool working = q0 < qlen && !(first_only && wave != 0);
+    f32x16_t o[2];
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int d = 32 * db + 8 * j + 4 * g;
-            bf16x4_t w = {(__bf16)(o[db][4 * j] * inv), (__bf16)(o[db][4 * j + 1] * inv),
-                          (__bf16)(o[db][4 * j + 2] * inv), (__bf16)(o[db][4 * j + 3] * inv)};
-            if (ctx_layout != kRowMajor)
-                *reinterpret_cast<bf16x4_t*>(ctx + operand_offset(ctx_layout, (int)row_base + qi, (h * 64 + d) * 2, (int)hidden * 2 / 64)) = w;
-            else
-                *reinterpret_cast<bf16x4_t*>(orow + d * 2) = w;
+        for (int e = 0; e < 16; ++e) o[db][e] = 0.0f;
+    float run_max = -INFINITY, run_sum = 0.0f;
+    // Where my 8-byte piece of a transposing read lies in a V block: row 4 g + (i >> 2), i = l32 & 15; 32-byte block
+    // 2 db + (l32 >> 4), permuted by (row >> 1) & 3, which the multiples of 8 that the reads add to the row do not change.
+    int vpiece[2];
+    {
+        const int i16 = l32 & 15, prow = 4 * g + (i16 >> 2), psw = (prow >> 1) & 3;
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+            vpiece[db] = prow * 128 + (((2 * db + (l32 >> 4)) ^ psw) << 5) + (i16 & 3) * 8;
+    }
+    for (int blk0 = 0; blk0 < nblk; blk0 += NW) {
+        if (((live >> blk0) & ((1u << NW) - 1u)) == 0u) continue;      // the same for every wave
+        if (blk0 > 0) {
+            __syncthreads();                             // everybody has read the previous chunk
+            stage(blk0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
         }
+        if (!working) continue;
+        for (int j = 0; j < NW && blk0 + j < nblk; ++j) {
+            if (!((live >> (blk0 + j)) & 1u)) continue;
+            const unsigned char* const vp[2] = {sV + j * 4096 + vpiece[0], sV + j * 4096 + vpiece[1]};
+            attend_block<true>(sK + (32 * j + l32) * 128, l32 & 7, qf, sM + (blk0 + j) * 32, (plain >> (blk0 + j)) & 1u, vp, scale_log2e, g, o,
+                               run_max, run_sum);
+        }
+    }
+    const int qi = q0 + l32;
+    if (!working || qi >= qlen || (first_only && qi != 0)) return;
+    store_context(ctx, ctx_layout, (first_only ? (size_t)b : (cu ? (size_t)cu[b] : (size_t)b * S) + qi), heads, h, g, o, run_sum);
 }
 
 
@@ -516,7 +622,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[db][e] = 0.0f;
     float run_max = -INFINITY, run_sum = 0.0f;
-    // where my 8-byte piece of a transposing read lies in a V block (see attention_lds_kernel)
+    // where my 8-byte piece of a transposing read lies in a V block (see attention_chunk_kernel)
     int vpiece[2];
     {
         const int i16 = l32 & 15, prow = 4 * g + (i16 >> 2), psw = (prow >> 1) & 3;
@@ -704,9 +810,19 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
         CUBERT_HIP_OK(hipGetLastError());
         return true;
     }
+    if (elt == kBF16 && S <= 512 && v_rowmajor) {
+        // one workgroup of fewer waves up to 64 keys, four waves beyond (see the kernel)
+        const dim3 grid(heads, B, first_only || S <= 64 ? 1 : (S + 127) / 128);
+        const float c = scale * 1.4426950408889634f;
+        if (S <= 32) hipLaunchKernelGGL(attention_chunk_kernel<1>, grid, dim3(64), 0, stream, qc, kc, vc, maskadd, cc, heads, S, Sp, c, cp, cu, fo);
+        else if (S <= 64) hipLaunchKernelGGL(attention_chunk_kernel<2>, grid, dim3(128), 0, stream, qc, kc, vc, maskadd, cc, heads, S, Sp, c, cp, cu, fo);
+        else hipLaunchKernelGGL(attention_chunk_kernel<4>, grid, dim3(256), 0, stream, qc, kc, vc, maskadd, cc, heads, S, Sp, c, cp, cu, fo);
+        CUBERT_HIP_OK(hipGetLastError());
+        return true;
+    }
     if (elt == kBF16 && S <= 512) {
         const int vstride = round_up(Sp * 2, 256) + 8;
-        const size_t lds = (size_t)Sp * 128 + (v_rowmajor ? (size_t)Sp * 128 : 64 * (size_t)vstride) + (size_t)Sp * 4 + 64;
+        const size_t lds = (size_t)Sp * 128 + 64 * (size_t)vstride + (size_t)Sp * 4 + 64;
         // More than 64 KiB of dynamic LDS has to be allowed once per device.
         // (Several host threads, one model each, may get here together: the flag is atomic and
         // setting the attribute twice is harmless.)
@@ -714,18 +830,12 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
         int dev = 0;
         CUBERT_HIP_OK(hipGetDevice(&dev));
         if (dev < 0 || dev >= 64 || !allowed[dev].load(std::memory_order_acquire)) {
-            CUBERT_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_lds_kernel<false>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            CUBERT_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_lds_kernel<true>),
+            CUBERT_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_lds_kernel),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             if (dev >= 0 && dev < 64) allowed[dev].store(true, std::memory_order_release);
         }
-        if (v_rowmajor)
-            hipLaunchKernelGGL(attention_lds_kernel<true>, dim3(heads, B), dim3(2 * Sp), lds, stream, qc, kc, vc, maskadd,
-                               cc, heads, S, Sp, vstride, scale * 1.4426950408889634f, cp, cu, fo);
-        else
-            hipLaunchKernelGGL(attention_lds_kernel<false>, dim3(heads, B), dim3(2 * Sp), lds, stream, qc, kc, vc, maskadd,
-                               cc, heads, S, Sp, vstride, scale * 1.4426950408889634f, cp, cu, fo);
+        hipLaunchKernelGGL(attention_lds_kernel, dim3(heads, B), dim3(2 * Sp), lds, stream, qc, kc, vc, maskadd,
+                           cc, heads, S, Sp, vstride, scale * 1.4426950408889634f, cp, cu, fo);
         CUBERT_HIP_OK(hipGetLastError());
         return true;
     }

@@ -126,7 +126,7 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
                       hipStream_t stream, const int* cu = nullptr, bool v_rowmajor = false, bool first_only = false,
                       int variant = kAttnAuto);
 // v_rowmajor (bf16, S <= 512 only): `vt` holds V as [B, heads, S, 64] like k.
-// variant (v_rowmajor only): kAttnPerHead = one workgroup per (batch, head); kAttnSplitKeys = one workgroup per
+// variant (v_rowmajor only): kAttnPerHead = a wave walks all keys of its 32 queries; kAttnSplitKeys = one workgroup per
 // (batch, head, 32 queries) whose four waves share the keys: the short-batch kernel; kAttnAuto picks by the number of such workgroups.
 // The variants agree to the last bit or two of the bf16 context, not bit for bit.
 // first_only: only the context of every sequence's first token is produced, as row b of ctx [B, heads*64] (same bits
