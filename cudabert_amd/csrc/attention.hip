@@ -764,11 +764,11 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const size_t row = first_only ? (size_t)b : (cu ? (size_t)cu[b] : (size_t)b * S) + qrow;
     const int kbyte = (h * 64 + fg * FPT) * 2;
     unsigned char* dst = ctx_layout != kRowMajor ? ctx + operand_offset(ctx_layout, (int)row, kbyte, (int)hidden * 2 / 64) : ctx + row * hidden * 2 + kbyte;
+    static_assert(FPT == 8, "a thread stores 16 bytes");
+    bf16x8_t w8;
 #pragma unroll
-    for (int e = 0; e < FPT; e += 4) {
-        const bf16x4_t w4 = {(__bf16)(acc[e] * inv), (__bf16)(acc[e + 1] * inv), (__bf16)(acc[e + 2] * inv), (__bf16)(acc[e + 3] * inv)};
-        *reinterpret_cast<bf16x4_t*>(dst + e * 2) = w4;
-    }
+    for (int e = 0; e < FPT; ++e) w8[e] = (__bf16)(acc[e] * inv);
+    *reinterpret_cast<bf16x8_t*>(dst) = w8;
 }
 
 }  // namespace

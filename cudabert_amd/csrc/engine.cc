@@ -520,7 +520,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     const Dims& D = opt_.dims;
     const int elt = opt_.precision;
     const size_t os = elt == kBF16 ? 2 : 6;      // bytes per element of a GEMM operand and of q, k, v
-    const int gelt = elt == kBF16 ? kBF16 : kF32Split, layout = elt == kBF16 ? kPacked : kSplit;
+    const int gelt = elt == kBF16 ? kBF16 : kF32Split;
     // rows of this part: every token, or (unpadded pass) the valid ones only, stored from row r0
     const int H = D.hidden, I = D.inter, N = cp ? cp->rows : B * S, Sp = round_up(S, 32);
     const size_t cap = (size_t)cap_tokens_, t0 = (size_t)b0 * S;
@@ -547,9 +547,13 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             max_splits = 16;
             while (max_splits > 1 && (long)max_splits * N > (long)N + kSplitRows) max_splits /= 2;
         }
-        return gemm_plan(N, H, K, gelt, max_splits, true, false);
+        return gemm_plan(N, H, K, gelt, max_splits, true, false, elt == kBF16);
     };
     const bool any_order = cur_parts_ == 1 && opt_.split_k;
+    // LayerNorm's bf16 copy: the units layout for the few rows at which QKV and FFN-in may take a skinny tile, which needs it
+    // (one line of 17 tokens, BERT-base: 435 -> 416 us), else the packed one, whose pieces of a row are 64 bytes instead of 16
+    // (one line of 200 tokens, BERT-large, no skinny tile: 1145 us packed, 1155 units).
+    const int layout = elt == kF32 ? kSplit : any_order && N <= kSkinnyMaxRows ? kUnits : kPacked;
     const GemmPlan plan_ao = plan_for(H), plan_fo = plan_for(I);
     const int sp_ao = plan_ao.splits, sp_fo = plan_fo.splits;
     // the attn-out / FFN-out GEMMs add the residual stream in their epilogue, so LayerNorm reads one operand
@@ -611,7 +615,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             g = GemmParams();
             g.elt = g.out_elt = gelt; g.X = xbc; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
             g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
-        g.x_units = layout == kUnits;
+            g.x_units = layout == kUnits;
             if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
             g = GemmParams();
             g.elt = gelt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;

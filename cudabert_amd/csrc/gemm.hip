@@ -390,8 +390,9 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 constexpr int kPlanSmallRows = 6144;
 
 namespace {
-// Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits).
-GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu) {
+// Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits).  skinny: the operands and the
+// epilogue suit the skinny kernel and the caller does not need the k order that the other tiles share.
+GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, bool skinny) {
     // launch: before the first workgroup runs; fixed + per_hs * half-steps: a workgroup alone on its CU (deep_k: what a
     // half-step costs more when K > 2048 and the weights stream from memory); rho, q: see above; out: weight of the
     // result traffic (bytes / 4 TB/s).  Least-squares fit (5 % mean error) to launches of the four linears of BERT-large
@@ -420,6 +421,16 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
             const double cost = c.launch + c.out * out_us * (sp > 1 ? 1.5 : 1.0) + T * g;
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
         }
+    }
+    // The skinny tile (32 features x 64 tokens) wins while every workgroup has a CU to itself; a second one on a CU competes for
+    // the same loads.  Microseconds, cold weights, skinny against the best of the others: 17 rows, QKV / FFN-in / FFN-out of
+    // BERT-base 5.0 / 5.0 / 4.9 against 6.1 / 6.0 / 5.3, of BERT-large 6.3 / 7.8 / 5.8 against 6.8 / 8.4 / 6.3; 128 rows of
+    // BERT-base 5.5 / 5.8 / 5.8 against 6.4 / 6.5 / 6.3; 200 rows (288 workgroups) 7.8 / 8.1 against 6.5 / 6.7.
+    for (int sp = min_splits; skinny && sp <= max_splits && sp <= 16; sp *= 2) {
+        if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
+        if ((long)((M + 63) / 64) * ((N + 31) / 32) * sp > 256) break;
+        const double cost = 3.2 + 0.1 * (K / 32.0 / sp) + (sp > 1 ? 0.6 : 0.0) + (gelu ? 0.8 : 0.0);
+        if (cost < best_cost) { best_cost = cost; best = GemmPlan{kTileSkinny12, sp}; }
     }
     return best;
 }
@@ -518,7 +529,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
 }
 }  // namespace
 
-GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu) {
+GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool units) {
     if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, max_splits > 1);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
@@ -532,7 +543,7 @@ GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result
         }
         return best;
     }
-    return plan_small(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu);
+    return plan_small(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, units && max_splits > 1 && N % 8 == 0);
 }
 
 bool launch_gemm(const GemmParams& p, hipStream_t stream) {
@@ -635,8 +646,11 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     int bt = p.tile;
     if (!bt) {
         // the caller has settled on the split count; the tile follows
-        if (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0)
-            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu).tile;
+        if (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0) {
+            const bool skinny = p.any_k_order && p.x_units && p.w_units && p.N % 8 == 0 && !p.compiler_scheduled && epi != kEpiBiasResLN &&
+                                (p.epilogue == kEpiQKV ? p.v_rowmajor : epi == kEpiBiasGeluUnits || ((epi == kEpiBias || epi == kEpiBiasRes) && out == kF32));
+            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu, skinny).tile;
+        }
         else
             bt = gemm_pick_tile(p.M, p.N, p.K, p.elt);
     }

@@ -43,6 +43,7 @@ constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 ker
 
 constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
 constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results)
+constexpr int kSkinnyMaxRows = 128;   // rows up to which QKV and FFN-in of the model may take a skinny tile in bf16 (engine.cc)
 
 struct GemmParams {
     const void* X = nullptr;
@@ -99,9 +100,9 @@ struct GemmParams {
 bool launch_gemm(const GemmParams& p, hipStream_t stream);
 // The tile (a GemmParams::tile value, never 0) and split count launch_gemm's cost model prefers for a problem.
 // max_splits > 1: the caller can take a float32 result as up to that many partial sums (a power of two is chosen).
-// f32_result / gelu: the launch will write float32 / use the GELU epilogue.
+// f32_result / gelu: the launch will write float32 / use the GELU epilogue.  units: both (bf16) operands are in the units layout.
 struct GemmPlan { int tile; int splits; };
-GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu);
+GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool units);
 // Workspace of a GEMM with the LayerNorm in its epilogue (GemmParams::ln_ws) for up to M rows.
 size_t gemm_ln_workspace_bytes(size_t M);
 // Test aid: puts a workspace into a state in which the workgroups of row band 0 can never see their band complete

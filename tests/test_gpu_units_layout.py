@@ -108,3 +108,33 @@ def test_skinny_qkv_matches_the_staged_tile(lib, tile, B, S, heads):
         ref = want[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
         lim = scale[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
         assert ((t.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + (H / 16 + 6) * U * lim).all()
+
+
+@pytest.fixture(scope="module")
+def two_layers(tmp_path_factory):
+    import dataclasses
+    from cudabert_amd import pybert
+    from cudabert_amd import weights as W
+    dims = dataclasses.replace(W.BASE, layers=2, vocab=500)
+    d = str(tmp_path_factory.mktemp("two_layers"))
+    W.export_npy_dir(W.bf16_representable(W.synth_state(dims, seed=3, degenerate=False)), d)
+    m = pybert.load_model_ex(d, dims.hidden, dims.layers, dims.heads, dims.inter, precision=1, max_batchsize=2, max_seq_length=300)
+    yield m, W.load_npy_dir(d), dims
+    pybert.unload_model(m)
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (1, 17), (1, 64), (1, 65), (1, 128), (1, 129), (1, 256), (1, 257), (2, 129)])
+def test_rows_at_which_the_model_changes_layout_and_tile(two_layers, B, S):
+    """The units layout and the skinny tiles end at 128 rows; eager and replayed pass against the float32 oracle at the bf16
+    mode's tolerance, 3e-2."""
+    from cudabert_amd import pybert, synth
+    from oracle import bert_oracle as O
+    m, npy, dims = two_layers
+    ids, seg, mask = synth.make_inputs(B, S, np.full(B, S), vocab=dims.vocab, seed=S, prune=False)
+    seq_ref, pooled_ref = O.forward_torch(npy, dims.heads, ids, seg, mask)
+    first = None
+    for _ in range(4):
+        pooled, seq, _ = pybert.encode(m, ids, seg, mask, want_seq=True)
+        assert np.abs(seq - seq_ref).max() < 3e-2 and np.abs(pooled - pooled_ref).max() < 3e-2
+        first = seq if first is None else first
+        assert np.array_equal(seq, first)
