@@ -158,14 +158,16 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
     normalise_store<LAYOUT>(v, H, lane, gamma, beta, xrow, xb, row);
 }
 
-// The same operation for a short batch whose addend comes as the partial sums of a split-K GEMM
+// The same operation for a short batch, whose addend may come as the partial sums of a split-K GEMM
 // ([part][rows][H] float32): one workgroup per row, so that the few rows still spread over the
-// chip.  Such a launch is a chain of round trips and little else, so everything it needs -- the row,
+// chip and a wave's chain is a quarter of a row long.  Such a launch is a chain of round trips and little else, so everything it needs -- the row,
 // every partial sum, gamma and beta -- is requested before the first value is used.  Wave w adds up the
 // parts of features 256 w .. 256 w + 255 and forms the statistics of its two slots; the waves exchange
 // those through the LDS, every wave combines them (the same arithmetic in the same order as
 // add_layernorm_kernel, hence the same bits) and normalises its own features.
-template <int LAYOUT>
+// MORE: parts after the first; 0, 1 and 3 are exact, any other number goes in rounds of 8 that repeat part 0 to fill up
+// (1600 x 1024, 4 parts: five needless loads out of eight, 9.8 us against 9.4; 2 parts 6.9 against 6.1).
+template <int LAYOUT, int MORE>
 __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restrict__ x, const float* __restrict__ y,
                                                                   const float* __restrict__ gamma,
                                                                   const float* __restrict__ beta,
@@ -185,16 +187,24 @@ __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restr
         f32x4_t t = *reinterpret_cast<const f32x4_t*>(y + (size_t)row * H + i);
         g4 = *reinterpret_cast<const f32x4_t*>(gamma + i);
         b4 = *reinterpret_cast<const f32x4_t*>(beta + i);
-        for (int p0 = 1; p0 < y_parts; p0 += 8) {
-            f32x4_t u[8];
+        if constexpr (MORE == 1 || MORE == 3) {
+            f32x4_t u[MORE];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int part = p0 + j < y_parts ? p0 + j : 0;        // a repeat of part 0 is not added
-                u[j] = *reinterpret_cast<const f32x4_t*>(y + ((size_t)part * rows + row) * H + i);
+            for (int j = 0; j < MORE; ++j) u[j] = *reinterpret_cast<const f32x4_t*>(y + ((size_t)(1 + j) * rows + row) * H + i);
+#pragma unroll
+            for (int j = 0; j < MORE; ++j) t += u[j];
+        } else if constexpr (MORE != 0) {
+            for (int p0 = 1; p0 < y_parts; p0 += 8) {
+                f32x4_t u[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int part = p0 + j < y_parts ? p0 + j : 0;        // a repeat of part 0 is not added
+                    u[j] = *reinterpret_cast<const f32x4_t*>(y + ((size_t)part * rows + row) * H + i);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (p0 + j < y_parts) t += u[j];
             }
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (p0 + j < y_parts) t += u[j];
         }
         a += t;
 #pragma unroll
@@ -594,6 +604,12 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
+// Rows up to which a whole (not split) addend takes the kernel with a workgroup per row, by what the copy's stores allow (the
+// split layout's 16-byte pieces of a row want neighbouring rows in one workgroup).  Microseconds, workgroup per row against
+// wave per row, H = 1024: packed copy 200 rows 2.8 / 5.3, 800 4.5 / 6.4, 1600 5.9 / 7.4, 3200 8.5 / 9.4, 6000 15.7 / 13.3;
+// split copy 128 rows 3.4 / 5.0, 800 7.0 / 7.7, 1600 10.5 / 9.7.
+constexpr int kRowPerGroup = 4096, kRowPerGroupSplit = 800;
+
 bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma, const float* beta,
                           void* xb, int xb_layout, int rows, int H, hipStream_t stream, int y_parts, bool add_x) {
     if (!add_x && !y) { set_error("layernorm: without the residual stream an addend is required"); return false; }
@@ -614,7 +630,11 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
         constexpr int L = decltype(layout)::value;
         const int ax = add_x ? 1 : 0;
         if (!y) hipLaunchKernelGGL((add_layernorm_kernel<-1, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
-        else if (y_elt == kF32 && y_parts > 1) hipLaunchKernelGGL(add_layernorm_parts_kernel<L>, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, y_parts, ax);
+        else if (y_elt == kF32 && (y_parts > 1 || rows <= (L == kSplit ? kRowPerGroupSplit : kRowPerGroup))) {
+            auto kernel = y_parts == 1 ? add_layernorm_parts_kernel<L, 0> : y_parts == 2 ? add_layernorm_parts_kernel<L, 1>
+                        : y_parts == 4 ? add_layernorm_parts_kernel<L, 3> : add_layernorm_parts_kernel<L, 7>;
+            hipLaunchKernelGGL(kernel, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, y_parts, ax);
+        }
         else if (y_elt == kF32) hipLaunchKernelGGL((add_layernorm_kernel<kF32, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
         else hipLaunchKernelGGL((add_layernorm_kernel<kBF16, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
     };
