@@ -97,6 +97,15 @@ __device__ __forceinline__ void ln_store4(const float (&v)[4], float mean, float
     }
 }
 
+// Mean and 1 / sigma of the row held in v[][] (lane owns elements c*256 + lane*4 + e).
+__device__ __forceinline__ void ln_row_stats(const float (&v)[kMaxChunks][4], int H, int lane, float* mean, float* rstd) {
+    float ssum[2 * kMaxChunks], sm2[2 * kMaxChunks];
+#pragma unroll
+    for (int c = 0; c < kMaxChunks; ++c)
+        ln_chunk_stats(v[c], c, H, lane, &ssum[2 * c], &sm2[2 * c], &ssum[2 * c + 1], &sm2[2 * c + 1]);
+    ln_combine_slots(ssum, sm2, H, mean, rstd);
+}
+
 // Normalises the row held in v[][] (lane owns elements c*256 + lane*4 + e) and
 // writes it to x (f32) and optionally xb (ln_store4).
 template <int LAYOUT>
@@ -104,12 +113,8 @@ __device__ __forceinline__ void normalise_store(float (&v)[kMaxChunks][4], int H
                                                 const float* __restrict__ gamma,
                                                 const float* __restrict__ beta, float* xrow,
                                                 void* xb, int row) {
-    float ssum[2 * kMaxChunks], sm2[2 * kMaxChunks];
-#pragma unroll
-    for (int c = 0; c < kMaxChunks; ++c)
-        ln_chunk_stats(v[c], c, H, lane, &ssum[2 * c], &sm2[2 * c], &ssum[2 * c + 1], &sm2[2 * c + 1]);
     float mean, rstd;
-    ln_combine_slots(ssum, sm2, H, &mean, &rstd);
+    ln_row_stats(v, H, lane, &mean, &rstd);
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c) {
         const int i = c * 256 + lane * 4;
@@ -156,6 +161,63 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
         }
     }
     normalise_store<LAYOUT>(v, H, lane, gamma, beta, xrow, xb, row);
+}
+
+// add_layernorm_kernel<kF32, kSplit> for many rows.  There a wave stores its row's copy in 16-byte pieces, one per unit half and
+// plane, and the memory system is handed a quarter of a 64-byte line at a time.  Here the eight waves of a workgroup hold eight
+// neighbouring rows, put the pieces side by side in the LDS (group of 8 features of a plane: 128 bytes, row r in slot
+// r ^ (group % 8), which spreads a wave's writes over the banks) and store whole 128-byte lines.  Same bits.
+// BERT-large fp32, 128 lines of up to 200 tokens: 58.8 -> 57.8 ms a pass; BERT-base, 16 of up to 512: 8.07 -> 8.01 ms.
+__global__ __launch_bounds__(512) void add_layernorm_split_rows_kernel(float* __restrict__ x, const float* __restrict__ y,
+                                                                       const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                                       unsigned char* __restrict__ xb, int rows, int H, int add_x) {
+    __shared__ __attribute__((aligned(16))) unsigned char pieces[3 * (kMaxChunks * 256 / 8) * 128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row0 = blockIdx.x * 8, row = row0 + wave, groups = H >> 3;
+    if (row < rows) {
+        float* xrow = x + (size_t)row * H;
+        const float* yrow = y + (size_t)row * H;
+        float v[kMaxChunks][4];
+#pragma unroll
+        for (int c = 0; c < kMaxChunks; ++c) {
+            const int i = c * 256 + lane * 4;
+            if (i < H) {
+                f32x4_t a = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(yrow + i));
+                if (add_x) a = *reinterpret_cast<const f32x4_t*>(xrow + i) + a;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[c][e] = a[e];
+            }
+        }
+        float mean, rstd;
+        ln_row_stats(v, H, lane, &mean, &rstd);
+#pragma unroll
+        for (int c = 0; c < kMaxChunks; ++c) {
+            const int i = c * 256 + lane * 4;
+            if (i < H) {
+                const f32x4_t g4 = *reinterpret_cast<const f32x4_t*>(gamma + i);
+                const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(beta + i);
+                f32x4_t o;
+                __bf16 s[3][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = ln_apply(v[c][e], mean, rstd, g4[e], b4[e]);
+                    split_bf16x3(o[e], s[0][e], s[1][e], s[2][e]);
+                }
+                __builtin_nontemporal_store(o, reinterpret_cast<f32x4_t*>(xrow + i));
+                const int grp = i >> 3;
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    *reinterpret_cast<bf16x4_t*>(pieces + (p * groups + grp) * 128 + (wave ^ (grp & 7)) * 16 + (i & 4) * 2) =
+                        bf16x4_t{s[p][0], s[p][1], s[p][2], s[p][3]};
+            }
+        }
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < 3 * groups * 8; c += 512) {
+        const int slot = c & 7, pg = c >> 3, p = (pg >= groups) + (pg >= 2 * groups), grp = pg - p * groups;
+        const int r = row0 + (slot ^ (grp & 7));
+        if (r < rows) *reinterpret_cast<f32x4_t*>(xb + split_offset(r, grp * 8, H) + p * 1024) = *reinterpret_cast<const f32x4_t*>(pieces + c * 16);
+    }
 }
 
 // The same operation for a short batch, whose addend may come as the partial sums of a split-K GEMM
@@ -635,6 +697,7 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
                         : y_parts == 4 ? add_layernorm_parts_kernel<L, 3> : add_layernorm_parts_kernel<L, 7>;
             hipLaunchKernelGGL(kernel, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, y_parts, ax);
         }
+        else if (y_elt == kF32 && L == kSplit && xb) hipLaunchKernelGGL(add_layernorm_split_rows_kernel, dim3((rows + 7) / 8), dim3(512), 0, stream, x, static_cast<const float*>(y), gamma, beta, static_cast<unsigned char*>(xb), rows, H, ax);
         else if (y_elt == kF32) hipLaunchKernelGGL((add_layernorm_kernel<kF32, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
         else hipLaunchKernelGGL((add_layernorm_kernel<kBF16, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, H, y_parts, ax);
     };
