@@ -357,7 +357,7 @@ int cubert_op_attention(const void* q, const void* k, const void* vt, const floa
     cubert::set_error("");
     if (elt == cubert::kF32Split)
         return cubert::launch_attention_f32(q, k, vt, maskadd, ctx, B, heads, S, cubert::round_up(S > 0 ? S : 1, 32), scale,
-                                            static_cast<hipStream_t>(stream)) ? 0 : 1;
+                                            static_cast<hipStream_t>(stream), nullptr, false, (flags >> 20) & 3) ? 0 : 1;
     return cubert::launch_attention(q, k, vt, maskadd, ctx, result_layout(flags & ~CUBERT_Y_SPLIT), B, heads, S,
                                     cubert::round_up(S > 0 ? S : 1, 32), scale, elt,
                                     static_cast<hipStream_t>(stream), nullptr, (flags & CUBERT_V_ROWMAJOR) != 0, false,

@@ -51,7 +51,7 @@ inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 // it as they are, and LDS fragment reads are linear in the lane; writers that hold whole rows (LayerNorm) prefer the
 // packed layout, whose pieces of a row are 64 bytes instead of 16.
 // Attention kernels (launch_attention's `variant`).
-constexpr int kAttnAuto = 0, kAttnPerHead = 1, kAttnSplitKeys = 2;
+constexpr int kAttnAuto = 0, kAttnPerHead = 1, kAttnSplitKeys = 2, kAttnSplitKeys8 = 3;      // 8: float32 only, eight waves instead of four
 constexpr int kAttnSplitMaxWorkgroups = 768; // B * heads * ceil(S / 32) up to which kAttnAuto takes the key-split kernel
 
 __host__ __device__ inline int packed_swizzle(int r) { return (r >> 2) & 3; }

@@ -373,7 +373,7 @@ bool Model::run_compact(const int* lens, int B, int S) {
     const size_t cu_off = cap + 256 * (kMaxParts - 1);
     CUBERT_HIP_OK(hipMemcpyAsync(d_meta_ + cu_off, h_meta_ + cu_off, (size_t)parts * kCuStride * 4, hipMemcpyHostToDevice, stream_));
     cur_parts_ = parts;
-    cur_attn_ = (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
+    cur_attn_ = pick_attention(B, S);
     if (parts == 1) return enqueue_part(0, 0, B, 0, S, false, stream_, &cp[0]);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));
     bool ok = true;
@@ -477,13 +477,18 @@ void Model::forget_uncaptured_shapes() {
         it = it->second.exec ? std::next(it) : graphs_.erase(it);
 }
 
+int Model::pick_attention(int B, int S) const {
+    if (opt_.precision == kF32) return attn_f32_variant(B, opt_.dims.heads, S, opt_.attn_split_workgroups);
+    return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
+}
+
 // One forward pass.  A large batch is cut into parts of whole sequences that run
 // the same launch sequence on separate streams: the parts are independent, and
 // while one part's GEMM is in its last, partly filled round of tiles (or in a
 // bandwidth-bound row kernel) another part's kernel takes the idle CUs.
 bool Model::enqueue(int B, int S, bool has_mask) {
     const long tokens = (long)B * S;
-    cur_attn_ = (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
+    cur_attn_ = pick_attention(B, S);
     int parts = opt_.split_parts < kMaxParts ? opt_.split_parts : kMaxParts;
     if (parts > B) parts = B;
     if (profiling_ || parts < 2 || opt_.split_min_tokens <= 0 || tokens < opt_.split_min_tokens) {
@@ -566,7 +571,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     if (ln_ao || ln_fo) ln_used_ = std::max(ln_used_, part + 1);
 
     auto attention = [&](void* out, bool vrow, bool first_only) {
-        if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only);
+        if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only, cur_attn_);
         return launch_attention(q, k, vt, maskadd, out, kUnits, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto);
     };
 

@@ -30,7 +30,7 @@ struct ModelOptions {
     bool fuse_residual = true;     // residual add in the epilogue of the GEMM before each LayerNorm
     bool fuse_layernorm = true;    // ... and the LayerNorm itself, where the GEMM kernel supports it (bf16, large batches)
     bool v_rowmajor = true;        // bf16, S <= 512: V is stored [B, heads, S, 64] like K; attention transposes on its LDS reads
-    int attn_split_workgroups = kAttnSplitMaxWorkgroups;   // bf16, S <= 512, row-major V: batches of up to this many
+    int attn_split_workgroups = kAttnSplitMaxWorkgroups;   // fp32, or bf16 with S <= 512 and row-major V: batches of up to this many
                                    // (batch, head, 32 queries) blocks run the attention kernel that splits a head's keys
                                    // over a workgroup's waves (0: never)
     bool split_k = true;           // short batches: split K of the hidden-wide GEMMs (changes the summation order)
@@ -98,6 +98,7 @@ class Model {
     bool init(const ModelOptions& opt);
     bool check_shape(int B, int S);
     bool run(int B, int S, bool has_mask);             // graph or eager
+    int pick_attention(int B, int S) const;            // cur_attn_ for a batch
     bool enqueue(int B, int S, bool has_mask);         // the launch sequence (one or two parts)
     bool enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp = nullptr);
     bool run_compact(const int* h_lens, int B, int S);

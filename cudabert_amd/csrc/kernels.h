@@ -136,7 +136,11 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
 // float32 attention on split operands: q, k, v as the QKV GEMM with elt == kF32Split writes them, [B, heads, Sp / 32] blocks
 // of twelve 1 KiB units each (attention_f32.hip); ctx in the split layout.  Other arguments as above.
 bool launch_attention_f32(const void* q, const void* k, const void* v, const float* maskadd, void* ctx, int B, int heads,
-                          int S, int Sp, float scale, hipStream_t stream, const int* cu = nullptr, bool first_only = false);
+                          int S, int Sp, float scale, hipStream_t stream, const int* cu = nullptr, bool first_only = false,
+                          int variant = kAttnAuto);
+// The kernel for a batch (kAttnPerHead, kAttnSplitKeys or kAttnSplitKeys8: waves walk all keys, or share them); decided on the
+// whole batch where it runs in parts, since the kernels sum in different orders.
+int attn_f32_variant(int B, int heads, int S, int max_blocks);
 
 // ----------------------------------------------------------- LayerNorm -----
 // x <- LayerNorm(x + y) * gamma + beta   over rows of length H, in place on the

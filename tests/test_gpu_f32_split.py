@@ -131,3 +131,44 @@ def test_qkv_projection_and_attention(lib, B, S, heads, tile):
     dscore = 26 * U * qk + 2 * proj * float(qkv[:2].abs().sum(-1).max()) * 0.125 + 4 * U * float(sc[sc > -5000].abs().max())
     bound = float(qkv[2].abs().max()) * (2 * dscore + (S + 26) * U) + proj
     assert float((unsplit(ctx, B * S, H).cpu() - want).abs().max()) < bound
+
+
+@pytest.mark.parametrize("B,S,heads", [(1, 1, 1), (2, 32, 1), (3, 33, 2), (2, 128, 1), (2, 129, 2), (1, 257, 1), (4, 300, 2), (1, 545, 1)])
+def test_attention_kernels_agree(lib, B, S, heads):
+    """The kernels whose four or eight waves share the keys and the one whose waves walk them, each against float64: masks that end early,
+    leave out keys in the middle or hide every key, padding rows of the last block that hold numbers of their own."""
+    H, Sp = heads * 64, (S + 31) // 32 * 32
+    X, W, b = operands(B * Sp, 3 * H, H)
+    X, W = X / X.abs().max() * 4, W * 2
+    mask = np.zeros((B, Sp), np.float32)
+    rng = np.random.default_rng(S)
+    for i in range(B):
+        if i == 1:
+            mask[i, :] = -10000.0                        # no visible key: a uniform shift, softmax over all of them
+        elif i == 2:
+            mask[i, rng.random(Sp) < 0.5] = -10000.0
+        elif i == 3:
+            mask[i, 1:] = -10000.0
+    mask[:, S:] = -np.inf
+    xs, ws, bd, md = split(lib, X.cuda()), split(lib, W.cuda()), b.cuda(), torch.from_numpy(mask).cuda()
+    q, k, v = (torch.zeros(B * heads * Sp * 384, dtype=torch.uint8, device="cuda") for _ in range(3))
+    # every position of the padded blocks is written, as a longer batch before this one would have left it
+    check(lib.cubert_op_gemm_qkv(xs.data_ptr(), ws.data_ptr(), bd.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), B, Sp, heads,
+                                 SPLIT, 128, 0, None))
+    qkv = (X.double() @ W.double().t() + b.double()).view(B, Sp, 3, heads, 64)[:, :S].permute(2, 0, 3, 1, 4)
+    sc = torch.matmul(qkv[0], qkv[1].transpose(-1, -2).contiguous()) * 0.125
+    want = torch.matmul(torch.softmax(sc + torch.from_numpy(mask[:, None, None, :S]).double(), -1), qkv[2]).permute(0, 2, 1, 3).reshape(B * S, H)
+    scale_in = float((X.double().abs() @ W.double().abs().t() + b.double().abs()).max())
+    proj = (6 * H / 16 + 2) * U * scale_in
+    qk = float(torch.matmul(qkv[0].abs(), qkv[1].abs().transpose(-1, -2).contiguous()).max()) * 0.125
+    # as above; where every key is masked (second sequence), a score near 10000 has an ulp of its own
+    offset = torch.tensor([10000.0 if i == 1 else 0.0 for i in range(B)], dtype=torch.float64).repeat_interleave(S)[:, None]
+    dscore = 26 * U * qk + 2 * proj * float(qkv[:2].abs().sum(-1).max()) * 0.125 + 4 * U * (float(sc.abs().max()) + offset)
+    bound = float(qkv[2].abs().max()) * (2 * dscore + (S + 26) * U) + proj
+    for variant in (1, 2, 3):
+        ctx = torch.full((lib.cubert_split_bytes(B * S, H),), 0x7f, dtype=torch.uint8, device="cuda")
+        check(lib.cubert_op_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), md.data_ptr(), ctx.data_ptr(), B, heads, S, 0.125, SPLIT,
+                                      variant << 20, None))
+        torch.cuda.synchronize()
+        got = unsplit(ctx, B * S, H).cpu()
+        assert ((got - want).abs() < bound).all(), variant
