@@ -643,12 +643,14 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
             return false;
         }
     }
+    // what the skinny kernel reads and writes, whoever asks for its tile
+    const bool skinny_fits = p.elt == kBF16 && p.x_units && p.w_units && p.N % 8 == 0 &&
+                             (p.epilogue == kEpiQKV ? p.v_rowmajor : epi == kEpiBiasGeluUnits || ((epi == kEpiBias || epi == kEpiBiasRes) && out == kF32));
     int bt = p.tile;
     if (!bt) {
         // the caller has settled on the split count; the tile follows
         if (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0) {
-            const bool skinny = p.any_k_order && p.x_units && p.w_units && p.N % 8 == 0 && !p.compiler_scheduled && epi != kEpiBiasResLN &&
-                                (p.epilogue == kEpiQKV ? p.v_rowmajor : epi == kEpiBiasGeluUnits || ((epi == kEpiBias || epi == kEpiBiasRes) && out == kF32));
+            const bool skinny = p.any_k_order && skinny_fits && !p.compiler_scheduled;
             bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu, skinny).tile;
         }
         else
@@ -670,7 +672,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
         return launch_gemm_bf16_t256x128(d, out, epi, stream);
     }
     if (bt == kTileSkinny12 || bt == kTileSkinny22) {
-        if (p.elt != kBF16 || !p.x_units || !p.w_units || p.N % 8 != 0 || (epi != kEpiQKV && epi != kEpiQKVMap && epi != kEpiBiasGeluUnits && out != kF32) || ((epi == kEpiQKV || epi == kEpiQKVMap) && !p.v_rowmajor)) {
+        if (!skinny_fits) {
             set_error("gemm: the skinny tiles need bf16 operands in the units layout and a GELU result in it, row-major QKV or float32 result");
             return false;
         }
