@@ -547,12 +547,12 @@ GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result
 }
 
 bool launch_gemm(const GemmParams& p, hipStream_t stream) {
+    if (p.xcd_partition != -1 && p.xcd_partition != 0 && p.xcd_partition != 2 && p.xcd_partition != 4) { set_error("gemm: the XCD partition is 0, 2 or 4"); return false; }
     if (p.elt == kF32Split) return launch_split_operands(p, stream);
     const int es = (p.elt == kBF16) ? 2 : 4;
     const int bk = 128 / es;
     if (p.elt != kBF16 && p.elt != kF32) { set_error("gemm: bad operand type"); return false; }
     if (p.M <= 0 || p.N <= 0 || p.K <= 0) { set_error("gemm: empty problem"); return false; }
-    if (p.xcd_partition != -1 && p.xcd_partition != 0 && p.xcd_partition != 2 && p.xcd_partition != 4) { set_error("gemm: the XCD partition is 0, 2 or 4"); return false; }
     if (p.K % bk != 0) { set_error("gemm: K must be a multiple of " + std::to_string(bk)); return false; }
     if (p.N % 4 != 0) { set_error("gemm: N must be a multiple of 4"); return false; }
     if (p.out_elt == kBF16 && p.N % 8 != 0) { set_error("gemm: N must be a multiple of 8 for bf16 results"); return false; }

@@ -30,3 +30,12 @@ def refused(pb, match, rc):
 ])
 def test_skinny_tile_takes_only_what_its_kernel_writes(pb, tile, epilogue, out, flags):
     refused(pb, "skinny", pb.lib.cubert_op_gemm(A, A, A, A, 1, 4096, 1024, 1024, BF16, out, epilogue, tile, flags, None))
+
+
+@pytest.mark.parametrize("partition", [1, 3, 5, 9, 14])
+@pytest.mark.parametrize("elt", [BF16, F32, SPLIT])
+def test_xcd_partition_is_checked_for_every_operand_type(pb, elt, partition):
+    """tile_of_block divides by the partition and takes block rows from it: another value leaves tiles out and reads past X."""
+    flags = (partition + 1) << 16
+    refused(pb, "XCD partition", pb.lib.cubert_op_gemm(A, A, A, A, 256, 256, 256, 256, elt, F32, 0, 128, flags, None))
+    refused(pb, "XCD partition", pb.lib.cubert_op_gemm_qkv(A, A, A, A, A, A, 2, 128, 4, elt, 128, flags, None))
