@@ -338,9 +338,8 @@ bool Model::run_compact(const int* lens, int B, int S) {
     if (lens != last_lens_.data()) last_lens_.assign(lens, lens + B);
     long tokens = 0;                  // rows this pass computes: the valid tokens
     for (int b = 0; b < B; ++b) tokens += lens[b];
-    int parts = opt_.split_parts < kMaxParts ? opt_.split_parts : kMaxParts;
-    if (parts > B) parts = B;
-    if (parts < 1 || opt_.split_min_tokens <= 0 || tokens < opt_.split_min_tokens) parts = 1;
+    const int parts = parts_for(tokens, B);
+    order_rows_ = opt_.split_k && parts == 1 ? (int)tokens : 0;
     // the pinned metadata of the previous call must have been consumed
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     const size_t cap = (size_t)cap_tokens_;
@@ -372,7 +371,6 @@ bool Model::run_compact(const int* lens, int B, int S) {
     CUBERT_HIP_OK(hipMemcpyAsync(d_meta_, h_meta_, rows_total * 4, hipMemcpyHostToDevice, stream_));
     const size_t cu_off = cap + 256 * (kMaxParts - 1);
     CUBERT_HIP_OK(hipMemcpyAsync(d_meta_ + cu_off, h_meta_ + cu_off, (size_t)parts * kCuStride * 4, hipMemcpyHostToDevice, stream_));
-    cur_parts_ = parts;
     cur_attn_ = pick_attention(B, S);
     if (parts == 1) return enqueue_part(0, 0, B, 0, S, false, stream_, &cp[0]);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));
@@ -482,20 +480,20 @@ int Model::pick_attention(int B, int S) const {
     return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
 }
 
+int Model::parts_for(long rows, int B) const {
+    const int parts = std::min(std::min(opt_.split_parts, (int)kMaxParts), B);
+    return parts < 2 || opt_.split_min_tokens <= 0 || rows < opt_.split_min_tokens ? 1 : parts;
+}
+
 // One forward pass.  A large batch is cut into parts of whole sequences that run
 // the same launch sequence on separate streams: the parts are independent, and
 // while one part's GEMM is in its last, partly filled round of tiles (or in a
 // bandwidth-bound row kernel) another part's kernel takes the idle CUs.
 bool Model::enqueue(int B, int S, bool has_mask) {
-    const long tokens = (long)B * S;
     cur_attn_ = pick_attention(B, S);
-    int parts = opt_.split_parts < kMaxParts ? opt_.split_parts : kMaxParts;
-    if (parts > B) parts = B;
-    if (profiling_ || parts < 2 || opt_.split_min_tokens <= 0 || tokens < opt_.split_min_tokens) {
-        cur_parts_ = 1;
-        return enqueue_part(0, 0, B, 0, S, has_mask, stream_);
-    }
-    cur_parts_ = parts;
+    const int parts = profiling_ ? 1 : parts_for((long)B * S, B);
+    order_rows_ = opt_.split_k && parts == 1 ? B * S : 0;
+    if (parts == 1) return enqueue_part(0, 0, B, 0, S, has_mask, stream_);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));
     bool ok = true;
     size_t r0 = 0;
@@ -543,24 +541,27 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     float* maskadd = maskadd_ + (size_t)b0 * Sp;
     const float scale = 1.0f / std::sqrt(64.0f);
 
+    // V stays row-major like K where the attention kernel that follows transposes on its own LDS reads
+    const bool vrow = opt_.v_rowmajor && elt == kBF16 && S <= 512;
     // Short batches: the two GEMMs with only `hidden` output features have too few tiles for the
     // chip; they split K over several workgroups and the LayerNorm that follows adds the parts.
     // (Not for the parts of a split batch, which sit side by side in y32; the parts of K need rows of y32.)
-    auto plan_for = [&](int K) {
-        int max_splits = 1;
-        if (cur_parts_ == 1 && opt_.split_k) {
-            max_splits = 16;
-            while (max_splits > 1 && (long)max_splits * N > (long)N + kSplitRows) max_splits /= 2;
-        }
-        return gemm_plan(N, H, K, gelt, max_splits, true, false, elt == kBF16);
-    };
-    const bool any_order = cur_parts_ == 1 && opt_.split_k;
+    const bool any_order = order_rows_ > 0;
+    const int R = any_order ? order_rows_ : N;      // N or more
+    int max_splits = any_order ? 16 : 1;
+    while (max_splits > 1 && (long)max_splits * R > (long)R + kSplitRows) max_splits /= 2;
     // LayerNorm's bf16 copy: the units layout for the few rows at which QKV and FFN-in may take a skinny tile, which needs it
     // (one line of 17 tokens, BERT-base: 435 -> 416 us), else the packed one, whose pieces of a row are 64 bytes instead of 16
     // (one line of 200 tokens, BERT-large, no skinny tile: 1145 us packed, 1155 units).
-    const int layout = elt == kF32 ? kSplit : any_order && N <= kSkinnyMaxRows ? kUnits : kPacked;
-    const GemmPlan plan_ao = plan_for(H), plan_fo = plan_for(I);
+    const int layout = elt == kF32 ? kSplit : any_order && R <= kSkinnyMaxRows ? kUnits : kPacked;
+    const bool any_x = any_order && layout != kPacked;
+    const GemmPlan plan_ao = gemm_plan(R, H, H, gelt, max_splits, true, false, any_order),
+                   plan_fo = gemm_plan(R, H, I, gelt, max_splits, true, false, any_order);
+    const int qkv_order = gemm_plan(R, 3 * H, H, gelt, 1, false, false, any_x && (elt == kF32 || vrow)).k_order();
+    const int fi_order = gemm_plan(R, I, H, gelt, 1, false, true, any_x).k_order();
     const int sp_ao = plan_ao.splits, sp_fo = plan_fo.splits;
+    // a tile that splits K is part of the order: tiles cut K at multiples of their own step
+    const int tile_ao = sp_ao > 1 || R == N ? plan_ao.tile : 0, tile_fo = sp_fo > 1 || R == N ? plan_fo.tile : 0;
     // the attn-out / FFN-out GEMMs add the residual stream in their epilogue, so LayerNorm reads one operand
     const bool fuse_res = opt_.fuse_residual;
     // ... and, where the GEMM kernel can, normalise there as well: x32 and its bf16 copy come straight out of
@@ -584,21 +585,19 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         const LayerDev& L = layers_[i];
         GemmParams g;
         g.elt = gelt;
-        // QKV projection, scattered per head (V transposed, unless the attention kernel that follows
-        // transposes on its own LDS reads)
-        const bool vrow = opt_.v_rowmajor && elt == kBF16 && S <= 512;
+        // QKV projection, scattered per head
         g.X = xb; g.ldx = H; g.W = L.w_qkv; g.bias = L.b_qkv; g.M = N; g.N = 3 * H; g.K = H;
         g.epilogue = kEpiQKV; g.q = q; g.k = k; g.vt = vt; g.S = S; g.Sp = Sp; g.heads = D.heads;
         g.v_rowmajor = vrow;
         g.rowmap = cp ? cp->rowmap : nullptr;
-        g.any_k_order = any_order;
+        g.k_order = qkv_order;
         g.x_packed = g.w_packed = g.w_units = pk;
         g.x_units = layout == kUnits;
         if (!mark(kPhQKV) || !launch_gemm(g, st)) return false;
         // The last layer of a pass whose caller gets no sequence output: keys and values are needed of every token,
-        // everything after them only of the first token of each sequence, which is all the pooler reads.  Its B rows
-        // go through the same kernels as row b * S of the full pass would (K is never split for them, and every
-        // kernel treats a row the same whatever else is in the launch), so the pooled output keeps its bits.
+        // everything after them only of the first token of each sequence, which is all the pooler reads.  Where the full
+        // pass would not split K, its B rows take kernels that sum over k in the order of the full pass's, and every kernel
+        // treats a row the same whatever else is in the launch, so the pooled output keeps its bits.
         const bool first = first_only_ && i == D.layers - 1 && sp_ao == 1 && sp_fo == 1;
         if (!mark(kPhAttention)) return false;
         if (first) {
@@ -614,6 +613,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             g.elt = gelt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
             g.M = B; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
+            g.k_order = plan_ao.k_order();
             if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
             if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, layout, B, H, st, 1, !fuse_res)) return false;
@@ -621,11 +621,13 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             g.elt = g.out_elt = gelt; g.X = xbc; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
             g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
             g.x_units = layout == kUnits;
+            g.k_order = fi_order;
             if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
             g = GemmParams();
             g.elt = gelt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;
             g.M = B; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
+            g.k_order = plan_fo.k_order();
             if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
             if (!launch_add_layernorm(xc, yc, kF32, L.g2, L.be2, nullptr, kRowMajor, B, H, st, 1, !fuse_res)) return false;
@@ -638,7 +640,8 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         g.elt = gelt; g.out_elt = kF32; g.X = ctx; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = y32;
         g.M = N; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk; g.splits = sp_ao;
         g.residual = fuse_res ? x32 : nullptr;
-        g.tile = plan_ao.tile;
+        g.tile = tile_ao;
+        g.k_order = plan_ao.k_order();
         if (ln_ao) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
@@ -648,13 +651,14 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         g.elt = g.out_elt = gelt; g.X = xb; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = h;
         g.M = N; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
         g.x_units = layout == kUnits;
-        g.any_k_order = any_order;
+        g.k_order = fi_order;
         if (!mark(kPhFFNIn) || !launch_gemm(g, st)) return false;
         g = GemmParams();
         g.elt = gelt; g.out_elt = kF32; g.X = h; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = y32;
         g.M = N; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk; g.splits = sp_fo;
         g.residual = fuse_res ? x32 : nullptr;
-        g.tile = plan_fo.tile;
+        g.tile = tile_fo;
+        g.k_order = plan_fo.k_order();
         if (ln_fo) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;

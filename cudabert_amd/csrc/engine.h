@@ -99,6 +99,7 @@ class Model {
     bool check_shape(int B, int S);
     bool run(int B, int S, bool has_mask);             // graph or eager
     int pick_attention(int B, int S) const;            // cur_attn_ for a batch
+    int parts_for(long rows, int B) const;             // parts a pass over that many token rows is cut into
     bool enqueue(int B, int S, bool has_mask);         // the launch sequence (one or two parts)
     bool enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp = nullptr);
     bool run_compact(const int* h_lens, int B, int S);
@@ -151,7 +152,9 @@ class Model {
     void *ctxc_ = nullptr, *hc_ = nullptr;         // attention context / FFN activation of those rows
     bool first_only_ = false;                      // the pass being enqueued (and the last one run) is of that kind
     bool last_compact_ = false;
-    int cur_parts_ = 1;          // parts of the pass being enqueued
+    // Rows on which split counts and skinny tiles, which regroup sums, are decided: those of the pass.
+    // 0: nothing is regrouped (split_k off, or a pass in parts).
+    int order_rows_ = 0;
     int cur_attn_ = kAttnPerHead;   // attention kernel of the pass being enqueued (decided on the whole batch)
     int B_ = 0, S_ = 0;
     // hipGraph cache: one entry per (B, S, mask) shape, captured on second sight, at most

@@ -390,9 +390,10 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 constexpr int kPlanSmallRows = 6144;
 
 namespace {
-// Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits).  skinny: the operands and the
-// epilogue suit the skinny kernel and the caller does not need the k order that the other tiles share.
-GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, bool skinny) {
+// Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits), all of one k order (kOrderAny:
+// the operands and the epilogue suit the skinny kernel).
+GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, int order) {
+    if (order == kOrderSkinny) return GemmPlan{kTileSkinny12, min_splits};
     // launch: before the first workgroup runs; fixed + per_hs * half-steps: a workgroup alone on its CU (deep_k: what a
     // half-step costs more when K > 2048 and the weights stream from memory); rho, q: see above; out: weight of the
     // result traffic (bytes / 4 TB/s).  Least-squares fit (5 % mean error) to launches of the four linears of BERT-large
@@ -426,7 +427,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
     // the same loads.  Microseconds, cold weights, skinny against the best of the others: 17 rows, QKV / FFN-in / FFN-out of
     // BERT-base 5.0 / 5.0 / 4.9 against 6.1 / 6.0 / 5.3, of BERT-large 6.3 / 7.8 / 5.8 against 6.8 / 8.4 / 6.3; 128 rows of
     // BERT-base 5.5 / 5.8 / 5.8 against 6.4 / 6.5 / 6.3; 200 rows (288 workgroups) 7.8 / 8.1 against 6.5 / 6.7.
-    for (int sp = min_splits; skinny && sp <= max_splits && sp <= 16; sp *= 2) {
+    for (int sp = min_splits; order == kOrderAny && sp <= max_splits && sp <= 16; sp *= 2) {
         if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
         if ((long)((M + 63) / 64) * ((N + 31) / 32) * sp > 256) break;
         const double cost = 3.2 + 0.1 * (K / 32.0 / sp) + (sp > 1 ? 0.6 : 0.0) + (gelu ? 0.8 : 0.0);
@@ -443,8 +444,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
 //   the skinny tiles: fixed + per_step * steps * (w > 1 ? w + 0.5 : 1), bound by what a CU fetches (60 - 65 GB/s of operands).
 // At 128 rows (QKV 3072 x 1024 / FFN-in 4096 x 1024 / FFN-out 1024 x 4096): 13.9 / 15.6 / 14.6 us with the skinny tile,
 // 35.2 / 40.7 / 24.0 with the 128 one; at 1600 rows 81 / 102 / 102 against 65 / 79 / 76.
-// any_order: the caller does not need the k order that all tiles but the skinny ones share.
-GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool any_order) {
+GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, int order) {
     struct Cand { int tile, bm, bn; double fixed, per_step; bool skinny; };
     static const Cand cands[] = {
         {128, 128, 128, 6.0, 0.455, false},
@@ -452,10 +452,11 @@ GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits
         {kTileSkinny12, 64, 32, 4.5, 0.144, true},
         {kTileSkinny22, 64, 64, 4.5, 0.214, true},
     };
-    GemmPlan best{128, min_splits};
+    GemmPlan best{order == kOrderSkinny ? kTileSkinny12 : 128, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
-        if (c.skinny && (!any_order || N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
+        if (order == (c.skinny ? kOrderShared : kOrderSkinny)) continue;
+        if (c.skinny && (N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;
             if (c.skinny && 4 * sp > K / 16) break;
@@ -514,7 +515,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
             d.R = p.residual;
         }
     }
-    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.any_k_order).tile;
+    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.k_order).tile;
     const bool skinny = tile == kTileSkinny12 || tile == kTileSkinny22;
     const int bn = tile == kTile256x128 ? 256 : tile == kTileSkinny12 ? 32 : tile == kTileSkinny22 ? 64 : 128, bm = skinny ? 64 : 128;
     d.tiles_n = (p.N + bn - 1) / bn;
@@ -529,8 +530,9 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
 }
 }  // namespace
 
-GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool units) {
-    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, max_splits > 1);
+GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order) {
+    const int order = any_order && N % 8 == 0 ? kOrderAny : kOrderShared;
+    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, order);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {
@@ -543,7 +545,7 @@ GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result
         }
         return best;
     }
-    return plan_small(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, units && max_splits > 1 && N % 8 == 0);
+    return plan_small(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, order);
 }
 
 bool launch_gemm(const GemmParams& p, hipStream_t stream) {
@@ -649,9 +651,9 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     int bt = p.tile;
     if (!bt) {
         // the caller has settled on the split count; the tile follows
-        if (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0) {
-            const bool skinny = p.any_k_order && skinny_fits && !p.compiler_scheduled;
-            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu, skinny).tile;
+        if (p.k_order == kOrderSkinny || (p.elt == kBF16 && p.M < kPlanSmallRows && p.K % 64 == 0)) {
+            const int order = p.k_order == kOrderAny && (!skinny_fits || p.compiler_scheduled) ? (int)kOrderShared : p.k_order;
+            bt = plan_small(p.M, p.N, p.K, d.splits, d.splits, out == kF32, p.epilogue == kEpiBiasGelu, order).tile;
         }
         else
             bt = gemm_pick_tile(p.M, p.N, p.K, p.elt);

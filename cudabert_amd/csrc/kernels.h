@@ -45,6 +45,11 @@ constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged
 constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results)
 constexpr int kSkinnyMaxRows = 128;   // rows up to which QKV and FFN-in of the model may take a skinny tile in bf16 (engine.cc)
 
+// How a launch groups the sums over k.  All kernels share one order (per split count) but the skinny tiles, whose four waves
+// each sum a share of K; among themselves those agree too.  Launches of a pass that have to give the same bits at different
+// row counts (the valid tokens alone, the first tokens alone) are given the same order.
+enum KOrder : int { kOrderShared = 0, kOrderSkinny = 1, kOrderAny = 2 };
+
 struct GemmParams {
     const void* X = nullptr;
     const void* W = nullptr;
@@ -85,9 +90,7 @@ struct GemmParams {
     // writes its partial result to Y + z * M * N; the bias goes into partial 0.  The consumer adds
     // them up (launch_add_layernorm's y_parts).  Y must hold splits * M * N floats.
     int splits = 1;
-    // A kernel may be chosen that groups the sums over k its own way (the skinny tiles do, as split K does): the result then
-    // depends, in its last bits, on which kernel the row count asks for.
-    bool any_k_order = false;
+    int k_order = kOrderShared;        // tile 0: which kernels may be chosen (a KOrder)
     bool compiler_scheduled = false;   // 256 tile: use the generic kernel, not the hand-scheduled one
     // Packed operand layout (common.h): X / W read from it, Y (bf16, plain epilogues) written in it.
     bool x_packed = false, w_packed = false, y_packed = false;
@@ -100,9 +103,13 @@ struct GemmParams {
 bool launch_gemm(const GemmParams& p, hipStream_t stream);
 // The tile (a GemmParams::tile value, never 0) and split count launch_gemm's cost model prefers for a problem.
 // max_splits > 1: the caller can take a float32 result as up to that many partial sums (a power of two is chosen).
-// f32_result / gelu: the launch will write float32 / use the GELU epilogue.  units: both (bf16) operands are in the units layout.
-struct GemmPlan { int tile; int splits; };
-GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool units);
+// f32_result / gelu: the launch will write float32 / use the GELU epilogue.  any_order: a skinny tile may be chosen (operands,
+// N and result suit it).
+struct GemmPlan {
+    int tile; int splits;
+    int k_order() const { return tile == kTileSkinny12 || tile == kTileSkinny22 ? kOrderSkinny : kOrderShared; }
+};
+GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order);
 // Workspace of a GEMM with the LayerNorm in its epilogue (GemmParams::ln_ws) for up to M rows.
 size_t gemm_ln_workspace_bytes(size_t M);
 // Test aid: puts a workspace into a state in which the workgroups of row band 0 can never see their band complete
