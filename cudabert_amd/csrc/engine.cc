@@ -287,10 +287,10 @@ bool Model::forward_host(const int* ids, const int* seg, const int* mask, int B,
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, h_in_ + cap, n * 4, hipMemcpyHostToDevice, stream_));
     if (mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * cap, h_in_ + 2 * cap, n * 4, hipMemcpyHostToDevice, stream_));
     // Masks that are 1 on a non-empty prefix and 0 after it allow the unpadded pass (valid tokens
-    // only; same pooled output bit for bit, zeros instead of values on the padding positions of the
-    // sequence output).  varlen = 1: whenever the masks allow it.  varlen = -1 (default): only when
-    // the caller cannot see the sequence output, the batch is too large for hipGraph replay and at
-    // least 5 % of it is padding.
+    // only; zeros instead of values on the padding positions of the sequence output).  varlen = 1: whenever the masks
+    // allow it.  varlen = -1 (default): only when the caller cannot see the sequence output, the batch is too large for
+    // hipGraph replay and at least 5 % of it is padding; the caller did not ask for it, so the pooled output is the padded
+    // pass's bit for bit.
     const bool too_big_for_graph = opt_.graph_max_tokens <= 0 || (long)n > opt_.graph_max_tokens;
     // The caller will not see the sequence output: the last layer only has to produce what the pooler reads.
     first_only_ = !need_seq && opt_.first_token_last_layer;
@@ -307,7 +307,7 @@ bool Model::forward_host(const int* ids, const int* seg, const int* mask, int B,
             lens[b] = len;
             valid += (size_t)len;
         }
-        if (prefix && (opt_.varlen == 1 || valid * 20 <= n * 19)) return run_compact(lens.data(), B, S);
+        if (prefix && (opt_.varlen == 1 || valid * 20 <= n * 19)) return run_compact(lens.data(), B, S, opt_.varlen < 0);
     }
     return run(B, S, mask != nullptr);
 }
@@ -324,22 +324,25 @@ bool Model::forward_device_lens(const int* d_ids, const int* d_seg, const int* h
     const size_t n = (size_t)B * S, cap = (size_t)cap_tokens_;
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_, d_ids, n * 4, hipMemcpyDeviceToDevice, stream_));
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
-    return run_compact(h_lens, B, S);
+    return run_compact(h_lens, B, S, false);
 }
 
 // Unpadded pass: the host lays out, per part, the token index of every compact row and the
 // row offset of every sequence, uploads both and enqueues the parts (never through a graph:
 // the row counts change from call to call).
-bool Model::run_compact(const int* lens, int B, int S) {
+bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     B_ = B;
     S_ = S;
     last_compact_ = true;
+    last_padded_bits_ = padded_bits;
     last_classified_ = false;
     if (lens != last_lens_.data()) last_lens_.assign(lens, lens + B);
     long tokens = 0;                  // rows this pass computes: the valid tokens
     for (int b = 0; b < B; ++b) tokens += lens[b];
     const int parts = parts_for(tokens, B);
-    order_rows_ = opt_.split_k && parts == 1 ? (int)tokens : 0;
+    // (a padded pass that runs in parts regroups nothing, and then neither does this one)
+    const long order_rows = padded_bits ? (long)B * S : tokens;
+    order_rows_ = opt_.split_k && parts_for(order_rows, B) == 1 ? (int)order_rows : 0;
     // the pinned metadata of the previous call must have been consumed
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     const size_t cap = (size_t)cap_tokens_;
@@ -727,7 +730,7 @@ bool Model::rerun_last() {
     const bool classified = last_classified_;
     bool ok;
     if (last_compact_) {
-        ok = run_compact(last_lens_.data(), B_, S_);
+        ok = run_compact(last_lens_.data(), B_, S_, last_padded_bits_);
     } else {
         last_classified_ = false;
         ok = enqueue(B_, S_, last_has_mask_);

@@ -61,8 +61,9 @@ class Model {
     bool forward_device(const int* d_ids, const int* d_seg, const int* d_mask, int B, int S);
     // Unpadded forward: only the first h_lens[b] >= 1 tokens of every sequence are computed (as if
     // the attention mask were 1 on exactly those).  Pooled output and the sequence output on
-    // the valid positions equal forward_device's bit for bit; the padding positions of the
-    // sequence output are zero.  h_lens is host memory.  Asynchronous after the metadata upload.
+    // the valid positions equal forward_device's, bit for bit unless short launches regroup sums by their
+    // row count (split_k); the padding positions of the sequence output are zero.  h_lens is host memory.  Asynchronous
+    // after the metadata upload.
     bool forward_device_lens(const int* d_ids, const int* d_seg, const int* h_lens, int B, int S);
     // softmax(pooled @ classifier_kernel + bias) for the last forward -> cls_probs().
     bool classify();
@@ -102,7 +103,8 @@ class Model {
     int parts_for(long rows, int B) const;             // parts a pass over that many token rows is cut into
     bool enqueue(int B, int S, bool has_mask);         // the launch sequence (one or two parts)
     bool enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp = nullptr);
-    bool run_compact(const int* h_lens, int B, int S);
+    // padded_bits: the sums are grouped as in the padded pass of the batch, else as the computed rows ask for
+    bool run_compact(const int* h_lens, int B, int S, bool padded_bits);
     bool rerun_last();                                 // the last pass once more, eagerly, from the inputs still on the device
     bool mark(int phase);                              // profiling: event before a launch
 
@@ -152,8 +154,9 @@ class Model {
     void *ctxc_ = nullptr, *hc_ = nullptr;         // attention context / FFN activation of those rows
     bool first_only_ = false;                      // the pass being enqueued (and the last one run) is of that kind
     bool last_compact_ = false;
-    // Rows on which split counts and skinny tiles, which regroup sums, are decided: those of the pass.
-    // 0: nothing is regrouped (split_k off, or a pass in parts).
+    bool last_padded_bits_ = false;
+    // Rows on which split counts and skinny tiles, which regroup sums, are decided: those of the pass, or of the padded pass
+    // whose bits it has to give.  0: nothing is regrouped (split_k off, or a pass in parts).
     int order_rows_ = 0;
     int cur_attn_ = kAttnPerHead;   // attention kernel of the pass being enqueued (decided on the whole batch)
     int B_ = 0, S_ = 0;

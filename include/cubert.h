@@ -129,16 +129,19 @@ int cubert_sync(void* model);
  * longest line, utils.py:3-13): only the first lengths[b] (1..seq_length) tokens of
  * every sequence are computed, as if the attention mask were 1 on exactly those.
  * d_words / d_token_types are device [B, S] as above; `lengths` is HOST memory [B].
- * The pooled output and the sequence output on the valid positions are bit-identical
- * to cubert_forward_device with the corresponding prefix mask; the sequence output is
- * zero on the padding positions (the padded pass computes values there that no caller
- * uses).  The host-input entry points take this path by themselves when every mask row
+ * The pooled output and the sequence output on the valid positions are those of
+ * cubert_forward_device with the corresponding prefix mask: bit for bit with
+ * CUBERT_SPLIT_K=0 and where neither pass is short; below about 8192 computed rows split K
+ * and the kernels for few rows group float32 sums by the rows a pass computes, and the two
+ * agree to the rounding of the precision.  The sequence output is zero on the padding
+ * positions (the padded pass computes values there that no caller uses).  The host-input entry points take this path by themselves when every mask row
  * is a non-empty prefix of ones and
  *   CUBERT_VARLEN=1:      always (Cuda_Bert, Cuda_Classify, Cuda_Inference, cubert_encode);
  *   CUBERT_VARLEN unset:  only for calls that return no sequence output (Cuda_Bert,
  *                         Cuda_Classify, cubert_encode with seq_out == NULL), on batches above
  *                         the hipGraph limit with at least 5 % padding -- the results such a
- *                         call returns are bit-identical either way;
+ *                         call returns are bit-identical either way (its sums are grouped as
+ *                         the padded pass groups them);
  *   CUBERT_VARLEN=0:      never.
  * Returns 0 on success. */
 int cubert_forward_device_lens(void* model, const int* d_words, const int* d_token_types,

@@ -1,5 +1,5 @@
 """Bit identity at the default settings, where split K and the skinny tiles regroup sums by a row count: the routes of one
-batch that compute fewer rows (the first tokens alone in the last layer) decide on the same rows.
+batch that compute fewer rows (the first tokens alone in the last layer, the valid tokens alone) decide on the same rows.
 Two layers of BERT-base, BERT-large and a small model; the row counts lie on both sides of the changes of plan (float32,
 BERT-base, 1300 rows and small, 2560: skinny tiles that do not split K)."""
 import numpy as np
@@ -51,4 +51,18 @@ def test_pooled_only_call_has_the_bits_of_the_full_pass(pb, models, size, precis
     ids, seg, _ = synth.make_inputs(B, S, [S] * B, vocab=500, seed=B)
     full, _, cls_full = pb.encode(m, ids, seg, None, want_seq=True, want_cls=True)
     pooled, _, cls = pb.encode(m, ids, seg, None, want_cls=True)
+    assert np.array_equal(pooled, full) and np.array_equal(cls, cls_full)
+
+
+@pytest.mark.parametrize("B,S,low,high", [(42, 200, 20, 60), (60, 150, 20, 150), (64, 150, 60, 150), (64, 200, 20, 70), (64, 512, 32, 120),
+                                          (64, 512, 8, 20)])
+@pytest.mark.parametrize("size,precision", SIZES)
+def test_padding_skipped_unasked_leaves_no_trace(pb, models, size, precision, B, S, low, high):
+    """More than 8192 tokens with padding: a pooled-only call computes the valid tokens alone, one that returns the sequence
+    output the padded batch."""
+    m = models(size, precision)
+    lens = np.random.default_rng(B + S).integers(low, high + 1, size=B)
+    ids, seg, mask = synth.make_inputs(B, S, lens, vocab=500, seed=S, prune=False)
+    full, _, cls_full = pb.encode(m, ids, seg, mask, want_seq=True, want_cls=True)
+    pooled, _, cls = pb.encode(m, ids, seg, mask, want_cls=True)
     assert np.array_equal(pooled, full) and np.array_equal(cls, cls_full)
