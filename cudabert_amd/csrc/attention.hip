@@ -719,8 +719,8 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
                 }
             }
         }
-        // the next round's memory-to-LDS loads stay behind this round's LDS reads
-        asm volatile("" ::: "memory");
+        // the next round's memory-to-LDS loads stay behind this round's LDS reads, and those are done
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 
     // ---- the partials meet: wave w's context as [query][feature] over its V space ----

@@ -317,7 +317,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void attention_f32_split_
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const bool plain = __ballot(reinterpret_cast<const float*>(myM)[l32] == 0.0f) == ~0ull;
         key_block([&](int kk, int p) { return kf[kk][p]; }, qf, myV, vpiece, myM, plain, g, scale_log2e, o, run_max, run_sum);
-        asm volatile("" ::: "memory");                   // the next round's memory-to-LDS loads stay behind this round's reads
+        // the next round's memory-to-LDS loads stay behind this round's LDS reads, and those are done
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 
     // ---- the partials meet: wave w's context as [query][feature] over its V space ----
