@@ -81,6 +81,7 @@ __global__ __launch_bounds__(256, 3) void gemm_bf16_t128_kernel(const GemmDev p)
 
 template <int OUT>
 bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
+    if (!epilogue_gives(OUT, epi)) { set_error("gemm: unknown epilogue"); return false; }
     const dim3 grid(d.tiles_n * d.tiles_m, d.splits), block(256);
     switch (epi) {
         case kEpiBias: hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBias>), grid, block, 0, stream, d); break;
@@ -89,17 +90,11 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiQKV: hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiQKV>), grid, block, 0, stream, d); break;
         case kEpiQKVMap: hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiQKVMap>), grid, block, 0, stream, d); break;
         case kEpiBiasRes:
-            if constexpr (OUT == kF32) {
-                hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+            break;
         case kEpiBiasGeluUnits:
-            if constexpr (OUT == kBF16) {
-                hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kBF16) hipLaunchKernelGGL((gemm_bf16_t128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+            break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());

@@ -239,6 +239,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256x128_deep_kernel(const Gemm
 
 template <int OUT>
 bool launch_epi_half_deep(const GemmDev& d, int epi, hipStream_t stream) {
+    if (!epilogue_gives(OUT, epi)) { set_error("gemm: unknown epilogue"); return false; }
     const dim3 grid(d.tiles_n * d.tiles_m), block(256);
     switch (epi) {
         case kEpiBias: hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBias>), grid, block, 0, stream, d); break;
@@ -247,17 +248,11 @@ bool launch_epi_half_deep(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiQKV: hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiQKV>), grid, block, 0, stream, d); break;
         case kEpiQKVMap: hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiQKVMap>), grid, block, 0, stream, d); break;
         case kEpiBiasRes:
-            if constexpr (OUT == kF32) {
-                hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+            break;
         case kEpiBiasGeluUnits:
-            if constexpr (OUT == kBF16) {
-                hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kBF16) hipLaunchKernelGGL((gemm_bf16_t256x128_deep_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+            break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());
@@ -270,6 +265,7 @@ dim3 ln_grid(const GemmDev& d) { return dim3(8 * d.tiles_n * ((d.tiles_m + 7) / 
 
 template <int OUT>
 bool launch_epi_half(const GemmDev& d, int epi, hipStream_t stream) {
+    if (!epilogue_gives(OUT, epi)) { set_error("gemm: unknown epilogue"); return false; }
     const dim3 grid(d.tiles_n * d.tiles_m), block(256);
     switch (epi) {
         case kEpiBias: hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBias>), grid, block, 0, stream, d); break;
@@ -278,25 +274,14 @@ bool launch_epi_half(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiQKV: hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiQKV>), grid, block, 0, stream, d); break;
         case kEpiQKVMap: hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiQKVMap>), grid, block, 0, stream, d); break;
         case kEpiBiasRes:
-            if constexpr (OUT == kF32) {
-                hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+            break;
         case kEpiBiasResLN:
-            if constexpr (OUT == kF32) {
-                if (epi == kEpiBiasResLN) {
-                    hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasResLN>), ln_grid(d), block, 0, stream, d);
-                    break;
-                }
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasResLN>), ln_grid(d), block, 0, stream, d);
+            break;
         case kEpiBiasGeluUnits:
-            if constexpr (OUT == kBF16) {
-                hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kBF16) hipLaunchKernelGGL((gemm_bf16_t256x128_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+            break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());
@@ -305,6 +290,7 @@ bool launch_epi_half(const GemmDev& d, int epi, hipStream_t stream) {
 
 template <int OUT>
 bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
+    if (!epilogue_gives(OUT, epi)) { set_error("gemm: unknown epilogue"); return false; }
     const dim3 grid(d.tiles_n * d.tiles_m), block(256);
     switch (epi) {
         case kEpiBias: hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBias>), grid, block, 0, stream, d); break;
@@ -313,25 +299,14 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
         case kEpiQKV: hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiQKV>), grid, block, 0, stream, d); break;
         case kEpiQKVMap: hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiQKVMap>), grid, block, 0, stream, d); break;
         case kEpiBiasRes:
-            if constexpr (OUT == kF32) {
-                hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasRes>), grid, block, 0, stream, d);
+            break;
         case kEpiBiasResLN:
-            if constexpr (OUT == kF32) {
-                if (epi == kEpiBiasResLN) {
-                    hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasResLN>), ln_grid(d), block, 0, stream, d);
-                    break;
-                }
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kF32) hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasResLN>), ln_grid(d), block, 0, stream, d);
+            break;
         case kEpiBiasGeluUnits:
-            if constexpr (OUT == kBF16) {
-                hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
-                break;
-            }
-            [[fallthrough]];
+            if constexpr (OUT == kBF16) hipLaunchKernelGGL((gemm_bf16_t256_kernel<OUT, kEpiBiasGeluUnits>), grid, block, 0, stream, d);
+            break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());

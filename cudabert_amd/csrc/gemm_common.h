@@ -41,6 +41,11 @@ struct GemmDev {
     int ln_bands;
 };
 
+// Results an epilogue exists for: residual and LayerNorm give float32, the units layout is bf16.
+constexpr bool epilogue_gives(int out, int epi) {
+    return epi == kEpiBiasRes || epi == kEpiBiasResLN ? out == kF32 : epi != kEpiBiasGeluUnits || out == kBF16;
+}
+
 // Where a lane's MFMA fragment (k-phase 0) of rows row0 .. row0 + 31 lies in a tile's LDS image (64 bytes per row), and what
 // leads to k-phase 1 (xor).
 __device__ __forceinline__ int frag_base(int row0, int units, int l32, int g) {
