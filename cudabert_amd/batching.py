@@ -24,16 +24,28 @@ What is kept, because it determines the (batch, seq) shapes the engine sees:
 Differences: ready batches of a bucket leave first-in first-out (the reference
 pops the newest one while ranking buckets by their oldest, engine.py:58-61); a
 line whose mask has no 1 at all has length 1 rather than 512; at the end of the
-input the lines left in the buckets are batched across bucket edges instead of
-bucket by bucket (``QueueManager.merge_rest``).
+input the lines left in neighbouring buckets share a batch where that costs less
+than a batch for each (``QueueManager.merge_rest``).
 """
 from __future__ import annotations
 
 import sys
+from bisect import bisect_left, bisect_right
 from collections import deque
+from itertools import accumulate
 from typing import Callable, Iterable, List, Optional, Sequence
 
 import numpy as np
+
+
+# What a batch costs whatever it holds, in tokens of padding that a pass computes in the same time.  Pooled-only calls on MI355X,
+# lines merged by cost with 360 / 1024 / 1536 tokens, one batch per bucket and batches filled whatever the padding beside them:
+#   2000 lines of 8 to 200 tokens  BERT-large bf16  204.8 / 193.8 / 193.4 ms, 291.8 and 190.9   fp32  745 / 736 / 733 ms, 862 and 726
+#   300 lines of 8 to 200          BERT-large bf16   40.3 /  35.7 /  33.3 ms, 104.4 and 28.8    fp32  126 / 115 / 113 ms, 229 and 99
+#   100 lines of 8 to 64           BERT-large bf16   7.37 /  7.32 /  6.24 ms, 13.4 and 6.28     fp32  19.9 / 20.0 / 22.1 ms, 29.6 and 22.1
+# From 1536 on the model whose tokens cost most (BERT-large fp32) loses; filled whatever the padding, 15 lines of 20 tokens and one
+# of 512 take 7.6 ms in bf16 and 24.6 in fp32 where a batch for each length takes 2.8 and 6.3.
+PASS_TOKENS = 1024
 
 
 def generate_splits(max_seq_length: int, start_split: int = 50, end_split: int = 180, split_size: int = 2) -> List[int]:
@@ -114,7 +126,11 @@ class BatchContainer:
             self.temp = []
 
     def emit(self, lines: List[TaggedLine]):
-        self.prepare.append(BatchPacked(lines, optimize_batch(lines)))
+        """Lines in input order; ready batches stay in the order of their first lines."""
+        at = len(self.prepare)
+        while at and self.prepare[at - 1].lines_list[0].num_line > lines[0].num_line:
+            at -= 1
+        self.prepare.insert(at, BatchPacked(lines, optimize_batch(lines)))
 
     def force_enqueue(self):
         self._batch()
@@ -134,6 +150,7 @@ class QueueManager:
         if len(seq_length_split) < 2 or any(b <= a for a, b in zip(seq_length_split, seq_length_split[1:])):
             raise ValueError("bucket edges must be strictly increasing")
         self.boardlines = list(seq_length_split)
+        self.batchsize = batchsize
         self.containers = [BatchContainer(a, b, batchsize) for a, b in zip(self.boardlines, self.boardlines[1:])]
 
     def put(self, line: TaggedLine):
@@ -150,19 +167,31 @@ class QueueManager:
             c.force_enqueue()
 
     def merge_rest(self):
-        """End of the input: the lines still waiting, shortest bucket first, in batches of batch_size lines that run across
-        bucket edges.  (A bucket is a few tokens wide and is left with a few dozen lines; the device is as good as idle on such
-        a batch, and a batch of neighbouring lengths costs no more padding than the engine skips.  2000 lines of 8 to 200
-        tokens, BERT-large bf16: 72 batches in 290 ms, 23 batches in 187 ms.)"""
-        rest: List[TaggedLine] = []
-        for c in self.containers:
-            rest.extend(c.temp)
-            c.temp.clear()
-            while len(rest) >= c.batchsize:
-                c.emit(rest[:c.batchsize])
-                rest = rest[c.batchsize:]
-        if rest:
-            self.containers[-1].emit(rest)
+        """End of the input: the lines still waiting, in order of length, in the batches that cost least, where a batch costs its
+        tokens, padding included, and ``PASS_TOKENS``, and ends at a bucket edge or full.  (A bucket is a few tokens wide and is
+        left with a few dozen lines, a batch on which the device is as good as idle.  Padding counts in full: the engine skips
+        it in some calls only, and the callback may be any.)  Never more batches than one per bucket, and never more tokens
+        than ``PASS_TOKENS`` for each batch less."""
+        rests = [c for c in self.containers if c.temp]
+        lines = sorted((l for c in rests for l in c.temp), key=lambda l: l.length)      # bucket after bucket
+        edges = list(accumulate(len(c.temp) for c in rests))
+        best = [(0, 0)] + [None] * len(lines)         # the first n lines: least cost, and where their last batch begins
+        for begin in range(len(lines)):
+            if best[begin] is None:
+                continue
+            full = begin + self.batchsize
+            ends = [e for e in edges[bisect_right(edges, begin):] if e < full]
+            for end in ends + [min(full, len(lines))]:
+                cost = best[begin][0] + (end - begin) * lines[end - 1].length + PASS_TOKENS
+                if best[end] is None or cost < best[end][0]:
+                    best[end] = (cost, begin)
+        end = len(lines)
+        while end:
+            begin = best[end][1]
+            rests[bisect_left(edges, end)].emit(sorted(lines[begin:end], key=lambda l: l.num_line))
+            end = begin
+        for c in rests:
+            c.temp = []
 
     def ready(self) -> int:
         return sum(len(c.prepare) for c in self.containers)

@@ -51,6 +51,58 @@ def test_bucket_routing_and_emission_order():
         qm.put(line(9, 41, total=48))
 
 
+def rest_batches(lens, max_seq, batch_size, finish, drain_first=True):
+    """The batches handed out for lines of these lengths after the last one has been put."""
+    qm = Bt.QueueManager(Bt.generate_splits(max_seq), batch_size)
+    for i, n in enumerate(lens):
+        qm.put(line(i, int(n), total=max_seq))
+        while drain_first and qm.get() is not None:
+            pass
+    getattr(qm, finish)()
+    out = []
+    while (b := qm.get()) is not None:
+        out.append(b)
+    assert not any(c.temp for c in qm.containers)
+    return out
+
+
+def tokens(batches):
+    return sum(b.tensor[0].size for b in batches)
+
+
+@pytest.mark.parametrize("lens", [[8] * 39 + [200], [20] * 15 + [512], [10] * 127 + [512], [512] + [10] * 127])
+def test_rest_keeps_a_few_long_lines_apart(lens):
+    """Lines far apart in length: a common batch would compute up to 37 times the tokens."""
+    assert [b.tensor[0].shape for b in rest_batches(lens, 512, 128, "merge_rest")] \
+        == [b.tensor[0].shape for b in rest_batches(lens, 512, 128, "force_enqueue")]
+
+
+@pytest.mark.parametrize("kind", ["uniform", "skewed", "narrow", "two_lengths"])
+@pytest.mark.parametrize("n,batch_size", [(1, 128), (40, 7), (300, 128), (1500, 128), (700, 1)])
+def test_rest_never_costs_more_than_bucket_by_bucket(kind, n, batch_size):
+    rng = np.random.default_rng(n)
+    lens = {"uniform": rng.integers(1, 201, n), "skewed": np.clip(rng.lognormal(3.4, 0.8, n), 1, 200).astype(int),
+            "narrow": rng.integers(100, 131, n), "two_lengths": rng.choice([9, 190], n)}[kind]
+    rest, by_bucket = rest_batches(lens, 200, batch_size, "merge_rest"), rest_batches(lens, 200, batch_size, "force_enqueue")
+    assert sorted(l.num_line for b in rest for l in b.lines_list) == sorted(l.num_line for b in by_bucket for l in b.lines_list)
+    assert all(len(b.lines_list) <= batch_size for b in rest)
+    saved = len(by_bucket) - len(rest)
+    assert saved >= 0 and tokens(rest) - tokens(by_bucket) <= saved * Bt.PASS_TOKENS
+    if kind == "uniform" and n == 1500 and batch_size == 128:
+        assert len(rest) * 3 < len(by_bucket)
+
+
+def test_rest_batches_leave_in_the_order_of_their_first_lines():
+    lens = [60, 9, 61, 150, 55, 8, 199, 57, 30, 151, 90, 9, 12, 92] + [9] * 4
+    for drain_first in (True, False):              # False: full batches of the same buckets are still waiting
+        batches = rest_batches(lens, 200, 4, "merge_rest", drain_first)
+        first = [b.lines_list[0].num_line for b in batches]
+        assert first == sorted(first)
+        assert all(min(l.num_line for l in b.lines_list) == f for b, f in zip(batches, first))
+        if not drain_first:
+            assert sorted(l.num_line for b in batches for l in b.lines_list) == list(range(len(lens)))
+
+
 def test_ordered_writer_rejects_duplicates():
     got = []
     w = Bt.OrderedWriter(lambda l: got.append(l.num_line))
