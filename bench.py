@@ -31,6 +31,9 @@ sys.path.insert(0, ROOT)
 # fp32: a float32 product is six bf16 matrix products (split operands); the float32 MFMA would reach 157.3
 PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 2500.0 / 6}
 PEAK_HBM_GBS = 8000.0
+# Operand layouts of the bf16 FFN-in GEMM as the model launches it above 128 rows (include/cubert.h): X and W packed, W and Y
+# in the units form.
+FFN_IN_FLAGS = 1 | 2 | 4 | 1 << 24 | 1 << 25
 
 
 def measured_traffic(precision, N, I, H):
@@ -52,8 +55,9 @@ def measured_traffic(precision, N, I, H):
 
 def roofline_leg(torch, pybert, lib, prec, precision, N, I, H):
     # ---- roofline of the dominant kernel: the FFN-in GEMM (bias+GELU epilogue) ----
-    # Same kind of launch as in the model: in bf16 mode all three matrices are in the packed operand layout, in fp32
-    # mode in the split one, three bf16 planes per element (their contents are random, only the layout matters for timing).
+    # Same kind of launch as in the model above 128 rows: in bf16 mode X in the packed operand layout, W and Y in its units
+    # form; in fp32 mode all three in the split layout, three bf16 planes per element (their contents are random, only the
+    # layout matters for timing).
     tdt = torch.bfloat16 if prec == pybert.BF16 else torch.float32
     packed = prec == pybert.BF16
     pad, planes = (256, 1) if packed else (32, 3)
@@ -65,7 +69,7 @@ def roofline_leg(torch, pybert, lib, prec, precision, N, I, H):
     Y = torch.empty((rows_x, I * planes), dtype=torch.bfloat16, device="cuda")
     st = torch.cuda.current_stream()
     elt = prec if packed else 2              # CUBERT_F32_SPLIT
-    gflags = (pybert.X_PACKED | pybert.W_PACKED | pybert.Y_PACKED) if packed else 0
+    gflags = FFN_IN_FLAGS if packed else 0
 
     def ffn_in():
         pybert.check(lib.cubert_op_gemm(X.data_ptr(), Wt.data_ptr(), bias.data_ptr(), Y.data_ptr(), N, I, H, H, elt,
@@ -82,7 +86,7 @@ def roofline_leg(torch, pybert, lib, prec, precision, N, I, H):
     k_ms = e0.elapsed_time(e1) / launches
     flops_per_launch = 2.0 * N * H * I
     achieved = flops_per_launch / k_ms / 1e9
-    kname = "gemm_bf16_t256x128_kernel<bf16, bias+GELU>" if precision == "bf16" else "gemm_split_kernel<bias+GELU>"
+    kname = "gemm_bf16_t256x128_kernel<bf16, bias+GELU in units>" if precision == "bf16" else "gemm_split_kernel<bias+GELU>"
     roofline = {"bound": "mfma", "kernel": "%s (FFN-in %dx%dx%d, tile chosen by the library)" % (kname, N, I, H), "achieved": round(achieved, 1), "peak": PEAK_TFLOPS[precision],
                 "unit": "TFLOP/s", "frac": round(achieved / PEAK_TFLOPS[precision], 4),
                 "avg_launch_ms": round(k_ms, 4), "flop_per_launch": flops_per_launch,
@@ -289,7 +293,7 @@ def power_leg(torch, pybert, lib, step, sync, prec, N, I, H):
         def launches():
             for _ in range(40):
                 pybert.check(lib.cubert_op_gemm(X.data_ptr(), Wt.data_ptr(), bias.data_ptr(), Y.data_ptr(), N, I, H, H,
-                                                1, 1, 1, tile, 7 | pflag, st.cuda_stream))
+                                                1, 1, 1, tile, FFN_IN_FLAGS | pflag, st.cuda_stream))
             torch.cuda.synchronize()
         r = ps.measure(launches, 1.2)
         if r:
@@ -472,31 +476,33 @@ def main():
         lib = pybert.lib
         roofline = roofline_leg(torch, pybert, lib, prec, args.precision, N, I, H)
         st = torch.cuda.current_stream()
-        tdt = torch.bfloat16 if prec == pybert.BF16 else torch.float32
         rows = (N + 255) // 256 * 256
-        # residual + LayerNorm as the pass launches it: reads the GEMM result, writes the float32 stream
-        # (+ the packed bf16 copy in bf16 mode)
+        # LayerNorm as the pass launches it where it is a kernel of its own: reads the GEMM result, which holds the residual,
+        # writes the float32 stream and the next GEMM's operand (bf16 packed, or float32 split)
         x = torch.randn((N, H), device="cuda")
         y = torch.randn((N, H), device="cuda")
         g, b = torch.ones(H, device="cuda"), torch.zeros(H, device="cuda")
-        xb = torch.empty((rows, H), dtype=torch.bfloat16, device="cuda")
+        bf16 = prec == pybert.BF16
+        planes = 1 if bf16 else 3
+        xb = torch.empty((rows, H * planes), dtype=torch.bfloat16, device="cuda")
         for _ in range(20):
             pybert.check(lib.cubert_op_add_layernorm(x.data_ptr(), y.data_ptr(), 0, g.data_ptr(), b.data_ptr(),
-                                                     xb.data_ptr() if prec == pybert.BF16 else None, N, H,
-                                                     (4 if prec == pybert.BF16 else 0) | 16, st.cuda_stream))
-        # fused attention on this configuration's ragged masks
+                                                     xb.data_ptr(), N, H, (4 if bf16 else 64) | 16, st.cuda_stream))
+        # fused attention on this configuration's ragged masks, operands and context in the model's layouts: head-major bf16 with
+        # V like K (transposed beyond 512 positions) and a context in units, or split float32
         Sp = (S + 31) // 32 * 32
-        q = torch.randn((B, A, S, 64), device="cuda").to(tdt)
-        k = torch.randn((B, A, S, 64), device="cuda").to(tdt)
-        vrow = prec == pybert.BF16 and S <= 512       # as in the model: V head-major like k, transposed by the kernel's LDS reads
-        vt = torch.randn((B, A, S, 64) if vrow else (B, A, 64, Sp), device="cuda").to(tdt)
+        vrow = bf16 and S <= 512
+        qshape = (B, A, S, 64) if bf16 else (B, A, Sp, 64 * planes)
+        q = torch.randn(qshape, device="cuda").to(torch.bfloat16)
+        k = torch.randn(qshape, device="cuda").to(torch.bfloat16)
+        vt = torch.randn(qshape if vrow or not bf16 else (B, A, 64, Sp), device="cuda").to(torch.bfloat16)
         madd = np.full((B, Sp), -np.inf, np.float32)
         madd[:, :S] = (1.0 - mask.astype(np.float32)) * -10000.0
         madd = torch.from_numpy(madd).cuda()
-        ctx = torch.empty((rows, H), dtype=tdt, device="cuda")
+        ctx = torch.empty((rows, H * planes), dtype=torch.bfloat16, device="cuda")
         for _ in range(20):
             pybert.check(lib.cubert_op_attention(q.data_ptr(), k.data_ptr(), vt.data_ptr(), madd.data_ptr(), ctx.data_ptr(),
-                                                 B, A, S, 0.125, prec, (4 if prec == pybert.BF16 else 0) | (32 if vrow else 0),
+                                                 B, A, S, 0.125, 1 if bf16 else 2, (1 << 25 if bf16 else 0) | (32 if vrow else 0),
                                                  st.cuda_stream))
         a = torch.empty(64 << 20, dtype=torch.float32, device="cuda")     # 256 MiB read + 256 MiB written
         c = torch.empty_like(a)
