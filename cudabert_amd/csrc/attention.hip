@@ -10,12 +10,13 @@
 // (8*(v/4) + 4*(lane/32) + v%4), so the row maximum and row sum of the softmax
 // are 16 in-register operations plus one exchange with lane ^ 32.  The
 // probabilities stay in registers and feed the second MFMA as its "B" operand
-// (k = key); V is read from a pre-transposed [64, Sp] layout (written by the
-// QKV GEMM epilogue) so that the "A" operand lane (d, g) picks up the keys
-// that match the probability lane's k slots with 8/16-byte loads.  The
-// context comes out transposed too: a lane holds one query and four
-// consecutive head features per accumulator quad -> vector stores into the
-// row-major [tokens, hidden] context matrix.
+// (k = key); the "A" operand lane (d, g) needs the keys that match the
+// probability lane's k slots of its feature: V comes as rows like K and is
+// transposed by the LDS reads, or (more than 512 positions, or on request)
+// pre-transposed as [64, Sp] by the QKV GEMM's epilogue and is read with
+// 8/16-byte loads.  The context comes out transposed too: a lane holds one
+// query and four consecutive head features per accumulator quad -> vector
+// stores into the next GEMM's operand or a row-major [tokens, hidden] matrix.
 #include <atomic>
 
 #include "kernels.h"
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(1024) void attention_lds_kernel(
 // Bound: the vector ALU's softmax work, and what is resident to hide the loads behind it.  A chunk of 128 keys is 34 KiB of
 // LDS, so a CU holds four workgroups whatever S is (a whole head of S = 512 is 130 KiB: one workgroup, whose waves past a short
 // sequence's end idle while they hold it), and the query blocks of a long sequence spread over CUs.  K and V are read again for
-// every 128 queries, out of the L2.  Measured against one workgroup per (batch, head) with all of K and V staged, 16 heads,
+// every 128 queries, mostly from behind the L2: B=128 S=200 fetches 234 MiB a launch where q, k and v are 150.  Measured against one workgroup per (batch, head) with all of K and V staged, 16 heads,
 // microseconds: B=64 S=512 114 -> 107, B=128 S=300 110 -> 92, B=128 S=200 50.8 -> 48.5, B=128 S=128 31.1 -> 25.9, B=23 S=77
 // 7.4 -> 6.7, B=1 S=512 22.5 -> 12.5; 64 lines of 32 to 512 valid tokens in compact rows (a pass of BERT-large) 9.2 -> 8.5 ms.
 // Up to 64 keys four waves would idle (S = 33: 8.5 -> 9.5), hence NW = ceil(S / 32) there.

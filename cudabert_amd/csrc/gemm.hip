@@ -385,8 +385,9 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 // workgroup that has its CU to itself (a constant plus a cost per half-step of 32 k), and g says how the launch
 // stretches when a CU gets w > 1 workgroups on average: g = 1 + (w - 1 + q) * rho; rho is what one more workgroup on a CU
 // costs relative to a lone one (1: nothing is gained from sharing a CU, the 128 x 128 tile saturates the LDS on its
-// own) and q allows for the uneven hand-out of coarse tiles.  From kPlanSmallRows rows on, and for float32 operands,
-// gemm_pick_tile decides (its costs were measured inside whole forward passes at the power limit) and K is not split.
+// own) and q allows for the uneven hand-out of coarse tiles.  From kPlanSmallRows rows on gemm_pick_tile decides (its costs were
+// measured inside whole forward passes at the power limit) and K is split only where 64 x 64 tiles would not give 512
+// workgroups, which takes fewer output features than any BERT has.
 constexpr int kPlanSmallRows = 6144;
 
 namespace {
@@ -424,9 +425,14 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         }
     }
     // The skinny tile (32 features x 64 tokens) wins while every workgroup has a CU to itself; a second one on a CU competes for
-    // the same loads.  Microseconds, cold weights, skinny against the best of the others: 17 rows, QKV / FFN-in / FFN-out of
-    // BERT-base 5.0 / 5.0 / 4.9 against 6.1 / 6.0 / 5.3, of BERT-large 6.3 / 7.8 / 5.8 against 6.8 / 8.4 / 6.3; 128 rows of
-    // BERT-base 5.5 / 5.8 / 5.8 against 6.4 / 6.5 / 6.3; 200 rows (288 workgroups) 7.8 / 8.1 against 6.5 / 6.7.
+    // the same loads.  Microseconds, cold weights, skinny against the best of the others: 17 rows, QKV / FFN-in of BERT-base
+    // 5.0 / 5.0 against 6.1 / 6.0, of BERT-large 6.3 / 7.8 against 6.8 / 8.4; 128 rows of BERT-base 5.5 / 5.8 against 6.4 / 6.5;
+    // 200 rows (288 workgroups) 7.8 / 8.1 against 6.5 / 6.7.
+    // attn-out and FFN-out stay with the 64 tile at every size of the model: by this estimate a finer split of it costs less
+    // (17 rows, FFN-out of BERT-base: 16 parts 4.4, skinny tile with 8 parts 5.0).  Measured with the LayerNorm that adds the
+    // parts, each tile with its best split, attn-out / FFN-out, 64 tile against skinny: 17 rows of BERT-base 8.8 / 10.3
+    // against 8.9 / 10.1, of BERT-large 9.1 / 11.4 against 9.2 / 11.0; 128 rows 9.8 / 12.1 against 9.9 / 11.1 and 10.3 / 13.5
+    // against 10.5 / 13.3: level on attn-out, up to a microsecond less on FFN-out that the estimate does not see.
     for (int sp = min_splits; order == kOrderAny && sp <= max_splits && sp <= 16; sp *= 2) {
         if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
         if ((long)((M + 63) / 64) * ((N + 31) / 32) * sp > 256) break;
@@ -536,7 +542,7 @@ GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {
-            // float32 operands: the rule the short batches were tuned with (64 x 64 tiles, at most 512 workgroups)
+            // many rows and few features, or a K that plan_small's tiles do not take: at most 512 workgroups of 64 x 64 tiles
             const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
             int sp = 1;
             while (sp * 2 <= max_splits && tiles * sp < 512 && K / (sp * 2) >= 256) sp *= 2;

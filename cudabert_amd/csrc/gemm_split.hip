@@ -5,7 +5,8 @@
 // (gemm_split_128_loop.inc, gemm_split_256x128_loop.inc; pipeline and register plan in gen_gemm_asm.py).
 //
 // Bound: the matrix pipe at the socket's power limit.  9800 x 4096 x 1024 with GELU: 377 us, 218 TFLOP/s, i.e. 1.31 PFLOP/s of
-// bf16 products (a large bf16 product reaches 1.28 on this card), against 668 us, 123 TFLOP/s with the float32 MFMA, whose
+// bf16 products; 25600 x 4096 x 1024 without it 1.43 at 1400 W of 1400 (a bf16 product of 8192^3 reaches 1.44 there: 0.97 pJ per
+// operation both, where a bf16 FFN-in, whose fragments serve one product instead of two, spends 1.35), against 668 us, 123 TFLOP/s with the float32 MFMA, whose
 // peak is 157; 19600 x 3072 x 1024: 535 us against 942.  Error against float64, root mean square of the result: 2.7e-7 at
 // K = 1024 and 8.0e-7 at K = 4096, with the float32 MFMA 3.1e-7 and 9.1e-7 (fewer, larger accumulation steps).
 #include "gemm_common.h"

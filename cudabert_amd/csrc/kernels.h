@@ -42,7 +42,9 @@ constexpr int kTile256x128Deep = 385; // ... of the 256 x 128 kernel with one wo
 constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 kernel (bf16, three workgroups per CU, splits K)
 
 constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
-constexpr int kTileSkinny22 = 98;     // ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results)
+// ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results; in bf16 the model's
+// plans take 32 x 64 alone, for QKV and FFN-in: the 64 x 64 tile and float32 results are there for callers that ask for them)
+constexpr int kTileSkinny22 = 98;
 constexpr int kSkinnyMaxRows = 128;   // rows up to which QKV and FFN-in of the model may take a skinny tile in bf16 (engine.cc)
 
 // How a launch groups the sums over k.  All kernels share one order (per split count) but the skinny tiles, whose four waves

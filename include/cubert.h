@@ -99,7 +99,8 @@ const char* cubert_last_error(void);
 
 typedef struct cubert_config {
     int hidden, layers, heads, intermediate; /* head dim (hidden/heads) must be 64 */
-    int precision;                           /* 0 = float32, 1 = bfloat16 operands / float32 accumulate */
+    int precision;                           /* 0 = float32 (Linear kernels and their operands take 6 bytes per element of
+                                                device memory: three bf16 planes), 1 = bfloat16 operands / float32 accumulate */
     int graph_max_tokens;                    /* hipGraph replay for batches up to this many tokens; 0 = off */
 } cubert_config;
 
@@ -206,7 +207,8 @@ long cubert_capacity_tokens(void* model);
  * multiple of 16; Y is float32 row-major, or (GELU epilogue) split, out_elt 2.  fp32 mode runs on this. */
 #define CUBERT_F32_SPLIT 2
 /* cubert_op_attention with CUBERT_V_ROWMAJOR: which kernel.  0 (no flag) = by batch size; 1 = one workgroup per
- * (batch, head); 2 = one workgroup per (batch, head, 32 queries) whose four waves share the keys (short batches).
+ * (batch, head, 128 queries), a wave walks all keys; 2 = one workgroup per (batch, head, 32 queries) whose four waves share
+ * the keys (short batches).
  * elt = CUBERT_F32_SPLIT: 1 = one workgroup per (batch, head, 128 queries); 2 as above; 3 = the same with eight waves. */
 #define CUBERT_ATTN_VARIANT(n) (((n) & 3) << 20)
 /* Split K (cubert_op_gemm, epilogue 0, float32 Y): n workgroups share a tile, each reduces 1/n of K

@@ -272,7 +272,7 @@ def test_layernorm_epilogue_timeout_is_recovered_not_fatal(pb, base_ckpt, monkey
 
 def test_cfg4_large_b64_s512_skewed(pb, large_ckpt):
     """BERT-large, batch 64, seq 512, 70 % short / 30 % long sequences, bf16: the attention kernel
-    with 1024-thread workgroups and the whole head in LDS over 24 layers.  The longest and the
+    that walks a head's keys in chunks of 128, four chunks, over 24 layers.  The longest and the
     shortest sequence against the oracle (padded and unpadded pass), and the size-independent
     properties on the full batch."""
     D = W.LARGE

@@ -12,7 +12,7 @@ F32, BF16 = 0, 1
 V_ROWMAJOR = 32          # CUBERT_V_ROWMAJOR
 
 
-def ATTN_VARIANT(n):      # CUBERT_ATTN_VARIANT: 1 = one workgroup per (batch, head), 2 = the waves of a workgroup share the keys
+def ATTN_VARIANT(n):      # CUBERT_ATTN_VARIANT: 1 = a wave walks all keys of its queries, 2 = the waves of a workgroup share the keys
     return (n & 3) << 20
 
 
