@@ -24,22 +24,28 @@ struct GemmDev {
     int M, N, K, ldx;
     int S, Sp, heads, hidden;
     int tiles_n, tiles_m;
-    int x_packed, w_packed, y_packed;     // operand / result in the packed or units layout (common.h)
-    int x_units, w_units, y_units;        // ... in the units layout
+    // one word: see the static_assert below
+    unsigned x_packed : 1, w_packed : 1, y_packed : 1;   // operand / result in the packed or units layout (common.h)
+    unsigned x_units : 1, w_units : 1, y_units : 1;      // ... in the units layout
+    unsigned v_rowmajor : 1;              // QKV epilogue: V is stored like q / k instead of transposed
+    unsigned ln_xb_packed : 1;            // ln_xb is in the packed layout
     int xn_parts;                         // how the XCDs divide the tile grid (tile_of_block)
     const int* rowmap;                    // QKV epilogue: row m -> token b * S + s (nullptr: m itself)
-    int v_rowmajor;                       // QKV epilogue: V is stored like q / k instead of transposed
     const float* R;                       // kEpiBiasRes: [M, N] float32 row-major, added to the result
     int splits;                           // split K: blockIdx.y owns a K range, results go to Y + y * M * N (f32)
     // kEpiBiasResLN: LayerNorm in the epilogue (gemm_epilogue_ln)
     const float* ln_gamma;
     const float* ln_beta;
     unsigned char* ln_xb;                 // bf16 copy of the result (may be null)
-    int ln_xb_packed;
     int* ln_cnt;                          // [0] error flag, [1] poll limit (0: default), [kLnCntFirst + band] arrivals, [.. + ln_bands + band] departures
     unsigned long long* ln_stats;         // [row][2 * tiles_n] (sum, M2 about the slot's mean) as two floats in 64 bits
     int ln_bands;
 };
+// A workgroup reads its arguments from memory, 64 bytes a line, before it can issue its first operand load, and in a pass of
+// short launches that is in the chain of every one of them.  One line of 200 tokens, BERT-large bf16: 1148 us with a word for
+// each flag (216 bytes), 1140 without the units flags (200), 1127 with all flags in one word (176); four lines of 200:
+// 2011 -> 1996 us, one of 512 1504 -> 1483 (216 against 176 bytes).
+static_assert(sizeof(GemmDev) <= 192, "the GEMM argument record fits three lines");
 
 // Results an epilogue exists for: residual and LayerNorm give float32, the units layout is bf16.
 constexpr bool epilogue_gives(int out, int epi) {
