@@ -117,8 +117,6 @@ template <int CTRL>
 __device__ __forceinline__ float ln_dpp_lanes(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
-// Sum over the 32 lanes that share lane / 32; every lane gets the same bits (the additions are
-// pairwise and commutative).
 // v combined with the value of the lane 32 further (or back): gfx950's v_permlane32_swap exchanges the upper half of
 // one register with the lower half of another, so of two copies of v one ends up holding v of the lower lane of each
 // pair in both halves and the other v of the upper lane; sum and maximum commute, so the result has the bits of
@@ -162,13 +160,23 @@ __device__ __forceinline__ float half_swap_max(float v) {
     half_swap(a, b);
     return fmaxf(a, b);
 }
+// Sum over the 32 lanes that share lane / 32; every lane gets the same bits (the additions are
+// pairwise and commutative).  The pairs: lanes 8, 4, 2, 16 and last 1 apart.  The GEMM epilogue that normalises
+// holds a row in the MFMA accumulator layout, where quad 8 i + 2 qd + g of a slot is block i, group qd of lane half g: with the
+// neighbours last it adds a lane's sixteen quads in registers and crosses lanes once (ln_tree16, then half_swap_sum).
 __device__ __forceinline__ float ln_half_wave_sum(float v) {
-    v += ln_dpp_lanes<0xB1>(v);       // quad_perm [1,0,3,2]: lane ^ 1
-    v += ln_dpp_lanes<0x4E>(v);       // quad_perm [2,3,0,1]: lane ^ 2
-    v += ln_dpp_lanes<0x141>(v);      // row_half_mirror: the other quad of 8 lanes
-    v += ln_dpp_lanes<0x140>(v);      // row_mirror: the other 8 of 16 lanes
+    v += ln_dpp_lanes<0x128>(v);      // row_ror 8: lane ^ 8
+    v += ln_dpp_lanes<0x124>(v);      // row_ror 4: lane ^ 4, now that lanes 8 apart agree
+    v += ln_dpp_lanes<0x122>(v);      // row_ror 2: lane ^ 2
     v += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));   // lane ^ 16
+    v += ln_dpp_lanes<0xB1>(v);       // quad_perm [1,0,3,2]: lane ^ 1
     return v;
+}
+// The same sum, but for the last step, of values one lane holds: v[4 i + qd] is what lane 8 i + 2 qd would hold above.
+__device__ __forceinline__ float ln_tree16(const float (&v)[16]) {
+    const float a = ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
+    const float b = ((v[8] + v[12]) + (v[10] + v[14])) + ((v[9] + v[13]) + (v[11] + v[15]));
+    return a + b;
 }
 __device__ __forceinline__ float ln_sum4(float a, float b, float c, float d) { return (a + b) + (c + d); }
 __device__ __forceinline__ float ln_sumsq4(float a, float b, float c, float d) {
@@ -200,9 +208,13 @@ __device__ __forceinline__ float ln_finalize(float m2, float inv_n) {
 #pragma clang fp contract(off)
     return 1.0f / sqrtf(m2 * inv_n + 1e-12f);
 }
-__device__ __forceinline__ float ln_apply(float x, float mean, float rstd, float gamma, float beta) {
+__device__ __forceinline__ float ln_scale(float x, float mean, float rstd) {
 #pragma clang fp contract(off)
-    return __builtin_fmaf(gamma, (x - mean) * rstd, beta);
+    return (x - mean) * rstd;
+}
+__device__ __forceinline__ float ln_affine(float z, float gamma, float beta) { return __builtin_fmaf(gamma, z, beta); }
+__device__ __forceinline__ float ln_apply(float x, float mean, float rstd, float gamma, float beta) {
+    return ln_affine(ln_scale(x, mean, rstd), gamma, beta);
 }
 #endif
 

@@ -26,7 +26,8 @@ template <int OUT, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
     constexpr int BT = 256;
     // Four stages of 32 KiB: W tile (256 rows x 64 B) then X tile.
-    __shared__ __attribute__((aligned(2048))) unsigned char lds[4 * 32768];
+    // (The LayerNorm epilogue has 512 bytes a wave of its own behind them.)
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[4 * 32768 + (EPI == kEpiBiasResLN ? 2048 : 0)];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -89,10 +90,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_t256_kernel(const GemmDev p) {
 
     // Stages 0 and 1 were last read two barriers ago; the tail of the loop only reads stages
     // 2 and 3, so the first 64 KiB are free for the epilogue's staging while slower waves finish.
-    // (The LayerNorm epilogue keeps its row statistics above them, after a barrier of its own.)
     if constexpr (EPI == kEpiBiasResLN)
         gemm_epilogue_ln<4, 4>(p, acc, n0 + wn * 128, m0 + wm * 128, l32, g, tile_m, 2 * tile_n + wn, lds + wave * 16384,
-                               reinterpret_cast<float*>(lds + 65536 + wave * 1024));
+                               reinterpret_cast<float*>(lds + 4 * 32768 + wave * 512));
     else
         gemm_epilogue<OUT, EPI, 4, 4, false, 8, true>(p, acc, bias, n0 + wn * 128, m0 + wm * 128, l32, g, lds + wave * 16384);
 }
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_t256x128_kernel(const GemmDe
     if constexpr (!gemm_bias_at_readout<OUT, EPI>()) gemm_load_bias<4>(p, n0 + wn * 128, g, bias);
     if constexpr (EPI == kEpiBiasResLN)
         gemm_epilogue_ln<4, 2>(p, acc, n0 + wn * 128, m0 + wm * 64, l32, g, tile_m, 2 * tile_n + wn, lds + wave * 16384,
-                               reinterpret_cast<float*>(lds + 65536 + wave * 1024));
+                               reinterpret_cast<float*>(lds + 65536 + wave * 512));
     else
         gemm_epilogue<OUT, EPI, 4, 2, false, 8, true>(p, acc, bias, n0 + wn * 128, m0 + wm * 64, l32, g, lds + wave * 16384);
 }

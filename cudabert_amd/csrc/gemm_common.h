@@ -452,10 +452,9 @@ __device__ __forceinline__ void gemm_epilogue(const GemmDev& p, f32x16_t (&acc)[
 // A workgroup holds 256 of a row's features, so the tiles_n workgroups of one band of rows have to
 // agree on the row statistics.  Every wave (128 features of its rows) publishes (sum, M2 about its own mean)
 // per row in device memory, the workgroup counts itself in on the band's arrival counter, waits until
-// all tiles_n workgroups have, and reads the 2 * tiles_n partial sums of its rows.  The accumulators go
-// through the wave's LDS staging once (whole row segments come out, bias and residual are added to
-// them); the sums go back into the registers the accumulators came from and wait there, in read-out
-// order, until the statistics are known, and are then normalised and stored.
+// all tiles_n workgroups have, and reads the 2 * tiles_n partial sums of its rows.  Bias and residual (which
+// comes through the LDS) are added where the accumulators lie; the sums wait in the same registers until the
+// statistics are known, are normalised there, and leave through the wave's LDS staging as whole row segments.
 //
 // Workgroup order (ln_tile_of_block): XCD x (= workgroup id % 8) owns the bands x, x + 8, ...; the
 // workgroups of a band have consecutive positions on that XCD, i.e. ids 8 apart.  Workgroups are
@@ -473,93 +472,106 @@ __device__ __forceinline__ void ln_tile_of_block(int pid, int tiles_n, int* tn, 
     *tn = idx % tiles_n;
 }
 
-// One trip of the accumulators through the wave's LDS staging block: block column j is written in
-// accumulator order (row = token, chunk swizzled by the row) and read back as whole row segments, lane
-// (rrow, rc) taking features 4 rc .. 4 rc + 3 of row 2 s + rrow in step s; bias and residual are added on
-// the way out and `use(j, s, d)` receives the sums.  The residual rows come in batches of PB steps, the
-// next batch requested before the current one is consumed.
-template <int NBI, int NBJ, int SCHED, typename Use>
-__device__ __forceinline__ void ln_stream_rows(f32x16_t (&acc)[NBI][NBJ], unsigned char* buf, int l32, int g, int rrow, int rc,
-                                               const f32x4_t& bias4, __amdgpu_buffer_rsrc_t r_rsrc, int lane_off, int row_bytes,
-                                               Use use) {
-    constexpr int RB = 512, RPI = 2, NIT = 16, PB = 8;
-    constexpr int NBATCH = NBJ * NIT / PB;
-    f32x4_t res[2][PB];
-    auto fetch_res = [&](int batch, f32x4_t (&r)[PB]) {
+// Residual rows for the first pass: 4 KiB pieces of 32 rows x 32 features (block column j, block i; piece index 4 j + i),
+// memory to LDS into slot i of the wave's buffer, no registers.  16-byte chunk c of row r lies in place c ^ ((r >> 1) & 7) of the
+// row's 128 bytes, so the reads of one chunk from 32 rows spread over the banks.  Rows past the matrix arrive as zeros.
+// The reads of the slot's previous contents are waited for first: the two are not ordered by themselves.
+__device__ __forceinline__ void ln_fetch_residual(const u32x4_t& rsrc, int lds_slot, int off_even, int off_odd, int row_bytes) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int u = 0; u < PB; ++u)      // row 32 j + 2 s (+ rrow) with j * NIT + s = batch * PB + u
-            r[u] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r_rsrc, lane_off + (batch * PB + u) * RPI * row_bytes, 0, 0));
-    };
-    fetch_res(0, res[0]);
-#pragma unroll
-    for (int j = 0; j < NBJ; ++j) {
-#pragma unroll
-        for (int i = 0; i < NBI; ++i)
-#pragma unroll
-            for (int qd = 0; qd < 4; ++qd) {
-                const int fb = (32 * i + 8 * qd + 4 * g) * 4;
-                const f32x4_t v = {acc[i][j][4 * qd], acc[i][j][4 * qd + 1], acc[i][j][4 * qd + 2], acc[i][j][4 * qd + 3]};
-                *reinterpret_cast<f32x4_t*>(buf + l32 * RB + ((((fb >> 4) ^ l32) & 31) << 4)) = v;
-            }
-#pragma unroll
-        for (int s = 0; s < NIT; ++s) {
-            const int batch = (j * NIT + s) / PB;             // compile-time after unrolling
-            if (s % PB == 0 && batch + 1 < NBATCH) fetch_res(batch + 1, res[(batch + 1) & 1]);
-            const int row = s * RPI + rrow;
-            const f32x4_t staged = *reinterpret_cast<const f32x4_t*>(buf + row * RB + (((rc ^ row) & 31) << 4));
-            use(j, s, (staged + bias4) + res[batch & 1][s % PB]);
-            if (s % SCHED == SCHED - 1) __builtin_amdgcn_sched_barrier(0);     // bounds how many steps the scheduler interleaves
-        }
-    }
+    for (int t = 0; t < 4; ++t)         // eight rows each
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :: "s"(lds_slot + 1024 * t), "v"((t & 1 ? off_odd : off_even) + 8 * t * row_bytes), "s"(rsrc)
+                     : "memory", "m0");
 }
 
+// The wave holds 128 features of 32 NBJ rows.  Statistics are formed in the accumulator layout, where a lane owns half of a row's
+// features (its lane ^ 32 the rest): 64 values in registers and one exchange per row, no reductions across lanes.  buf: 16 KiB of
+// LDS of the wave's own, which no load in flight and no other wave touches; bias_buf: room for its 128 bias values.
+// Bound: vector instructions and the way of residual and result to and from memory, with nothing beside them where the CU holds one
+// workgroup.  Sums read out as rows first and reduced across 32 lanes, step by step, took 12.5 us of such a launch (10947 x 1024 x
+// 1024, 256 x 256 tile) before the exchange between workgroups; the whole launch 51.8 -> 42.9 us, with K = 4096 103.9 -> 95.4,
+// 8192 x 768 x 768 with the 256 x 128 tile 29.0 -> 26.2.
 template <int NBI, int NBJ>
 __device__ __forceinline__ void gemm_epilogue_ln(const GemmDev& p, f32x16_t (&acc)[NBI][NBJ], int n_base, int m_base,
                                                  int l32, int g, int band, int slot, unsigned char* buf,
-                                                 float* statbuf) {
-    static_assert(NBI == 4 && NBJ % 2 == 0, "a wave holds 128 features and a multiple of 64 rows");
-    constexpr int RPI = 2;                   // rows one read-out step covers
-    constexpr int NIT = 16;                  // read-out steps per block column of 32 rows
-    constexpr int NP = NBJ * NIT / 32;       // (block column, step) pairs whose row a lane publishes
+                                                 float* bias_buf) {
+    static_assert(NBI == 4, "a wave holds one slot of 128 features");
     const int slots = 2 * p.tiles_n;
     const float invn = 1.0f / (float)p.N;
-    // Residual and result through buffer descriptors: a row's address is one lane offset plus a
-    // wave-uniform row term, rows past M read as zero and are not stored.  (The whole offset goes
+    // Residual and result through buffer descriptors: rows past M read as zero and are not stored.  (The whole offset goes
     // into the lane operand: the descriptor's range check does not look at the scalar offset.)
     const int row_bytes = p.N * 4;
-    const __amdgpu_buffer_rsrc_t r_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.R), 0, p.M * row_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t y_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, p.M * row_bytes, 0x00020000);
 
-    // ---- first pass: row sums of (acc + bias + R) over this wave's 128 features ----
-    float ksum[NP], ksq[NP];
-#pragma unroll
-    for (int t = 0; t < NP; ++t) ksum[t] = ksq[t] = 0.0f;
+    // ---- first pass: acc + bias + R, which stays in the accumulators' registers, and its slot statistics ----
     {
-        const int lane = l32 + 32 * g, rrow = lane >> 5, rc = lane & 31;
-        const int n = n_base + rc * 4;           // this lane's four features on the way out (N % 256 == 0: in range)
-        const f32x4_t bias4 = *reinterpret_cast<const f32x4_t*>(p.bias + n);
-        ln_stream_rows<NBI, NBJ, 4>(acc, buf, l32, g, rrow, rc, bias4, r_rsrc, (m_base + rrow) * row_bytes + n * 4, row_bytes,
-                                 [&](int j, int s, const f32x4_t& d) {
-            float t, q;                                       // the slot's sum and M2 about the slot's mean
-            ln_slot_stats(d[0], d[1], d[2], d[3], true, 0.0078125f, &t, &q);
-            const int pair = j * NIT + s;                     // compile-time after unrolling
-            if (rc == (pair & 31)) { ksum[pair >> 5] = t; ksq[pair >> 5] = q; }
-            // The sums stay in the registers of the accumulators they were made from (block column j
-            // has been staged completely by now): step s of column j in acc[s / 4][j][4 (s % 4) ..].
+#pragma clang fp contract(off)
+        const int lane = l32 + 32 * g;
+        const unsigned long long ra = reinterpret_cast<unsigned long long>(p.R);
+        const u32x4_t r_rsrc = {(unsigned)ra, (unsigned)(ra >> 32) & 0xffffu, (unsigned)(p.M * row_bytes), 0x00020000u};
+        const int lds_buf = __builtin_amdgcn_readfirstlane((int)(size_t)(__attribute__((address_space(3))) unsigned char*)buf);
+        const int off = (m_base + (lane >> 3)) * row_bytes + n_base * 4;
+        const int off_even = off + (((lane & 7) ^ (lane >> 4)) << 4), off_odd = off + (((lane & 7) ^ (4 + (lane >> 4))) << 4);
+        float sums[NBJ], m2s[NBJ];
+        // the bias from the LDS, quad by quad (two addresses a read): sixteen quads in registers are 64 the two-per-CU kernel lacks
+        *reinterpret_cast<u32x2_t*>(bias_buf + 2 * lane) = *reinterpret_cast<const u32x2_t*>(p.bias + n_base + 2 * lane);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[s / 4][j][4 * (s % 4) + e] = d[e];
-            // the selection happens here (left to itself the compiler postpones all of them past the
-            // loop and spills every step's sums until then)
-            asm volatile("" : "+v"(ksum[pair >> 5]), "+v"(ksq[pair >> 5]));
-        });
-        // lane (rrow, rc) publishes the rows of the pairs t * 32 + rc
+        for (int i = 0; i < 4; ++i) ln_fetch_residual(r_rsrc, lds_buf + 4096 * i, off_even + 128 * i, off_odd + 128 * i, row_bytes);
+        const unsigned char* mine = buf + l32 * 128;
+        const int swz = (l32 >> 1) & 7;
 #pragma unroll
-        for (int t = 0; t < NP; ++t) {
-            const int pair = t * 32 + rc;
-            const int mm = m_base + 32 * (pair / NIT) + RPI * (pair % NIT) + rrow;
-            if (mm < p.M) {
-                const unsigned long long bits = (unsigned long long)__builtin_bit_cast(unsigned, ksum[t]) |
-                                                ((unsigned long long)__builtin_bit_cast(unsigned, ksq[t]) << 32);
+        for (int j = 0; j < NBJ; ++j) {
+            float qsum[16];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // younger loads than this piece's: up to three pieces of four
+                const int left = 4 * NBJ - 1 - (4 * j + i);           // compile-time after unrolling
+                if (left >= 3) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+                else if (left == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+                else if (left == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                f32x4_t r[4], bias[4];
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) bias[qd] = *reinterpret_cast<const f32x4_t*>(bias_buf + 32 * i + 8 * qd + 4 * g);
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) r[qd] = *reinterpret_cast<const f32x4_t*>(mine + 4096 * i + (((2 * qd + g) ^ swz) << 4));
+                if (j + 1 < NBJ) {
+                    const int next = (32 * (j + 1)) * row_bytes + 128 * i;
+                    ln_fetch_residual(r_rsrc, lds_buf + 4096 * i, off_even + next, off_odd + next, row_bytes);
+                }
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {
+                    float d[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        d[e] = (acc[i][j][4 * qd + e] + bias[qd][e]) + r[qd][e];
+                        acc[i][j][4 * qd + e] = d[e];
+                    }
+                    qsum[4 * i + qd] = ln_sum4(d[0], d[1], d[2], d[3]);
+                }
+            }
+            const float sum = half_swap_sum(ln_tree16(qsum));
+            const float mu = sum * 0.0078125f;
+            float qsq[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                const int e0 = 4 * (t & 3);
+                qsq[t] = ln_sumsq4(acc[t >> 2][j][e0] - mu, acc[t >> 2][j][e0 + 1] - mu, acc[t >> 2][j][e0 + 2] - mu, acc[t >> 2][j][e0 + 3] - mu);
+            }
+            const float m2 = half_swap_sum(ln_tree16(qsq));
+            const int mm = m_base + 32 * j + l32;
+            sums[j] = sum;
+            m2s[j] = m2;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // (Published at the end: a store counts among the loads in flight that are waited for by number above.)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) {
+            const int mm = m_base + 32 * j + l32;
+            if (g == 0 && mm < p.M) {
+                const unsigned long long bits = (unsigned long long)__builtin_bit_cast(unsigned, sums[j]) |
+                                                ((unsigned long long)__builtin_bit_cast(unsigned, m2s[j]) << 32);
                 __hip_atomic_store(p.ln_stats + (size_t)mm * slots + slot, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
@@ -583,7 +595,7 @@ __device__ __forceinline__ void gemm_epilogue_ln(const GemmDev& p, f32x16_t (&ac
     }
     __syncthreads();
 
-    // What the registers of the accumulators hold now (the sums, in read-out order) has to survive
+    // What the registers of the accumulators hold now (the sums) has to survive
     // the wait in place: the empty statements keep the compiler from moving the values elsewhere.
 #pragma unroll
     for (int i = 0; i < NBI; ++i)
@@ -600,40 +612,35 @@ __device__ __forceinline__ void gemm_epilogue_ln(const GemmDev& p, f32x16_t (&ac
     // The partners' sums are read with cache-bypassing buffer loads (sc0 | sc1), all requested before the
     // first one is used.  A row's slots are contiguous: a load past 2 * tiles_n reads the next row's or,
     // at the end, nothing (zero); those values are not added.
+    float mean[NBJ], rstd[NBJ];
     {
         const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.ln_stats, 0, p.M * slots * 8, 0x00020000);
-        f32x4_t raw[NP][4];
+        f32x4_t raw[NBJ][4];
 #pragma unroll
-        for (int t = 0; t < NP; ++t) {
-            const int pair = t * 32 + rc;
-            const int mm = m_base + 32 * (pair / NIT) + RPI * (pair % NIT) + rrow;
+        for (int j = 0; j < NBJ; ++j)
 #pragma unroll
             for (int c = 0; c < 4; ++c)          // two slots per load; rows past M fall outside the descriptor as well
-                raw[t][c] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, (mm * slots + 2 * c) * 8, 0, 17));
-        }
+                raw[j][c] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((m_base + 32 * j + l32b) * slots + 2 * c) * 8, 0, 17));
 #pragma unroll
-        for (int t = 0; t < NP; ++t) {
-            const int pair = t * 32 + rc;
-            const int rl = 32 * (pair / NIT) + RPI * (pair % NIT) + rrow;     // row within the wave's rows
+        for (int j = 0; j < NBJ; ++j) {
             float sum = 0.0f;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 if (2 * c < slots) {          // a wave-uniform branch; slots is even
-                    sum += raw[t][c][0];
-                    sum += raw[t][c][2];
+                    sum += raw[j][c][0];
+                    sum += raw[j][c][2];
                 }
             }
-            const float mean = ln_row_mean(sum, invn);
+            mean[j] = ln_row_mean(sum, invn);
             float m2 = 0.0f;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 if (2 * c < slots) {
-                    m2 = ln_merge_slot(m2, raw[t][c][0], raw[t][c][1], 128.0f, 0.0078125f, mean);
-                    m2 = ln_merge_slot(m2, raw[t][c][2], raw[t][c][3], 128.0f, 0.0078125f, mean);
+                    m2 = ln_merge_slot(m2, raw[j][c][0], raw[j][c][1], 128.0f, 0.0078125f, mean[j]);
+                    m2 = ln_merge_slot(m2, raw[j][c][2], raw[j][c][3], 128.0f, 0.0078125f, mean[j]);
                 }
             }
-            statbuf[2 * rl] = mean;
-            statbuf[2 * rl + 1] = ln_finalize(m2, invn);
+            rstd[j] = ln_finalize(m2, invn);
         }
     }
     __syncthreads();                                       // every wave holds its statistics: the band can be left
@@ -644,40 +651,49 @@ __device__ __forceinline__ void gemm_epilogue_ln(const GemmDev& p, f32x16_t (&ac
         }
     }
 
-    // ---- second pass: normalise the kept sums and store ----
+    // ---- second pass: (sum - mean) / sigma through the LDS, out as whole row segments with gamma and beta applied ----
+    // In step s of block column j lane (rrow, rc) takes features 4 rc .. + 3 of row 32 j + 2 s + rrow.
     const f32x4_t gamma4 = *reinterpret_cast<const f32x4_t*>(p.ln_gamma + n);
     const f32x4_t beta4 = *reinterpret_cast<const f32x4_t*>(p.ln_beta + n);
     // bf16 copy: row-major, or packed (common.h): block of 256 rows x 64 bytes, chunk c of row r in slot
-    // c ^ ((r >> 2) & 3).  The wave's rows start at a multiple of 64, so with r = m_base + 32 j + 2 s + rrow
-    // the row's block and its swizzle (s >> 1) & 3 are known per step; only the chunk is the lane's.
+    // c ^ ((r >> 2) & 3).  A block column's rows start at a multiple of 32, so its block and, per step, the swizzle
+    // (s >> 1) & 3 are known; only the chunk is the lane's.
     const bool xb_on = p.ln_xb != nullptr;
     const int xb_size = p.ln_xb_packed ? (int)packed_bytes(p.M, (size_t)p.N * 2) : p.M * p.N * 2;
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(xb_on ? p.ln_xb : p.Y, 0, xb_on ? xb_size : 0, 0x00020000);
     const int kb_per_row = p.N * 2 / 64;
     const int xb_chunk = (n * 2 >> 4) & 3;
-    const int xb_lane = p.ln_xb_packed
-        ? (((m_base >> 8) * kb_per_row + (n * 2 >> 6)) * 16384 + ((m_base & 255) + rrow) * 64 + ((n * 2) & 15))
-        : ((m_base + rrow) * p.N + n) * 2;
+    const int xb_lane = p.ln_xb_packed ? (n * 2 >> 6) * 16384 + rrow * 64 + ((n * 2) & 15) : ((m_base + rrow) * p.N + n) * 2;
     const int lane_off = (m_base + rrow) * row_bytes + n * 4;
 #pragma unroll
     for (int j = 0; j < NBJ; ++j) {
 #pragma unroll
-        for (int s = 0; s < NIT; ++s) {
-            const int step_rows = 32 * j + s * RPI;
-            const int rl = step_rows + rrow;
-            const float mean = statbuf[2 * rl], rstd = statbuf[2 * rl + 1];
+        for (int i = 0; i < NBI; ++i)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                f32x4_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = ln_scale(acc[i][j][4 * qd + e], mean[j], rstd[j]);
+                *reinterpret_cast<f32x4_t*>(buf + l32b * 512 + (((8 * i + 2 * qd + gb) ^ l32b) << 4)) = v;
+            }
+        const int m_col = m_base + 32 * j;
+        const int xb_col = p.ln_xb_packed ? (m_col >> 8) * kb_per_row * 16384 + (m_col & 255) * 64 : 32 * j * p.N * 2;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const int row = 2 * s + rrow;
+            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(buf + row * 512 + ((rc ^ row) << 4));
             f32x4_t o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = ln_apply(acc[s / 4][j][4 * (s % 4) + e], mean, rstd, gamma4[e], beta4[e]);
+            for (int e = 0; e < 4; ++e) o[e] = ln_affine(v[e], gamma4[e], beta4[e]);
             // rows past M: the descriptor drops the float32 store; the copy is predicated
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), y_rsrc, lane_off + step_rows * row_bytes, 0, 0);
-            if (xb_on && m_base + rl < p.M) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), y_rsrc, lane_off + (32 * j + 2 * s) * row_bytes, 0, 0);
+            if (xb_on && m_col + row < p.M) {
                 const bf16x4_t ob = {(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
-                const int off = p.ln_xb_packed ? xb_lane + step_rows * 64 + ((xb_chunk ^ ((s >> 1) & 3)) << 4)
-                                               : xb_lane + step_rows * p.N * 2;
+                const int off = xb_lane + xb_col + (p.ln_xb_packed ? 128 * s + ((xb_chunk ^ ((s >> 1) & 3)) << 4) : 2 * s * p.N * 2);
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, ob), x_rsrc, off, 0, 0);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
