@@ -40,6 +40,7 @@ bool launch_gemm_bf16_t256(const gemm_detail::GemmDev& d, int out_elt, int epilo
 bool launch_gemm_bf16_t256x128(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
 bool launch_gemm_bf16_t128(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
 bool launch_gemm_bf16_t256x128_deep(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
+bool launch_gemm_bf16_t256x192_ln(const gemm_detail::GemmDev& d, hipStream_t stream);
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream);
 bool launch_gemm_split(const gemm_detail::GemmDev& d, int tile, int epilogue, hipStream_t stream);
 int gemm_pick_tile(int M, int N, int K, int elt);
@@ -332,15 +333,20 @@ bool gemm_ln_workspace_force_expiry(void* ln_ws) {
     return true;
 }
 
-// Tile of a GEMM with the LayerNorm in its epilogue, 0 if the separate kernels are the better choice.
-// Measured on MI355X (N = 768 and 1024, K = N and 4 N): from about 6000 rows on the fused kernel beats
-// GEMM + LayerNorm launch.  Inside a forward pass (two half-batches on two streams) the 256 x 256 tile wins
-// once its tiles cover half of the CUs (152 and 200 tiles: +7 % on the pass over the 256 x 128 tile), below
-// that the 256 x 128 tile, two workgroups per CU and half as coarse (96 tiles: +3 %).
+// Tile of a GEMM with the LayerNorm in its epilogue, 0 if the separate kernels are the better choice (below about 6000
+// rows; N = 768 and 1024, K = N and 4 N).  The smallest tile that still makes one round of at most one workgroup per CU, since a
+// launch lasts as long as its slowest CU; beyond that the 256 x 256 one.  Microseconds, cold weights, N = 1024, K = 1024 / 4096,
+// with 128 / 192 / 256 tokens:  8192 rows 35.3 / 35.5 / 39.4 and 76.1 / 78.9 / 89.7;  8448 (264 tiles of 128 tokens) 43.4 / 36.6 /
+// 39.9 and 101 / 81.2 / 90.3;  10947 48.5 / 41.2 / 43.8 and 112 / 89.6 / 96.6;  12288 51.3 / 44.0 / 45.7 and 116 / 96.4 / 99.9;
+// 12416 (260 tiles of 192 tokens) 51.9 / 65.4 / 46.7 and 116 / 150 / 102.  N = 768, K = 768 / 3072, 12170 rows 40.6 / 33.4 / 37.6 and
+// 83.8 / 66.5 / 74.2.  The parts of a pass on two streams take the same tiles: 18009 rows of BERT-large 12.76 ms against 12.80, 20926
+// rows 15.17 against 15.27 with 256 tokens.
 int gemm_ln_pick_tile(int M, int N, int K, int elt) {
     if (M < 6144 || !ln_shape_ok(N, K, elt)) return 0;
-    const long tiles256 = (long)((M + 255) / 256) * (N / 256);
-    return (K % 128 == 0 && tiles256 >= 128) ? 256 : kTile256x128;
+    auto tiles = [&](int rows) { return (long)((M + rows - 1) / rows) * (N / 256); };
+    if (K % 128 != 0 || tiles(128) <= 256) return kTile256x128;
+    if (tiles(192) <= 256) return kTile256x192;
+    return tiles(256) >= 128 ? 256 : kTile256x128;
 }
 
 bool gemm_ln_supported(int M, int N, int K, int elt) { return gemm_ln_pick_tile(M, N, K, elt) != 0; }
@@ -604,7 +610,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     if (p.ln_gamma) {
         if (!p.residual || !p.ln_beta || !p.ln_ws || p.splits > 1 || !ln_shape_ok(p.N, p.K, p.elt) ||
             ((size_t)p.M + 256) * p.N * 4 >= (1ull << 31) || (size_t)(p.M + 127) / 128 > kLnMaxBands ||
-            (p.tile ? (p.tile != 256 && p.tile != kTile256x128) || (p.tile == 256 && p.K % 128 != 0)
+            (p.tile ? (p.tile != 256 && p.tile != kTile256x192 && p.tile != kTile256x128) || (p.tile != kTile256x128 && p.K % 128 != 0)
                     : !gemm_ln_supported(p.M, p.N, p.K, p.elt)) ||
             ((reinterpret_cast<uintptr_t>(p.ln_gamma) | reinterpret_cast<uintptr_t>(p.ln_beta) |
               reinterpret_cast<uintptr_t>(p.ln_xb) | reinterpret_cast<uintptr_t>(p.ln_ws)) & 15)) {
@@ -667,6 +673,12 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
     if (epi == kEpiBiasResLN && !p.tile) bt = gemm_ln_pick_tile(p.M, p.N, p.K, p.elt);
     if (d.splits > 1 && (bt == 256 || bt == kTile256x128 || bt == kTile256x128Deep) && !p.tile) bt = 128;      // those kernels do not split
     if (epi == kEpiBiasResLN && p.compiler_scheduled) { set_error("gemm: the LayerNorm epilogue has no compiler-scheduled kernel"); return false; }
+    if (bt == kTile256x192) {
+        if (epi != kEpiBiasResLN) { set_error("gemm: the 256x192 tile is there for the LayerNorm epilogue only"); return false; }
+        d.tiles_n = p.N / 256;
+        d.tiles_m = (p.M + 191) / 192;
+        return launch_gemm_bf16_t256x192_ln(d, stream);
+    }
     if (bt == kTile256x128 || bt == kTile256x128Deep) {
         if (p.elt != kBF16 || d.splits != 1) { set_error("gemm: the 256x128 tile is bf16 only and does not split K"); return false; }
         d.tiles_n = (p.N + 255) / 256;

@@ -259,6 +259,71 @@ bool launch_epi_half_deep(const GemmDev& d, int epi, hipStream_t stream) {
     return true;
 }
 
+// ---------------------------------------------------------------------------
+// 256 features x 192 tokens, one workgroup per CU: the pipeline of the 256 x 256 kernel (loop gemm_bf16_256x192_loop.inc,
+// "rows192" mode of gen_gemm_asm.py), with LayerNorm in the epilogue.  For launches whose 256 x 256 tiles are one round with
+// CUs to spare: three quarters of the tile on a third more CUs (gemm_ln_pick_tile has the measurements).  K a multiple of 128.
+#define CUBERT_ACC_OPERANDS_43 CUBERT_ACC_OPERANDS_H, [c02] "=&a"(acc[0][2]), [c12] "=&a"(acc[1][2]), [c22] "=&a"(acc[2][2]), [c32] "=&a"(acc[3][2])
+
+__global__ __launch_bounds__(256) void gemm_bf16_t256x192_ln_kernel(const GemmDev p) {
+    // Four stages of 28 KiB: W tile (256 rows x 64 B) at +0, X tile (192 rows x 64 B) at +0x4000; the epilogue's bias.
+    __shared__ __attribute__((aligned(2048))) unsigned char lds[4 * 28672 + 2048];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave >> 1, wm = wave & 1;
+    const int l32 = lane & 31, g = lane >> 5;
+
+    int tile_n, tile_m;
+    ln_tile_of_block(blockIdx.x, p.tiles_n, &tile_n, &tile_m);
+    if (tile_m >= p.tiles_m) return;          // the grid is padded to whole groups of eight bands
+    const int n0 = tile_n * 256, m0 = tile_m * 192;
+
+    const unsigned long long wa = reinterpret_cast<unsigned long long>(p.W);
+    const unsigned long long xa = reinterpret_cast<unsigned long long>(p.X);
+    const unsigned wsize = p.w_packed ? (unsigned)packed_bytes(p.N, (size_t)p.K * 2) : (unsigned)((size_t)p.N * p.K * 2);
+    const unsigned xsize = p.x_packed ? (unsigned)packed_bytes(p.M, (size_t)p.K * 2)
+                                      : (unsigned)((((size_t)p.M - 1) * p.ldx + p.K) * 2);
+    const u32x4_t wres = {(unsigned)wa, (unsigned)(wa >> 32) & 0xffffu, wsize, 0x00020000u};
+    const u32x4_t xres = {(unsigned)xa, (unsigned)(xa >> 32) & 0xffffu, xsize, 0x00020000u};
+    const int w_rowb = p.K * 2, x_rowb = p.ldx * 2;
+    const int KB = p.K * 2 / 64;
+    const int dc = (lane & 3) ^ packed_swizzle(lane >> 2);
+    const int w_v0 = p.w_packed ? (tile_n * KB * 16384 + wave * 1024 + lane * 16)
+                                : ((n0 + 16 * wave + (lane >> 2)) * w_rowb + (dc << 4));
+    int x_v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int m = m0 + 64 * k;            // 64 rows never straddle a packed block
+        x_v[k] = p.x_packed ? (m >> 8) * KB * 16384 + (m & 255) * 64 + wave * 1024 + lane * 16
+                            : (m + 16 * wave + (lane >> 2)) * x_rowb + (dc << 4);
+    }
+    const int w64 = p.w_packed ? 4096 : 64 * w_rowb;
+    const int wkstep = p.w_packed ? 16384 : 64, xkstep = p.x_packed ? 16384 : 64;
+    const int lds_base = (int)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    const int wb = lds_base + frag_base(wn * 128, p.w_units, l32, g), wx = frag_kphase(p.w_units);
+    const int xb = lds_base + 0x4000 + frag_base(wm * 96, p.x_units, l32, g), xx = frag_kphase(p.x_units);
+    const int m0b = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
+    const int ht = p.K / 32;          // half-steps; a multiple of 4
+
+    f32x16_t acc[4][3];       // zeroed inside the asm block
+
+    asm volatile(
+#include "gemm_bf16_256x192_loop.inc"
+        : CUBERT_ACC_OPERANDS_43
+        : [wb] "v"(wb), [xb] "v"(xb), [wx] "s"(wx), [xx] "s"(xx), [wv0] "v"(w_v0), [xv0] "v"(x_v[0]), [xv1] "v"(x_v[1]), [xv2] "v"(x_v[2]),
+          [wres] "s"(wres), [xres] "s"(xres), [w64] "s"(w64), [ht] "s"(ht), [m0b] "s"(m0b), [wkstep] "s"(wkstep), [xkstep] "s"(xkstep)
+        : "memory", "scc", "m0", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "v104", "v105", "v106", "v107", "v108", "v109",
+          CUBERT_V10(11), CUBERT_V10(12), CUBERT_V10(13), CUBERT_V10(14), CUBERT_V10(15), CUBERT_V10(16), "v170", "v171", "v172",
+          "v173", "v174");
+
+    // Slower waves may still be multiplying out of the last two stages, which reach into the first 64 KiB.
+    __syncthreads();
+    gemm_epilogue_ln<4, 3>(p, acc, n0 + wn * 128, m0 + wm * 96, l32, g, tile_m, 2 * tile_n + wn, lds + wave * 16384,
+                           reinterpret_cast<float*>(lds + 4 * 28672 + wave * 512));
+}
+
 // LayerNorm epilogue: eight XCDs x whole groups of bands x the workgroups of a band (ln_tile_of_block);
 // workgroups whose band does not exist leave at once.
 dim3 ln_grid(const GemmDev& d) { return dim3(8 * d.tiles_n * ((d.tiles_m + 7) / 8)); }
@@ -326,6 +391,14 @@ bool launch_gemm_bf16_t256(const gemm_detail::GemmDev& d, int out_elt, int epilo
 bool launch_gemm_bf16_t256x128_deep(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream) {
     if (d.K % 128 != 0 || d.K < 128) { set_error("gemm: the one-per-CU 256x128 tile needs K to be a multiple of 128"); return false; }
     return out_elt == kBF16 ? launch_epi_half_deep<kBF16>(d, epilogue, stream) : launch_epi_half_deep<kF32>(d, epilogue, stream);
+}
+
+// 256 x 192 tile with LayerNorm in the epilogue: d.tiles_n for 256 features, d.tiles_m for 192 tokens; d.K % 128 == 0.
+bool launch_gemm_bf16_t256x192_ln(const gemm_detail::GemmDev& d, hipStream_t stream) {
+    if (d.K % 128 != 0 || d.K < 128) { set_error("gemm: the 256x192 tile needs K to be a multiple of 128"); return false; }
+    hipLaunchKernelGGL(gemm_bf16_t256x192_ln_kernel, ln_grid(d), dim3(256), 0, stream, d);
+    CUBERT_HIP_OK(hipGetLastError());
+    return true;
 }
 
 // 256 x 128 tile: d.tiles_n for 256 features, d.tiles_m for 128 tokens; d.K % 32 == 0, K >= 64.

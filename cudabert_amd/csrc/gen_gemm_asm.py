@@ -6,6 +6,7 @@ string) of the bf16 GEMM macro tiles:
     python gen_gemm_asm.py half > gemm_bf16_256x128_loop.inc    # 256 x 128, two per CU (end of file)
     python gen_gemm_asm.py quarter > gemm_bf16_128_loop.inc     # 128 x 128, three per CU (end of file)
     python gen_gemm_asm.py deep > gemm_bf16_256x128_deep_loop.inc  # 256 x 128, one per CU, the 256 x 256 pipeline
+    python gen_gemm_asm.py rows192 > gemm_bf16_256x192_loop.inc    # 256 x 192, likewise
 
 and of the float32 GEMM on operands split into three bf16 planes (end of file):
 
@@ -177,6 +178,12 @@ FULL = Deep("", 4, 4, 112, 128, 144, 160, 96, 104, 108, 0x8000)
 #   v64..v79 / v80..v87  W / X fragments, set A      v88..v103 / v104..v111  set B
 #   v112..v119  fragment row addresses (stages 0-1, 2-3)   v120..v123 / v124..v125  W / X lane offsets
 DEEP = Deep("deep", 4, 2, 64, 80, 88, 104, 112, 120, 124, 0x6000)
+# "rows192" mode: python gen_gemm_asm.py rows192 > gemm_bf16_256x192_loop.inc
+# 256 features x 192 tokens (4 x 3 accumulator blocks per wave), stages of 28 KiB.  A tile's three groups of 64 token rows may
+# lie in two of the packed layout's blocks of 256 rows, so the kernel hands in a lane offset for each (%[xv0] .. %[xv2]).
+#   v104..v119 / v120..v131  W / X fragments, set A      v132..v147 / v148..v159  set B
+#   v160..v167  fragment row addresses (stages 0-1, 2-3)   v168..v171 / v172..v174  W / X lane offsets
+ROWS192 = Deep("rows192", 4, 3, 104, 120, 132, 148, 160, 168, 172, 0x7000)
 
 
 def main(c=FULL):
@@ -194,7 +201,8 @@ def main(c=FULL):
         if i < c.nwb:
             e.emit("v_add_u32 v%d, %%[w64], v%d" % (c.wvoff + i, c.wvoff + i - 1))
         if i < c.nxb:
-            e.emit("v_add_u32 v%d, %%[x64], v%d" % (c.xvoff + i, c.xvoff + i - 1))
+            e.emit("v_mov_b32 v%d, %%[xv%d]" % (c.xvoff + i, i) if c is ROWS192 else
+                   "v_add_u32 v%d, %%[x64], v%d" % (c.xvoff + i, c.xvoff + i - 1))
     # zero the accumulators: 0 * 0 + 0 through the matrix pipe (the accumulator
     # operands are write-only for the compiler, which halves the operand count)
     for r in range(4):
@@ -578,6 +586,8 @@ if __name__ == "__main__":
         main_skewed(HALF)
     elif len(sys.argv) > 1 and sys.argv[1] == "deep":
         main(DEEP)
+    elif len(sys.argv) > 1 and sys.argv[1] == "rows192":
+        main(ROWS192)
     elif len(sys.argv) > 1 and sys.argv[1] == "quarter":
         if len(sys.argv) > 2:
             QUARTER.nstage = int(sys.argv[2])

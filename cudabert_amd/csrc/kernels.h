@@ -39,6 +39,7 @@ struct Compact {
 
 constexpr int kTile256x128 = 384;     // GemmParams::tile value of the 256 features x 128 tokens kernel
 constexpr int kTile256x128Deep = 385; // ... of the 256 x 128 kernel with one workgroup per CU and the deeper pipeline (K % 128 == 0)
+constexpr int kTile256x192 = 386;     // ... of the 256 features x 192 tokens kernel (LayerNorm epilogue only; K % 128 == 0)
 constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 kernel (bf16, three workgroups per CU, splits K)
 
 constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
@@ -77,7 +78,7 @@ struct GemmParams {
     // kEpiBias with a residual and ln_gamma set: the LayerNorm that follows the linear runs in the
     // epilogue.  Y (float32 row-major, may be the residual buffer itself) receives
     // LayerNorm(acc + bias + R) * gamma + beta over each row of N features, ln_xb (optional) a bf16
-    // copy of it (row-major, or packed with ln_xb_packed).  bf16 operands, the 256 x 256 or 256 x 128
+    // copy of it (row-major, or packed with ln_xb_packed).  bf16 operands, the 256 x 256, 256 x 192 or 256 x 128
     // tile, N a multiple of 256 up to 1024, no split K.  The N / 256 workgroups that hold one band
     // of rows exchange their partial row sums through ln_ws: gemm_ln_workspace_bytes(M) bytes of
     // device memory that are all zero before the first launch (each launch leaves the words it
