@@ -56,6 +56,7 @@ void* make_model(const cubert_config& cfg, int gpu, int maxB, int maxS, const ch
     // measured: one stream is the faster choice below about 14 thousand token rows in bf16 mode
     // (11 - 12 thousand rows: +3 ... 7 %), two streams already from 8 thousand in fp32 mode (+6 ... 13 %)
     opt.split_min_tokens = env_int("CUBERT_SPLIT_MIN_TOKENS", cfg.precision == cubert::kBF16 ? 14336 : 8192);
+    opt.split_keeps_one_round = cfg.precision == cubert::kBF16 && !std::getenv("CUBERT_SPLIT_MIN_TOKENS");
     opt.split_parts = env_int("CUBERT_SPLIT_PARTS", 2);
     opt.varlen = env_int("CUBERT_VARLEN", -1);
     opt.split_k = env_int("CUBERT_SPLIT_K", 1) != 0;
