@@ -4,6 +4,9 @@
 // Same operand roles and epilogues as the other kernels (gemm.hip).  The K loops are hand-scheduled inline asm
 // (gemm_split_128_loop.inc, gemm_split_256x128_loop.inc; pipeline and register plan in gen_gemm_asm.py).
 //
+// The 128 x 128 loop reads a step's fragments during the step before: 1024 x 768 x 768 (48 workgroups) 26.5 -> 23.8 us, 1024 x 3072 x
+// 768 32.3 -> 30.6, 12800 x 1024 x 4096 513 -> 504; at 192 workgroups and more its loop runs at the rate the power limit allows.
+//
 // Bound: the matrix pipe at the socket's power limit.  9800 x 4096 x 1024 with GELU: 377 us, 218 TFLOP/s, i.e. 1.31 PFLOP/s of
 // bf16 products; 25600 x 4096 x 1024 without it 1.43 at 1400 W of 1400 (a bf16 product of 8192^3 reaches 1.44 there: 0.97 pJ per
 // operation both, where a bf16 FFN-in, whose fragments serve one product instead of two, spends 1.35), against 668 us, 123 TFLOP/s with the float32 MFMA, whose
@@ -115,7 +118,8 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(const GemmDev p) {
             : [wb] "v"(wb), [xb] "v"(xb), [wv0] "v"(v0), [xv0] "v"(v0), [wres] "s"(wres), [xres] "s"(xres),
               [m0b] "s"(m0b), [k0] "s"(k0), [kmax] "s"(kmax), [steps] "s"(steps)
             : "memory", "scc", "m0", "s92", "s93", "s94", "s95", "s96", "s97", CUBERT_V10(4), CUBERT_V10(5), CUBERT_V10(6),
-              CUBERT_V10(7), CUBERT_V10(8), "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97");
+              CUBERT_V10(7), CUBERT_V10(8), CUBERT_V10(9), CUBERT_V10(10), CUBERT_V10(11), CUBERT_V10(12), CUBERT_V10(13), "v140",
+              "v141", "v142", "v143", "v144", "v145");
     } else {
         asm volatile(
 #include "gemm_split_256x128_loop.inc"

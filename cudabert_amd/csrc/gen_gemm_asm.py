@@ -453,8 +453,9 @@ def main_skewed(c):
 # are exactly the MFMA operand (lane l's 16 bytes at 16 l), so a global->LDS load moves one unit and a fragment read
 # is linear in the lane.  A wave multiplies nwb x 2 blocks with the six plane products that reach float32 precision:
 # 12 nwb MFMAs on 3 (nwb + 2) fragments, i.e. a quarter to a half of a fragment read per MFMA, where the bf16 loops
-# need three quarters to one.  With two or three waves per SIMD the matrix pipe always has another wave's work while one
-# waits for its first fragments, so nothing is read ahead of the barrier.
+# need three quarters to one.  The 256 x 128 loop reads nothing ahead of the barrier: a SIMD holds two of its waves, and one
+# multiplies while the other waits for its first fragments.  The 128 x 128 loop, which serves launches with one workgroup on
+# a CU as well, reads a step ahead (main_split_ahead).
 #   s92  stage offset of the tile being multiplied   s93  of the tile being fetched   s94  M0 base (LDS base + wave * 3072)
 #   s95  M0 base of the tile being fetched   s96  K byte offset (the same for both operands)   s97  counter
 class Split:
@@ -468,6 +469,7 @@ class Split:
         self.stage = self.x_lds + 4 * 3072
         self.n = 3 * (nwb // 2) + 3                  # global->LDS loads per step and wave
         self.last = self.voff + self.n - 1
+        self.second = self.last + 1                  # split128: the other fragment set, laid out like the first
 
 
 SPLIT128 = Split("split128", 2, 3, 40)
@@ -520,6 +522,8 @@ def main_split(c):
         e.emit("s_add_u32 s96, s96, 0xc00")
         e.emit("s_min_u32 s96, s96, %[kmax]")
 
+    if c is SPLIT128:
+        return main_split_ahead(c, e, wf, xf, dma, rotate, advance)
     e.emit("; ======== prologue ========")
     for t in range(c.nstage - 1):
         e.emit("s_add_u32 s95, s94, s93")
@@ -571,6 +575,88 @@ def main_split(c):
     e.emit("s_add_u32 s97, s97, 1")
     e.emit("s_cmp_lt_u32 s97, %[steps]")
     e.emit("s_cbranch_scc1 L_loop_%=")
+    e.emit("s_waitcnt vmcnt(0)")
+    e.emit("s_barrier")
+    print("// Generated by gen_gemm_asm.py %s -- do not edit." % c.name)
+    for ln in e.lines:
+        print('"%s\\n"' % ln)
+
+
+def main_split_ahead(c, e, wf, xf, dma, rotate, advance):
+    """The 128 x 128 loop: a step's fragments are read one step ahead, into a second register set, behind the MFMAs of the step
+    before.  (Read after the barrier, with one workgroup on the CU, every step began with an idle matrix pipe.)  Two steps per turn
+    of the loop, left in the middle when the count is odd.  The tile of step s is in registers when step s begins, so its stage
+    takes the loads of step s + 3 while the tile of s + 1 is read and that of s + 2 is on its way."""
+    e.emit("; ======== prologue: tiles 0, 1, 2 -> stages 0, 1, 2 ========")
+    for t in range(3):
+        e.emit("s_add_u32 s95, s94, s93")
+        for k in range(c.n):
+            m0, ld = dma(k)
+            e.emit(m0)
+            e.emit("s_nop 0")
+            e.emit(ld)
+        rotate(93)
+        advance()
+
+    def addresses():
+        e.emit("v_add_u32 v%d, s92, v%d" % (c.base + 2, c.base))
+        e.emit("v_add_u32 v%d, s92, v%d" % (c.base + 3, c.base + 1))
+
+    def reads(shift):
+        out = []
+        for p in range(3):
+            for kind, b in [("w", 0)] + [("x", b) for b in range(c.nxb)] + [("w", b) for b in range(1, c.nwb)]:
+                out.append((wf(p, b) + shift, c.base + 2, b * 3072 + p * 1024) if kind == "w" else
+                           (xf(p, b) + shift, c.base + 3, c.x_lds + b * 3072 + p * 1024))
+        return out
+
+    e.emit("s_waitcnt vmcnt(%d)" % (2 * c.n))        # tile 0 has landed
+    e.emit("s_barrier")
+    addresses()
+    for r in reads(0):
+        e.read(*r)
+    rotate(92)
+    e.emit("s_waitcnt vmcnt(%d) lgkmcnt(0)" % c.n)   # tile 1 has landed; tile 0 is in registers
+    e.emit("s_barrier")
+    e.emit("s_mov_b32 s97, 0")
+    e.emit("L_loop_%=:")
+    other = c.second - c.w
+    for half, (cur, nxt) in enumerate(((0, other), (other, 0))):
+        addresses()
+        e.emit("s_add_u32 s95, s94, s93")
+        pending = reads(nxt)
+        total = len(PLANE_PRODUCTS) * c.nwb * c.nxb
+        every = (total - 4) // c.n
+        m = d = 0
+        for wp, xp in PLANE_PRODUCTS:
+            for i in range(c.nwb):
+                for j in range(c.nxb):
+                    load = m % every == 1 and d < c.n
+                    if load:
+                        e.emit(dma(d)[0])
+                    e.emit("v_mfma_f32_32x32x16_bf16 %%[c%d%d], %s, %s, %%[c%d%d]" %
+                           (i, j, vreg4(wf(wp, i) + cur), vreg4(xf(xp, j) + cur), i, j))
+                    if load:
+                        e.emit(dma(d)[1])
+                        d += 1
+                    if m < len(pending):
+                        e.read(*pending[m])
+                    m += 1
+        assert d == c.n
+        rotate(92)
+        rotate(93)
+        advance()
+        # the tile after the next has landed; the next one is in registers (and its stage free once everybody says so)
+        e.emit("s_waitcnt vmcnt(%d) lgkmcnt(0)" % c.n)
+        e.emit("s_barrier")
+        e.emit("s_add_u32 s97, s97, 1")
+        if half == 0:
+            e.emit("s_cmp_ge_u32 s97, %[steps]")
+            e.emit("s_cbranch_scc1 L_end_%=")
+        else:
+            e.emit("s_cmp_lt_u32 s97, %[steps]")
+            e.emit("s_cbranch_scc1 L_loop_%=")
+    e.emit("L_end_%=:")
     e.emit("s_waitcnt vmcnt(0)")
     e.emit("s_barrier")
     print("// Generated by gen_gemm_asm.py %s -- do not edit." % c.name)
