@@ -608,14 +608,16 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         if (!mark(kPhQKV) || !launch_gemm(g, st)) return false;
         // The last layer of a pass whose caller gets no sequence output: keys and values are needed of every token,
         // everything after them only of the first token of each sequence, which is all the pooler reads.  Where the full
-        // pass would not split K, its B rows take kernels that sum over k in the order of the full pass's, and every kernel
-        // treats a row the same whatever else is in the launch, so the pooled output keeps its bits.
-        const bool first = first_only_ && i == D.layers - 1 && sp_ao == 1 && sp_fo == 1;
+        // pass would not split K, its B rows take kernels that sum over k in the order of the full pass's, where it would they
+        // take its tile and its split (the partial sums lie in y32, which has room for those of all N rows), and every kernel
+        // treats a row the same whatever else is in the launch, so the pooled output keeps its bits.  Up to kSkinnyMaxRows rows
+        // the layer's launches are as long for one row as for all, and there is one more (the gather).
+        const bool first = first_only_ && i == D.layers - 1 && ((sp_ao == 1 && sp_fo == 1) || N > kSkinnyMaxRows);
         if (!mark(kPhAttention)) return false;
         if (first) {
             const size_t c0 = (size_t)part * 1024;
             float* xc = xc32_ + c0 * H;
-            float* yc = yc32_ + c0 * H;
+            float* yc = any_order ? y32 : yc32_ + c0 * H;
             unsigned char* xbc = xbc_ + c0 * H * os;
             unsigned char* ctxc = static_cast<unsigned char*>(ctxc_) + c0 * H * os;
             unsigned char* hc = static_cast<unsigned char*>(hc_) + c0 * I * os;
@@ -625,10 +627,12 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             g.elt = gelt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
             g.M = B; g.N = H; g.K = H; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
+            g.splits = sp_ao;
+            g.tile = sp_ao > 1 ? plan_ao.tile : 0;
             g.k_order = plan_ao.k_order();
             if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
-            if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, layout, B, H, st, 1, !fuse_res)) return false;
+            if (!launch_add_layernorm(xc, yc, kF32, L.g1, L.be1, xbc, layout, B, H, st, sp_ao, !fuse_res)) return false;
             g = GemmParams();
             g.elt = g.out_elt = gelt; g.X = xbc; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = hc;
             g.M = B; g.N = I; g.K = H; g.epilogue = kEpiBiasGelu; g.x_packed = g.w_packed = g.y_packed = g.w_units = g.y_units = pk;
@@ -639,10 +643,12 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             g.elt = gelt; g.out_elt = kF32; g.X = hc; g.ldx = I; g.W = L.w_out; g.bias = L.b_out; g.Y = yc;
             g.M = B; g.N = H; g.K = I; g.epilogue = kEpiBias; g.x_packed = g.w_packed = g.x_units = g.w_units = pk;
             g.residual = fuse_res ? xc : nullptr;
+            g.splits = sp_fo;
+            g.tile = sp_fo > 1 ? plan_fo.tile : 0;
             g.k_order = plan_fo.k_order();
             if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
             if (!mark(kPhLayerNorm)) return false;
-            if (!launch_add_layernorm(xc, yc, kF32, L.g2, L.be2, nullptr, kRowMajor, B, H, st, 1, !fuse_res)) return false;
+            if (!launch_add_layernorm(xc, yc, kF32, L.g2, L.be2, nullptr, kRowMajor, B, H, st, sp_fo, !fuse_res)) return false;
             if (!mark(kPhPooler)) return false;
             return launch_pooler(xc, w_pool_, elt, b_pool_, pooled_ + (size_t)b0 * H, B, 1, H, st, nullptr);
         }
