@@ -126,6 +126,12 @@ __device__ __forceinline__ float ln_dpp_lanes(float v) {
 __device__ __forceinline__ void half_swap(float& a, float& b) {
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
 }
+// The same for lanes 16 apart (rows of 16 lanes: the odd rows of one register with the even rows of the other).
+__device__ __forceinline__ float row_swap_sum(float v) {
+    float a = v, b = v;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    return a + b;
+}
 // Accumulator layout -> split layout.  x: four consecutive values (features or k) of group 2 u and four of group 2 u + 1 of
 // my row, the halves lane / 32 of the two groups of eight; after exchanging with lane ^ 32 a lane holds all eight of group
 // 2 u + lane / 32, i.e. the 16 bytes per plane of a unit that are its own.  Every lane of the wave takes part.
@@ -168,7 +174,7 @@ __device__ __forceinline__ float ln_half_wave_sum(float v) {
     v += ln_dpp_lanes<0x128>(v);      // row_ror 8: lane ^ 8
     v += ln_dpp_lanes<0x124>(v);      // row_ror 4: lane ^ 4, now that lanes 8 apart agree
     v += ln_dpp_lanes<0x122>(v);      // row_ror 2: lane ^ 2
-    v += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));   // lane ^ 16
+    v = row_swap_sum(v);              // lane ^ 16
     v += ln_dpp_lanes<0xB1>(v);       // quad_perm [1,0,3,2]: lane ^ 1
     return v;
 }
