@@ -265,7 +265,7 @@ bool Model::check_shape(int B, int S) {
 bool Model::forward_host(const int* ids, const int* seg, const int* mask, int B, int S, bool need_seq) {
     if (!check_shape(B, S)) return false;
     if (!ids || !seg) { set_error("input_ids and token_type_ids must not be null"); return false; }
-    const size_t n = (size_t)B * S, cap = (size_t)cap_tokens_;
+    const size_t n = (size_t)B * S;
     const Dims& D = opt_.dims;
     for (size_t i = 0; i < n; ++i) {
         if ((unsigned)ids[i] >= (unsigned)D.vocab) {
@@ -281,11 +281,10 @@ bool Model::forward_host(const int* ids, const int* seg, const int* mask, int B,
     // must have left it before it is overwritten.
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     std::memcpy(h_in_, ids, n * 4);
-    std::memcpy(h_in_ + cap, seg, n * 4);
-    if (mask) std::memcpy(h_in_ + 2 * cap, mask, n * 4);
-    CUBERT_HIP_OK(hipMemcpyAsync(d_in_, h_in_, n * 4, hipMemcpyHostToDevice, stream_));
-    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, h_in_ + cap, n * 4, hipMemcpyHostToDevice, stream_));
-    if (mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * cap, h_in_ + 2 * cap, n * 4, hipMemcpyHostToDevice, stream_));
+    std::memcpy(h_in_ + n, seg, n * 4);
+    if (mask) std::memcpy(h_in_ + 2 * n, mask, n * 4);
+    // One upload: each is a launch of its own at the head of the pass.
+    CUBERT_HIP_OK(hipMemcpyAsync(d_in_, h_in_, (mask ? 3 : 2) * n * 4, hipMemcpyHostToDevice, stream_));
     // Masks that are 1 on a non-empty prefix and 0 after it allow the unpadded pass (valid tokens
     // only; zeros instead of values on the padding positions of the sequence output).  varlen = 1: whenever the masks
     // allow it.  varlen = -1 (default): only when the caller cannot see the sequence output, the batch is too large for
@@ -321,9 +320,9 @@ bool Model::forward_device_lens(const int* d_ids, const int* d_seg, const int* h
             set_error("length " + std::to_string(h_lens[b]) + " of sequence " + std::to_string(b) + " is outside 1.." + std::to_string(S));
             return false;
         }
-    const size_t n = (size_t)B * S, cap = (size_t)cap_tokens_;
+    const size_t n = (size_t)B * S;
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_, d_ids, n * 4, hipMemcpyDeviceToDevice, stream_));
-    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
+    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + n, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
     return run_compact(h_lens, B, S, false);
 }
 
@@ -394,10 +393,10 @@ bool Model::forward_device(const int* d_ids, const int* d_seg, const int* d_mask
     if (!check_shape(B, S)) return false;
     first_only_ = false;
     if (!d_ids || !d_seg) { set_error("input_ids and token_type_ids must not be null"); return false; }
-    const size_t n = (size_t)B * S, cap = (size_t)cap_tokens_;
+    const size_t n = (size_t)B * S;
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_, d_ids, n * 4, hipMemcpyDeviceToDevice, stream_));
-    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
-    if (d_mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * cap, d_mask, n * 4, hipMemcpyDeviceToDevice, stream_));
+    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + n, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
+    if (d_mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * n, d_mask, n * 4, hipMemcpyDeviceToDevice, stream_));
     return run(B, S, d_mask != nullptr);
 }
 
@@ -538,9 +537,9 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     const int gelt = elt == kBF16 ? kBF16 : kF32Split;
     // rows of this part: every token, or (unpadded pass) the valid ones only, stored from row r0
     const int H = D.hidden, I = D.inter, N = cp ? cp->rows : B * S, Sp = round_up(S, 32);
-    const size_t cap = (size_t)cap_tokens_, t0 = (size_t)b0 * S;
+    const size_t n_in = (size_t)B_ * S, t0 = (size_t)b0 * S;      // inputs lie one after the other, all tokens of the pass each
     const int* cu = cp ? cp->cu : nullptr;
-    const int *ids = d_in_ + t0, *seg = d_in_ + cap + t0, *mask = has_mask ? d_in_ + 2 * cap + t0 : nullptr;
+    const int *ids = d_in_ + t0, *seg = d_in_ + n_in + t0, *mask = has_mask ? d_in_ + 2 * n_in + t0 : nullptr;
     float* x32 = x32_ + (cp ? r0 : t0) * H;
     float* y32 = y32_ + r0 * H;
     unsigned char* xb = xb_ + r0 * H * os;
@@ -706,10 +705,10 @@ bool Model::profile_device(const int* d_ids, const int* d_seg, const int* d_mask
     if (!phase_ms) { set_error("profile: null output"); return false; }
     if (!check_shape(B, S)) return false;
     if (!d_ids || !d_seg) { set_error("input_ids and token_type_ids must not be null"); return false; }
-    const size_t n = (size_t)B * S, cap = (size_t)cap_tokens_;
+    const size_t n = (size_t)B * S;
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_, d_ids, n * 4, hipMemcpyDeviceToDevice, stream_));
-    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + cap, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
-    if (d_mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * cap, d_mask, n * 4, hipMemcpyDeviceToDevice, stream_));
+    CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + n, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
+    if (d_mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * n, d_mask, n * 4, hipMemcpyDeviceToDevice, stream_));
     B_ = B;
     S_ = S;
     first_only_ = false;

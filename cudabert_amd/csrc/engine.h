@@ -134,7 +134,7 @@ class Model {
     float* maskadd_ = nullptr;   // [B, Sp]
     float* pooled_ = nullptr;    // [B, H]
     float* cls_ = nullptr;       // [B, C]
-    int* d_in_ = nullptr;        // ids | seg | mask, cap_tokens each
+    int* d_in_ = nullptr;        // ids | seg | mask, B * S of the pass each
     int* h_in_ = nullptr;        // pinned staging, same layout
     // unpadded passes: per part a row map (token index of every compact row) and cu (row offsets)
     static constexpr int kSplitRows = 8192;   // extra rows of y32 for the partial results of split-K GEMMs
