@@ -48,6 +48,7 @@ Model::~Model() {
     if (ablock_) (void)hipFree(ablock_);
     if (h_in_) (void)hipHostFree(h_in_);
     if (h_meta_) (void)hipHostFree(h_meta_);
+    if (h_out_) (void)hipHostFree(h_out_);
     if (ev_fork_) (void)hipEventDestroy(ev_fork_);
     for (int i = 1; i < kMaxParts; ++i) {
         if (ev_join_[i]) (void)hipEventDestroy(ev_join_[i]);
@@ -232,6 +233,7 @@ bool Model::init(const ModelOptions& opt_in) {
     ctxc_ = ablock_ + o_ctxc;
     hc_ = ablock_ + o_hc;
     CUBERT_HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_meta_), meta_ints * 4, hipHostMallocDefault));
+    CUBERT_HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_out_), kStagedFloats * 4, hipHostMallocDefault));
     CUBERT_HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_in_), 3 * N * 4, hipHostMallocDefault));
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     return true;
@@ -786,13 +788,17 @@ bool Model::sync() {
     return true;
 }
 
+// Small results come down through pinned memory: into pageable memory of the caller a copy of 3 KiB takes 23 us, into pinned
+// memory 13; from 92 KiB on both take the same.
 bool Model::copy_out(float* out, const float* dev, size_t floats) {
-    CUBERT_HIP_OK(hipMemcpyAsync(out, dev, floats * 4, hipMemcpyDeviceToHost, stream_));
+    float* to = floats <= kStagedFloats ? h_out_ : out;
+    CUBERT_HIP_OK(hipMemcpyAsync(to, dev, floats * 4, hipMemcpyDeviceToHost, stream_));
     if (!sync()) return false;
     if (recovered_) {       // the copy above ran before the pass was repeated
-        CUBERT_HIP_OK(hipMemcpyAsync(out, dev, floats * 4, hipMemcpyDeviceToHost, stream_));
+        CUBERT_HIP_OK(hipMemcpyAsync(to, dev, floats * 4, hipMemcpyDeviceToHost, stream_));
         CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     }
+    if (to != out) std::memcpy(out, to, floats * 4);
     return true;
 }
 

@@ -136,6 +136,8 @@ class Model {
     float* cls_ = nullptr;       // [B, C]
     int* d_in_ = nullptr;        // ids | seg | mask, B * S of the pass each
     int* h_in_ = nullptr;        // pinned staging, same layout
+    static constexpr size_t kStagedFloats = 16384;
+    float* h_out_ = nullptr;     // pinned staging of results of up to kStagedFloats
     // unpadded passes: per part a row map (token index of every compact row) and cu (row offsets)
     static constexpr int kSplitRows = 8192;   // extra rows of y32 for the partial results of split-K GEMMs
     static constexpr int kCuStride = 1032;    // B <= 1024 per part, + 1
