@@ -236,13 +236,35 @@ __global__ __launch_bounds__(512) void add_layernorm_split_rows_kernel(float* __
     }
 }
 
+// A row held by a workgroup of four waves, wave w the features i = 256 w + lane * 4 .. + 3 (v; zeros past H): statistics of its two
+// slots, exchanged through the LDS, combined by every wave (the arithmetic and order of ln_row_stats, hence the same bits), and its
+// own features normalised and stored.
+template <int LAYOUT>
+__device__ __forceinline__ void ln_group_row(const float (&v)[4], const LnDims& d, int lane, int wave, const f32x4_t& g4,
+                                             const f32x4_t& b4, float* xrow, void* xb, int row) {
+    __shared__ float stats[kMaxChunks][4];
+    float s_lo, q_lo, s_hi, q_hi;
+    ln_chunk_stats(v, wave, d, lane, &s_lo, &q_lo, &s_hi, &q_hi);
+    if (lane == 0) {
+        stats[wave][0] = s_lo; stats[wave][1] = q_lo; stats[wave][2] = s_hi; stats[wave][3] = q_hi;
+    }
+    __syncthreads();
+    float ssum[2 * kMaxChunks], sm2[2 * kMaxChunks];
+#pragma unroll
+    for (int c = 0; c < kMaxChunks; ++c) {
+        ssum[2 * c] = stats[c][0]; sm2[2 * c] = stats[c][1]; ssum[2 * c + 1] = stats[c][2]; sm2[2 * c + 1] = stats[c][3];
+    }
+    float mean, rstd;
+    ln_combine_slots(ssum, sm2, d, &mean, &rstd);
+    const int i = wave * 256 + lane * 4;
+    if (i < d.H) ln_store4<LAYOUT>(v, mean, rstd, g4, b4, xrow, xb, row, i, d.H);
+}
+
 // The same operation for a short batch, whose addend may come as the partial sums of a split-K GEMM
 // ([part][rows][H] float32): one workgroup per row, so that the few rows still spread over the
 // chip and a wave's chain is a quarter of a row long.  Such a launch is a chain of round trips and little else, so everything it needs -- the row,
 // every partial sum, gamma and beta -- is requested before the first value is used.  Wave w adds up the
-// parts of features 256 w .. 256 w + 255 and forms the statistics of its two slots; the waves exchange
-// those through the LDS, every wave combines them (the same arithmetic in the same order as
-// add_layernorm_kernel, hence the same bits) and normalises its own features.
+// parts of features 256 w .. 256 w + 255 (ln_group_row).
 // MORE: parts after the first; 0, 1 and 3 are exact, any other number goes in rounds of 8 that repeat part 0 to fill up
 // (1600 x 1024, 4 parts: five needless loads out of eight, 9.8 us against 9.4; 2 parts 6.9 against 6.1).
 template <int LAYOUT, int MORE>
@@ -252,7 +274,6 @@ __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restr
                                                                   void* __restrict__ xb, int rows, LnDims d,
                                                                   int y_parts, int add_x) {
     const int H = d.H;
-    __shared__ float stats[kMaxChunks][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = blockIdx.x;
     float* xrow = x + (size_t)row * H;
@@ -289,20 +310,7 @@ __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restr
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = a[e];
     }
-    float s_lo, q_lo, s_hi, q_hi;
-    ln_chunk_stats(v, wave, d, lane, &s_lo, &q_lo, &s_hi, &q_hi);
-    if (lane == 0) {
-        stats[wave][0] = s_lo; stats[wave][1] = q_lo; stats[wave][2] = s_hi; stats[wave][3] = q_hi;
-    }
-    __syncthreads();
-    float ssum[2 * kMaxChunks], sm2[2 * kMaxChunks];
-#pragma unroll
-    for (int c = 0; c < kMaxChunks; ++c) {
-        ssum[2 * c] = stats[c][0]; sm2[2 * c] = stats[c][1]; ssum[2 * c + 1] = stats[c][2]; sm2[2 * c + 1] = stats[c][3];
-    }
-    float mean, rstd;
-    ln_combine_slots(ssum, sm2, d, &mean, &rstd);
-    if (in) ln_store4<LAYOUT>(v, mean, rstd, g4, b4, xrow, xb, row, i, H);
+    ln_group_row<LAYOUT>(v, d, lane, wave, g4, b4, xrow, xb, row);
 }
 
 template <int LAYOUT>
@@ -351,6 +359,49 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
         }
     }
     normalise_store<LAYOUT>(v, d, lane, gamma, beta, x + (size_t)row * H, xb, row);
+}
+
+// The same for a short batch: such a launch is a chain of round trips (id, word row, result), so a workgroup per row, a wave's chain
+// a quarter of a row long, gamma, beta and the position's row requested before the token's id has arrived.  A wave per row against
+// this: 17 x 768 6.3 -> 3.8 us, 1600 x 1024 11.5 -> 9.3, 128 x 1024 with the split copy 8.9 -> 5.3.
+template <int LAYOUT>
+__global__ __launch_bounds__(256) void embed_layernorm_row_kernel(
+    const int* __restrict__ ids, const int* __restrict__ seg, const int* __restrict__ mask,
+    const float* __restrict__ word, const float* __restrict__ pos, const float* __restrict__ type,
+    const float* __restrict__ gamma, const float* __restrict__ beta, float* __restrict__ x,
+    void* __restrict__ xb, float* __restrict__ maskadd, int B, int S, int Sp, LnDims d, int vocab,
+    int type_vocab, const int* __restrict__ rowmap, const int* __restrict__ cu, int nrows) {
+    const int H = d.H, row = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tok = rowmap ? rowmap[row] : row;
+    int id = ids[tok];
+    int tt = seg ? seg[tok] : 0;
+    const int b = tok / S, s = tok - b * S;
+    const int i = wave * 256 + lane * 4;
+    f32x4_t g4 = {0.0f, 0.0f, 0.0f, 0.0f}, b4 = g4, p4 = g4;
+    if (i < H) {
+        p4 = *reinterpret_cast<const f32x4_t*>(pos + (size_t)s * H + i);
+        g4 = *reinterpret_cast<const f32x4_t*>(gamma + i);
+        b4 = *reinterpret_cast<const f32x4_t*>(beta + i);
+    }
+    id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
+    tt = tt < 0 ? 0 : (tt >= type_vocab ? type_vocab - 1 : tt);
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (i < H) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(word + (size_t)id * H + i);
+        const f32x4_t t4 = *reinterpret_cast<const f32x4_t*>(type + (size_t)tt * H + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (a[e] + p4[e]) + t4[e];
+    }
+    float* mrow = maskadd + (size_t)b * Sp;                     // as in embed_layernorm_kernel
+    if (!rowmap) {
+        if (threadIdx.x == 0) mrow[s] = (1.0f - (float)(mask ? mask[tok] : 1)) * -10000.0f;
+        if (s == 0 && wave == 0 && S + lane < Sp) mrow[S + lane] = -INFINITY;
+    } else if (s == 0) {
+        const int len = cu[b + 1] - cu[b];
+        for (int k = threadIdx.x; k < Sp; k += 256) mrow[k] = k < len ? 0.0f : (k < S ? -10000.0f : -INFINITY);
+    }
+    ln_group_row<LAYOUT>(v, d, lane, wave, g4, b4, x + (size_t)row * H, xb, row);
 }
 
 // One wave per score row of length S <= 512 (8 elements per lane, strided by
@@ -752,8 +803,15 @@ bool launch_embed_layernorm(const int* ids, const int* seg, const int* mask, con
         return false;
     }
     const long rows = compact ? compact->rows : (long)B * S;
-    dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    auto kernel = xb_layout == kSplit ? embed_layernorm_kernel<kSplit> : xb_layout == kUnits ? embed_layernorm_kernel<kUnits> : xb_layout == kPacked ? embed_layernorm_kernel<kPacked> : embed_layernorm_kernel<kRowMajor>;
+    // (the lines of the LayerNorm that adds: with the split copy a row's own pieces are 16 bytes, and many rows are bound by those)
+    const bool group = rows <= (xb_layout == kSplit ? kRowPerGroupSplit : kRowPerGroup);
+    dim3 grid((unsigned)(group ? rows : (rows + 3) / 4)), block(256);
+    auto pick = [&](auto layout) {
+        constexpr int L = decltype(layout)::value;
+        return group ? embed_layernorm_row_kernel<L> : embed_layernorm_kernel<L>;
+    };
+    auto kernel = xb_layout == kSplit ? pick(std::integral_constant<int, kSplit>()) : xb_layout == kUnits ? pick(std::integral_constant<int, kUnits>())
+                : xb_layout == kPacked ? pick(std::integral_constant<int, kPacked>()) : pick(std::integral_constant<int, kRowMajor>());
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, ids, seg, mask, word, pos, type, gamma,
                        beta, x, xb, maskadd, B, S, Sp, ln_dims(H), vocab, type_vocab,
                        compact ? compact->rowmap : nullptr, compact ? compact->cu : nullptr, (int)rows);
