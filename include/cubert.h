@@ -246,7 +246,7 @@ int cubert_op_gemm_residual(const void* X, const void* W, const float* bias, con
  * cuda_bert/ops/layernorm.cu:136-206, after op_Linear::forward, ops/linear.cu:91-148):
  *   Y[M,N] (float32, may be R itself) = LayerNorm(X * W^T + bias + R) * gamma + beta   per row,
  * eps 1e-12 inside the square root, biased variance; xb (optional) receives a bf16 copy of Y, row-major
- * or (CUBERT_Y_PACKED) in the packed operand layout.  bf16 operands, tile 256 or 384 (0 = automatic,
+ * or (CUBERT_Y_PACKED) in the packed operand layout.  bf16 operands, tile 256, 386 or 384 (0 = automatic,
  * which needs a problem large enough for one of them), N a multiple of 256 up to 1024, no split K.
  * The N / 256 workgroups that hold the same rows exchange partial row sums through `workspace`:
  * cubert_gemm_layernorm_workspace_bytes(M) bytes of device memory, all zero before the first launch
