@@ -109,11 +109,12 @@ class BatchPacked:
 class BatchContainer:
     """Lines of one length bucket (engine.py:12-61)."""
 
-    def __init__(self, base_length: int, top_length: int, batchsize: int, on_ready: Callable[[int], None] = lambda num_line: None):
+    def __init__(self, base_length: int, top_length: int, batchsize: int, queue: Optional[List[tuple]] = None, index: int = 0):
         self.base_length = base_length
         self.top_length = top_length
         self.batchsize = batchsize
-        self.on_ready = on_ready             # told the first line of every batch that becomes ready
+        self.queue = [] if queue is None else queue      # heap that every batch joins when it becomes ready: (first line, index)
+        self.index = index
         self.temp: List[TaggedLine] = []
         self.prepare: deque = deque()
 
@@ -133,7 +134,7 @@ class BatchContainer:
         while at and self.prepare[at - 1].lines_list[0].num_line > lines[0].num_line:
             at -= 1
         self.prepare.insert(at, BatchPacked(lines, optimize_batch(lines)))
-        self.on_ready(lines[0].num_line)
+        heappush(self.queue, (lines[0].num_line, self.index))
 
     def force_enqueue(self):
         self._batch()
@@ -157,7 +158,7 @@ class QueueManager:
         # (first line, bucket) of every ready batch.  The loop asks for one after every line it reads: looking at all the buckets
         # each time took 40 ms of host time for a file of 2000 lines, during which the device had nothing to do.
         self.queue: List[tuple] = []
-        self.containers = [BatchContainer(a, b, batchsize, lambda num_line, q=q: heappush(self.queue, (num_line, q)))
+        self.containers = [BatchContainer(a, b, batchsize, self.queue, q)
                            for q, (a, b) in enumerate(zip(self.boardlines, self.boardlines[1:]))]
 
     def put(self, line: TaggedLine):

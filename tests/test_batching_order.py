@@ -1,4 +1,5 @@
 """The ready batch with the earliest line goes first, however the batches became ready and whoever took some of them."""
+import copy
 import random
 
 import numpy as np
@@ -43,3 +44,11 @@ def test_earliest_line_first(seed):
 def test_length_above_the_last_edge_is_refused():
     with pytest.raises(ValueError):
         Bt.QueueManager([0, 8], batchsize=2).put(line(0, 9))
+
+
+def test_a_copy_is_a_manager_of_its_own():
+    qm = Bt.QueueManager([2, 8, 40], batchsize=2)
+    qm.put(line(0, 5))
+    twin = copy.deepcopy(qm)
+    twin.put(line(1, 5))
+    assert qm.get() is None and [l.num_line for l in twin.get().lines_list] == [0, 1]
