@@ -333,20 +333,28 @@ bool gemm_ln_workspace_force_expiry(void* ln_ws) {
     return true;
 }
 
+// A launch of the LayerNorm GEMM with tiles of `rows` tokens gives every CU at most one workgroup.  Counted for the XCD with most
+// of them: ln_tile_of_block hands out whole bands, band b and its N / 256 workgroups to XCD b % 8, and an XCD has 32 CUs.  With
+// N = 768, 81 to 85 bands are 243 to 255 workgroups, but 33 on up to five of the XCDs.
+bool gemm_ln_one_round(int M, int N, int rows) {
+    const long bands = ((long)M + rows - 1) / rows;
+    return (bands + 7) / 8 * (N / 256) <= 32;
+}
+
 // Tile of a GEMM with the LayerNorm in its epilogue, 0 if the separate kernels are the better choice (below about 6000
 // rows; N = 768 and 1024, K = N and 4 N).  The smallest tile that still makes one round of at most one workgroup per CU, since a
 // launch lasts as long as its slowest CU; beyond that the 256 x 256 one.  Microseconds, cold weights, N = 1024, K = 1024 / 4096,
 // with 128 / 192 / 256 tokens:  8192 rows 35.3 / 35.5 / 39.4 and 76.1 / 78.9 / 89.7;  8448 (264 tiles of 128 tokens) 43.4 / 36.6 /
 // 39.9 and 101 / 81.2 / 90.3;  10947 48.5 / 41.2 / 43.8 and 112 / 89.6 / 96.6;  12288 51.3 / 44.0 / 45.7 and 116 / 96.4 / 99.9;
-// 12416 (260 tiles of 192 tokens) 51.9 / 65.4 / 46.7 and 116 / 150 / 102.  N = 768, K = 768 / 3072, 12170 rows 40.6 / 33.4 / 37.6 and
-// 83.8 / 66.5 / 74.2.  The parts of a pass on two streams take the same tiles: 18009 rows of BERT-large 12.76 ms against 12.80, 20926
+// 12416 (260 tiles of 192 tokens) 51.9 / 65.4 / 46.7 and 116 / 150 / 102.  N = 768, K = 768 / 3072:  10240 rows 30.0 / 32.5 / 37.2
+// and 54.8 / 57.8 / 66.2;  10241 (81 bands of 128 tokens) 35.3 / 31.2 / 35.9 and 76.3 / 57.9 / 66.4;  12170 40.6 / 33.4 / 37.6 and
+// 83.8 / 66.5 / 74.2;  15360 42.4 / 36.2 / 40.2 and 88.0 / 73.9 / 81.6;  15361 (81 bands of 192) 42.6 / 53.7 / 40.0 and 88.4 / 115 /
+// 81.5.  The parts of a pass on two streams take the same tiles: 18009 rows of BERT-large 12.76 ms against 12.80, 20926
 // rows 15.17 against 15.27 with 256 tokens.
 int gemm_ln_pick_tile(int M, int N, int K, int elt) {
     if (M < 6144 || !ln_shape_ok(N, K, elt)) return 0;
-    auto tiles = [&](int rows) { return (long)((M + rows - 1) / rows) * (N / 256); };
-    if (K % 128 != 0 || tiles(128) <= 256) return kTile256x128;
-    if (tiles(192) <= 256) return kTile256x192;
-    return tiles(256) >= 128 ? 256 : kTile256x128;
+    if (K % 128 != 0 || gemm_ln_one_round(M, N, 128)) return kTile256x128;
+    return gemm_ln_one_round(M, N, 192) ? kTile256x192 : 256;
 }
 
 bool gemm_ln_supported(int M, int N, int K, int elt) { return gemm_ln_pick_tile(M, N, K, elt) != 0; }
