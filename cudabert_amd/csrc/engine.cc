@@ -484,16 +484,16 @@ int Model::pick_attention(int B, int S) const {
     return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
 }
 
-int Model::parts_for(long rows, int B) const {
-    const int parts = std::min(std::min(opt_.split_parts, (int)kMaxParts), B);
-    if (parts < 2 || opt_.split_min_tokens <= 0 || rows < opt_.split_min_tokens) return 1;
+int Model::parts_of(const ModelOptions& opt, long rows, int B) {
+    const int parts = std::min(std::min(opt.split_parts, (int)kMaxParts), B);
+    if (parts < 2 || opt.split_min_tokens <= 0 || rows < opt.split_min_tokens) return 1;
     // One stream while the 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) fill one round of the
     // 256 CUs to seven eighths: there is little left for a second stream to fill, and halves would need two rounds of smaller
     // launches.  BERT-large, one stream against two: 14783 rows 10.50 / 10.91 ms, 16325 (256 tiles) 11.85 / 12.68, 17036
-    // (268 tiles) 14.40 / 12.19; BERT-base, 16384 rows (192 tiles) 3.94 / 3.66, 19877 (234) 4.69 / 4.67.
-    if (opt_.split_keeps_one_round && opt_.fuse_layernorm && opt_.dims.hidden % 256 == 0) {
-        const long tiles = (rows + 255) / 256 * (opt_.dims.hidden / 256);
-        if (tiles >= 224 && tiles <= 256) return 1;
+    // (268 tiles) 14.40 / 12.19; BERT-base, 16384 rows (192 tiles) 3.94 / 3.66, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
+    if (opt.split_keeps_one_round && opt.fuse_layernorm && opt.dims.hidden % 256 == 0) {
+        const long tiles = (rows + 255) / 256 * (opt.dims.hidden / 256);
+        if (tiles >= 224 && gemm_ln_one_round((int)rows, opt.dims.hidden, 256)) return 1;
     }
     return parts;
 }

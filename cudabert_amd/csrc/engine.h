@@ -27,7 +27,7 @@ struct ModelOptions {
     int split_parts = 2;           // number of parts (1..4) a large batch is cut into
     int split_min_tokens = 14336;  // passes over at least this many token rows run as two halves on two streams (0: never);
                                    // the C API's default follows the precision
-    bool split_keeps_one_round = false;   // ... but not where one launch's tiles cover the chip once (bf16; parts_for)
+    bool split_keeps_one_round = false;   // ... but not where one launch's tiles cover the chip once (bf16; parts_of)
     bool fuse_residual = true;     // residual add in the epilogue of the GEMM before each LayerNorm
     bool fuse_layernorm = true;    // ... and the LayerNorm itself, where the GEMM kernel supports it (bf16, large batches)
     bool v_rowmajor = true;        // bf16, S <= 512: V is stored [B, heads, S, 64] like K; attention transposes on its LDS reads
@@ -53,6 +53,7 @@ struct LayerDev {
 class Model {
   public:
     static Model* create(const ModelOptions& opt);     // nullptr + error text on failure
+    static int parts_of(const ModelOptions& opt, long rows, int B);   // parts a pass over that many token rows of B sequences is cut into
     ~Model();
 
     // Host inputs [B, S] int32 (mask may be nullptr).  Asynchronous.
@@ -101,7 +102,7 @@ class Model {
     bool check_shape(int B, int S);
     bool run(int B, int S, bool has_mask);             // graph or eager
     int pick_attention(int B, int S) const;            // cur_attn_ for a batch
-    int parts_for(long rows, int B) const;             // parts a pass over that many token rows is cut into
+    int parts_for(long rows, int B) const { return parts_of(opt_, rows, B); }
     bool enqueue(int B, int S, bool has_mask);         // the launch sequence (one or two parts)
     bool enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp = nullptr);
     // padded_bits: the sums are grouped as in the padded pass of the batch, else as the computed rows ask for
