@@ -491,10 +491,10 @@ int Model::parts_of(const ModelOptions& opt, long rows, int B) {
     // 256 CUs to seven eighths: there is little left for a second stream to fill, and halves would need two rounds of smaller
     // launches.  BERT-large, one stream against two: 14783 rows 10.50 / 10.91 ms, 16325 (256 tiles) 11.85 / 12.68, 17036
     // (268 tiles) 14.40 / 12.19; BERT-base, 16384 rows (192 tiles) 3.94 / 3.66, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
-    if (opt.split_keeps_one_round && opt.fuse_layernorm && opt.dims.hidden % 256 == 0) {
-        const long tiles = (rows + 255) / 256 * (opt.dims.hidden / 256);
-        if (tiles >= 224 && gemm_ln_one_round((int)rows, opt.dims.hidden, 256)) return 1;
-    }
+    const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
+    if (opt.split_keeps_one_round && opt.fuse_residual && opt.fuse_layernorm && gemm_ln_pick_tile(M, H, H, opt.precision) == 256 &&
+        gemm_ln_pick_tile(M, H, I, opt.precision) == 256 && (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256))
+        return 1;
     return parts;
 }
 

@@ -44,7 +44,6 @@ bool launch_gemm_bf16_t256x192_ln(const gemm_detail::GemmDev& d, hipStream_t str
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream);
 bool launch_gemm_split(const gemm_detail::GemmDev& d, int tile, int epilogue, hipStream_t stream);
 int gemm_pick_tile(int M, int N, int K, int elt);
-int gemm_ln_pick_tile(int M, int N, int K, int elt);
 
 namespace {
 

@@ -122,6 +122,8 @@ bool gemm_ln_workspace_force_expiry(void* ln_ws);
 // True if launch_gemm can run the LayerNorm of a [M, N] float32 result in the epilogue of a
 // bf16 GEMM with reduction length K.
 bool gemm_ln_supported(int M, int N, int K, int elt);
+// GemmParams::tile value that it takes for the problem (0: none, the LayerNorm is better a kernel of its own).
+int gemm_ln_pick_tile(int M, int N, int K, int elt);
 // True if that GEMM, with tiles of 256 features x `rows` tokens, puts at most one workgroup on every CU.
 bool gemm_ln_one_round(int M, int N, int rows);
 

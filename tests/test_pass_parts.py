@@ -12,8 +12,10 @@ int main(int argc, char** argv) {
     opt.precision = cubert::kBF16;
     opt.split_keeps_one_round = true;
     opt.dims.hidden = std::atoi(argv[1]);
-    opt.dims.inter = 4 * opt.dims.hidden;
-    for (int i = 2; i < argc; ++i) std::printf("%d\n", cubert::Model::parts_of(opt, std::atol(argv[i]), 128));
+    opt.dims.inter = std::atoi(argv[2]);
+    opt.fuse_residual = std::atoi(argv[3]);
+    opt.fuse_layernorm = std::atoi(argv[4]);
+    for (int i = 5; i < argc; ++i) std::printf("%d\n", cubert::Model::parts_of(opt, std::atol(argv[i]), 128));
 }
 """
 
@@ -23,8 +25,8 @@ def program(tmp_path_factory):
     return compile_program(PROGRAM, tmp_path_factory.mktemp("parts"))
 
 
-def parts(program, hidden, rows):
-    return list(map(int, lines(program, hidden, *rows)))
+def parts(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1):
+    return list(map(int, lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, *rows)))
 
 
 def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
@@ -35,3 +37,9 @@ def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
 
 def test_one_round_of_1024_features(program):
     assert parts(program, 1024, [14335, 14336, 16384, 16385]) == [1, 1, 1, 2]
+
+
+@pytest.mark.parametrize("without", [dict(fuse_residual=0), dict(fuse_layernorm=0), dict(inter=4128)])
+def test_one_stream_asks_for_the_gemms_it_counts(program, without):
+    """No residual or no LayerNorm in the epilogue, or an FFN-out (K not a multiple of 128) that does not have the 256 x 256 tile."""
+    assert parts(program, 1024, [14336, 16384], **without) == [2, 2]
