@@ -310,7 +310,7 @@ bool Model::forward_host(const int* ids, const int* seg, const int* mask, int B,
         }
         if (prefix && (opt_.varlen == 1 || valid * 20 <= n * 19)) return run_compact(lens.data(), B, S, opt_.varlen < 0);
     }
-    return run(B, S, mask != nullptr);
+    return run(B, S, mask != nullptr, true);
 }
 
 bool Model::forward_device_lens(const int* d_ids, const int* d_seg, const int* h_lens, int B, int S) {
@@ -334,6 +334,7 @@ bool Model::forward_device_lens(const int* d_ids, const int* d_seg, const int* h
 bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     B_ = B;
     S_ = S;
+    waited_ = true;                   // for the metadata, below
     last_compact_ = true;
     last_padded_bits_ = padded_bits;
     last_classified_ = false;
@@ -399,12 +400,13 @@ bool Model::forward_device(const int* d_ids, const int* d_seg, const int* d_mask
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_, d_ids, n * 4, hipMemcpyDeviceToDevice, stream_));
     CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + n, d_seg, n * 4, hipMemcpyDeviceToDevice, stream_));
     if (d_mask) CUBERT_HIP_OK(hipMemcpyAsync(d_in_ + 2 * n, d_mask, n * 4, hipMemcpyDeviceToDevice, stream_));
-    return run(B, S, d_mask != nullptr);
+    return run(B, S, d_mask != nullptr, false);
 }
 
-bool Model::run(int B, int S, bool has_mask) {
+bool Model::run(int B, int S, bool has_mask, bool waited) {
     B_ = B;
     S_ = S;
+    waited_ = waited && (opt_.graph_max_tokens <= 0 || (long)B * S > opt_.graph_max_tokens);
     last_compact_ = false;
     last_has_mask_ = has_mask;
     last_classified_ = false;
@@ -484,16 +486,21 @@ int Model::pick_attention(int B, int S) const {
     return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
 }
 
-int Model::parts_of(const ModelOptions& opt, long rows, int B) {
+int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
     const int parts = std::min(std::min(opt.split_parts, (int)kMaxParts), B);
     if (parts < 2 || opt.split_min_tokens <= 0 || rows < opt.split_min_tokens) return 1;
     // One stream while the 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) fill one round of the
-    // 256 CUs to seven eighths: there is little left for a second stream to fill, and halves would need two rounds of smaller
-    // launches.  BERT-large, one stream against two: 14783 rows 10.50 / 10.91 ms, 16325 (256 tiles) 11.85 / 12.68, 17036
-    // (268 tiles) 14.40 / 12.19; BERT-base, 16384 rows (192 tiles) 3.94 / 3.66, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
+    // 256 CUs to seven eighths: there is little left for a second stream to fill, and it starts late, since its launches are
+    // enqueued after all of the first one's.  One stream / two, in ms:  BERT-large, valid tokens, 14498 rows 10.65 / 11.71, 16323
+    // 12.04 / 12.78; pooled output on the host, 15360 rows 10.72 / 10.97, 16384 11.03 / 11.81; BERT-base, the same, 19072 rows
+    // 4.08 / 4.13, 20480 4.30 / 4.36.  Not for passes that queue up on the device, where the second stream is as early as the first
+    // (BERT-large, 14336 rows 9.51 / 9.36, 15360 10.87 / 10.51, BERT-base, 19456 4.29 / 4.24), nor for narrower models (host, hidden
+    // 512, 30720 rows 3.63 / 3.51; hidden 256, 61440 rows 3.17 / 3.07), nor beyond the one round: BERT-large, 16512 rows (260 tiles)
+    // 13.73 / 11.26, BERT-base, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
     const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
-    if (opt.split_keeps_one_round && opt.fuse_residual && opt.fuse_layernorm && gemm_ln_pick_tile(M, H, H, opt.precision) == 256 &&
-        gemm_ln_pick_tile(M, H, I, opt.precision) == 256 && (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256))
+    if (waited && opt.split_keeps_one_round && H >= 768 && opt.fuse_residual && opt.fuse_layernorm &&
+        gemm_ln_pick_tile(M, H, H, opt.precision) == 256 && gemm_ln_pick_tile(M, H, I, opt.precision) == 256 &&
+        (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256))
         return 1;
     return parts;
 }
@@ -714,6 +721,7 @@ bool Model::profile_device(const int* d_ids, const int* d_seg, const int* d_mask
     B_ = B;
     S_ = S;
     first_only_ = false;
+    waited_ = false;
     last_compact_ = false;
     last_has_mask_ = d_mask != nullptr;
     last_classified_ = false;

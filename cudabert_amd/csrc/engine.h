@@ -53,7 +53,8 @@ struct LayerDev {
 class Model {
   public:
     static Model* create(const ModelOptions& opt);     // nullptr + error text on failure
-    static int parts_of(const ModelOptions& opt, long rows, int B);   // parts a pass over that many token rows of B sequences is cut into
+    // Parts a pass over that many token rows of B sequences is cut into.  waited: its launches reach an idle device one by one.
+    static int parts_of(const ModelOptions& opt, long rows, int B, bool waited);
     ~Model();
 
     // Host inputs [B, S] int32 (mask may be nullptr).  Asynchronous.
@@ -100,9 +101,9 @@ class Model {
     Model() = default;
     bool init(const ModelOptions& opt);
     bool check_shape(int B, int S);
-    bool run(int B, int S, bool has_mask);             // graph or eager
+    bool run(int B, int S, bool has_mask, bool waited);   // graph or eager
     int pick_attention(int B, int S) const;            // cur_attn_ for a batch
-    int parts_for(long rows, int B) const { return parts_of(opt_, rows, B); }
+    int parts_for(long rows, int B) const { return parts_of(opt_, rows, B, waited_); }
     bool enqueue(int B, int S, bool has_mask);         // the launch sequence (one or two parts)
     bool enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mask, hipStream_t st, const Compact* cp = nullptr);
     // padded_bits: the sums are grouped as in the padded pass of the batch, else as the computed rows ask for
@@ -157,6 +158,7 @@ class Model {
     unsigned char* xbc_ = nullptr;                 // GEMM-operand copy
     void *ctxc_ = nullptr, *hc_ = nullptr;         // attention context / FFN activation of those rows
     bool first_only_ = false;                      // the pass being enqueued (and the last one run) is of that kind
+    bool waited_ = false;                          // the host waited for the pass before this one, and this one is not a graph
     bool last_compact_ = false;
     bool last_padded_bits_ = false;
     // Rows on which split counts and skinny tiles, which regroup sums, are decided: those of the pass, or of the padded pass

@@ -15,7 +15,8 @@ int main(int argc, char** argv) {
     opt.dims.inter = std::atoi(argv[2]);
     opt.fuse_residual = std::atoi(argv[3]);
     opt.fuse_layernorm = std::atoi(argv[4]);
-    for (int i = 5; i < argc; ++i) std::printf("%d\n", cubert::Model::parts_of(opt, std::atol(argv[i]), 128));
+    const bool waited = std::atoi(argv[5]);
+    for (int i = 6; i < argc; ++i) std::printf("%d\n", cubert::Model::parts_of(opt, std::atol(argv[i]), 128, waited));
 }
 """
 
@@ -25,8 +26,8 @@ def program(tmp_path_factory):
     return compile_program(PROGRAM, tmp_path_factory.mktemp("parts"))
 
 
-def parts(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1):
-    return list(map(int, lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, *rows)))
+def parts(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1, waited=1):
+    return list(map(int, lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, waited, *rows)))
 
 
 def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
@@ -43,3 +44,14 @@ def test_one_round_of_1024_features(program):
 def test_one_stream_asks_for_the_gemms_it_counts(program, without):
     """No residual or no LayerNorm in the epilogue, or an FFN-out (K not a multiple of 128) that does not have the 256 x 256 tile."""
     assert parts(program, 1024, [14336, 16384], **without) == [2, 2]
+
+
+@pytest.mark.parametrize("hidden", [768, 1024])
+def test_passes_that_queue_up_on_the_device_run_on_two_streams(program, hidden):
+    rows = [14336, 16384, 18945, 20480]
+    assert parts(program, hidden, rows, waited=0) == [2] * 4 != parts(program, hidden, rows)
+
+
+@pytest.mark.parametrize("hidden", [256, 512])
+def test_narrow_models_run_on_two_streams(program, hidden):
+    assert set(parts(program, hidden, range(14336, 70000, 256))) == {2}
