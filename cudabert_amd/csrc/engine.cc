@@ -342,6 +342,7 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     long tokens = 0;                  // rows this pass computes: the valid tokens
     for (int b = 0; b < B; ++b) tokens += lens[b];
     const int parts = parts_for(tokens, B);
+    ln_tile_ = ln_tile_of_parts(opt_, tokens, parts);
     // (a padded pass that runs in parts regroups nothing, and then neither does this one)
     const long order_rows = padded_bits ? (long)B * S : tokens;
     order_rows_ = opt_.split_k && parts_for(order_rows, B) == 1 ? (int)order_rows : 0;
@@ -486,23 +487,34 @@ int Model::pick_attention(int B, int S) const {
     return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
 }
 
+// The 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) of all the rows of a pass fill one round of the
+// 256 CUs, to seven eighths at least.  Models of hidden 768 and more: see the figures of the two rules below.
+static bool ln_tiles_are_one_round(const ModelOptions& opt, long rows) {
+    const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
+    return H >= 768 && opt.fuse_residual && opt.fuse_layernorm && gemm_ln_pick_tile(M, H, H, opt.precision) == 256 &&
+           gemm_ln_pick_tile(M, H, I, opt.precision) == 256 && (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256);
+}
+
 int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
     const int parts = std::min(std::min(opt.split_parts, (int)kMaxParts), B);
     if (parts < 2 || opt.split_min_tokens <= 0 || rows < opt.split_min_tokens) return 1;
-    // One stream while the 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) fill one round of the
-    // 256 CUs to seven eighths: there is little left for a second stream to fill, and it starts late, since its launches are
-    // enqueued after all of the first one's.  One stream / two, in ms:  BERT-large, valid tokens, 14498 rows 10.65 / 11.71, 16323
-    // 12.04 / 12.78; pooled output on the host, 15360 rows 10.72 / 10.97, 16384 11.03 / 11.81; BERT-base, the same, 19072 rows
-    // 4.08 / 4.13, 20480 4.30 / 4.36.  Not for passes that queue up on the device, where the second stream is as early as the first
-    // (BERT-large, 14336 rows 9.51 / 9.36, 15360 10.87 / 10.51, BERT-base, 19456 4.29 / 4.24), nor for narrower models (host, hidden
-    // 512, 30720 rows 3.63 / 3.51; hidden 256, 61440 rows 3.17 / 3.07), nor beyond the one round: BERT-large, 16512 rows (260 tiles)
-    // 13.73 / 11.26, BERT-base, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
-    const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
-    if (waited && opt.split_keeps_one_round && H >= 768 && opt.fuse_residual && opt.fuse_layernorm &&
-        gemm_ln_pick_tile(M, H, H, opt.precision) == 256 && gemm_ln_pick_tile(M, H, I, opt.precision) == 256 &&
-        (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256))
-        return 1;
-    return parts;
+    // One stream while the LayerNorm GEMMs are one round: there is little left for a second stream to fill, and it starts late,
+    // since its launches are enqueued after all of the first one's.  One stream / two, in ms:  BERT-large, valid tokens, 14498 rows
+    // 10.65 / 11.71, 16323 12.04 / 12.78; pooled output on the host, 15360 rows 10.72 / 10.97, 16384 11.03 / 11.81; BERT-base, the
+    // same, 19072 rows 4.08 / 4.13, 20480 4.30 / 4.36.  Not for passes that queue up on the device, where the second stream is as
+    // early as the first (BERT-large, 14336 rows 9.51 / 9.36, 15360 10.87 / 10.51, BERT-base, 19456 4.29 / 4.24), nor for narrower
+    // models (host, hidden 512, 30720 rows 3.63 / 3.51; hidden 256, 61440 rows 3.17 / 3.07), nor beyond the one round: BERT-large,
+    // 16512 rows (260 tiles) 13.73 / 11.26, BERT-base, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
+    return waited && opt.split_keeps_one_round && ln_tiles_are_one_round(opt, rows) ? 1 : parts;
+}
+
+// Parts of such a pass run their LayerNorm GEMMs beside each other, so that the 256 x 256 tiles of all parts cover the chip once;
+// chosen for a part alone, the tile would be the one that covers it with the part.  Queued passes of 128 lines in two parts, tiles of
+// 128 / 192 / 256 tokens, in ms:  BERT-large, 14464 rows 9.56 / 9.63 / 9.38, 15360 10.63 / 10.22 / 10.48, 16384 11.13 / 10.97 /
+// 10.61; BERT-base, 19072 4.17 / 4.34 / 4.16, 20480 4.36 / 4.43 / 4.25.  Narrower models: hidden 512, 28672 rows 3.36 / 3.42 / 3.55;
+// hidden 256, 65536 rows 3.29 / 3.22 / 3.42.
+int Model::ln_tile_of_parts(const ModelOptions& opt, long rows, int parts) {
+    return parts > 1 && ln_tiles_are_one_round(opt, rows) ? 256 : 0;
 }
 
 // One forward pass.  A large batch is cut into parts of whole sequences that run
@@ -512,6 +524,7 @@ int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
 bool Model::enqueue(int B, int S, bool has_mask) {
     cur_attn_ = pick_attention(B, S);
     const int parts = profiling_ ? 1 : parts_for((long)B * S, B);
+    ln_tile_ = ln_tile_of_parts(opt_, (long)B * S, parts);
     order_rows_ = opt_.split_k && parts == 1 ? B * S : 0;
     if (parts == 1) return enqueue_part(0, 0, B, 0, S, has_mask, stream_);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));
@@ -668,7 +681,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = tile_ao;
         g.k_order = plan_ao.k_order();
-        if (ln_ao) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
+        if (ln_ao) { g.tile = ln_tile_; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
         if (!ln_ao && !launch_add_layernorm(x32, y32, kF32, L.g1, L.be1, xb, layout, N, H, st, sp_ao, !fuse_res)) return false;
@@ -685,7 +698,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         g.residual = fuse_res ? x32 : nullptr;
         g.tile = tile_fo;
         g.k_order = plan_fo.k_order();
-        if (ln_fo) { g.tile = 0; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
+        if (ln_fo) { g.tile = ln_tile_; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
         if (!ln_fo && !launch_add_layernorm(x32, y32, kF32, L.g2, L.be2, xb, layout, N, H, st, sp_fo, !fuse_res)) return false;

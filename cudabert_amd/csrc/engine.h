@@ -55,6 +55,8 @@ class Model {
     static Model* create(const ModelOptions& opt);     // nullptr + error text on failure
     // Parts a pass over that many token rows of B sequences is cut into.  waited: its launches reach an idle device one by one.
     static int parts_of(const ModelOptions& opt, long rows, int B, bool waited);
+    // GemmParams::tile of the LayerNorm GEMMs of a pass over that many rows in that many parts (0: chosen for each launch alone).
+    static int ln_tile_of_parts(const ModelOptions& opt, long rows, int parts);
     ~Model();
 
     // Host inputs [B, S] int32 (mask may be nullptr).  Asynchronous.
@@ -164,6 +166,7 @@ class Model {
     // Rows on which split counts and skinny tiles, which regroup sums, are decided: those of the pass, or of the padded pass
     // whose bits it has to give.  0: nothing is regrouped (split_k off, or a pass in parts).
     int order_rows_ = 0;
+    int ln_tile_ = 0;               // ln_tile_of_parts of the pass being enqueued
     int cur_attn_ = kAttnPerHead;   // attention kernel of the pass being enqueued (decided on the whole batch)
     int B_ = 0, S_ = 0;
     // hipGraph cache: one entry per (B, S, mask) shape, captured on second sight, at most

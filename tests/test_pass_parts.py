@@ -16,7 +16,11 @@ int main(int argc, char** argv) {
     opt.fuse_residual = std::atoi(argv[3]);
     opt.fuse_layernorm = std::atoi(argv[4]);
     const bool waited = std::atoi(argv[5]);
-    for (int i = 6; i < argc; ++i) std::printf("%d\n", cubert::Model::parts_of(opt, std::atol(argv[i]), 128, waited));
+    for (int i = 6; i < argc; ++i) {
+        const long rows = std::atol(argv[i]);
+        const int parts = cubert::Model::parts_of(opt, rows, 128, waited);
+        std::printf("%d %d\n", parts, cubert::Model::ln_tile_of_parts(opt, rows, parts));
+    }
 }
 """
 
@@ -26,8 +30,14 @@ def program(tmp_path_factory):
     return compile_program(PROGRAM, tmp_path_factory.mktemp("parts"))
 
 
-def parts(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1, waited=1):
-    return list(map(int, lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, waited, *rows)))
+def plan(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1, waited=1):
+    """(parts, tile of the LayerNorm GEMMs that the pass prescribes) for every row count."""
+    out = lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, waited, *rows)
+    return [tuple(map(int, l.split())) for l in out]
+
+
+def parts(*args, **kw):
+    return [p for p, _ in plan(*args, **kw)]
 
 
 def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
@@ -55,3 +65,13 @@ def test_passes_that_queue_up_on_the_device_run_on_two_streams(program, hidden):
 @pytest.mark.parametrize("hidden", [256, 512])
 def test_narrow_models_run_on_two_streams(program, hidden):
     assert set(parts(program, hidden, range(14336, 70000, 256))) == {2}
+
+
+@pytest.mark.parametrize("hidden,first,last", [(1024, 14336, 16384), (768, 18945, 20480)])
+def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, first, last):
+    rows = range(first, last + 1, 7)
+    assert set(plan(program, hidden, rows, waited=0)) == {(2, 256)}
+    assert set(plan(program, hidden, rows)) == {(1, 0)}
+    beside = [14335, first - 1, last + 1, 25600, 32768]
+    assert {t for _, t in plan(program, hidden, beside, waited=0)} == {0}
+    assert {t for _, t in plan(program, hidden, rows, waited=0, fuse_layernorm=0)} == {0}
