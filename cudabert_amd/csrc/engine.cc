@@ -343,9 +343,7 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     for (int b = 0; b < B; ++b) tokens += lens[b];
     const int parts = parts_for(tokens, B);
     ln_tile_ = ln_tile_of_parts(opt_, tokens, parts);
-    // (a padded pass that runs in parts regroups nothing, and then neither does this one)
-    const long order_rows = padded_bits ? (long)B * S : tokens;
-    order_rows_ = opt_.split_k && parts_for(order_rows, B) == 1 ? (int)order_rows : 0;
+    order_rows_ = (int)order_rows_of(opt_, tokens, padded_bits ? (long)B * S : tokens, B, waited_);
     // the pinned metadata of the previous call must have been consumed
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
     const size_t cap = (size_t)cap_tokens_;
@@ -506,6 +504,13 @@ int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
     // models (host, hidden 512, 30720 rows 3.63 / 3.51; hidden 256, 61440 rows 3.17 / 3.07), nor beyond the one round: BERT-large,
     // 16512 rows (260 tiles) 13.73 / 11.26, BERT-base, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
     return waited && opt.split_keeps_one_round && ln_tiles_are_one_round(opt, rows) ? 1 : parts;
+}
+
+// Parts regroup nothing: they sit side by side in y32, which has no room for partial sums there.  A pass in one part gives the bits
+// of one in parts, and the other way round (a pass of the valid rows may be in more parts than the padded one: 15000 valid rows of
+// 20000 of BERT-base), only if neither regroups.
+long Model::order_rows_of(const ModelOptions& opt, long rows, long bits_of, int B, bool waited) {
+    return opt.split_k && parts_of(opt, rows, B, waited) == 1 && parts_of(opt, bits_of, B, waited) == 1 ? bits_of : 0;
 }
 
 // Parts of such a pass run their LayerNorm GEMMs beside each other, so that the 256 x 256 tiles of all parts cover the chip once;

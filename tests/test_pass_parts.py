@@ -19,7 +19,10 @@ int main(int argc, char** argv) {
     for (int i = 6; i < argc; ++i) {
         const long rows = std::atol(argv[i]);
         const int parts = cubert::Model::parts_of(opt, rows, 128, waited);
-        std::printf("%d %d\n", parts, cubert::Model::ln_tile_of_parts(opt, rows, parts));
+        std::printf("%d %d", parts, cubert::Model::ln_tile_of_parts(opt, rows, parts));
+        for (long bits_of : {1000, 12000, 14336, 16000, 19000, 20000, 20480, 22000})
+            std::printf(" %ld", cubert::Model::order_rows_of(opt, rows, bits_of, 128, waited));
+        std::puts("");
     }
 }
 """
@@ -33,7 +36,7 @@ def program(tmp_path_factory):
 def plan(program, hidden, rows, inter=None, fuse_residual=1, fuse_layernorm=1, waited=1):
     """(parts, tile of the LayerNorm GEMMs that the pass prescribes) for every row count."""
     out = lines(program, hidden, inter or 4 * hidden, fuse_residual, fuse_layernorm, waited, *rows)
-    return [tuple(map(int, l.split())) for l in out]
+    return [tuple(map(int, l.split()[:2])) for l in out]
 
 
 def parts(*args, **kw):
@@ -75,3 +78,13 @@ def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, f
     beside = [14335, first - 1, last + 1, 25600, 32768]
     assert {t for _, t in plan(program, hidden, beside, waited=0)} == {0}
     assert {t for _, t in plan(program, hidden, rows, waited=0, fuse_layernorm=0)} == {0}
+
+
+@pytest.mark.parametrize("hidden", [256, 768, 1024])
+def test_a_pass_in_parts_regroups_no_sums(program, hidden):
+    """Nor does one that gives the bits of a pass in parts.  (768: 20000 padded rows are one part, 15000 valid ones two.)"""
+    rows, bits_of = [900, 11000, 14335, 14336, 15000, 18000, 18945, 20000], [1000, 12000, 14336, 16000, 19000, 20000, 20480, 22000]
+    of = dict(zip(rows + bits_of, parts(program, hidden, rows + bits_of)))
+    for n, l in zip(rows, lines(program, hidden, 4 * hidden, 1, 1, 1, *rows)):
+        for padded, order in zip(bits_of, map(int, l.split()[2:])):
+            assert order == (padded if of[n] == of[padded] == 1 else 0), (n, padded)
