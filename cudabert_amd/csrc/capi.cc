@@ -53,11 +53,7 @@ void* make_model(const cubert_config& cfg, int gpu, int maxB, int maxS, const ch
     opt.precision = cfg.precision;
     opt.graph_max_tokens = cfg.graph_max_tokens;
     opt.graph_cache = env_int("CUBERT_GRAPH_CACHE", 64);
-    // measured: one stream is the faster choice below about 14 thousand token rows in bf16 mode
-    // (11 - 12 thousand rows: +3 ... 7 %), two streams already from 8 thousand in fp32 mode (+6 ... 13 %)
-    opt.split_min_tokens = env_int("CUBERT_SPLIT_MIN_TOKENS", cfg.precision == cubert::kBF16 ? 14336 : 8192);
-    opt.split_keeps_one_round = cfg.precision == cubert::kBF16 && !std::getenv("CUBERT_SPLIT_MIN_TOKENS");
-    opt.split_parts = env_int("CUBERT_SPLIT_PARTS", 2);
+    cubert::read_split_options(&opt);
     opt.varlen = env_int("CUBERT_VARLEN", -1);
     opt.split_k = env_int("CUBERT_SPLIT_K", 1) != 0;
     opt.fuse_residual = env_int("CUBERT_FUSE_RESIDUAL", 1) != 0;
@@ -87,6 +83,18 @@ cubert_config preset(bool large) {
 const char* default_dir(bool large) { return large ? "model_npy/large_uncased" : "model_npy/base_uncased"; }
 
 }  // namespace
+
+namespace cubert {
+void read_split_options(ModelOptions* opt) {
+    // measured: one stream is the faster choice below about 14 thousand token rows in bf16 mode
+    // (11 - 12 thousand rows: +3 ... 7 %), two streams already from 8 thousand in fp32 mode (+6 ... 13 %)
+    const int least = opt->precision == kBF16 ? 14336 : 8192, parts = 2;
+    opt->split_min_tokens = env_int("CUBERT_SPLIT_MIN_TOKENS", least);
+    opt->split_parts = env_int("CUBERT_SPLIT_PARTS", parts);
+    // a caller who asks for other rows or another number of parts gets those
+    opt->split_keeps_one_round = env_int("CUBERT_SPLIT_ONE_ROUND", 1) != 0 && opt->split_min_tokens == least && opt->split_parts == parts;
+}
+}  // namespace cubert
 
 extern "C" {
 

@@ -27,7 +27,7 @@ struct ModelOptions {
     int split_parts = 2;           // number of parts (1..4) a large batch is cut into
     int split_min_tokens = 14336;  // passes over at least this many token rows run as two halves on two streams (0: never);
                                    // the C API's default follows the precision
-    bool split_keeps_one_round = false;   // ... but not where one launch's tiles cover the chip once (bf16; parts_of)
+    bool split_keeps_one_round = false;   // ... but not where one launch's tiles cover the chip once (parts_of)
     bool fuse_residual = true;     // residual add in the epilogue of the GEMM before each LayerNorm
     bool fuse_layernorm = true;    // ... and the LayerNorm itself, where the GEMM kernel supports it (bf16, large batches)
     bool v_rowmajor = true;        // bf16, S <= 512: V is stored [B, heads, S, 64] like K; attention transposes on its LDS reads
@@ -43,6 +43,9 @@ struct ModelOptions {
     int graph_cache = 64;          // instantiated hipGraphs kept per model (least recently used is dropped)
     std::string dir;
 };
+
+// split_parts, split_min_tokens and split_keeps_one_round from the environment and the precision.
+void read_split_options(ModelOptions* opt);
 
 struct LayerDev {
     void *w_qkv, *w_ao, *w_in, *w_out;            // [out, in] as GEMM operands: bf16 packed, or float32 split (common.h)

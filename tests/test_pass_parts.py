@@ -9,6 +9,12 @@ PROGRAM = r"""
 #include "engine.h"
 int main(int argc, char** argv) {
     cubert::ModelOptions opt;
+    if (argc == 2) {
+        opt.precision = std::atoi(argv[1]);
+        cubert::read_split_options(&opt);
+        std::printf("%d %d %d\n", opt.split_min_tokens, opt.split_parts, (int)opt.split_keeps_one_round);
+        return 0;
+    }
     opt.precision = cubert::kBF16;
     opt.split_keeps_one_round = true;
     opt.dims.hidden = std::atoi(argv[1]);
@@ -88,3 +94,20 @@ def test_a_pass_in_parts_regroups_no_sums(program, hidden):
     for n, l in zip(rows, lines(program, hidden, 4 * hidden, 1, 1, 1, *rows)):
         for padded, order in zip(bits_of, map(int, l.split()[2:])):
             assert order == (padded if of[n] == of[padded] == 1 else 0), (n, padded)
+
+
+@pytest.mark.parametrize("precision,least", [(0, 8192), (1, 14336)])
+def test_a_setting_of_the_default_value_changes_nothing(program, monkeypatch, precision, least):
+    for name in ("MIN_TOKENS", "PARTS", "ONE_ROUND"):
+        monkeypatch.delenv("CUBERT_SPLIT_" + name, raising=False)
+
+    def options(**env):
+        return tuple(map(int, lines(program, precision, **env)[0].split()))
+
+    own = options()
+    assert own == (least, 2, 1)
+    assert own == options(CUBERT_SPLIT_MIN_TOKENS=str(least)) == options(CUBERT_SPLIT_PARTS="2") == options(CUBERT_SPLIT_ONE_ROUND="1") \
+        == options(CUBERT_SPLIT_MIN_TOKENS="")
+    assert options(CUBERT_SPLIT_ONE_ROUND="0") == (least, 2, 0)
+    assert options(CUBERT_SPLIT_MIN_TOKENS="10000") == (10000, 2, 0)
+    assert options(CUBERT_SPLIT_PARTS="3") == (least, 3, 0)
