@@ -461,6 +461,10 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
 //   128 x 128, 256 x 128: (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly
 //     what the first did, and the hand-out is uneven by half a workgroup; the larger tile wins from about 900 tiles on;
 //   the skinny tiles: fixed + per_step * steps * (w > 1 ? w + 0.5 : 1), bound by what a CU fetches (60 - 65 GB/s of operands).
+// The 128 x 128 constants are those of its loop before it read fragments a step ahead (gemm_split.hip), which takes less from launches
+// of few workgroups: 1024 x 768 x 768 in 23.6 us for an estimate of 27.8.  At the lines they draw, skinny / 128 x 128 in us (* is
+// taken): 512 x 3072 x 1024 32.4* / 31.0, 512 x 4096 x 1024 35.6 / 34.7*, 768 x 2304 x 768 23.7* / 25.4, 1024 x 2304 x 768 30.8 /
+// 26.4*, 1024 x 3072 x 768 34.6 / 29.2*, and in 16 parts 192 x 1024 x 4096 21.4 / 23.2*, 256 x 1024 x 4096 27.1 / 23.6*.
 // At 128 rows (QKV 3072 x 1024 / FFN-in 4096 x 1024 / FFN-out 1024 x 4096): 13.9 / 15.6 / 14.6 us with the skinny tile,
 // 35.2 / 40.7 / 24.0 with the 128 one; at 1600 rows 81 / 102 / 102 against 65 / 79 / 76.
 GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, int order) {
@@ -622,7 +626,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
             ((reinterpret_cast<uintptr_t>(p.ln_gamma) | reinterpret_cast<uintptr_t>(p.ln_beta) |
               reinterpret_cast<uintptr_t>(p.ln_xb) | reinterpret_cast<uintptr_t>(p.ln_ws)) & 15)) {
             set_error("gemm: the LayerNorm epilogue needs a residual, bf16 operands, N a multiple of 256 up to 1024, the "
-                      "256 or 256x128 tile, no split K, a workspace and 16-byte aligned gamma / beta / copy");
+                      "256, 256x192 or 256x128 tile, no split K, a workspace and 16-byte aligned gamma / beta / copy");
             return false;
         }
         epi = kEpiBiasResLN;

@@ -560,7 +560,6 @@ __device__ __forceinline__ void gemm_epilogue_ln(const GemmDev& p, f32x16_t (&ac
                 qsq[t] = ln_sumsq4(acc[t >> 2][j][e0] - mu, acc[t >> 2][j][e0 + 1] - mu, acc[t >> 2][j][e0 + 2] - mu, acc[t >> 2][j][e0 + 3] - mu);
             }
             const float m2 = half_swap_sum(ln_tree16(qsq));
-            const int mm = m_base + 32 * j + l32;
             sums[j] = sum;
             m2s[j] = m2;
             __builtin_amdgcn_sched_barrier(0);
