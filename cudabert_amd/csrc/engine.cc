@@ -496,19 +496,18 @@ static bool ln_tiles_are_one_round(const ModelOptions& opt, long rows) {
 int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
     const int parts = std::min(std::min(opt.split_parts, (int)kMaxParts), B);
     if (parts < 2 || opt.split_min_tokens <= 0 || rows < opt.split_min_tokens) return 1;
-    // One stream while the LayerNorm GEMMs are one round: there is little left for a second stream to fill, and it starts late,
-    // since its launches are enqueued after all of the first one's.  One stream / two, in ms:  BERT-large, valid tokens, 14498 rows
-    // 10.65 / 11.71, 16323 12.04 / 12.78; pooled output on the host, 15360 rows 10.72 / 10.97, 16384 11.03 / 11.81; BERT-base, the
-    // same, 19072 rows 4.08 / 4.13, 20480 4.30 / 4.36.  Not for passes that queue up on the device, where the second stream is as
-    // early as the first (BERT-large, 14336 rows 9.51 / 9.36, 15360 10.87 / 10.51, BERT-base, 19456 4.29 / 4.24), nor for narrower
-    // models (host, hidden 512, 30720 rows 3.63 / 3.51; hidden 256, 61440 rows 3.17 / 3.07), nor beyond the one round: BERT-large,
-    // 16512 rows (260 tiles) 13.73 / 11.26, BERT-base, 20608 (243 tiles, 33 on one XCD) 5.38 / 4.64.
-    return waited && opt.split_keeps_one_round && ln_tiles_are_one_round(opt, rows) ? 1 : parts;
+    // One stream while the LayerNorm GEMMs of a pass of hidden 1024 are one round and the host waits for it: there is little left for
+    // a second stream to fill, and it starts late, since its launches are enqueued after all of the first one's.  Two streams / one,
+    // BERT-large, pooled output on the host and valid tokens, every 128 rows: 1.00 to 1.04 up to 14976 rows, 0.95 to 1.02 from 15104
+    // on (QKV and FFN-in change to 256 x 256 tiles there, which cost the one stream more), 1.00 to 1.03 from 16256 to 16384; 1.00 on
+    // average, and beyond the one round, 16512 rows, 0.82.  BERT-base, the same, 0.985 (bands of three workgroups leave a sixteenth
+    // of the chip idle); hidden 512, 30720 rows 0.97; hidden 256, 61440 rows 0.97.  Passes that queue up on the device, where the
+    // second stream is as early as the first: BERT-large 14336 rows 0.98, 15360 0.95, 16384 0.96, BERT-base 0.95 to 0.97.
+    return waited && opt.split_keeps_one_round && opt.dims.hidden >= 1024 && ln_tiles_are_one_round(opt, rows) ? 1 : parts;
 }
 
-// Parts regroup nothing: they sit side by side in y32, which has no room for partial sums there.  A pass in one part gives the bits
-// of one in parts, and the other way round (a pass of the valid rows may be in more parts than the padded one: 15000 valid rows of
-// 20000 of BERT-base), only if neither regroups.
+// Parts regroup nothing: they sit side by side in y32, which has no room for partial sums there.  And a pass in parts and one in one
+// part have the same bits only if neither regroups.
 long Model::order_rows_of(const ModelOptions& opt, long rows, long bits_of, int B, bool waited) {
     return opt.split_k && parts_of(opt, rows, B, waited) == 1 && parts_of(opt, bits_of, B, waited) == 1 ? bits_of : 0;
 }

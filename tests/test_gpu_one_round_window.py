@@ -80,8 +80,7 @@ def test_same_bits_whoever_calls(pb, models, i):
 @pytest.mark.parametrize("B,S,low,high", [(128, 157, 90, 140), (128, 160, 60, 160), (128, 168, 150, 159), (128, 128, 100, 128),
                                           (128, 126, 112, 120), (128, 140, 110, 120)])
 def test_padding_skipped_unasked_leaves_no_trace(pb, models, B, S, low, high):
-    """A pooled-only call computes the valid tokens alone.  Padded and valid rows lie inside and outside the window in turn (128 lines
-    of up to 157 tokens of BERT-base: one part padded, two parts of the valid rows)."""
+    """A pooled-only call computes the valid tokens alone.  Padded and valid rows lie inside and outside the window in turn."""
     size, kept = models
     lens = np.random.default_rng(B + S).integers(low, high + 1, size=B)
     ids, seg, mask = synth.make_inputs(B, S, lens, vocab=500, seed=S, prune=False)

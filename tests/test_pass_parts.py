@@ -52,7 +52,6 @@ def parts(*args, **kw):
 def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
     """768 features: band b of 256 rows and its three workgroups belong to XCD b % 8, and 81 bands are 33 workgroups on one."""
     assert parts(program, 768, [14335, 14336, 20481, 20608, 21760, 21761]) == [1, 2, 2, 2, 2, 2]
-    assert parts(program, 768, [20480]) == [1]
 
 
 def test_one_round_of_1024_features(program):
@@ -67,11 +66,10 @@ def test_one_stream_asks_for_the_gemms_it_counts(program, without):
 
 @pytest.mark.parametrize("hidden", [768, 1024])
 def test_passes_that_queue_up_on_the_device_run_on_two_streams(program, hidden):
-    rows = [14336, 16384, 18945, 20480]
-    assert parts(program, hidden, rows, waited=0) == [2] * 4 != parts(program, hidden, rows)
+    assert parts(program, hidden, [14336, 16384, 18945, 20480], waited=0) == [2] * 4
 
 
-@pytest.mark.parametrize("hidden", [256, 512])
+@pytest.mark.parametrize("hidden", [256, 512, 768])
 def test_narrow_models_run_on_two_streams(program, hidden):
     assert set(parts(program, hidden, range(14336, 70000, 256))) == {2}
 
@@ -80,7 +78,7 @@ def test_narrow_models_run_on_two_streams(program, hidden):
 def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, first, last):
     rows = range(first, last + 1, 7)
     assert set(plan(program, hidden, rows, waited=0)) == {(2, 256)}
-    assert set(plan(program, hidden, rows)) == {(1, 0)}
+    assert set(plan(program, hidden, rows)) == ({(1, 0)} if hidden == 1024 else {(2, 256)})
     beside = [14335, first - 1, last + 1, 25600, 32768]
     assert {t for _, t in plan(program, hidden, beside, waited=0)} == {0}
     assert {t for _, t in plan(program, hidden, rows, waited=0, fuse_layernorm=0)} == {0}
@@ -88,7 +86,7 @@ def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, f
 
 @pytest.mark.parametrize("hidden", [256, 768, 1024])
 def test_a_pass_in_parts_regroups_no_sums(program, hidden):
-    """Nor does one that gives the bits of a pass in parts.  (768: 20000 padded rows are one part, 15000 valid ones two.)"""
+    """Nor does one that gives the bits of a pass in parts."""
     rows, bits_of = [900, 11000, 14335, 14336, 15000, 18000, 18945, 20000], [1000, 12000, 14336, 16000, 19000, 20000, 20480, 22000]
     of = dict(zip(rows + bits_of, parts(program, hidden, rows + bits_of)))
     for n, l in zip(rows, lines(program, hidden, 4 * hidden, 1, 1, 1, *rows)):
