@@ -342,7 +342,6 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     long tokens = 0;                  // rows this pass computes: the valid tokens
     for (int b = 0; b < B; ++b) tokens += lens[b];
     const int parts = parts_for(tokens, B);
-    ln_tile_ = ln_tile_of_parts(opt_, tokens, parts);
     order_rows_ = (int)order_rows_of(opt_, tokens, padded_bits ? (long)B * S : tokens, B, waited_);
     // the pinned metadata of the previous call must have been consumed
     CUBERT_HIP_OK(hipStreamSynchronize(stream_));
@@ -351,6 +350,7 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     Compact cp[kMaxParts];
     size_t r0[kMaxParts];
     int b0s[kMaxParts], Bs[kMaxParts];
+    std::vector<int> part_rows(parts);
     size_t rows_total = 0, r = 0;
     for (int i = 0, b0 = 0; i < parts; ++i) {
         const int Bi = B / parts + (i < B % parts ? 1 : 0);
@@ -364,7 +364,7 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
         cu[Bi] = rows;
         cp[i].rowmap = d_meta_ + rows_total;
         cp[i].cu = d_meta_ + cap + 256 * (kMaxParts - 1) + (size_t)i * kCuStride;
-        cp[i].rows = rows;
+        cp[i].rows = part_rows[i] = rows;
         r0[i] = r;
         b0s[i] = b0;
         Bs[i] = Bi;
@@ -376,6 +376,7 @@ bool Model::run_compact(const int* lens, int B, int S, bool padded_bits) {
     const size_t cu_off = cap + 256 * (kMaxParts - 1);
     CUBERT_HIP_OK(hipMemcpyAsync(d_meta_ + cu_off, h_meta_ + cu_off, (size_t)parts * kCuStride * 4, hipMemcpyHostToDevice, stream_));
     cur_attn_ = pick_attention(B, S);
+    ln_tile_ = ln_tile_of_parts(opt_, part_rows);
     if (parts == 1) return enqueue_part(0, 0, B, 0, S, false, stream_, &cp[0]);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));
     bool ok = true;
@@ -485,12 +486,13 @@ int Model::pick_attention(int B, int S) const {
     return (long)B * opt_.dims.heads * ((S + 31) / 32) <= opt_.attn_split_workgroups ? kAttnSplitKeys : kAttnPerHead;
 }
 
-// The 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) of all the rows of a pass fill one round of the
-// 256 CUs, to seven eighths at least.  Models of hidden 768 and more: see the figures of the two rules below.
+// The 256 x 256 tiles of the attn-out and FFN-out GEMMs (LayerNorm in the epilogue) of all the rows of a pass are one round of the
+// 256 CUs, seven eighths full at least.
 static bool ln_tiles_are_one_round(const ModelOptions& opt, long rows) {
     const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
-    return H >= 768 && opt.fuse_residual && opt.fuse_layernorm && gemm_ln_pick_tile(M, H, H, opt.precision) == 256 &&
-           gemm_ln_pick_tile(M, H, I, opt.precision) == 256 && (rows + 255) / 256 * (H / 256) >= 224 && gemm_ln_one_round(M, H, 256);
+    return opt.fuse_residual && opt.fuse_layernorm && gemm_ln_pick_tile(M, H, H, opt.precision) == 256 &&
+           gemm_ln_pick_tile(M, H, I, opt.precision) == 256 && (rows + 255) / 256 * (H / 256) >= 224 &&
+           gemm_ln_xcd_workgroups(M, H, 256) <= kXcdCus;
 }
 
 int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
@@ -512,13 +514,23 @@ long Model::order_rows_of(const ModelOptions& opt, long rows, long bits_of, int 
     return opt.split_k && parts_of(opt, rows, B, waited) == 1 && parts_of(opt, bits_of, B, waited) == 1 ? bits_of : 0;
 }
 
-// Parts of such a pass run their LayerNorm GEMMs beside each other, so that the 256 x 256 tiles of all parts cover the chip once;
-// chosen for a part alone, the tile would be the one that covers it with the part.  Queued passes of 128 lines in two parts, tiles of
-// 128 / 192 / 256 tokens, in ms:  BERT-large, 14464 rows 9.56 / 9.63 / 9.38, 15360 10.63 / 10.22 / 10.48, 16384 11.13 / 10.97 /
-// 10.61; BERT-base, 19072 4.17 / 4.34 / 4.16, 20480 4.36 / 4.43 / 4.25.  Narrower models: hidden 512, 28672 rows 3.36 / 3.42 / 3.55;
-// hidden 256, 65536 rows 3.29 / 3.22 / 3.42.
-int Model::ln_tile_of_parts(const ModelOptions& opt, long rows, int parts) {
-    return parts > 1 && ln_tiles_are_one_round(opt, rows) ? 256 : 0;
+// Parts run their LayerNorm GEMMs beside each other: where 256 x 256 tiles of the whole pass are one round, a tile chosen for a part
+// alone, the one that covers the chip with that part, is too small.  The 256 x 256 one if the parts' workgroups leave no XCD with two
+// on a CU, else 256 x 192 (bands are rounded up in each part, and lines of uneven length make uneven parts).  Passes in two parts,
+// in ms, tiles of 128 / 192 / 256 tokens.  Parts of equal lines, queued:  BERT-large, 14464 rows 9.56 / 9.63 / 9.38, 15360 10.63 /
+// 10.22 / 10.48, 16384 11.13 / 10.97 / 10.61; BERT-base, 19072 4.17 / 4.34 / 4.16, 20480 4.36 / 4.43 / 4.25.  Uneven parts, valid
+// tokens: BERT-large, 7964 + 7601 rows 12.31 / 11.92 / 11.74, 8193 + 7823 (36 workgroups of 256 x 256 on an XCD) 12.84 / 11.94 /
+// 12.29; BERT-base, 10009 + 9485 4.97 / 4.82 / 4.68, 10313 + 9196 (33) 5.05 / 4.79 / 4.95.  Narrower models, queued: hidden 512,
+// 28672 rows 3.36 / 3.42 / 3.55; hidden 256, 65536 rows 3.29 / 3.22 / 3.42.
+int Model::ln_tile_of_parts(const ModelOptions& opt, const std::vector<int>& part_rows) {
+    long rows = 0;
+    int workgroups = 0;
+    for (int n : part_rows) {
+        rows += n;
+        workgroups += gemm_ln_xcd_workgroups(n, opt.dims.hidden, 256);
+    }
+    if (part_rows.size() < 2 || opt.dims.hidden < 768 || !ln_tiles_are_one_round(opt, rows)) return 0;
+    return workgroups <= kXcdCus ? 256 : kTile256x192;
 }
 
 // One forward pass.  A large batch is cut into parts of whole sequences that run
@@ -528,7 +540,9 @@ int Model::ln_tile_of_parts(const ModelOptions& opt, long rows, int parts) {
 bool Model::enqueue(int B, int S, bool has_mask) {
     cur_attn_ = pick_attention(B, S);
     const int parts = profiling_ ? 1 : parts_for((long)B * S, B);
-    ln_tile_ = ln_tile_of_parts(opt_, (long)B * S, parts);
+    std::vector<int> part_rows(parts);
+    for (int i = 0; i < parts; ++i) part_rows[i] = (B / parts + (i < B % parts ? 1 : 0)) * S;
+    ln_tile_ = ln_tile_of_parts(opt_, part_rows);
     order_rows_ = opt_.split_k && parts == 1 ? B * S : 0;
     if (parts == 1) return enqueue_part(0, 0, B, 0, S, has_mask, stream_);
     CUBERT_HIP_OK(hipEventRecord(ev_fork_, stream_));

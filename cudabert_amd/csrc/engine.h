@@ -60,8 +60,8 @@ class Model {
     static int parts_of(const ModelOptions& opt, long rows, int B, bool waited);
     // Rows on which a pass over `rows` token rows may decide how to regroup sums (order_rows_), given those of the pass whose bits it gives.
     static long order_rows_of(const ModelOptions& opt, long rows, long bits_of, int B, bool waited);
-    // GemmParams::tile of the LayerNorm GEMMs of a pass over that many rows in that many parts (0: chosen for each launch alone).
-    static int ln_tile_of_parts(const ModelOptions& opt, long rows, int parts);
+    // GemmParams::tile of the LayerNorm GEMMs of a pass whose parts have that many rows (0: chosen for each launch alone).
+    static int ln_tile_of_parts(const ModelOptions& opt, const std::vector<int>& part_rows);
     ~Model();
 
     // Host inputs [B, S] int32 (mask may be nullptr).  Asynchronous.

@@ -332,12 +332,12 @@ bool gemm_ln_workspace_force_expiry(void* ln_ws) {
     return true;
 }
 
-// A launch of the LayerNorm GEMM with tiles of `rows` tokens gives every CU at most one workgroup.  Counted for the XCD with most
-// of them: ln_tile_of_block hands out whole bands, band b and its N / 256 workgroups to XCD b % 8, and an XCD has 32 CUs.  With
-// N = 768, 81 to 85 bands are 243 to 255 workgroups, but 33 on up to five of the XCDs.
-bool gemm_ln_one_round(int M, int N, int rows) {
-    const long bands = ((long)M + rows - 1) / rows;
-    return (bands + 7) / 8 * (N / 256) <= 32;
+// A launch gives every CU at most one workgroup if no XCD gets more workgroups than it has CUs: ln_tile_of_block hands out whole
+// bands, band b and its N / 256 workgroups to XCD b % 8.  With N = 768, 81 to 85 bands are 243 to 255 workgroups, but 33 on up to
+// five of the XCDs.
+int gemm_ln_xcd_workgroups(int M, int N, int rows) {
+    const int bands = (M + rows - 1) / rows;
+    return (bands + 7) / 8 * (N / 256);
 }
 
 // Tile of a GEMM with the LayerNorm in its epilogue, 0 if the separate kernels are the better choice (below about 6000
@@ -352,8 +352,8 @@ bool gemm_ln_one_round(int M, int N, int rows) {
 // rows 15.17 against 15.27 with 256 tokens.
 int gemm_ln_pick_tile(int M, int N, int K, int elt) {
     if (M < 6144 || !ln_shape_ok(N, K, elt)) return 0;
-    if (K % 128 != 0 || gemm_ln_one_round(M, N, 128)) return kTile256x128;
-    return gemm_ln_one_round(M, N, 192) ? kTile256x192 : 256;
+    if (K % 128 != 0 || gemm_ln_xcd_workgroups(M, N, 128) <= kXcdCus) return kTile256x128;
+    return gemm_ln_xcd_workgroups(M, N, 192) <= kXcdCus ? kTile256x192 : 256;
 }
 
 bool gemm_ln_supported(int M, int N, int K, int elt) { return gemm_ln_pick_tile(M, N, K, elt) != 0; }

@@ -124,8 +124,9 @@ bool gemm_ln_workspace_force_expiry(void* ln_ws);
 bool gemm_ln_supported(int M, int N, int K, int elt);
 // GemmParams::tile value that it takes for the problem (0: none, the LayerNorm is better a kernel of its own).
 int gemm_ln_pick_tile(int M, int N, int K, int elt);
-// True if that GEMM, with tiles of 256 features x `rows` tokens, puts at most one workgroup on every CU.
-bool gemm_ln_one_round(int M, int N, int rows);
+// Workgroups of that GEMM, with tiles of 256 features x `rows` tokens, on the XCD that gets most of them; an XCD has kXcdCus CUs.
+constexpr int kXcdCus = 32;
+int gemm_ln_xcd_workgroups(int M, int N, int rows);
 
 // ----------------------------------------------------------- attention -----
 // Fused QK^T * scale + mask -> softmax -> P V for head dim 64.

@@ -22,10 +22,18 @@ int main(int argc, char** argv) {
     opt.fuse_residual = std::atoi(argv[3]);
     opt.fuse_layernorm = std::atoi(argv[4]);
     const bool waited = std::atoi(argv[5]);
+    if (argc > 6 && std::atoi(argv[6]) == 0) {                    // a pass of parts of these rows
+        std::vector<int> part_rows;
+        for (int i = 7; i < argc; ++i) part_rows.push_back(std::atoi(argv[i]));
+        std::printf("%d\n", cubert::Model::ln_tile_of_parts(opt, part_rows));
+        return 0;
+    }
     for (int i = 6; i < argc; ++i) {
         const long rows = std::atol(argv[i]);
         const int parts = cubert::Model::parts_of(opt, rows, 128, waited);
-        std::printf("%d %d", parts, cubert::Model::ln_tile_of_parts(opt, rows, parts));
+        std::vector<int> part_rows(parts, rows / parts);
+        part_rows[0] += rows % parts;
+        std::printf("%d %d", parts, cubert::Model::ln_tile_of_parts(opt, part_rows));
         for (long bits_of : {1000, 12000, 14336, 16000, 19000, 20000, 20480, 22000})
             std::printf(" %ld", cubert::Model::order_rows_of(opt, rows, bits_of, 128, waited));
         std::puts("");
@@ -76,12 +84,24 @@ def test_narrow_models_run_on_two_streams(program, hidden):
 
 @pytest.mark.parametrize("hidden,first,last", [(1024, 14336, 16384), (768, 18945, 20480)])
 def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, first, last):
-    rows = range(first, last + 1, 7)
+    rows = range(first + first % 2, last + 1, 14)
     assert set(plan(program, hidden, rows, waited=0)) == {(2, 256)}
     assert set(plan(program, hidden, rows)) == ({(1, 0)} if hidden == 1024 else {(2, 256)})
     beside = [14335, first - 1, last + 1, 25600, 32768]
     assert {t for _, t in plan(program, hidden, beside, waited=0)} == {0}
     assert {t for _, t in plan(program, hidden, rows, waited=0, fuse_layernorm=0)} == {0}
+
+
+@pytest.mark.parametrize("hidden,part_rows,tile", [
+    (1024, (8192, 8192), 256), (1024, (7937, 7937), 256), (1024, (8193, 7823), 386), (1024, (8769, 6683), 386),
+    (768, (10240, 10240), 256), (768, (10241, 9629), 386), (768, (8752, 10317), 386), (768, (9618, 10687), 386),
+    (768, (10753, 10753), 0), (1024, (8193, 8192), 0), (512, (16384, 16384), 0)])
+def test_uneven_parts(program, hidden, part_rows, tile):
+    """Bands are rounded up in each part: where the 256 x 256 workgroups of both parts are more than an XCD's 32, 256 x 192."""
+    assert lines(program, hidden, 4 * hidden, 1, 1, 0, 0, *part_rows) == [str(tile)]
+    xcd = sum(-(-(-(-n // 256)) // 8) * (hidden // 256) for n in part_rows)
+    assert tile != 256 or xcd <= 32
+    assert tile != 386 or xcd > 32
 
 
 @pytest.mark.parametrize("hidden", [256, 768, 1024])
