@@ -498,14 +498,18 @@ static bool ln_tiles_are_one_round(const ModelOptions& opt, long rows) {
 int Model::parts_of(const ModelOptions& opt, long rows, int B, bool waited) {
     const int parts = std::min(std::min(opt.split_parts, (int)kMaxParts), B);
     if (parts < 2 || opt.split_min_tokens <= 0 || rows < opt.split_min_tokens) return 1;
-    // One stream while the LayerNorm GEMMs of a pass of hidden 1024 are one round and the host waits for it: there is little left for
-    // a second stream to fill, and it starts late, since its launches are enqueued after all of the first one's.  Two streams / one,
-    // BERT-large, pooled output on the host and valid tokens, every 128 rows: 1.00 to 1.04 up to 14976 rows, 0.95 to 1.02 from 15104
-    // on (QKV and FFN-in change to 256 x 256 tiles there, which cost the one stream more), 1.00 to 1.03 from 16256 to 16384; 1.00 on
-    // average, and beyond the one round, 16512 rows, 0.82.  BERT-base, the same, 0.985 (bands of three workgroups leave a sixteenth
-    // of the chip idle); hidden 512, 30720 rows 0.97; hidden 256, 61440 rows 0.97.  Passes that queue up on the device, where the
-    // second stream is as early as the first: BERT-large 14336 rows 0.98, 15360 0.95, 16384 0.96, BERT-base 0.95 to 0.97.
-    return waited && opt.split_keeps_one_round && opt.dims.hidden >= 1024 && ln_tiles_are_one_round(opt, rows) ? 1 : parts;
+    // One stream while the LayerNorm GEMMs of a pass of hidden 1024 are one round, QKV and FFN-in have the 256 x 128 tile, two on a CU,
+    // and the host waits for the pass: there is little left for a second stream to fill, and it starts late, since its launches are
+    // enqueued after all of the first one's.  Two streams / one, BERT-large, pooled output on the host and valid tokens, every 128
+    // rows: 1.00 to 1.04 up to 14976 rows, 0.95 to 1.01 from 15104 on, where QKV and FFN-in change to 256 x 256 tiles, and 1.00 to
+    // 1.03 again at 64 bands of them; beyond the one round, 16512 rows, 0.82.  BERT-base, the same, 0.985 (bands of three workgroups
+    // leave a sixteenth of the chip idle); hidden 512, 30720 rows 0.97; hidden 256, 61440 rows 0.97.  Passes that queue up on the
+    // device, where the second stream is as early as the first: BERT-large 14336 rows 0.98, 15360 0.95, 16384 0.96, BERT-base 0.95 to 0.97.
+    const int H = opt.dims.hidden, I = opt.dims.inter, M = (int)rows;
+    const bool one = waited && opt.split_keeps_one_round && H >= 1024 && ln_tiles_are_one_round(opt, rows) &&
+                     gemm_plan(M, 3 * H, H, opt.precision, 1, false, false, false).tile == kTile256x128 &&
+                     gemm_plan(M, I, H, opt.precision, 1, false, true, false).tile == kTile256x128;
+    return one ? 1 : parts;
 }
 
 // Parts regroup nothing: they sit side by side in y32, which has no room for partial sums there.  And a pass in parts and one in one

@@ -63,13 +63,14 @@ def test_two_rounds_on_an_xcd_are_no_reason_for_one_stream(program):
 
 
 def test_one_round_of_1024_features(program):
-    assert parts(program, 1024, [14335, 14336, 16384, 16385]) == [1, 1, 1, 2]
+    """... while QKV and FFN-in have the tile of which a CU holds two, up to 15000 rows."""
+    assert parts(program, 1024, [14335, 14336, 14976, 15104, 16384, 16385]) == [1, 1, 1, 2, 2, 2]
 
 
 @pytest.mark.parametrize("without", [dict(fuse_residual=0), dict(fuse_layernorm=0), dict(inter=4128)])
 def test_one_stream_asks_for_the_gemms_it_counts(program, without):
     """No residual or no LayerNorm in the epilogue, or an FFN-out (K not a multiple of 128) that does not have the 256 x 256 tile."""
-    assert parts(program, 1024, [14336, 16384], **without) == [2, 2]
+    assert parts(program, 1024, [14336, 14976], **without) == [2, 2]
 
 
 @pytest.mark.parametrize("hidden", [768, 1024])
@@ -86,7 +87,7 @@ def test_narrow_models_run_on_two_streams(program, hidden):
 def test_parts_that_cover_the_chip_together_take_the_256_tile(program, hidden, first, last):
     rows = range(first + first % 2, last + 1, 14)
     assert set(plan(program, hidden, rows, waited=0)) == {(2, 256)}
-    assert set(plan(program, hidden, rows)) == ({(1, 0)} if hidden == 1024 else {(2, 256)})
+    assert set(plan(program, hidden, rows)) == ({(1, 0), (2, 256)} if hidden == 1024 else {(2, 256)})
     beside = [14335, first - 1, last + 1, 25600, 32768]
     assert {t for _, t in plan(program, hidden, beside, waited=0)} == {0}
     assert {t for _, t in plan(program, hidden, rows, waited=0, fuse_layernorm=0)} == {0}
