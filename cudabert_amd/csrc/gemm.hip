@@ -348,8 +348,8 @@ int gemm_ln_xcd_workgroups(int M, int N, int rows) {
 // 12416 (260 tiles of 192 tokens) 51.9 / 65.4 / 46.7 and 116 / 150 / 102.  N = 768, K = 768 / 3072:  10240 rows 30.0 / 32.5 / 37.2
 // and 54.8 / 57.8 / 66.2;  10241 (81 bands of 128 tokens) 35.3 / 31.2 / 35.9 and 76.3 / 57.9 / 66.4;  12170 40.6 / 33.4 / 37.6 and
 // 83.8 / 66.5 / 74.2;  15360 42.4 / 36.2 / 40.2 and 88.0 / 73.9 / 81.6;  15361 (81 bands of 192) 42.6 / 53.7 / 40.0 and 88.4 / 115 /
-// 81.5.  The parts of a pass on two streams take the same tiles: 18009 rows of BERT-large 12.76 ms against 12.80, 20926
-// rows 15.17 against 15.27 with 256 tokens.
+// 81.5.  The parts of a pass on two streams take the same tiles (18009 rows of BERT-large 12.76 ms against 12.80, 20926
+// rows 15.17 against 15.27 with 256 tokens), except where those of the whole pass are one round (Model::ln_tile_of_parts).
 int gemm_ln_pick_tile(int M, int N, int K, int elt) {
     if (M < 6144 || !ln_shape_ok(N, K, elt)) return 0;
     if (K % 128 != 0 || gemm_ln_xcd_workgroups(M, N, 128) <= kXcdCus) return kTile256x128;
