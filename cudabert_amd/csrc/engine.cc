@@ -605,15 +605,13 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     const int R = any_order ? order_rows_ : N;      // N or more
     int max_splits = any_order ? 16 : 1;
     while (max_splits > 1 && (long)max_splits * R > (long)R + kSplitRows) max_splits /= 2;
-    // LayerNorm's bf16 copy: the units layout for the few rows at which QKV and FFN-in may take a skinny tile, which needs it
-    // (one line of 17 tokens, BERT-base: 435 -> 416 us), else the packed one, whose pieces of a row are 64 bytes instead of 16
-    // (one line of 200 tokens, BERT-large, no skinny tile: 1145 us packed, 1155 units).
-    const int layout = elt == kF32 ? kSplit : any_order && R <= kSkinnyMaxRows ? kUnits : kPacked;
-    const bool any_x = any_order && layout != kPacked;
     const GemmPlan plan_ao = gemm_plan(R, H, H, gelt, max_splits, true, false, any_order),
                    plan_fo = gemm_plan(R, H, I, gelt, max_splits, true, false, any_order);
-    const int qkv_order = gemm_plan(R, 3 * H, H, gelt, 1, false, false, any_x && (elt == kF32 || vrow)).k_order();
-    const int fi_order = gemm_plan(R, I, H, gelt, 1, false, true, any_x).k_order();
+    const int qkv_order = gemm_plan(R, 3 * H, H, gelt, 1, false, false, any_order).k_order();
+    const int fi_order = gemm_plan(R, I, H, gelt, 1, false, true, any_order).k_order();
+    // LayerNorm's bf16 copy: the units layout where QKV or FFN-in take a skinny tile, which needs it, else the packed one, whose pieces
+    // of a row are 64 bytes instead of 16.
+    const int layout = elt == kF32 ? kSplit : qkv_order == kOrderSkinny || fi_order == kOrderSkinny ? kUnits : kPacked;
     const int sp_ao = plan_ao.splits, sp_fo = plan_fo.splits;
     // a tile that splits K is part of the order: tiles cut K at multiples of their own step
     const int tile_ao = sp_ao > 1 || R == N ? plan_ao.tile : 0, tile_fo = sp_fo > 1 || R == N ? plan_fo.tile : 0;

@@ -404,10 +404,27 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 constexpr int kPlanSmallRows = 6144;
 
 namespace {
+constexpr int kSkinnyTiles[] = {kTileSkinny11, kTileSkinny21, kTileSkinny12, kTileSkinny22};
+
+// Estimated time (microseconds) of a launch of the skinny kernel.  q workgroups share the busiest CU.  Terms: what those fetch, at 148
+// GB/s (64 bytes a clock), their MFMAs, the weights from memory at 6.1 TB/s, the result at 4 TB/s.  Least squares over launches of
+// 17 to 400 rows of the four linears of BERT-base and BERT-large, each tile, 1 to 16 parts, halfway between weights from memory and
+// weights in the L2 (mean error 6 %; the tile chosen by it is 1.2 % slower than the best in bf16, 0.2 % on split operands).
+double skinny_cost(int M, int N, int K, bool split_operands, int tile, int sp, bool f32_result) {
+    const int bn = skinny_features(tile), bm = skinny_tokens(tile), step = split_operands ? 16 : 32, es = split_operands ? 6 : 2;
+    const long tiles = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
+    const double q = (double)(((tiles + 7) / 8 * sp + kXcdCus - 1) / kXcdCus);
+    const double k = (double)((K / step + 8 * sp - 1) / (8 * sp)) * 8 * step;      // of a workgroup, whole steps of its eight waves
+    const double fetch = k * es * (bn + bm) / 148e3, weights = (double)N * K * es / 6.1e6, blocks = bn * bm / 1024.0;
+    const double mfma = k / 16 * blocks * (split_operands ? 6 : 1) * 32 / 4 / 2400.0;
+    const double out = (double)M * N * (f32_result ? 4.0 * sp : split_operands ? 6.0 : 2.0) / 4.0e6;
+    return split_operands ? 2.47 + q * (1.25 * fetch + 0.61 * mfma + 2.48) - 2.48 + 0.33 * weights + 1.94 * out + 0.08 * (sp - 1)
+                          : 1.67 + q * (1.08 * fetch + 0.73 * mfma) + 0.70 * weights + 0.135 * blocks + 4.03 * out + 0.02 * (sp - 1);
+}
+
 // Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits), all of one k order (kOrderAny:
 // the operands and the epilogue suit the skinny kernel).
 GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, int order) {
-    if (order == kOrderSkinny) return GemmPlan{kTileSkinny12, min_splits};
     // launch: before the first workgroup runs; fixed + per_hs * half-steps: a workgroup alone on its CU (deep_k: what a
     // half-step costs more when K > 2048 and the weights stream from memory); rho, q: see above; out: weight of the
     // result traffic (bytes / 4 TB/s).  Least-squares fit (5 % mean error) to launches of the four linears of BERT-large
@@ -420,9 +437,10 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         {kTile256x128Deep, 128, 256, 6.25, 1.33, 0.263, 1.50, 0.62, 0.86, 0.43, false, true},
         {256, 256, 256, 8.00, 3.43, 0.448, 1.15, 0.85, 0.97, 0.11, false, true},
     };
-    GemmPlan best{64, min_splits};
+    GemmPlan best{order == kOrderSkinny ? (int)kTileSkinny12 : 64, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
+        if (order == kOrderSkinny) break;
         if ((!c.splits && min_splits > 1) || (c.k128 && K % 128 != 0)) continue;
         for (int sp = min_splits; sp <= (c.splits ? max_splits : 1) && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;             // at least four half-steps per share
@@ -437,20 +455,19 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
         }
     }
-    // The skinny tile (32 features x 64 tokens) wins while every workgroup has a CU to itself; a second one on a CU competes for
-    // the same loads.  Microseconds, cold weights, skinny against the best of the others: 17 rows, QKV / FFN-in of BERT-base
-    // 5.0 / 5.0 against 6.1 / 6.0, of BERT-large 6.3 / 7.8 against 6.8 / 8.4; 128 rows of BERT-base 5.5 / 5.8 against 6.4 / 6.5;
-    // 200 rows (288 workgroups) 7.8 / 8.1 against 6.5 / 6.7.
-    // attn-out and FFN-out stay with the 64 tile at every size of the model: by this estimate a finer split of it costs less
-    // (17 rows, FFN-out of BERT-base: 16 parts 4.4, skinny tile with 8 parts 5.0).  Measured with the LayerNorm that adds the
-    // parts, each tile with its best split, attn-out / FFN-out, 64 tile against skinny: 17 rows of BERT-base 8.8 / 10.3
-    // against 8.9 / 10.1, of BERT-large 9.1 / 11.4 against 9.2 / 11.0; 128 rows 9.8 / 12.1 against 9.9 / 11.1 and 10.3 / 13.5
-    // against 10.5 / 13.3: level on attn-out, up to a microsecond less on FFN-out that the estimate does not see.
-    for (int sp = min_splits; order == kOrderAny && sp <= max_splits && sp <= 16; sp *= 2) {
-        if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
-        if ((long)((M + 63) / 64) * ((N + 31) / 32) * sp > 256) break;
-        const double cost = 3.2 + 0.1 * (K / 32.0 / sp) + (sp > 1 ? 0.6 : 0.0) + (gelu ? 0.8 : 0.0);
-        if (cost < best_cost) { best_cost = cost; best = GemmPlan{kTileSkinny12, sp}; }
+    // The skinny tiles win up to a few hundred rows.  Microseconds, weights from memory / in the L2, best skinny tile against the best of
+    // the others, attn-out and FFN-out with the LayerNorm that adds the parts.  BERT-base, QKV 17 rows 3.6 / 3.0 against 5.9 / 5.6,
+    // 128 rows 4.4 / 3.7 against 6.3 / 5.9, 400 rows 5.7 / 4.9 against 6.1 / 5.8, 600 rows 8.9 / 8.1 against 8.5 / 7.8; FFN-out 17 rows
+    // 6.9 / 6.0 against 8.3 / 7.5, 200 rows 9.7 / 8.9 against 10.5 / 9.9, 600 rows 13.1 / 13.2 against 13.9 / 14.2.  BERT-large, FFN-in
+    // 128 rows 6.4 / 4.1 against 8.4 / 6.6, 200 rows 8.2 / 5.3 against 8.3 / 6.9, 400 rows 13.4 / 9.2 against 12.0 / 8.6; attn-out 128
+    // rows 7.2 / 6.3 against 8.9 / 8.2, 600 rows 10.9 / 10.2 against 12.3 / 11.8.
+    for (int tile : kSkinnyTiles) {
+        if (order == kOrderShared) break;
+        for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
+            if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
+            const double cost = skinny_cost(M, N, K, false, tile, sp, f32_result);
+            if (cost < best_cost) { best_cost = cost; best = GemmPlan{tile, sp}; }
+        }
     }
     return best;
 }
@@ -460,20 +477,20 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
 // 1600 rows of the linears of BERT-base and BERT-large, and up to 19600 rows for the large tiles):
 //   128 x 128, 256 x 128: (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly
 //     what the first did, and the hand-out is uneven by half a workgroup; the larger tile wins from about 900 tiles on;
-//   the skinny tiles: fixed + per_step * steps * (w > 1 ? w + 0.5 : 1), bound by what a CU fetches (60 - 65 GB/s of operands).
+//   the skinny tiles: skinny_cost.
 // The 128 x 128 constants are those of its loop before it read fragments a step ahead (gemm_split.hip), which takes less from launches
-// of few workgroups: 1024 x 768 x 768 in 23.6 us for an estimate of 27.8.  At the lines they draw, skinny / 128 x 128 in us (* is
-// taken): 512 x 3072 x 1024 32.4* / 31.0, 512 x 4096 x 1024 35.6 / 34.7*, 768 x 2304 x 768 23.7* / 25.4, 1024 x 2304 x 768 30.8 /
-// 26.4*, 1024 x 3072 x 768 34.6 / 29.2*, and in 16 parts 192 x 1024 x 4096 21.4 / 23.2*, 256 x 1024 x 4096 27.1 / 23.6*.
-// At 128 rows (QKV 3072 x 1024 / FFN-in 4096 x 1024 / FFN-out 1024 x 4096): 13.9 / 15.6 / 14.6 us with the skinny tile,
-// 35.2 / 40.7 / 24.0 with the 128 one; at 1600 rows 81 / 102 / 102 against 65 / 79 / 76.
-GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, int order) {
+// of few workgroups: 1024 x 768 x 768 in 23.6 us for an estimate of 27.8.  Best skinny tile against 128 x 128, us, weights from memory:
+// 128 rows, QKV / FFN-in of BERT-large 13.5 / 14.0 against 33.4 / 34.9; 400 rows 29.2 / 30.4 against 32.6 / 34.8; 600 rows 30.4 / 42.5
+// against 33.2 / 35.3; of BERT-base 600 rows 23.1 / 23.9 against 26.6 / 28.5.
+GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool f32_result, int order) {
     struct Cand { int tile, bm, bn; double fixed, per_step; bool skinny; };
     static const Cand cands[] = {
         {128, 128, 128, 6.0, 0.455, false},
         {kTile256x128, 128, 256, 8.0, 0.98, false},
-        {kTileSkinny12, 64, 32, 4.5, 0.144, true},
-        {kTileSkinny22, 64, 64, 4.5, 0.214, true},
+        {kTileSkinny11, 0, 0, 0.0, 0.0, true},
+        {kTileSkinny21, 0, 0, 0.0, 0.0, true},
+        {kTileSkinny12, 0, 0, 0.0, 0.0, true},
+        {kTileSkinny22, 0, 0, 0.0, 0.0, true},
     };
     GemmPlan best{order == kOrderSkinny ? kTileSkinny12 : 128, min_splits};
     double best_cost = 1e30;
@@ -483,11 +500,15 @@ GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;
             if (c.skinny && 4 * sp > K / 16) break;
-            const double w = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * sp / 256.0, g = w > 1.0 ? w + 0.5 : 1.0;
-            const double loop = c.per_step * (K / 16.0 / sp);
-            double cost = c.skinny ? c.fixed + loop * g : (c.fixed + loop) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
-            // every part of a split result is written and read again by the consumer
-            if (sp > 1) cost += 0.6 + (double)M * N * 4.0 * sp / 4.0e6;
+            double cost;
+            if (c.skinny) {
+                cost = skinny_cost(M, N, K, true, c.tile, sp, f32_result);
+            } else {
+                const double w = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * sp / 256.0, g = w > 1.0 ? w + 0.5 : 1.0;
+                cost = (c.fixed + c.per_step * (K / 16.0 / sp)) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
+                // every part of a split result is written and read again by the consumer
+                if (sp > 1) cost += 0.6 + (double)M * N * 4.0 * sp / 4.0e6;
+            }
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
         }
     }
@@ -502,7 +523,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
         return false;
     }
     if ((size_t)p.K * 6 * 256 >= (1ull << 31)) { set_error("gemm: K too large"); return false; }
-    if (p.ln_gamma || p.compiler_scheduled || (p.tile != 0 && p.tile != 128 && p.tile != kTile256x128 && p.tile != kTileSkinny12 && p.tile != kTileSkinny22)) {
+    if (p.ln_gamma || p.compiler_scheduled || (p.tile != 0 && p.tile != 128 && p.tile != kTile256x128 && !is_skinny(p.tile))) {
         set_error("gemm: split operands take the 128, the 256x128 or a skinny tile and no LayerNorm epilogue");
         return false;
     }
@@ -538,24 +559,26 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
             d.R = p.residual;
         }
     }
-    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.k_order).tile;
-    const bool skinny = tile == kTileSkinny12 || tile == kTileSkinny22;
-    const int bn = tile == kTile256x128 ? 256 : tile == kTileSkinny12 ? 32 : tile == kTileSkinny22 ? 64 : 128, bm = skinny ? 64 : 128;
+    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.out_elt == kF32 && epi != kEpiQKV && epi != kEpiQKVMap, p.k_order).tile;
+    if (is_skinny(tile)) {
+        if (split_bytes(p.M, p.K) >= (1ull << 31) || split_bytes(p.N, p.K) >= (1ull << 31)) {
+            set_error("gemm: operand exceeds the 2 GiB addressable through one buffer descriptor");
+            return false;
+        }
+        return launch_gemm_skinny(d, kF32Split, tile, epi, stream);
+    }
+    const int bn = tile == kTile256x128 ? 256 : 128;
     d.tiles_n = (p.N + bn - 1) / bn;
-    d.tiles_m = (p.M + bm - 1) / bm;
+    d.tiles_m = (p.M + 127) / 128;
     d.xn_parts = gemm_pick_partition((double)p.M * p.K * 6, (double)p.N * p.K * 6, d.tiles_n, d.tiles_m, 8);
     if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
-    if (skinny && (split_bytes(p.M, p.K) >= (1ull << 31) || split_bytes(p.N, p.K) >= (1ull << 31))) {
-        set_error("gemm: operand exceeds the 2 GiB addressable through one buffer descriptor");
-        return false;
-    }
-    return skinny ? launch_gemm_skinny(d, kF32Split, tile, epi, stream) : launch_gemm_split(d, tile, epi, stream);
+    return launch_gemm_split(d, tile, epi, stream);
 }
 }  // namespace
 
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order) {
     const int order = any_order && N % 8 == 0 ? kOrderAny : kOrderShared;
-    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, order);
+    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, order);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {
@@ -668,9 +691,9 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
             return false;
         }
     }
-    // what the skinny kernel reads and writes, whoever asks for its tile
+    // what the skinny kernel reads and writes, whoever asks for its tile (which those who do not want V row-major may not)
     const bool skinny_fits = p.elt == kBF16 && p.x_units && p.w_units && p.N % 8 == 0 &&
-                             (p.epilogue == kEpiQKV ? p.v_rowmajor : epi == kEpiBiasGeluUnits || ((epi == kEpiBias || epi == kEpiBiasRes) && out == kF32));
+                             (p.epilogue == kEpiQKV ? p.v_rowmajor || !p.tile : epi == kEpiBiasGeluUnits || ((epi == kEpiBias || epi == kEpiBiasRes) && out == kF32));
     int bt = p.tile;
     if (!bt) {
         // the caller has settled on the split count; the tile follows
@@ -702,16 +725,11 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
         }
         return launch_gemm_bf16_t256x128(d, out, epi, stream);
     }
-    if (bt == kTileSkinny12 || bt == kTileSkinny22) {
+    if (is_skinny(bt)) {
         if (!skinny_fits) {
             set_error("gemm: the skinny tiles need bf16 operands in the units layout and a GELU result in it, row-major QKV or float32 result");
             return false;
         }
-        const int bn = bt == kTileSkinny12 ? 32 : 64;
-        d.tiles_n = (p.N + bn - 1) / bn;
-        d.tiles_m = (p.M + 63) / 64;
-        d.xn_parts = gemm_pick_partition((double)p.M * p.K * es, (double)p.N * p.K * es, d.tiles_n, d.tiles_m, 8);
-        if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
         return launch_gemm_skinny(d, kBF16, bt, epi == kEpiBiasGeluUnits ? (int)kEpiBiasGelu : epi, stream);
     }
     if (bt == kTile128Hand) {

@@ -1,11 +1,19 @@
 // GEMM for launches of a few hundred rows (gfx950):  Y = epilogue(X * W^T + bias), bf16 (units layout) or float32 (split layout) operands.
 //
 // Such a launch is bound by latency: a workgroup that streams its tile through the LDS spends most of every short K step
-// on the barrier and the round trip of the loads.  Here nothing is staged and the K loop has no barrier: the four waves of a
+// on the barrier and the round trip of the loads.  Here nothing is staged and the K loop has no barrier: the eight waves of a
 // workgroup share the K range of one (32 NBI) x (32 NBJ) tile, each requests its MFMA operands straight into registers
 // (both operand layouts are made of units a wave can load as they are, common.h), several steps ahead, and multiplies on its
-// own.  The four partial tiles meet in the LDS once, at the end, where every thread adds up (wave 0 first) the eight
-// consecutive features of one row that it then finishes and stores.  K may be split over blockIdx.y on top (float32 results).
+// own.  The partial tiles meet in the LDS once, at the end, where every thread adds up the four consecutive features of one row
+// that it then finishes and stores.  K may be split over workgroups on top (float32 results).
+//
+// What such a launch lasts (time stamps, bf16, 17 x 4096 x 1024, weights in the L2): 0.1 us until a wave runs, 0.55 until it has
+// addresses where the kernel divides (the workgroup's number by tiles, the wave's by parts), 1.3 until operands arrive, a CU taking 64 bytes a
+// clock (148 GB/s) from its L2; 0.3 for products, 0.2 for the exchange, 0.65 for results where 128 threads finish eight features each, and
+// 1.3 between launches.  Weights that are not in the L2: 2.3 more in bf16, 5 with split operands.  Hence no division on the device, four
+// features a thread, and eight waves with the whole of a K of 1024 in flight.  With four waves, eight features and divisions -> now, weights
+// from memory, smallest tile that gives each CU one workgroup: bf16 17 x 2304 x 768 4.8 -> 3.6 us, 17 x 4096 x 1024 7.8 -> 5.5, 128 x 3072 x 768
+// 5.5 -> 4.6, 128 x 4096 x 1024 7.9 -> 6.4; split operands 17 x 4096 x 1024 11.4 -> 10.3, 64 x 3072 x 1024 13.1 -> 9.8.
 #include "gemm_common.h"
 
 namespace cubert {
@@ -38,27 +46,49 @@ struct Operand<kBF16> {
     static __device__ int frag_offset(int lane_off, int f) { return lane_off + f * 1024; }
 };
 
+constexpr int kWaves = 8;
+
+// What the kernel needs of a GemmDev, with every division done by the host.
+struct SkinnyDev {
+    const unsigned char *X, *W;
+    const float *bias, *R;
+    unsigned char *Y, *k, *vt;          // QKV: Y is q
+    const int* rowmap;
+    int M, N, K, S, Sp, heads;
+    int tiles_m, per_xcd, more;         // tiles of an XCD: per_xcd, one more on the first `more` of the eight
+    int splits, share, extra;           // K steps of a wave: `share`, one more for the first `extra` of the kWaves * splits waves
+    unsigned split_magic, m_magic, s_magic;      // divisors splits, tiles_m and S (magic_of)
+    int v_rowmajor;                     // bf16 QKV: V like k; else [B, heads, 64, Sp]
+};
+
+// x / d as a multiplication, for x d < 2^32; 0 stands for d = 1.
+unsigned magic_of(unsigned d) { return d <= 1 ? 0u : (unsigned)((1ull << 32) / d + 1); }
+__device__ __forceinline__ int div_by(int x, unsigned magic) { return magic ? (int)__umulhi((unsigned)x, magic) : x; }
+
+// Workgroup ids go round the XCDs.  Each of them owns a run of the tiles, all rows of a band of features before the next band, so
+// that a weight row is fetched into one L2 (two at the ends of a run); the K shares of a tile follow each other.
 template <int ELT, int EPI, int NBI, int NBJ, int DEPTH>
-__global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const SkinnyDev p) {
     typedef Operand<ELT> Op;
-    constexpr int FR = Op::kFrags;
+    constexpr int FR = Op::kFrags, THREADS = 64 * kWaves;
     constexpr bool QKV = EPI == kEpiQKV || EPI == kEpiQKVMap;
     constexpr bool F32OUT = EPI == kEpiBias || EPI == kEpiBiasRes;
-    constexpr int ITEMS = NBI * NBJ / 2;                 // (row, eight features) pairs per thread at the end
-    static_assert(NBI * NBJ % 2 == 0, "every thread finishes whole items");
+    // the result leaves in units of 32 rows x 16 features, or in row segments
+    constexpr bool UNITS = EPI == kEpiBiasGelu || (QKV && ELT == kF32Split);
+    constexpr int ALL = 256 * NBI * NBJ, ITEMS = (ALL + THREADS - 1) / THREADS;      // (row, four features) pairs: all, and per thread
     // [wave][block column of 32 features][row][128 bytes], 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7)
-    __shared__ __attribute__((aligned(16))) unsigned char part[4 * NBI * NBJ * 4096];
+    constexpr int PART = NBI * NBJ * 4096;
+    __shared__ __attribute__((aligned(16))) unsigned char part[kWaves * PART];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    int tile_n, tile_m;
-    tile_of_block<8>(blockIdx.x, p.tiles_n * p.tiles_m, p.tiles_n, p.xn_parts, &tile_n, &tile_m);
-    const int n0 = tile_n * 32 * NBI, m0 = tile_m * 32 * NBJ;
+    const int xcd = blockIdx.x & 7, is = blockIdx.x >> 3, idx0 = div_by(is, p.split_magic), split = is - idx0 * p.splits;
+    if (idx0 >= p.per_xcd + (xcd < p.more ? 1 : 0)) return;            // the whole workgroup: no barrier has been met
+    const int tile = xcd * p.per_xcd + (xcd < p.more ? xcd : p.more) + idx0, tile_n = div_by(tile, p.m_magic);
+    const int n0 = tile_n * 32 * NBI, m0 = (tile - tile_n * p.tiles_m) * 32 * NBJ;
 
-    // steps of this wave: the wave-th quarter of the blockIdx.y-th share of K
-    const int all = p.K / Op::kStepK;
-    const int parts = 4 * p.splits, me = 4 * blockIdx.y + wave;
-    const int s0 = (int)((long)all * me / parts), s1 = (int)((long)all * (me + 1) / parts);
+    const int me = kWaves * split + wave;
+    const int s0 = me * p.share + (me < p.extra ? me : p.extra), s1 = s0 + p.share + (me < p.extra ? 1 : 0);
 
     // rows past the operand (padded to 32 or 256 rows in memory) read as zero
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(p.W), 0, (int)Op::bytes(p.N, p.K), 0x00020000);
@@ -66,8 +96,8 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
     const int w_off = Op::lane_offset(n0, p.K, l32, g), x_off = Op::lane_offset(m0, p.K, l32, g), stride = Op::block_stride(p.K);
     u32x4_t wf[DEPTH][NBI][FR], xf[DEPTH][NBJ][FR];
     auto load = [&](int d, int step) {
-        // Loads past the wave's share lie outside the descriptor (bit 31 of the lane offset): no traffic, zeros to multiply.
-        // They are issued all the same: with a fixed number of loads per step the compiler waits for exactly the oldest ones.
+        // Loads past the wave's share lie outside the descriptor (bit 31 of the lane offset): no traffic.
+        // They are issued all the same: with a fixed number of loads in flight the compiler waits for exactly the oldest ones.
         const int k = step * Op::kStepBytes, none = step < s1 ? 0 : (int)0x80000000u;
 #pragma unroll
         for (int i = 0; i < NBI; ++i)
@@ -86,33 +116,29 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // what my items add at the end, requested now
-    int row[ITEMS], c8[ITEMS];
+    // what my items add at the end, requested now, and where they go
+    int row[ITEMS], c4[ITEMS];
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-        const int idx = tid + it * 256;
-        if constexpr (EPI == kEpiBiasGelu) {       // units of 32 rows x 16 features
-            const int unit = idx >> 6;
-            row[it] = 32 * (unit / (2 * NBI)) + l32;
-            c8[it] = 2 * (unit % (2 * NBI)) + g;
-        } else {                                                       // row segments
-            row[it] = idx / (4 * NBI);
-            c8[it] = idx % (4 * NBI);
+        const int idx = (tid + it * THREADS) % ALL;                    // (threads past the last item repeat one and do not store it)
+        if constexpr (UNITS) {                                         // half unit by half unit, 512 bytes each
+            const int unit = idx >> 7;
+            row[it] = 32 * (unit / (2 * NBI)) + ((idx >> 1) & 31);
+            c4[it] = 4 * (unit % (2 * NBI)) + 2 * ((idx >> 6) & 1) + (idx & 1);
+        } else {
+            row[it] = idx / (8 * NBI);
+            c4[it] = idx % (8 * NBI);
         }
     }
-    f32x4_t bias[ITEMS][2], res[ITEMS][2];
+    f32x4_t bias[ITEMS], res[ITEMS];
     int tok[ITEMS];
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-        const int n = n0 + c8[it] * 8, m = m0 + row[it], mc = m < p.M ? m : p.M - 1;
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const int nc = n + 4 * hh < p.N ? n + 4 * hh : p.N - 4;
-            bias[it][hh] = res[it][hh] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            if (!F32OUT || blockIdx.y == 0) {                          // split K: bias and residual are added once
-                bias[it][hh] = *reinterpret_cast<const f32x4_t*>(p.bias + nc);
-                if constexpr (EPI == kEpiBiasRes) res[it][hh] = *reinterpret_cast<const f32x4_t*>(p.R + (size_t)mc * p.N + nc);
-            }
+        const int n = n0 + c4[it] * 4, m = m0 + row[it], mc = m < p.M ? m : p.M - 1, nc = n < p.N ? n : p.N - 4;
+        bias[it] = res[it] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (!F32OUT || split == 0) {                                   // split K: bias and residual are added once
+            bias[it] = *reinterpret_cast<const f32x4_t*>(p.bias + nc);
+            if constexpr (EPI == kEpiBiasRes) res[it] = *reinterpret_cast<const f32x4_t*>(p.R + (size_t)mc * p.N + nc);
         }
         tok[it] = mc;
         if constexpr (EPI == kEpiQKVMap) tok[it] = p.rowmap[mc];
@@ -143,7 +169,8 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
                     for (int j = 0; j < NBJ; ++j) mfma_chunk<kBF16>(wf[d][i][wp[t]], xf[d][j][xp[t]], acc[i][j]);
         }
     };
-    for (int s = s0; s < s1; s += DEPTH) {
+    int s = s0;
+    for (; s + DEPTH < s1; s += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             multiply(d);
@@ -151,8 +178,11 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
             __builtin_amdgcn_sched_barrier(0);       // left to itself the scheduler puts a round's loads together at its end
         }
     }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+        if (s + d < s1) multiply(d);
 
-    unsigned char* mine = part + wave * (NBI * NBJ * 4096);
+    unsigned char* mine = part + wave * PART;
 #pragma unroll
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
@@ -166,71 +196,86 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(const GemmDev p) {
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-        const int r = row[it], m = m0 + r, n = n0 + c8[it] * 8;
-        f32x4_t x[2];
+        const int r = row[it], m = m0 + r, n = n0 + c4[it] * 4;
+        const unsigned char* src = part + ((c4[it] >> 3) * NBJ * 32 + r) * 128 + (((c4[it] & 7) ^ ((r >> 1) & 7)) << 4);
+        f32x4_t p8[kWaves];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const int c = 2 * (c8[it] & 3) + hh;
-            const unsigned char* src = part + ((c8[it] >> 2) * NBJ * 32 + r) * 128 + ((c ^ ((r >> 1) & 7)) << 4);
-            x[hh] = *reinterpret_cast<const f32x4_t*>(src);
-#pragma unroll
-            for (int w = 1; w < 4; ++w) x[hh] += *reinterpret_cast<const f32x4_t*>(src + w * (NBI * NBJ * 4096));
-            x[hh] += bias[it][hh];
-            if constexpr (EPI == kEpiBiasRes) x[hh] += res[it][hh];
-        }
+        for (int w = 0; w < kWaves; ++w) p8[w] = *reinterpret_cast<const f32x4_t*>(src + w * PART);
+        f32x4_t x = ((p8[0] + p8[1]) + (p8[2] + p8[3])) + ((p8[4] + p8[5]) + (p8[6] + p8[7]));
+        x += bias[it];
+        if constexpr (EPI == kEpiBiasRes) x += res[it];
         if constexpr (EPI == kEpiBiasGelu) {
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[hh][e] = ELT == kBF16 ? gelu_fast(x[hh][e]) : gelu_erf(x[hh][e]);
+            for (int e = 0; e < 4; ++e) x[e] = ELT == kBF16 ? gelu_fast(x[e]) : gelu_erf(x[e]);
         }
-        if (m >= p.M || n >= p.N) continue;                            // N % 8 == 0
+        if (m >= p.M || n >= p.N || (ALL < THREADS && tid >= ALL)) continue;
         if constexpr (F32OUT) {
-            float* dst = reinterpret_cast<float*>(p.Y) + ((size_t)blockIdx.y * p.M + m) * p.N + n;
-            *reinterpret_cast<f32x4_t*>(dst) = x[0];
-            *reinterpret_cast<f32x4_t*>(dst + 4) = x[1];
+            *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.Y) + ((size_t)split * p.M + m) * p.N + n) = x;
         } else {
-            bf16x8_t pl[FR == 3 ? 3 : 1];
+            bf16x4_t pl[FR == 3 ? 3 : 1];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            for (int e = 0; e < 4; ++e) {
                 if constexpr (ELT == kBF16) {
-                    pl[0][e] = (__bf16)x[e >> 2][e & 3];
+                    pl[0][e] = (__bf16)x[e];
                 } else {
-                    __bf16 s0, s1, s2;
-                    split_bf16x3(x[e >> 2][e & 3], s0, s1, s2);
-                    pl[0][e] = s0; pl[1][e] = s1; pl[2][e] = s2;
+                    __bf16 a0, a1, a2;
+                    split_bf16x3(x[e], a0, a1, a2);
+                    pl[0][e] = a0; pl[1][e] = a1; pl[2][e] = a2;
                 }
             }
             unsigned char* dst;
             if constexpr (QKV) {
-                const int which = n >= 2 * p.hidden ? 2 : n >= p.hidden ? 1 : 0;
-                const int hn = n - which * p.hidden, b = tok[it] / p.S, s = tok[it] - b * p.S;
-                unsigned char* base = which == 2 ? p.vt : which ? p.k : p.q;
+                const int hidden = p.heads * 64;                       // a tile lies in one head: hidden and n0 are multiples of its width
+                const int which = n0 >= 2 * hidden ? 2 : n0 >= hidden ? 1 : 0, head = (n0 - which * hidden) >> 6;
+                const int hn = n & 63, b = div_by(tok[it], p.s_magic), s = tok[it] - b * p.S;
+                unsigned char* base = which == 2 ? p.vt : which ? p.k : p.Y;
                 if constexpr (ELT == kBF16) {
-                    dst = base + ((((size_t)b * p.heads + (hn >> 6)) * p.S + s) * 64 + (hn & 63)) * 2;
+                    if (which == 2 && !p.v_rowmajor) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) *reinterpret_cast<__bf16*>(base + ((((size_t)b * p.heads + head) * 64 + hn + e) * p.Sp + s) * 2) = pl[0][e];
+                        continue;
+                    }
+                    dst = base + ((((size_t)b * p.heads + head) * p.S + s) * 64 + hn) * 2;
                 } else {
-                    const int kk = (hn & 63) >> 4, half = (hn >> 3) & 1, pos = s & 31;
-                    const size_t unit = ((((size_t)b * p.heads + (hn >> 6)) * (p.Sp >> 5) + (s >> 5)) * 4 + kk) * 3;
-                    dst = base + unit * 1024 + half * 512 + (which == 2 ? attn_v_slot(pos, half, kk) : pos) * 16;
+                    const int kk = hn >> 4, half = (hn >> 3) & 1, pos = s & 31;
+                    const size_t unit = ((((size_t)b * p.heads + head) * (p.Sp >> 5) + (s >> 5)) * 4 + kk) * 3;
+                    dst = base + unit * 1024 + half * 512 + (which == 2 ? attn_v_slot(pos, half, kk) : pos) * 16 + (hn & 4) * 2;
                 }
             } else {
                 dst = p.Y + (ELT == kBF16 ? units_offset(m, n * 2, p.N * 2 / 64) : split_offset(m, n, p.N));
             }
 #pragma unroll
-            for (int q = 0; q < (FR == 3 ? 3 : 1); ++q) *reinterpret_cast<bf16x8_t*>(dst + q * 1024) = pl[q];
+            for (int q = 0; q < (FR == 3 ? 3 : 1); ++q) *reinterpret_cast<bf16x4_t*>(dst + q * 1024) = pl[q];
         }
     }
 }
 
 template <int ELT, int NBI, int NBJ, int DEPTH>
 bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
-    const dim3 grid(d.tiles_n * d.tiles_m, d.splits), block(256);
+    SkinnyDev p{};
+    p.X = d.X; p.W = d.W; p.bias = d.bias; p.R = d.R;
+    p.Y = epi == kEpiQKV || epi == kEpiQKVMap ? d.q : d.Y;
+    p.k = d.k; p.vt = d.vt; p.rowmap = d.rowmap;
+    p.M = d.M; p.N = d.N; p.K = d.K; p.S = d.S; p.Sp = d.Sp; p.heads = d.heads;
+    p.tiles_m = (d.M + 32 * NBJ - 1) / (32 * NBJ);
+    const int tiles = (d.N + 32 * NBI - 1) / (32 * NBI) * p.tiles_m;
+    p.per_xcd = tiles / 8;
+    p.more = tiles % 8;
+    p.splits = d.splits;
+    const int steps = d.K / Operand<ELT>::kStepK;
+    p.share = steps / (kWaves * d.splits);
+    p.extra = steps % (kWaves * d.splits);
+    p.split_magic = magic_of(d.splits);
+    p.m_magic = magic_of(p.tiles_m);
+    p.s_magic = magic_of(d.S);
+    p.v_rowmajor = d.v_rowmajor;
+    const dim3 grid(8 * ((tiles + 7) / 8) * d.splits), block(64 * kWaves);
     switch (epi) {
-        case kEpiBias: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBias, NBI, NBJ, DEPTH>), grid, block, 0, stream, d); break;
-        case kEpiBiasGelu: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasGelu, NBI, NBJ, DEPTH>), grid, block, 0, stream, d); break;
-        case kEpiQKV: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKV, NBI, NBJ, DEPTH>), grid, block, 0, stream, d); break;
-        case kEpiQKVMap: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKVMap, NBI, NBJ, DEPTH>), grid, block, 0, stream, d); break;
-        case kEpiBiasRes: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasRes, NBI, NBJ, DEPTH>), grid, block, 0, stream, d); break;
+        case kEpiBias: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBias, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
+        case kEpiBiasGelu: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasGelu, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
+        case kEpiQKV: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKV, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
+        case kEpiQKVMap: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKVMap, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
+        case kEpiBiasRes: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasRes, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
     CUBERT_HIP_OK(hipGetLastError());
@@ -239,18 +284,29 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
 
 }  // namespace
 
-// elt kBF16 (both operands and a GELU result in the units layout; per-head row-major Q, K, V; float32 results) or kF32Split; tile kTileSkinny12 (32
-// features x 64 tokens) or kTileSkinny22 (64 x 64); d.tiles_n / d.tiles_m for it; d.N % 8 == 0.
+// elt kBF16 (both operands and a GELU result in the units layout; per-head Q, K, V; float32 results) or kF32Split; tile a
+// skinny one; d.N % 8 == 0.
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream) {
     const int step = elt == kBF16 ? 32 : 16;
     if (d.K % step != 0 || d.N % 8 != 0 || d.splits < 1 || 4 * d.splits > d.K / step) {
         set_error("gemm: the skinny kernel needs N a multiple of 8 and at least four K steps per split");
         return false;
     }
+    // (depth: the steps a wave has in flight, as many as its 256 registers hold)
     if (elt == kBF16) {
-        return tile == kTileSkinny12 ? launch_epi<kBF16, 1, 2, 6>(d, epilogue, stream) : launch_epi<kBF16, 2, 2, 4>(d, epilogue, stream);
+        switch (tile) {
+            case kTileSkinny11: return launch_epi<kBF16, 1, 1, 4>(d, epilogue, stream);
+            case kTileSkinny21: return launch_epi<kBF16, 2, 1, 4>(d, epilogue, stream);
+            case kTileSkinny12: return launch_epi<kBF16, 1, 2, 4>(d, epilogue, stream);
+            default: return launch_epi<kBF16, 2, 2, 4>(d, epilogue, stream);
+        }
     }
-    return tile == kTileSkinny12 ? launch_epi<kF32Split, 1, 2, 4>(d, epilogue, stream) : launch_epi<kF32Split, 2, 2, 3>(d, epilogue, stream);
+    switch (tile) {
+        case kTileSkinny11: return launch_epi<kF32Split, 1, 1, 8>(d, epilogue, stream);
+        case kTileSkinny21: return launch_epi<kF32Split, 2, 1, 5>(d, epilogue, stream);
+        case kTileSkinny12: return launch_epi<kF32Split, 1, 2, 5>(d, epilogue, stream);
+        default: return launch_epi<kF32Split, 2, 2, 3>(d, epilogue, stream);
+    }
 }
 
 }  // namespace cubert

@@ -42,13 +42,15 @@ constexpr int kTile256x128Deep = 385; // ... of the 256 x 128 kernel with one wo
 constexpr int kTile256x192 = 386;     // ... of the 256 features x 192 tokens kernel (LayerNorm epilogue only; K % 128 == 0)
 constexpr int kTile128Hand = 192;     // ... of the hand-scheduled 128 x 128 kernel (bf16, three workgroups per CU, splits K)
 
-constexpr int kTileSkinny12 = 97;     // ... of the kernel without an LDS-staged loop whose waves share K: 32 features x 64 tokens
-// ... 64 x 64 (both: bf16 operands in the units layout or split float32 ones, any K split for float32 results; in bf16 the model's
-// plans take 32 x 64 alone, for QKV and FFN-in: the 64 x 64 tile and float32 results are there for callers that ask for them)
-constexpr int kTileSkinny22 = 98;
-constexpr int kSkinnyMaxRows = 128;   // rows up to which QKV and FFN-in of the model may take a skinny tile in bf16 (engine.cc)
+// ... of the kernel without an LDS-staged loop whose waves share K (bf16 operands in the units layout or split float32 ones, any K split
+// for float32 results): 32 x 32 (features x tokens), 64 x 32, 32 x 64, 64 x 64.
+constexpr int kTileSkinny11 = 95, kTileSkinny21 = 96, kTileSkinny12 = 97, kTileSkinny22 = 98;
+constexpr bool is_skinny(int tile) { return tile >= kTileSkinny11 && tile <= kTileSkinny22; }
+constexpr int skinny_features(int tile) { return tile == kTileSkinny11 || tile == kTileSkinny12 ? 32 : 64; }
+constexpr int skinny_tokens(int tile) { return tile == kTileSkinny11 || tile == kTileSkinny21 ? 32 : 64; }
+constexpr int kSkinnyMaxRows = 128;   // rows up to which the last layer runs whole although only its first tokens are wanted (engine.cc)
 
-// How a launch groups the sums over k.  All kernels share one order (per split count) but the skinny tiles, whose four waves
+// How a launch groups the sums over k.  All kernels share one order (per split count) but the skinny tiles, whose eight waves
 // each sum a share of K; among themselves those agree too.  Launches of a pass that have to give the same bits at different
 // row counts (the valid tokens alone, the first tokens alone) are given the same order.
 enum KOrder : int { kOrderShared = 0, kOrderSkinny = 1, kOrderAny = 2 };
@@ -110,7 +112,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream);
 // N and result suit it).
 struct GemmPlan {
     int tile; int splits;
-    int k_order() const { return tile == kTileSkinny12 || tile == kTileSkinny22 ? kOrderSkinny : kOrderShared; }
+    int k_order() const { return is_skinny(tile) ? kOrderSkinny : kOrderShared; }
 };
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order);
 // Workspace of a GEMM with the LayerNorm in its epilogue (GemmParams::ln_ws) for up to M rows.

@@ -1,0 +1,61 @@
+"""GEMM tiles whose eight waves share K, at the edges of what the host hands to them: tile counts that the eight XCDs do not share
+evenly (or that leave some without a tile), K steps that the waves of all parts do not, numbers of parts that are no power of two,
+rows past a 256-row block, features that end inside a tile.
+
+Bounds as in the tests of the two operand layouts: K / 16 float32 accumulations (six of them per float32 product of split operands)
+and a few additions against float64."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+import test_gpu_f32_split as f32  # noqa: E402
+import test_gpu_units_layout as b16  # noqa: E402
+from test_gpu_f32_split import lib as lib  # noqa: E402,F401
+
+TILES = (95, 96, 97, 98)
+U = 2.0 ** -24
+SHAPES = [(1, 32, 64, 1), (17, 264, 512, 3), (33, 72, 1088, 5), (65, 328, 192, 1), (300, 96, 1088, 1), (257, 1160, 256, 2)]
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K,splits", SHAPES)
+@pytest.mark.parametrize("split_operands", [False, True])
+def test_float32_result_in_parts(lib, tile, M, N, K, splits, split_operands):  # noqa: F811
+    steps = K // (16 if split_operands else 32)
+    if 4 * splits > steps:
+        pytest.skip("at least four K steps a part")
+    X, W, b = (f32.operands(M, N, K) if split_operands else b16.operands(M, N, K))[:3]
+    R = torch.randn(M, N, generator=torch.Generator().manual_seed(2))
+    want = X.double() @ W.double().t() + b.double() + R.double()
+    scale = X.double().abs() @ W.double().abs().t() + b.double().abs() + R.double().abs()
+    if split_operands:
+        xp, wp, elt, flags = f32.split(lib, X.cuda()), f32.split(lib, W.cuda()), f32.SPLIT, 0
+    else:
+        xp, wp, elt, flags = b16.pack(lib, X, True), b16.pack(lib, W, True), 1, 3 | b16.UNITS["X"] | b16.UNITS["W"]
+    bd, Rd = b.cuda(), R.cuda()
+    Y = torch.full((splits + 1, M, N), float("nan"), device="cuda")
+    f32.check(lib.cubert_op_gemm_residual(xp.data_ptr(), wp.data_ptr(), bd.data_ptr(), Rd.data_ptr(), Y.data_ptr(), M, N, K, K, elt, tile,
+                                          flags | (splits << 8 if splits > 1 else 0), None))
+    torch.cuda.synchronize()
+    assert torch.isnan(Y[splits]).all()                  # nothing past the last part
+    products = 6 if split_operands else 1
+    assert ((Y[:splits].double().sum(0).cpu() - want).abs() <= (products * K / 16 + 6 + splits) * U * scale).all()
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("B,S,heads", [(1, 1, 1), (3, 11, 1), (2, 150, 3)])
+def test_qkv_rows(lib, tile, B, S, heads):  # noqa: F811
+    """Token and head of every row from multiplications instead of divisions (a line of one token: no division at all)."""
+    H = max(heads, 2) * 64
+    X, W, b, want, scale = b16.operands(B * S, 3 * H, H)
+    xp, wp, bd = b16.pack(lib, X, True), b16.pack(lib, W, True), b.cuda()
+    heads = H // 64
+    out = [torch.zeros(B, heads, S, 64, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+    f32.check(lib.cubert_op_gemm_qkv(xp.data_ptr(), wp.data_ptr(), bd.data_ptr(), *[t.data_ptr() for t in out], B, S, heads, 1, tile,
+                                     3 | b16.UNITS["X"] | b16.UNITS["W"] | 32, None))
+    torch.cuda.synchronize()
+    for i, t in enumerate(out):
+        ref = want[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
+        lim = scale[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
+        assert ((t.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + (H / 16 + 6) * U * lim).all()
