@@ -20,6 +20,7 @@
 #include <atomic>
 
 #include "kernels.h"
+#include "l2_touch.h"
 
 namespace cubert {
 namespace {
@@ -582,9 +583,8 @@ __global__ __launch_bounds__(64 * NW, 4) void attention_chunk_kernel(
 template <int NW>
 __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
-    const unsigned char* __restrict__ v, const float* __restrict__ maskadd,
-    unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale_log2e, int ctx_layout,
-    const int* __restrict__ cu, int first_only) {
+    const unsigned char* __restrict__ v, const float* __restrict__ maskadd, const int* __restrict__ cu, int heads, int S, int Sp,
+    int query_blocks, unsigned char* __restrict__ ctx, float scale_log2e, int ctx_layout, int first_only, const WeightsAhead ahead) {
     constexpr int OSTRIDE = 68;                          // floats per query row of a partial context
     constexpr int OBYTES = 32 * OSTRIDE * 4;             // two V blocks (8 KiB) first, the partial context later
     constexpr int WBYTES = OBYTES + 256;                 // + the mask values of the two key blocks in flight
@@ -596,6 +596,12 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
     const int h = blockIdx.x, b = blockIdx.y, q0 = blockIdx.z * 32;
+    if ((int)blockIdx.z >= query_blocks) {               // the workgroups after the queries: weights for the next launch
+        const int plane = gridDim.x * gridDim.y, id = h + gridDim.x * b + plane * blockIdx.z, e = id - plane * query_blocks;
+        const int per_xcd = plane * (int)(gridDim.z - query_blocks) / 8;
+        if ((e >> 3) < per_xcd) l2_touch<false>(ahead, id & 7, (e >> 3) * NW + wave, per_xcd * NW, lane);
+        return;
+    }
     const int qlen = cu ? cu[b + 1] - cu[b] : S;
     if (q0 >= qlen) return;                              // the whole workgroup: no barrier has been met
     const int nblk = Sp >> 5;
@@ -776,7 +782,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
 
 bool launch_attention(const void* q, const void* k, const void* vt, const float* maskadd, void* ctx,
                       int ctx_layout, int B, int heads, int S, int Sp, float scale, int elt, hipStream_t stream,
-                      const int* cu, bool v_rowmajor, bool first_only, int variant) {
+                      const int* cu, bool v_rowmajor, bool first_only, int variant, const WeightsAhead& ahead) {
     const int fo = first_only ? 1 : 0;
     if (variant < kAttnAuto || variant > kAttnSplitKeys || (variant > kAttnPerHead && !(v_rowmajor && elt == kBF16 && S <= 512))) {
         set_error("attention: the key-split variants need bf16 operands, S <= 512 and V as [B, heads, S, 64]");
@@ -804,10 +810,11 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
     unsigned char* cc = static_cast<unsigned char*>(ctx);
     if (elt == kBF16 && S <= 512 && v_rowmajor &&
         (variant == kAttnSplitKeys || (variant == kAttnAuto && (long)B * heads * ((S + 31) / 32) <= kAttnSplitMaxWorkgroups))) {
-        const dim3 grid(heads, B, first_only ? 1 : (S + 31) / 32);
+        const int blocks = first_only ? 1 : (S + 31) / 32;
+        const dim3 grid(heads, B, blocks + (l2_touch_workgroups<false>(ahead) + heads * B - 1) / (heads * B));
         if (grid.z > 65535) { set_error("attention: grid too large"); return false; }
-        hipLaunchKernelGGL(attention_split_kernel<4>, grid, dim3(256), 0, stream, qc, kc, vc, maskadd, cc, heads, S, Sp,
-                           scale * 1.4426950408889634f, cp, cu, fo);
+        hipLaunchKernelGGL(attention_split_kernel<4>, grid, dim3(256), 0, stream, qc, kc, vc, maskadd, cu, heads, S, Sp, blocks, cc,
+                           scale * 1.4426950408889634f, cp, fo, ahead);
         CUBERT_HIP_OK(hipGetLastError());
         return true;
     }

@@ -17,7 +17,10 @@
 //
 // 128 sequences of up to 200 positions, 16 heads, a quarter of it padding: 137 us; 16 x 512, 12 heads: 73 us.  (Float32 MFMA,
 // K and V read from memory by every wave, attention.hip: 310 and 157 us.)
+#include <algorithm>
+
 #include "kernels.h"
+#include "l2_touch.h"
 
 namespace cubert {
 namespace {
@@ -265,8 +268,8 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(
 template <int NW>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void attention_f32_split_kernel(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
-    const float* __restrict__ maskadd, unsigned char* __restrict__ ctx, int heads, int S, int Sp, float scale_log2e,
-    const int* __restrict__ cu, int first_only) {
+    const float* __restrict__ maskadd, const int* __restrict__ cu, int heads, int S, int Sp, int query_blocks,
+    unsigned char* __restrict__ ctx, float scale_log2e, int first_only, const WeightsAhead ahead) {
     constexpr int OSTRIDE = 68;                          // floats per query row of a partial context
     constexpr int WBYTES = kBlockBytes + 256;            // a block of V, later the partial context (8.5 KiB), and 64 mask terms
     static_assert(32 * OSTRIDE * 4 <= kBlockBytes, "the partial context takes the place of V");
@@ -276,6 +279,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void attention_f32_split_
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
     const int h = blockIdx.x, b = blockIdx.y, q0 = blockIdx.z * 32;
+    if ((int)blockIdx.z >= query_blocks) {               // the workgroups after the queries: weights for the next launch
+        const int plane = gridDim.x * gridDim.y, id = h + gridDim.x * b + plane * blockIdx.z, e = id - plane * query_blocks;
+        const int per_xcd = plane * (int)(gridDim.z - query_blocks) / 8;
+        if ((e >> 3) < per_xcd) l2_touch<true>(ahead, id & 7, (e >> 3) * NW + wave, per_xcd * NW, lane);
+        return;
+    }
     const int qlen = cu ? cu[b + 1] - cu[b] : S;
     if (q0 >= qlen) return;                              // the whole workgroup: no barrier has been met
     const int nblk = Sp >> 5;
@@ -381,7 +390,7 @@ int attn_f32_variant(int B, int heads, int S, int max_blocks) {
 }
 
 bool launch_attention_f32(const void* q, const void* k, const void* v, const float* maskadd, void* ctx, int B, int heads,
-                          int S, int Sp, float scale, hipStream_t stream, const int* cu, bool first_only, int variant) {
+                          int S, int Sp, float scale, hipStream_t stream, const int* cu, bool first_only, int variant, const WeightsAhead& ahead) {
     if (B <= 0 || heads <= 0 || S <= 0) { set_error("attention: empty problem"); return false; }
     if (!(scale > 0.0f)) { set_error("attention: scale must be positive"); return false; }
     if (Sp % 32 != 0 || Sp < S || Sp - S >= 32 || (long)Sp * 384 >= (1L << 31)) {
@@ -400,11 +409,12 @@ bool launch_attention_f32(const void* q, const void* k, const void* v, const flo
     if (variant != kAttnPerHead) {
         if ((S + 31) / 32 > 65535) { set_error("attention: grid too large"); return false; }
         const bool eight = variant == kAttnSplitKeys8;
-        const dim3 sgrid(heads, B, first_only ? 1 : (S + 31) / 32);
+        const int blocks = first_only ? 1 : (S + 31) / 32;
+        const dim3 sgrid(heads, B, std::min(65535, blocks + (l2_touch_workgroups<true>(ahead) / (eight ? 2 : 1) + heads * B - 1) / (heads * B)));
         auto kernel = eight ? attention_f32_split_kernel<8> : attention_f32_split_kernel<4>;
         hipLaunchKernelGGL(kernel, sgrid, dim3(eight ? 512 : 256), 0, stream, static_cast<const unsigned char*>(q), static_cast<const unsigned char*>(k),
-                           static_cast<const unsigned char*>(v), maskadd, static_cast<unsigned char*>(ctx), heads, S, Sp,
-                           scale * 1.4426950408889634f, cu, first_only ? 1 : 0);
+                           static_cast<const unsigned char*>(v), maskadd, cu, heads, S, Sp, blocks, static_cast<unsigned char*>(ctx),
+                           scale * 1.4426950408889634f, first_only ? 1 : 0, ahead);
         CUBERT_HIP_OK(hipGetLastError());
         return true;
     }

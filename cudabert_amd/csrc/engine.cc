@@ -624,9 +624,14 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
     void* ln_ws = ln_ws_ + (size_t)part * ln_ws_bytes_;
     if (ln_ao || ln_fo) ln_used_ = std::max(ln_used_, part + 1);
 
-    auto attention = [&](void* out, bool vrow, bool first_only) {
-        if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only, cur_attn_);
-        return launch_attention(q, k, vt, maskadd, out, kUnits, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto);
+    auto attention = [&](void* out, bool vrow, bool first_only, const WeightsAhead& ahead) {
+        if (elt == kF32) return launch_attention_f32(q, k, vt, maskadd, out, B, D.heads, S, Sp, scale, st, cu, first_only, cur_attn_, ahead);
+        return launch_attention(q, k, vt, maskadd, out, kUnits, B, D.heads, S, Sp, scale, elt, st, cu, vrow, first_only, vrow ? cur_attn_ : kAttnAuto, ahead);
+    };
+    // weights that the launch before brings into the L2s: of GEMMs with a skinny tile
+    const WeightsAhead none;
+    auto ahead = [&](bool skinny, const void* w, int features, int k) {
+        return skinny && k % 32 == 0 && features % 32 == 0 ? WeightsAhead{w, k, features / 32} : none;
     };
 
     if (!mark(kPhEmbed)) return false;
@@ -662,7 +667,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             unsigned char* xbc = xbc_ + c0 * H * os;
             unsigned char* ctxc = static_cast<unsigned char*>(ctxc_) + c0 * H * os;
             unsigned char* hc = static_cast<unsigned char*>(hc_) + c0 * I * os;
-            if (!attention(ctxc, vrow, true)) return false;
+            if (!attention(ctxc, vrow, true, none)) return false;
             if (!launch_gather_first_rows(x32, cu, xc, B, S, H, st)) return false;
             g = GemmParams();
             g.elt = gelt; g.out_elt = kF32; g.X = ctxc; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = yc;
@@ -693,7 +698,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
             if (!mark(kPhPooler)) return false;
             return launch_pooler(xc, w_pool_, elt, b_pool_, pooled_ + (size_t)b0 * H, B, 1, H, st, nullptr);
         }
-        if (!attention(ctx, vrow, false)) return false;
+        if (!attention(ctx, vrow, false, ahead(is_skinny(plan_ao.tile), L.w_ao, H, H))) return false;
         // attention output projection -> f32, then residual add + LayerNorm
         g = GemmParams();
         g.elt = gelt; g.out_elt = kF32; g.X = ctx; g.ldx = H; g.W = L.w_ao; g.bias = L.b_ao; g.Y = y32;
@@ -704,7 +709,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         if (ln_ao) { g.tile = ln_tile_; g.Y = x32; g.ln_gamma = L.g1; g.ln_beta = L.be1; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhAttnOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
-        if (!ln_ao && !launch_add_layernorm(x32, y32, kF32, L.g1, L.be1, xb, layout, N, H, st, sp_ao, !fuse_res)) return false;
+        if (!ln_ao && !launch_add_layernorm(x32, y32, kF32, L.g1, L.be1, xb, layout, N, H, st, sp_ao, !fuse_res, ahead(fi_order == kOrderSkinny, L.w_in, I, H))) return false;
         // feed-forward
         g = GemmParams();
         g.elt = g.out_elt = gelt; g.X = xb; g.ldx = H; g.W = L.w_in; g.bias = L.b_in; g.Y = h;
@@ -721,7 +726,7 @@ bool Model::enqueue_part(int part, int b0, int B, size_t r0, int S, bool has_mas
         if (ln_fo) { g.tile = ln_tile_; g.Y = x32; g.ln_gamma = L.g2; g.ln_beta = L.be2; g.ln_xb = xb; g.ln_xb_packed = pk; g.ln_ws = ln_ws; }
         if (!mark(kPhFFNOut) || !launch_gemm(g, st)) return false;
         if (!mark(kPhLayerNorm)) return false;
-        if (!ln_fo && !launch_add_layernorm(x32, y32, kF32, L.g2, L.be2, xb, layout, N, H, st, sp_fo, !fuse_res)) return false;
+        if (!ln_fo && !launch_add_layernorm(x32, y32, kF32, L.g2, L.be2, xb, layout, N, H, st, sp_fo, !fuse_res, ahead(qkv_order == kOrderSkinny && i + 1 < D.layers, i + 1 < D.layers ? layers_[i + 1].w_qkv : nullptr, 3 * H, H))) return false;
     }
     // pooler: first-token gather + dense + tanh on the float32 sequence output
     if (!mark(kPhPooler)) return false;

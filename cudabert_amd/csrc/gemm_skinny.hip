@@ -48,16 +48,14 @@ struct Operand<kBF16> {
 
 constexpr int kWaves = 8;
 
-// What the kernel needs of a GemmDev, with every division done by the host.
-struct SkinnyDev {
-    const unsigned char *X, *W;
+// What the kernel needs of a GemmDev, with every division done by the host.  What the operands' addresses take comes as arguments of
+// its own, fourteen words that arrive in registers; the rest, loaded, is needed when the operands are under way.
+struct SkinnyRest {
     const float *bias, *R;
     unsigned char *Y, *k, *vt;          // QKV: Y is q
     const int* rowmap;
-    int M, N, K, S, Sp, heads;
-    int tiles_m, per_xcd, more;         // tiles of an XCD: per_xcd, one more on the first `more` of the eight
-    int splits, share, extra;           // K steps of a wave: `share`, one more for the first `extra` of the kWaves * splits waves
-    unsigned split_magic, m_magic, s_magic;      // divisors splits, tiles_m and S (magic_of)
+    int S, Sp, heads;
+    unsigned s_magic;                   // divisor S (magic_of)
     int v_rowmajor;                     // bf16 QKV: V like k; else [B, heads, 64, Sp]
 };
 
@@ -67,8 +65,12 @@ __device__ __forceinline__ int div_by(int x, unsigned magic) { return magic ? (i
 
 // Workgroup ids go round the XCDs.  Each of them owns a run of the tiles, all rows of a band of features before the next band, so
 // that a weight row is fetched into one L2 (two at the ends of a run); the K shares of a tile follow each other.
+// An XCD has per_xcd tiles, one more on the first `more`; tiles_m: tiles in a band of features (divisor m_magic).  A wave has `share` K
+// steps, one more for the first `extra` of the kWaves * splits (divisor split_magic) waves of a tile.
 template <int ELT, int EPI, int NBI, int NBJ, int DEPTH>
-__global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const SkinnyDev p) {
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsigned char* W, const unsigned char* X, int M, int N, int K,
+                                                                     int per_xcd, int tiles_m, unsigned m_magic, unsigned split_magic,
+                                                                     int splits_more, int share_extra, const SkinnyRest p) {
     typedef Operand<ELT> Op;
     constexpr int FR = Op::kFrags, THREADS = 64 * kWaves;
     constexpr bool QKV = EPI == kEpiQKV || EPI == kEpiQKVMap;
@@ -82,18 +84,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const Skinn
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    const int xcd = blockIdx.x & 7, is = blockIdx.x >> 3, idx0 = div_by(is, p.split_magic), split = is - idx0 * p.splits;
-    if (idx0 >= p.per_xcd + (xcd < p.more ? 1 : 0)) return;            // the whole workgroup: no barrier has been met
-    const int tile = xcd * p.per_xcd + (xcd < p.more ? xcd : p.more) + idx0, tile_n = div_by(tile, p.m_magic);
-    const int n0 = tile_n * 32 * NBI, m0 = (tile - tile_n * p.tiles_m) * 32 * NBJ;
+    const int splits = splits_more >> 3, more = splits_more & 7, share = share_extra >> 11, extra = share_extra & 2047;
+    const int xcd = blockIdx.x & 7, is = blockIdx.x >> 3, idx0 = div_by(is, split_magic), split = is - idx0 * splits;
+    if (idx0 >= per_xcd + (xcd < more ? 1 : 0)) return;                // the whole workgroup: no barrier has been met
+    const int tile = xcd * per_xcd + (xcd < more ? xcd : more) + idx0, tile_n = div_by(tile, m_magic);
+    const int n0 = tile_n * 32 * NBI, m0 = (tile - tile_n * tiles_m) * 32 * NBJ;
 
     const int me = kWaves * split + wave;
-    const int s0 = me * p.share + (me < p.extra ? me : p.extra), s1 = s0 + p.share + (me < p.extra ? 1 : 0);
+    const int s0 = me * share + (me < extra ? me : extra), s1 = s0 + share + (me < extra ? 1 : 0);
 
     // rows past the operand (padded to 32 or 256 rows in memory) read as zero
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(p.W), 0, (int)Op::bytes(p.N, p.K), 0x00020000);
-    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(p.X), 0, (int)Op::bytes(p.M, p.K), 0x00020000);
-    const int w_off = Op::lane_offset(n0, p.K, l32, g), x_off = Op::lane_offset(m0, p.K, l32, g), stride = Op::block_stride(p.K);
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(W), 0, (int)Op::bytes(N, K), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(X), 0, (int)Op::bytes(M, K), 0x00020000);
+    const int w_off = Op::lane_offset(n0, K, l32, g), x_off = Op::lane_offset(m0, K, l32, g), stride = Op::block_stride(K);
     u32x4_t wf[DEPTH][NBI][FR], xf[DEPTH][NBJ][FR];
     auto load = [&](int d, int step) {
         // Loads past the wave's share lie outside the descriptor (bit 31 of the lane offset): no traffic.
@@ -134,11 +137,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const Skinn
     int tok[ITEMS];
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-        const int n = n0 + c4[it] * 4, m = m0 + row[it], mc = m < p.M ? m : p.M - 1, nc = n < p.N ? n : p.N - 4;
+        const int n = n0 + c4[it] * 4, m = m0 + row[it], mc = m < M ? m : M - 1, nc = n < N ? n : N - 4;
         bias[it] = res[it] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         if (!F32OUT || split == 0) {                                   // split K: bias and residual are added once
             bias[it] = *reinterpret_cast<const f32x4_t*>(p.bias + nc);
-            if constexpr (EPI == kEpiBiasRes) res[it] = *reinterpret_cast<const f32x4_t*>(p.R + (size_t)mc * p.N + nc);
+            if constexpr (EPI == kEpiBiasRes) res[it] = *reinterpret_cast<const f32x4_t*>(p.R + (size_t)mc * N + nc);
         }
         tok[it] = mc;
         if constexpr (EPI == kEpiQKVMap) tok[it] = p.rowmap[mc];
@@ -208,9 +211,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const Skinn
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] = ELT == kBF16 ? gelu_fast(x[e]) : gelu_erf(x[e]);
         }
-        if (m >= p.M || n >= p.N || (ALL < THREADS && tid >= ALL)) continue;
+        if (m >= M || n >= N || (ALL < THREADS && tid >= ALL)) continue;
         if constexpr (F32OUT) {
-            *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.Y) + ((size_t)split * p.M + m) * p.N + n) = x;
+            *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.Y) + ((size_t)split * M + m) * N + n) = x;
         } else {
             bf16x4_t pl[FR == 3 ? 3 : 1];
 #pragma unroll
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const Skinn
                     dst = base + unit * 1024 + half * 512 + (which == 2 ? attn_v_slot(pos, half, kk) : pos) * 16 + (hn & 4) * 2;
                 }
             } else {
-                dst = p.Y + (ELT == kBF16 ? units_offset(m, n * 2, p.N * 2 / 64) : split_offset(m, n, p.N));
+                dst = p.Y + (ELT == kBF16 ? units_offset(m, n * 2, N * 2 / 64) : split_offset(m, n, N));
             }
 #pragma unroll
             for (int q = 0; q < (FR == 3 ? 3 : 1); ++q) *reinterpret_cast<bf16x4_t*>(dst + q * 1024) = pl[q];
@@ -252,32 +255,29 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const Skinn
 
 template <int ELT, int NBI, int NBJ, int DEPTH>
 bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
-    SkinnyDev p{};
-    p.X = d.X; p.W = d.W; p.bias = d.bias; p.R = d.R;
+    SkinnyRest p{};
+    p.bias = d.bias; p.R = d.R;
     p.Y = epi == kEpiQKV || epi == kEpiQKVMap ? d.q : d.Y;
     p.k = d.k; p.vt = d.vt; p.rowmap = d.rowmap;
-    p.M = d.M; p.N = d.N; p.K = d.K; p.S = d.S; p.Sp = d.Sp; p.heads = d.heads;
-    p.tiles_m = (d.M + 32 * NBJ - 1) / (32 * NBJ);
-    const int tiles = (d.N + 32 * NBI - 1) / (32 * NBI) * p.tiles_m;
-    p.per_xcd = tiles / 8;
-    p.more = tiles % 8;
-    p.splits = d.splits;
-    const int steps = d.K / Operand<ELT>::kStepK;
-    p.share = steps / (kWaves * d.splits);
-    p.extra = steps % (kWaves * d.splits);
-    p.split_magic = magic_of(d.splits);
-    p.m_magic = magic_of(p.tiles_m);
+    p.S = d.S; p.Sp = d.Sp; p.heads = d.heads;
     p.s_magic = magic_of(d.S);
     p.v_rowmajor = d.v_rowmajor;
+    const int tiles_m = (d.M + 32 * NBJ - 1) / (32 * NBJ), tiles = (d.N + 32 * NBI - 1) / (32 * NBI) * tiles_m;
+    const int waves = kWaves * d.splits, steps = d.K / Operand<ELT>::kStepK;
+    const unsigned m_magic = magic_of(tiles_m), split_magic = magic_of(d.splits);
+    const int splits_more = d.splits << 3 | tiles % 8, share_extra = steps / waves << 11 | steps % waves;      // (splits < 256)
     const dim3 grid(8 * ((tiles + 7) / 8) * d.splits), block(64 * kWaves);
+#define CUBERT_SKINNY(E) hipLaunchKernelGGL((gemm_skinny_kernel<ELT, E, NBI, NBJ, DEPTH>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, \
+                                            tiles / 8, tiles_m, m_magic, split_magic, splits_more, share_extra, p)
     switch (epi) {
-        case kEpiBias: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBias, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
-        case kEpiBiasGelu: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasGelu, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
-        case kEpiQKV: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKV, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
-        case kEpiQKVMap: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiQKVMap, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
-        case kEpiBiasRes: hipLaunchKernelGGL((gemm_skinny_kernel<ELT, kEpiBiasRes, NBI, NBJ, DEPTH>), grid, block, 0, stream, p); break;
+        case kEpiBias: CUBERT_SKINNY(kEpiBias); break;
+        case kEpiBiasGelu: CUBERT_SKINNY(kEpiBiasGelu); break;
+        case kEpiQKV: CUBERT_SKINNY(kEpiQKV); break;
+        case kEpiQKVMap: CUBERT_SKINNY(kEpiQKVMap); break;
+        case kEpiBiasRes: CUBERT_SKINNY(kEpiBiasRes); break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
+#undef CUBERT_SKINNY
     CUBERT_HIP_OK(hipGetLastError());
     return true;
 }
@@ -288,7 +288,7 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
 // skinny one; d.N % 8 == 0.
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream) {
     const int step = elt == kBF16 ? 32 : 16;
-    if (d.K % step != 0 || d.N % 8 != 0 || d.splits < 1 || 4 * d.splits > d.K / step) {
+    if (d.K % step != 0 || d.N % 8 != 0 || d.splits < 1 || d.splits > 255 || 4 * d.splits > d.K / step) {
         set_error("gemm: the skinny kernel needs N a multiple of 8 and at least four K steps per split");
         return false;
     }

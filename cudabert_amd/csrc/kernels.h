@@ -55,6 +55,13 @@ constexpr int kSkinnyMaxRows = 128;   // rows up to which the last layer runs wh
 // row counts (the valid tokens alone, the first tokens alone) are given the same order.
 enum KOrder : int { kOrderShared = 0, kOrderSkinny = 1, kOrderAny = 2 };
 
+// Weights [32 groups, K] (bf16 in units, or split float32) that a launch brings into the L2s for the one that follows it (l2_touch.h).
+// w null: none.
+struct WeightsAhead {
+    const void* w = nullptr;
+    int K = 0, groups = 0;
+};
+
 struct GemmParams {
     const void* X = nullptr;
     const void* W = nullptr;
@@ -142,7 +149,8 @@ int gemm_ln_xcd_workgroups(int M, int N, int rows);
 bool launch_attention(const void* q, const void* k, const void* vt, const float* maskadd,
                       void* ctx, int ctx_layout, int B, int heads, int S, int Sp, float scale, int elt,
                       hipStream_t stream, const int* cu = nullptr, bool v_rowmajor = false, bool first_only = false,
-                      int variant = kAttnAuto);
+                      int variant = kAttnAuto, const WeightsAhead& ahead = WeightsAhead());
+// ahead: weights to bring into the L2s meanwhile (kernels whose waves share the keys; the others leave them).
 // v_rowmajor (bf16, S <= 512 only): `vt` holds V as [B, heads, S, 64] like k.
 // variant (v_rowmajor only): kAttnPerHead = a wave walks all keys of its 32 queries; kAttnSplitKeys = one workgroup per
 // (batch, head, 32 queries) whose four waves share the keys: the short-batch kernel; kAttnAuto picks by the number of such workgroups.
@@ -154,7 +162,7 @@ bool launch_attention(const void* q, const void* k, const void* vt, const float*
 // of twelve 1 KiB units each (attention_f32.hip); ctx in the split layout.  Other arguments as above.
 bool launch_attention_f32(const void* q, const void* k, const void* v, const float* maskadd, void* ctx, int B, int heads,
                           int S, int Sp, float scale, hipStream_t stream, const int* cu = nullptr, bool first_only = false,
-                          int variant = kAttnAuto);
+                          int variant = kAttnAuto, const WeightsAhead& ahead = WeightsAhead());
 // The kernel for a batch (kAttnPerHead, kAttnSplitKeys or kAttnSplitKeys8: waves walk all keys, or share them); decided on the
 // whole batch where it runs in parts, since the kernels sum in different orders.
 int attn_f32_variant(int B, int heads, int S, int max_blocks);
@@ -166,11 +174,12 @@ int attn_f32_variant(int B, int heads, int S, int max_blocks);
 // LayerNorm).  eps = 1e-12 inside the square root, biased variance
 // (cuda_bert/ops/layernorm.cu:136-182; modeling.py:168-172).
 // xb_layout: an OperandLayout (common.h).
+// ahead: weights to bring into the L2s meanwhile (short batches; the kernels for more rows leave them).
 // add_x = false: x <- LayerNorm(y): y is already the sum with the residual stream (a GEMM with
 // GemmParams::residual produced it) and x is only written.
 bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma,
                           const float* beta, void* xb, int xb_layout, int rows, int H,
-                          hipStream_t stream, int y_parts = 1, bool add_x = true);
+                          hipStream_t stream, int y_parts = 1, bool add_x = true, const WeightsAhead& ahead = WeightsAhead());
 
 // --------------------------------------------------- embedding + LN --------
 // x[t] = LayerNorm(word[ids[t]] + pos[t % S] + type[seg[t]]); also writes the

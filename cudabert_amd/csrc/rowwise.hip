@@ -3,6 +3,7 @@
 // load-time weight transpose.  One wave64 owns one row; reductions are
 // butterfly shuffles over the 64 lanes, no LDS.
 #include "kernels.h"
+#include "l2_touch.h"
 #include <type_traits>
 
 namespace cubert {
@@ -271,11 +272,16 @@ template <int LAYOUT, int MORE>
 __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restrict__ x, const float* __restrict__ y,
                                                                   const float* __restrict__ gamma,
                                                                   const float* __restrict__ beta,
-                                                                  void* __restrict__ xb, int rows, LnDims d,
-                                                                  int y_parts, int add_x) {
-    const int H = d.H;
+                                                                  void* __restrict__ xb, int rows, int H,
+                                                                  int y_parts, int add_x, float inv_n, int rem, int inv_rem,
+                                                                  const WeightsAhead ahead) {
+    const LnDims d = {H, inv_n, rem, inv_rem};
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = blockIdx.x;
+    if (row >= rows) {                     // the workgroups after the rows: weights for the next launch
+        l2_touch<LAYOUT == kSplit>(ahead, row & 7, ((row - rows) >> 3) * 4 + wave, (int)(gridDim.x - rows) / 8 * 4, lane);
+        return;
+    }
     float* xrow = x + (size_t)row * H;
     const int i = wave * 256 + lane * 4;
     const bool in = i < H;
@@ -742,7 +748,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 constexpr int kRowPerGroup = 4096, kRowPerGroupSplit = 800;
 
 bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma, const float* beta,
-                          void* xb, int xb_layout, int rows, int H, hipStream_t stream, int y_parts, bool add_x) {
+                          void* xb, int xb_layout, int rows, int H, hipStream_t stream, int y_parts, bool add_x, const WeightsAhead& ahead) {
     if (!add_x && !y) { set_error("layernorm: without the residual stream an addend is required"); return false; }
     if (y_parts < 1 || (y_parts > 1 && (!y || y_elt != kF32))) { set_error("layernorm: partial addends must be float32"); return false; }
     if (xb && xb_layout != kRowMajor && H % 32 != 0) { set_error("layernorm: a packed copy needs H to be a multiple of 32"); return false; }
@@ -762,9 +768,10 @@ bool launch_add_layernorm(float* x, const void* y, int y_elt, const float* gamma
         const int ax = add_x ? 1 : 0;
         if (!y) hipLaunchKernelGGL((add_layernorm_kernel<-1, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, ln_dims(H), y_parts, ax);
         else if (y_elt == kF32 && (y_parts > 1 || rows <= (L == kSplit ? kRowPerGroupSplit : kRowPerGroup))) {
+            const LnDims d = ln_dims(H);
             auto kernel = y_parts == 1 ? add_layernorm_parts_kernel<L, 0> : y_parts == 2 ? add_layernorm_parts_kernel<L, 1>
                         : y_parts == 4 ? add_layernorm_parts_kernel<L, 3> : add_layernorm_parts_kernel<L, 7>;
-            hipLaunchKernelGGL(kernel, dim3(rows), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, ln_dims(H), y_parts, ax);
+            hipLaunchKernelGGL(kernel, dim3(rows + l2_touch_workgroups<L == kSplit>(ahead)), block, 0, stream, x, static_cast<const float*>(y), gamma, beta, xb, rows, H, y_parts, ax, d.inv_n, d.rem, d.inv_rem, ahead);
         }
         else if (y_elt == kF32 && L == kSplit && xb) hipLaunchKernelGGL(add_layernorm_split_rows_kernel, dim3((rows + 7) / 8), dim3(512), 0, stream, x, static_cast<const float*>(y), gamma, beta, static_cast<unsigned char*>(xb), rows, ln_dims(H), ax);
         else if (y_elt == kF32) hipLaunchKernelGGL((add_layernorm_kernel<kF32, L>), grid, block, 0, stream, x, yc, gamma, beta, xb, rows, ln_dims(H), y_parts, ax);
