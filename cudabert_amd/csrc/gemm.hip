@@ -32,6 +32,8 @@
 //
 // The 256 tile in bf16 has a hand-scheduled twin (gemm_bf16_256.hip); this
 // file is the general kernel (any tile, f32, odd step counts).
+#include <cmath>
+
 #include "gemm_common.h"
 
 namespace cubert {
@@ -42,6 +44,7 @@ bool launch_gemm_bf16_t128(const gemm_detail::GemmDev& d, int out_elt, int epilo
 bool launch_gemm_bf16_t256x128_deep(const gemm_detail::GemmDev& d, int out_elt, int epilogue, hipStream_t stream);
 bool launch_gemm_bf16_t256x192_ln(const gemm_detail::GemmDev& d, hipStream_t stream);
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream);
+bool launch_gemm_split_share(const gemm_detail::GemmDev& d, int tile, int epilogue, hipStream_t stream);
 bool launch_gemm_split(const gemm_detail::GemmDev& d, int tile, int epilogue, hipStream_t stream);
 int gemm_pick_tile(int M, int N, int K, int elt);
 
@@ -472,42 +475,68 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
     return best;
 }
 
+// Estimated time (microseconds) of a launch on split operands, w workgroups per CU, of a tile whose four waves share K (one workgroup to a
+// CU, so whole rounds, which last as long as their fetches and products; a round's GELU is not hidden) or of 128 x 128 (two to a CU).
+// out: the result at 4 TB/s; parts: what the consumer reads beside the first part.  Least squares over launches of 160 to 6000 rows of the four
+// linears of BERT-base and BERT-large, 1 to 8 parts, weights from memory, float32 results with the LayerNorm that adds the parts (mean error
+// 6 %; what is chosen by it and skinny_cost is 0.3 % slower on average than the best, 8 % at the worst).
+double share_or_128_cost(int M, int N, int K, int tile, int sp, double w, bool f32_result, bool gelu) {
+    const double out = (double)M * N * (f32_result ? 4.0 : 6.0) / 4.0e6, parts = (double)M * N * 4.0 * (sp - 1) / 4.0e6, rounds = std::ceil(w);
+    if (tile == 128) {
+        const double g = w > 1.0 ? w : 1.0, steps = K / 16.0 / sp;
+        return 9.44 + g * (0.476 * steps - 5.83 + (gelu ? 2.54 : 0.0)) + (w > 1.0 ? 0.38 * (rounds - g) * steps : 0.0) + 1.51 * out + 3.59 * parts;
+    }
+    const double blocks = share_features(tile) / 32, steps = (K / 16 + 4 * sp - 1) / (4 * sp);
+    return 2.75 + rounds * (steps * (0.475 + 0.281 * blocks) + (gelu ? 1.35 : 0.0) * blocks) + 2.38 * out + 4.56 * parts - 0.34 * w;
+}
+
 // float32 operands in the split layout.  Estimated time (microseconds) of a launch from that of a workgroup alone on its CU
 // and w = workgroups / 256, with constants measured on MI355X (cold weights: launches that cycle through 24 matrices, 17 to
 // 1600 rows of the linears of BERT-base and BERT-large, and up to 19600 rows for the large tiles):
 //   128 x 128, 256 x 128: (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly
 //     what the first did, and the hand-out is uneven by half a workgroup; the larger tile wins from about 900 tiles on;
-//   the skinny tiles: skinny_cost.
-// The 128 x 128 constants are those of its loop before it read fragments a step ahead (gemm_split.hip), which takes less from launches
+//   where tiles whose waves share K may be chosen too: skinny_cost, and share_or_128_cost for 128 x 128 as well.  LayerNorm included, us, best
+//   share tile / best of the others: 512 rows, BERT-base 18.8 / 19.7 (QKV), 22.9 / 25.4 (FFN-in), 25.0 / 25.9 (FFN-out); 1024 rows 24.4 / 27.7,
+//   17.3 / 23.2 (attn-out), 31.9 / 35.3, 34.1 / 39.3; 2048 rows, BERT-large 67.1 / 72.3, 31.4 / 42.0, 107.7 / 85.1 (FFN-in stays), 83.4 / 95.3;
+//   6000 rows 186.8 / 172.2, 82.5 / 85.7, 279.7 / 227.8, 232.8 / 251.1.
+// The 128 x 128 constants here are those of its loop before it read fragments a step ahead (gemm_split.hip), which takes less from launches
 // of few workgroups: 1024 x 768 x 768 in 23.6 us for an estimate of 27.8.  Best skinny tile against 128 x 128, us, weights from memory:
 // 128 rows, QKV / FFN-in of BERT-large 13.5 / 14.0 against 33.4 / 34.9; 400 rows 29.2 / 30.4 against 32.6 / 34.8; 600 rows 30.4 / 42.5
 // against 33.2 / 35.3; of BERT-base 600 rows 23.1 / 23.9 against 26.6 / 28.5.
-GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool f32_result, int order) {
-    struct Cand { int tile, bm, bn; double fixed, per_step; bool skinny; };
+GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, int order) {
+    struct Cand { int tile, bm, bn; double fixed, per_step; int order; };
     static const Cand cands[] = {
-        {128, 128, 128, 6.0, 0.455, false},
-        {kTile256x128, 128, 256, 8.0, 0.98, false},
-        {kTileSkinny11, 0, 0, 0.0, 0.0, true},
-        {kTileSkinny21, 0, 0, 0.0, 0.0, true},
-        {kTileSkinny12, 0, 0, 0.0, 0.0, true},
-        {kTileSkinny22, 0, 0, 0.0, 0.0, true},
+        {128, 128, 128, 6.0, 0.455, kOrderShared},
+        {kTile256x128, 128, 256, 8.0, 0.98, kOrderShared},
+        {kTileSkinny11, 0, 0, 0.0, 0.0, kOrderSkinny},
+        {kTileSkinny21, 0, 0, 0.0, 0.0, kOrderSkinny},
+        {kTileSkinny12, 0, 0, 0.0, 0.0, kOrderSkinny},
+        {kTileSkinny22, 0, 0, 0.0, 0.0, kOrderSkinny},
+        {kTileShare1, 128, 32, 0.0, 0.0, kOrderShare4},
+        {kTileShare2, 128, 64, 0.0, 0.0, kOrderShare4},
+        {kTileShare3, 128, 96, 0.0, 0.0, kOrderShare4},
     };
-    GemmPlan best{order == kOrderSkinny ? kTileSkinny12 : 128, min_splits};
+    GemmPlan best{order == kOrderSkinny ? (int)kTileSkinny12 : order == kOrderShare4 ? (int)kTileShare3 : 128, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
-        if (order == (c.skinny ? kOrderShared : kOrderSkinny)) continue;
-        if (c.skinny && (N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
+        if (order != kOrderAny && order != c.order) continue;
+        const bool skinny = c.order == kOrderSkinny;
+        if (skinny && (N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;
-            if (c.skinny && 4 * sp > K / 16) break;
+            if (c.order != kOrderShared && 4 * sp > K / 16) break;
             double cost;
-            if (c.skinny) {
+            if (skinny) {
                 cost = skinny_cost(M, N, K, true, c.tile, sp, f32_result);
             } else {
                 const double w = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * sp / 256.0, g = w > 1.0 ? w + 0.5 : 1.0;
-                cost = (c.fixed + c.per_step * (K / 16.0 / sp)) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
-                // every part of a split result is written and read again by the consumer
-                if (sp > 1) cost += 0.6 + (double)M * N * 4.0 * sp / 4.0e6;
+                if (order != kOrderShared && c.tile != kTile256x128) {
+                    cost = share_or_128_cost(M, N, K, c.tile, sp, w, f32_result, gelu);
+                } else {
+                    cost = (c.fixed + c.per_step * (K / 16.0 / sp)) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
+                    // every part of a split result is written and read again by the consumer
+                    if (sp > 1) cost += 0.6 + (double)M * N * 4.0 * sp / 4.0e6;
+                }
             }
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
         }
@@ -523,8 +552,8 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
         return false;
     }
     if ((size_t)p.K * 6 * 256 >= (1ull << 31)) { set_error("gemm: K too large"); return false; }
-    if (p.ln_gamma || p.compiler_scheduled || (p.tile != 0 && p.tile != 128 && p.tile != kTile256x128 && !is_skinny(p.tile))) {
-        set_error("gemm: split operands take the 128, the 256x128 or a skinny tile and no LayerNorm epilogue");
+    if (p.ln_gamma || p.compiler_scheduled || (p.tile != 0 && p.tile != 128 && p.tile != kTile256x128 && !is_skinny(p.tile) && !is_share(p.tile))) {
+        set_error("gemm: split operands take the 128, the 256x128 or a tile whose waves share K and no LayerNorm epilogue");
         return false;
     }
     GemmDev d{};
@@ -559,7 +588,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
             d.R = p.residual;
         }
     }
-    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.out_elt == kF32 && epi != kEpiQKV && epi != kEpiQKVMap, p.k_order).tile;
+    const int tile = p.tile ? p.tile : plan_split_operands(p.M, p.N, p.K, d.splits, d.splits, p.out_elt == kF32 && epi != kEpiQKV && epi != kEpiQKVMap, epi == kEpiBiasGelu, p.k_order).tile;
     if (is_skinny(tile)) {
         if (split_bytes(p.M, p.K) >= (1ull << 31) || split_bytes(p.N, p.K) >= (1ull << 31)) {
             set_error("gemm: operand exceeds the 2 GiB addressable through one buffer descriptor");
@@ -567,18 +596,18 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
         }
         return launch_gemm_skinny(d, kF32Split, tile, epi, stream);
     }
-    const int bn = tile == kTile256x128 ? 256 : 128;
+    const int bn = is_share(tile) ? share_features(tile) : tile == kTile256x128 ? 256 : 128;
     d.tiles_n = (p.N + bn - 1) / bn;
     d.tiles_m = (p.M + 127) / 128;
     d.xn_parts = gemm_pick_partition((double)p.M * p.K * 6, (double)p.N * p.K * 6, d.tiles_n, d.tiles_m, 8);
     if (p.xcd_partition >= 0) d.xn_parts = p.xcd_partition;
-    return launch_gemm_split(d, tile, epi, stream);
+    return is_share(tile) ? launch_gemm_split_share(d, tile, epi, stream) : launch_gemm_split(d, tile, epi, stream);
 }
 }  // namespace
 
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order) {
     const int order = any_order && N % 8 == 0 ? kOrderAny : kOrderShared;
-    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, order);
+    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, order);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {

@@ -12,7 +12,7 @@
 // operation both, where a bf16 FFN-in, whose fragments serve one product instead of two, spends 1.35), against 668 us, 123 TFLOP/s with the float32 MFMA, whose
 // peak is 157; 19600 x 3072 x 1024: 535 us against 942.  Error against float64, root mean square of the result: 2.7e-7 at
 // K = 1024 and 8.0e-7 at K = 4096, with the float32 MFMA 3.1e-7 and 9.1e-7 (fewer, larger accumulation steps).
-#include "gemm_common.h"
+#include "gemm_split_epilogue.h"
 
 namespace cubert {
 namespace {
@@ -22,56 +22,6 @@ using namespace gemm_detail;
 #define CUBERT_V10(b) "v" #b "0", "v" #b "1", "v" #b "2", "v" #b "3", "v" #b "4", "v" #b "5", "v" #b "6", "v" #b "7", "v" #b "8", "v" #b "9"
 #define CUBERT_ACC_22 [c00] "=&a"(acc[0][0]), [c01] "=&a"(acc[0][1]), [c10] "=&a"(acc[1][0]), [c11] "=&a"(acc[1][1])
 #define CUBERT_ACC_42 CUBERT_ACC_22, [c20] "=&a"(acc[2][0]), [c21] "=&a"(acc[2][1]), [c30] "=&a"(acc[3][0]), [c31] "=&a"(acc[3][1])
-
-// Epilogues whose result is an operand in MFMA register layout: bias + GELU in the split layout (the next GEMM's operand), and
-// Q, K, V as the attention kernel reads them.  split_unit_rows turns accumulator layout into 16 bytes per lane and plane;
-// they leave in 1 KiB units (Q, K, V: two runs of up to 512 bytes) without a trip through the LDS.
-template <int EPI, int NBI, int NBJ>
-__device__ __forceinline__ void split_epilogue(const GemmDev& p, f32x16_t (&acc)[NBI][NBJ], const f32x4_t (&bias)[4 * NBI],
-                                               int n_base, int m_base, int l32, int g) {
-    const int row_blocks = (p.M + 31) / 32, nblk = p.Sp >> 5;
-#pragma unroll
-    for (int j = 0; j < NBJ; ++j) {
-        const int rb = (m_base >> 5) + j;
-        if (rb >= row_blocks) continue;                    // wave-uniform
-        const int m = m_base + 32 * j + l32;
-        int bidx = 0, sidx = 0;
-        if constexpr (EPI != kEpiBiasGelu) {
-            const int mc = m < p.M ? m : p.M - 1;
-            const int tok = EPI == kEpiQKVMap ? p.rowmap[mc] : mc;
-            bidx = tok / p.S;
-            sidx = tok - bidx * p.S;
-        }
-#pragma unroll
-        for (int i = 0; i < NBI; ++i) {
-            if (n_base + 32 * i >= p.N) continue;          // N % 32 == 0
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int n = n_base + 32 * i + 16 * u;
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    x[e] = acc[i][j][8 * u + e] + bias[4 * i + 2 * u + e / 4][e % 4];
-                    if constexpr (EPI == kEpiBiasGelu) x[e] = gelu_erf(x[e]);
-                }
-                u32x4_t pl[3];
-                split_unit_rows(x, pl);
-                unsigned char* dst;
-                if constexpr (EPI == kEpiBiasGelu) {
-                    dst = p.Y + ((size_t)rb * (p.N / 16) + n / 16) * 3072 + (l32 + 32 * g) * 16;
-                } else {
-                    const int which = n >= 2 * p.hidden ? 2 : n >= p.hidden ? 1 : 0;
-                    const int hn = n - which * p.hidden, kk = (hn & 63) >> 4, pos = sidx & 31;
-                    const size_t unit = ((((size_t)bidx * p.heads + (hn >> 6)) * nblk + (sidx >> 5)) * 4 + kk) * 3;
-                    dst = (which == 2 ? p.vt : which ? p.k : p.q) + unit * 1024 + g * 512 + (which == 2 ? attn_v_slot(pos, g, kk) : pos) * 16;
-                    if (m >= p.M) continue;
-                }
-#pragma unroll
-                for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4_t*>(dst + q * 1024) = pl[q];
-            }
-        }
-    }
-}
 
 // NBI x 2 accumulator blocks per wave: 2 for the 128 x 128 tile, 4 for the 256 features x 128 tokens one.
 template <int EPI, int NBI>

@@ -48,12 +48,16 @@ constexpr int kTileSkinny11 = 95, kTileSkinny21 = 96, kTileSkinny12 = 97, kTileS
 constexpr bool is_skinny(int tile) { return tile >= kTileSkinny11 && tile <= kTileSkinny22; }
 constexpr int skinny_features(int tile) { return tile == kTileSkinny11 || tile == kTileSkinny12 ? 32 : 64; }
 constexpr int skinny_tokens(int tile) { return tile == kTileSkinny11 || tile == kTileSkinny21 ? 32 : 64; }
+// ... of the kernel on split operands whose four waves share K (gemm_split_share.hip): 32, 64 or 96 features x 128 tokens, any K split.
+constexpr int kTileShare1 = 101, kTileShare2 = 102, kTileShare3 = 103;
+constexpr bool is_share(int tile) { return tile >= kTileShare1 && tile <= kTileShare3; }
+constexpr int share_features(int tile) { return 32 * (tile - kTileShare1 + 1); }
 constexpr int kSkinnyMaxRows = 128;   // rows up to which the last layer runs whole although only its first tokens are wanted (engine.cc)
 
 // How a launch groups the sums over k.  All kernels share one order (per split count) but the skinny tiles, whose eight waves
-// each sum a share of K; among themselves those agree too.  Launches of a pass that have to give the same bits at different
+// each sum a share of K, and those whose four waves do; among themselves those agree too.  Launches of a pass that have to give the same bits at different
 // row counts (the valid tokens alone, the first tokens alone) are given the same order.
-enum KOrder : int { kOrderShared = 0, kOrderSkinny = 1, kOrderAny = 2 };
+enum KOrder : int { kOrderShared = 0, kOrderSkinny = 1, kOrderAny = 2, kOrderShare4 = 3 };
 
 // Weights [32 groups, K] (bf16 in units, or split float32) that a launch brings into the L2s for the one that follows it (l2_touch.h).
 // w null: none.
@@ -111,15 +115,15 @@ struct GemmParams {
                               // runs of the tile sequence, 2 / 4 = 4 x 2 / 2 x 4 cells (for measurements)
 };
 // elt == kF32Split: X and W in the split layout (common.h), K a multiple of 16; Y is float32 row-major, or, with the GELU
-// epilogue, split as well (out_elt kF32Split, N a multiple of 32); tile 0, 128, kTile256x128 or a skinny one.
+// epilogue, split as well (out_elt kF32Split, N a multiple of 32); tile 0, 128, kTile256x128, a skinny one or a kTileShare one.
 bool launch_gemm(const GemmParams& p, hipStream_t stream);
 // The tile (a GemmParams::tile value, never 0) and split count launch_gemm's cost model prefers for a problem.
 // max_splits > 1: the caller can take a float32 result as up to that many partial sums (a power of two is chosen).
-// f32_result / gelu: the launch will write float32 / use the GELU epilogue.  any_order: a skinny tile may be chosen (operands,
-// N and result suit it).
+// f32_result / gelu: the launch will write float32 / use the GELU epilogue.  any_order: a tile whose waves share K may be chosen
+// (operands, N and result suit it).
 struct GemmPlan {
     int tile; int splits;
-    int k_order() const { return is_skinny(tile) ? kOrderSkinny : kOrderShared; }
+    int k_order() const { return is_skinny(tile) ? kOrderSkinny : is_share(tile) ? kOrderShare4 : kOrderShared; }
 };
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order);
 // Workspace of a GEMM with the LayerNorm in its epilogue (GemmParams::ln_ws) for up to M rows.
