@@ -62,8 +62,30 @@ __device__ __forceinline__ int frag_kphase(int units) { return units ? 0x400 : 0
 constexpr int kLnCntFirst = 64;           // first counter word of the workspace (the words before it: flags)
 constexpr int kLnSpinLimit = 1 << 21;     // polls of a band's arrival counter before a workgroup gives up
 
+// GELU in float32:  gelu(x) = x / 2 + a G,  a = |x|,  G = erf(a / sqrt 2) / 2 = 1/2 - e / 2 + e a Q,  e = exp(-a^2 / 2),
+// Q a degree-11 polynomial in 2 a / 5 - 1 fitted (minimax of e a Q) to (1/2 - erfc(a / sqrt 2) / (2 e)) / a on [0, 5] and kept at its value beyond,
+// where e a is below 2e-5 and falls: G is 1/2 there and x / 2 + a G is exactly x or 0.  The halves that cancel near 0 do so before anything is
+// rounded.  24 issue slots a value, no branch; with the library's erff, both of whose branches a wave takes, 4.8 of the 30 us of
+// 1024 x 3072 x 768 were this function (gemm_split_share.hip).  Error against float64 over four million normal inputs of deviation 0.02 /
+// 0.3 / 1 / 2, root mean square relative to that of the results: 3.1e-8 / 3.3e-8 / 3.3e-8 / 3.1e-8, with x / 2 (1 + erff) 3.7e-8 / 4.1e-8 /
+// 3.9e-8 / 3.5e-8; the largest over |x| 1.0e-7 against 1.2e-7.
 __device__ __forceinline__ float gelu_erf(float x) {
-    return x * 0.5f * (1.0f + erff(x * 0.70710678118654752440f));
+#pragma clang fp contract(off)
+    const float a = fminf(fabsf(x), 5.0f), s = fmaf(a, 0.4f, -1.0f), e = __builtin_amdgcn_exp2f(x * x * -0.72134752044448170368f);
+    float q = -1.142469118e-03f;
+    q = fmaf(q, s, 5.211298703e-04f);
+    q = fmaf(q, s, 3.688280995e-04f);
+    q = fmaf(q, s, 2.818360692e-03f);
+    q = fmaf(q, s, -5.052679684e-03f);
+    q = fmaf(q, s, 7.229824085e-03f);
+    q = fmaf(q, s, -1.370374672e-02f);
+    q = fmaf(q, s, 2.401246130e-02f);
+    q = fmaf(q, s, -3.978192806e-02f);
+    q = fmaf(q, s, 6.372629851e-02f);
+    q = fmaf(q, s, -9.785424173e-02f);
+    q = fmaf(q, s, 1.434675008e-01f);
+    const float half = fmaf(-0.5f, e, 0.5f);
+    return fmaf(fabsf(x), fmaf(a * e, q, half), x * 0.5f);
 }
 
 // GELU for results that are stored as bf16, without transcendentals:
