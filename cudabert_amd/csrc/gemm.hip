@@ -405,6 +405,7 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 // measured inside whole forward passes at the power limit) and K is split only where 64 x 64 tiles would not give 512
 // workgroups, which takes fewer output features than any BERT has.
 constexpr int kPlanSmallRows = 6144;
+constexpr int kMidFirst = 257, kMidLast = 1280;      // bf16: rows from and up to which mid_cost estimates; others: skinny_cost and the table in plan_small
 
 namespace {
 constexpr int kSkinnyTiles[] = {kTileSkinny11, kTileSkinny21, kTileSkinny12, kTileSkinny22};
@@ -425,6 +426,38 @@ double skinny_cost(int M, int N, int K, bool split_operands, int tile, int sp, b
                           : 1.67 + q * (1.08 * fetch + 0.73 * mfma) + 0.70 * weights + 0.135 * blocks + 4.03 * out + 0.02 * (sp - 1);
 }
 
+// The same for kMidFirst to kMidLast rows, the skinny tiles and the others on one scale.  w: workgroups per CU; a tile's time grows with w (1 at
+// least), half-steps of 32 k and with how much of its last round is empty.  The skinny kernel as above, with what the average CU fetches beside
+// the busiest one.  Least squares, then a search for the fewest microseconds lost by the choice, over 300 to 6000 rows of the four linears of
+// BERT-base and BERT-large, every tile with 1 to 8 parts, weights from memory (40 matrices in turn), float32 results with the LayerNorm that
+// adds the parts.  Up to 1280 rows the tile chosen is 0.6 % slower than the best on average (8 % at the worst), with the costs for fewer rows 8 % (39 %).
+// Microseconds, LayerNorm included, their choice -> this one's:  FFN-out of BERT-base 1200 rows 22.0 -> 17.8, of BERT-large 800 rows 27.7 -> 22.1;
+// attn-out of BERT-large 640 rows 12.5 -> 9.0, 1000 rows 12.3 -> 10.7.  Passes, pooled output on the host, 400 / 640 / 1024 / 1280 rows: BERT-base
+// 526 -> 497, 586 -> 559, 696 -> 680, 730 -> 710; BERT-large 1350 -> 1309, 1640 -> 1587, 1858 -> 1818, 2286 -> 2199.  Beyond kMidLast the launches
+// come out the same or, in a pass, slower than the table's choice (1600 rows 2467 -> 2495, 1771 rows 2588 -> 2645).
+double mid_cost(int M, int N, int K, int tile, int bn, int bm, int sp, bool f32_result, bool gelu) {
+    const double tiles = (double)((N + bn - 1) / bn) * ((M + bm - 1) / bm), w = tiles * sp / 256.0;
+    const double out = (double)M * N * (f32_result ? 4.0 : 2.0) / 4.0e6, parts = (double)M * N * 4.0 * (sp - 1) / 4.0e6;
+    if (is_skinny(tile)) {
+        const double q = (double)((((long)tiles + 7) / 8 * sp + kXcdCus - 1) / kXcdCus), k = (double)((K / 32 + 8 * sp - 1) / (8 * sp)) * 256;
+        const double fetch = k * 2 * (bn + bm) / 148e3, weights = (double)N * K * 2 / 6.1e6, blocks = bn * bm / 1024.0, mfma = k / 16 * blocks * 8 / 2400.0;
+        return 0.732 + q * (0.829 * fetch + 0.431 * mfma + 0.459 * blocks - 0.352) + 0.843 * w * fetch + 1.15 * weights + 0.652 * out + 1.346 * parts;
+    }
+    struct Tile { int tile; double fixed, per_wg, per_hs, empty, empty_hs, deep_k, out, parts, gelu; };
+    static const Tile costs[] = {
+        {64, 4.271, -2.308, 0.158, 1.137, 0.03, -0.052, 1.559, 3.125, 0.094},
+        {kTile128Hand, 8.238, -5.257, 0.327, 0.924, 0.018, -0.039, 1.256, 1.885, 0.165},
+        {kTile256x128, 5.554, -0.844, 0.387, 0, 0.194, -0.053, 0.871, 0, 0.405},
+        {kTile256x128Deep, 0.437, -1.31, 0.563, 7.845, 0.116, -0.204, 0.854, 0, 1.006},
+        {256, 3.55, 1.415, 0.636, 10.54, 0.441, -0.105, 0.889, 0, 1.501},
+    };
+    const Tile* t = costs;
+    while (t->tile != tile) ++t;
+    const double g = w > 1.0 ? w : 1.0, empty = std::ceil(w) - g, hs = K / 32.0 / sp;
+    return t->fixed + g * (t->per_wg + hs * (t->per_hs + (K > 2048 ? t->deep_k : 0.0)) + (gelu ? t->gelu : 0.0)) + empty * (t->empty + t->empty_hs * hs) +
+           t->out * out + t->parts * parts;
+}
+
 // Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits), all of one k order (kOrderAny:
 // the operands and the epilogue suit the skinny kernel).
 GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, int order) {
@@ -440,6 +473,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         {kTile256x128Deep, 128, 256, 6.25, 1.33, 0.263, 1.50, 0.62, 0.86, 0.43, false, true},
         {256, 256, 256, 8.00, 3.43, 0.448, 1.15, 0.85, 0.97, 0.11, false, true},
     };
+    const bool mid = M >= kMidFirst && M <= kMidLast;
     GemmPlan best{order == kOrderSkinny ? (int)kTileSkinny12 : 64, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
@@ -454,7 +488,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
                              (gelu ? 0.8 : 0.0);
             const double out_us = (double)M * N * (f32_result ? 4.0 : 2.0) * sp / 4.0e6;
             // the consumer of split results reads every part again
-            const double cost = c.launch + c.out * out_us * (sp > 1 ? 1.5 : 1.0) + T * g;
+            const double cost = mid ? mid_cost(M, N, K, c.tile, c.bn, c.bm, sp, f32_result, gelu) : c.launch + c.out * out_us * (sp > 1 ? 1.5 : 1.0) + T * g;
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{c.tile, sp}; }
         }
     }
@@ -468,7 +502,8 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         if (order == kOrderShared) break;
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
-            const double cost = skinny_cost(M, N, K, false, tile, sp, f32_result);
+            const double cost = mid ? mid_cost(M, N, K, tile, skinny_features(tile), skinny_tokens(tile), sp, f32_result, gelu)
+                                                    : skinny_cost(M, N, K, false, tile, sp, f32_result);
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{tile, sp}; }
         }
     }
