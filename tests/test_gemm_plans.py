@@ -1,0 +1,44 @@
+"""Tile and number of parts that the library's rule gives a GEMM: ones that its kernel takes, for every row count about the rule's own limits,
+model widths from 64 to 1024 and any number of parts that the caller has room for.  No GPU needed."""
+import pytest
+
+from host_program import compile_program, lines
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "kernels.h"
+using namespace cubert;
+int main(int argc, char** argv) {
+    const int elt = std::atoi(argv[1]) ? kF32Split : kBF16, hidden = std::atoi(argv[2]), inter = std::atoi(argv[3]), step = elt == kBF16 ? 32 : 16;
+    const int shapes[4][2] = {{3 * hidden, hidden}, {hidden, hidden}, {inter, hidden}, {hidden, inter}};
+    int bad = 0, share = 0, skinny = 0;
+    for (int M : {1, 17, 31, 128, 255, 256, 257, 258, 400, 512, 640, 1000, 1024, 1279, 1280, 1281, 1600, 2048, 3000, 4096, 6143, 6144, 8191, 40000})
+        for (int s = 0; s < 4; ++s)
+            for (int max_splits : {1, 2, 3, 8, 16})
+                for (bool any : {false, true}) {
+                    const int N = shapes[s][0], K = shapes[s][1], most = s % 2 ? max_splits : 1;
+                    const GemmPlan p = gemm_plan(M, N, K, elt, most, s % 2 == 1, s == 2, any);
+                    bool ok = p.splits >= 1 && p.splits <= most && K % step == 0;
+                    if (is_skinny(p.tile)) ok = ok && any && 4 * p.splits <= K / step, ++skinny;
+                    else if (is_share(p.tile)) ok = ok && any && elt == kF32Split && 4 * p.splits <= K / 16, ++share;
+                    else if (p.tile == 256 || p.tile == kTile256x128Deep) ok = ok && elt == kBF16 && p.splits == 1 && K % 128 == 0;
+                    else if (p.tile == kTile256x128) ok = ok && (elt == kF32Split ? p.splits <= K / 16 : p.splits == 1);
+                    else ok = ok && (p.tile == 128 || (elt == kBF16 && (p.tile == 64 || p.tile == kTile128Hand))) && p.splits <= K / step;
+                    bad += !ok;
+                }
+    std::printf("%d %d %d\n", bad, share, skinny);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    return compile_program(PROGRAM, tmp_path_factory.mktemp("plans"))
+
+
+@pytest.mark.parametrize("split_operands", [0, 1])
+@pytest.mark.parametrize("hidden,inter", [(64, 64), (64, 256), (192, 768), (320, 1216), (768, 3072), (1024, 4096)])
+def test_plans_fit_their_kernels(program, split_operands, hidden, inter):
+    bad, share, skinny = map(int, lines(program, split_operands, hidden, inter)[0].split())
+    assert bad == 0 and (skinny > 0 or hidden < 128) and (share > 0 or not (split_operands and hidden >= 768))
