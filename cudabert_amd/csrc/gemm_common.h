@@ -153,6 +153,10 @@ __device__ __forceinline__ void store1(unsigned char* base, size_t elem_index, f
     }
 }
 
+// x / d as a multiplication, for x d < 2^32; 0 stands for d = 1.
+inline unsigned magic_of(unsigned d) { return d <= 1 ? 0u : (unsigned)((1ull << 32) / d + 1); }
+__device__ __forceinline__ int div_by(int x, unsigned magic) { return magic ? (int)__umulhi((unsigned)x, magic) : x; }
+
 // Workgroup id -> (tile_n, tile_m).  Hardware hands consecutive workgroup ids to
 // the eight XCDs round-robin, and every XCD has its own 4 MiB L2.  xn_parts = 4 or
 // 2 (chosen by gemm_pick_partition on the host, only when the grid divides): the

@@ -59,10 +59,6 @@ struct SkinnyRest {
     int v_rowmajor;                     // bf16 QKV: V like k; else [B, heads, 64, Sp]
 };
 
-// x / d as a multiplication, for x d < 2^32; 0 stands for d = 1.
-unsigned magic_of(unsigned d) { return d <= 1 ? 0u : (unsigned)((1ull << 32) / d + 1); }
-__device__ __forceinline__ int div_by(int x, unsigned magic) { return magic ? (int)__umulhi((unsigned)x, magic) : x; }
-
 // Workgroup ids go round the XCDs.  Each of them owns a run of the tiles, all rows of a band of features before the next band, so
 // that a weight row is fetched into one L2 (two at the ends of a run); the K shares of a tile follow each other.
 // An XCD has per_xcd tiles, one more on the first `more`; tiles_m: tiles in a band of features (divisor m_magic).  A wave has `share` K

@@ -12,7 +12,11 @@
 // Microseconds, weights from memory, LayerNorm included, against 128 x 128 with its best split:  1024 rows of BERT-base, QKV 27.7 -> 24.4,
 // attn-out 23.2 -> 17.3, FFN-in 35.3 -> 31.9, FFN-out 39.3 -> 34.1; 512 rows of BERT-large, QKV 33.6 -> 23.9, FFN-in 39.7 -> 29.4.
 // Bound: 1.05 us a step of the 96 x 128 tile (0.96 at the peak rate of the matrix pipe), 0.9 of 64 x 128 and 0.7 of 32 x 128, which their fetches
-// bound (80 to 90 GB/s a CU); around the loop some 12 us (first operands from memory, exchange, GELU and splitting, results of 6 bytes an element to memory).
+// bound (80 to 90 GB/s a CU) where few CUs work; with all of them 1.3 to 1.5 us, the socket being at its power limit (1.6 PFLOP/s of bf16 products).
+// Around the loop (time stamps, 1024 x 3072 x 768): 2.1 us until it begins, 1.1 for its first operands, 1.1 for the exchange, 2.6 for Q, K and V, 1.6
+// for a float32 result, GELU 7.3 with the library's erff and some 4 with gelu_erf; 3.6 between launches.  Without divisions on the device and with what
+// addresses take in registers at the start, against tile_of_block and the argument record: passes of 270 to 2048 rows 1.1 to 2.4 % (8 lines of 128,
+// BERT-base, 1665 -> 1626 us).
 // Steps in flight beside the one at work: one; two are 2 % slower.
 #include "gemm_split_epilogue.h"
 
@@ -23,29 +27,46 @@ using namespace gemm_detail;
 
 constexpr int kWaves = 4, kNBJ = 4, kDepth = 2;
 
-// A wave has `share` steps of 16 k, one more for the first `extra` of the kWaves * splits waves of a tile.
+constexpr int kGroupM = 8;
+
+// What the operands' addresses take comes as arguments of its own, fourteen words that arrive in registers, with every division done by the host.
+// Workgroup -> tile as in tile_of_block: xn = log2(xn_parts) + 1 or 0, cell = features' tiles << 16 | tokens' tiles of an XCD's cell (xn > 0) or of the
+// grid, run = tiles / 8 << 3 | tiles % 8; divisors kGroupM * features' tiles of the cell and the bands of its last group.
+// A wave has share >> 16 steps of 16 k, one more for the first share & 65535 of the kWaves * splits waves of a tile.
 template <int EPI, int NBI>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_share_kernel(const GemmDev p, int share, int extra) {
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_share_kernel(
+    const unsigned char* W, const unsigned char* X, int M, int N, int K, unsigned share_extra, int xn, unsigned cell, int run, unsigned group_magic,
+    unsigned last_magic, const GemmDev p) {
     constexpr bool F32OUT = EPI == kEpiBias || EPI == kEpiBiasRes;
     // [token block][source wave ^ token block, less one][block of 32 features][quad][lane]
     __shared__ __attribute__((aligned(16))) unsigned char part[kNBJ * 3 * NBI * 4096];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    int tile_n, tile_m;
-    tile_of_block<8>(blockIdx.x, p.tiles_n * p.tiles_m, p.tiles_n, p.xn_parts, &tile_n, &tile_m);
+    const int xcd = blockIdx.x & 7, n_count = cell >> 16, m_count = cell & 65535;
+    int t = blockIdx.x >> 3, tile_n = 0, tile_m = 0;
+    if (xn) {
+        tile_n = (xcd & ((1 << (xn - 1)) - 1)) * n_count;
+        tile_m = (xcd >> (xn - 1)) * m_count;
+    } else {
+        t += xcd * (run >> 3) + (xcd < (run & 7) ? xcd : run & 7);
+    }
+    const int group = div_by(t, group_magic), r = t - group * kGroupM * n_count, bands = m_count - group * kGroupM;
+    const int c = bands >= kGroupM ? r / kGroupM : div_by(r, last_magic);
+    tile_n += c;
+    tile_m += group * kGroupM + r - c * (bands >= kGroupM ? kGroupM : bands);
     const int n0 = tile_n * 32 * NBI, m0 = tile_m * 32 * kNBJ;
 
-    const int split = blockIdx.y, me = kWaves * split + wave;
+    const int split = blockIdx.y, me = kWaves * split + wave, share = share_extra >> 16, extra = share_extra & 65535;
     const int s0 = me * share + (me < extra ? me : extra), s1 = s0 + share + (me < extra ? 1 : 0);
 
     // descriptors that start at the tile's first row block, so that no operand size reaches 32 bits; row blocks past the end read as zero
-    const int rb_stride = p.K / 16 * 3072;
-    const int wleft = (p.N + 31) / 32 - (n0 >> 5), xleft = (p.M + 31) / 32 - (m0 >> 5);
+    const int rb_stride = K / 16 * 3072;
+    const int wleft = (N + 31) / 32 - (n0 >> 5), xleft = (M + 31) / 32 - (m0 >> 5);
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<unsigned char*>(p.W) + (size_t)(n0 >> 5) * rb_stride, 0, (wleft < NBI ? wleft : NBI) * rb_stride, 0x00020000);
+        const_cast<unsigned char*>(W) + (size_t)(n0 >> 5) * rb_stride, 0, (wleft < NBI ? wleft : NBI) * rb_stride, 0x00020000);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<unsigned char*>(p.X) + (size_t)(m0 >> 5) * rb_stride, 0, (xleft < kNBJ ? xleft : kNBJ) * rb_stride, 0x00020000);
+        const_cast<unsigned char*>(X) + (size_t)(m0 >> 5) * rb_stride, 0, (xleft < kNBJ ? xleft : kNBJ) * rb_stride, 0x00020000);
 
     int off[kNBJ];                                                     // of my 16 bytes in each row block (NBI <= kNBJ)
 #pragma unroll
@@ -186,15 +207,24 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 
 template <int NBI>
 bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
     const dim3 grid(d.tiles_n * d.tiles_m, d.splits), block(64 * kWaves);
-    const int share = d.K / 16 / (kWaves * d.splits), extra = d.K / 16 % (kWaves * d.splits);
+    const int total = d.tiles_n * d.tiles_m, steps = d.K / 16, waves = kWaves * d.splits;
+    int xn = d.xn_parts == 4 ? 3 : d.xn_parts == 2 ? 2 : 0;
+    if (xn && (total % 8 != 0 || d.tiles_n % d.xn_parts != 0 || d.tiles_m % (8 / d.xn_parts) != 0)) xn = 0;
+    const int n_count = xn ? d.tiles_n / d.xn_parts : d.tiles_n, m_count = xn ? d.tiles_m / (8 / d.xn_parts) : d.tiles_m;
+    if (n_count > 65535 || m_count > 65535 || steps / waves > 65535 || (double)total * kGroupM * n_count >= 4294967296.0) { set_error("gemm: too many tiles"); return false; }
+    const unsigned share = (unsigned)(steps / waves) << 16 | steps % waves, cell = (unsigned)n_count << 16 | m_count;
+    const unsigned group_magic = magic_of(kGroupM * n_count), last_magic = magic_of(m_count % kGroupM);
+#define CUBERT_SHARE(E) hipLaunchKernelGGL((gemm_split_share_kernel<E, NBI>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, share, xn, cell, \
+                                           total / 8 << 3 | total % 8, group_magic, last_magic, d)
     switch (epi) {
-        case kEpiBias: hipLaunchKernelGGL((gemm_split_share_kernel<kEpiBias, NBI>), grid, block, 0, stream, d, share, extra); break;
-        case kEpiBiasGelu: hipLaunchKernelGGL((gemm_split_share_kernel<kEpiBiasGelu, NBI>), grid, block, 0, stream, d, share, extra); break;
-        case kEpiQKV: hipLaunchKernelGGL((gemm_split_share_kernel<kEpiQKV, NBI>), grid, block, 0, stream, d, share, extra); break;
-        case kEpiQKVMap: hipLaunchKernelGGL((gemm_split_share_kernel<kEpiQKVMap, NBI>), grid, block, 0, stream, d, share, extra); break;
-        case kEpiBiasRes: hipLaunchKernelGGL((gemm_split_share_kernel<kEpiBiasRes, NBI>), grid, block, 0, stream, d, share, extra); break;
+        case kEpiBias: CUBERT_SHARE(kEpiBias); break;
+        case kEpiBiasGelu: CUBERT_SHARE(kEpiBiasGelu); break;
+        case kEpiQKV: CUBERT_SHARE(kEpiQKV); break;
+        case kEpiQKVMap: CUBERT_SHARE(kEpiQKVMap); break;
+        case kEpiBiasRes: CUBERT_SHARE(kEpiBiasRes); break;
         default: set_error("gemm: unknown epilogue"); return false;
     }
+#undef CUBERT_SHARE
     CUBERT_HIP_OK(hipGetLastError());
     return true;
 }
