@@ -405,6 +405,7 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 // measured inside whole forward passes at the power limit) and K is split only where 64 x 64 tiles would not give 512
 // workgroups, which takes fewer output features than any BERT has.
 constexpr int kPlanSmallRows = 6144;
+constexpr int kShareRows = 8192;         // split operands: rows from which no tile whose waves share K is taken (a pass runs in parts there, in one k order)
 constexpr int kMidFirst = 257, kMidLast = 1280;      // bf16: rows from and up to which mid_cost estimates; others: skinny_cost and the table in plan_small
 
 namespace {
@@ -642,7 +643,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
 
 GemmPlan gemm_plan(int M, int N, int K, int elt, int max_splits, bool f32_result, bool gelu, bool any_order) {
     const int order = any_order && N % 8 == 0 ? kOrderAny : kOrderShared;
-    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, order);
+    if (elt == kF32Split) return plan_split_operands(M, N, K, 1, max_splits > 1 ? max_splits : 1, f32_result, gelu, M < kShareRows ? order : (int)kOrderShared);
     GemmPlan best{gemm_pick_tile(M, N, K, elt), 1};
     if (elt != kBF16 || M >= kPlanSmallRows || K % 64 != 0) {
         if (max_splits > 1) {

@@ -13,7 +13,7 @@ int main(int argc, char** argv) {
     const int elt = std::atoi(argv[1]) ? kF32Split : kBF16, hidden = std::atoi(argv[2]), inter = std::atoi(argv[3]), step = elt == kBF16 ? 32 : 16;
     const int shapes[4][2] = {{3 * hidden, hidden}, {hidden, hidden}, {inter, hidden}, {hidden, inter}};
     int bad = 0, share = 0, skinny = 0;
-    for (int M : {1, 17, 31, 128, 255, 256, 257, 258, 400, 512, 640, 1000, 1024, 1279, 1280, 1281, 1600, 2048, 3000, 4096, 6143, 6144, 8191, 40000})
+    for (int M : {1, 17, 31, 128, 255, 256, 257, 258, 400, 512, 640, 1000, 1024, 1279, 1280, 1281, 1600, 2048, 3000, 4096, 6143, 6144, 8191, 8192, 40000})
         for (int s = 0; s < 4; ++s)
             for (int max_splits : {1, 2, 3, 8, 16})
                 for (bool any : {false, true}) {
@@ -21,7 +21,7 @@ int main(int argc, char** argv) {
                     const GemmPlan p = gemm_plan(M, N, K, elt, most, s % 2 == 1, s == 2, any);
                     bool ok = p.splits >= 1 && p.splits <= most && K % step == 0;
                     if (is_skinny(p.tile)) ok = ok && any && 4 * p.splits <= K / step, ++skinny;
-                    else if (is_share(p.tile)) ok = ok && any && elt == kF32Split && 4 * p.splits <= K / 16, ++share;
+                    else if (is_share(p.tile)) ok = ok && any && elt == kF32Split && M < 8192 && 4 * p.splits <= K / 16, ++share;
                     else if (p.tile == 256 || p.tile == kTile256x128Deep) ok = ok && elt == kBF16 && p.splits == 1 && K % 128 == 0;
                     else if (p.tile == kTile256x128) ok = ok && (elt == kF32Split ? p.splits <= K / 16 : p.splits == 1);
                     else ok = ok && (p.tile == 128 || (elt == kBF16 && (p.tile == 64 || p.tile == kTile128Hand))) && p.splits <= K / step;
