@@ -558,6 +558,7 @@ GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits
         if (order != kOrderAny && order != c.order) continue;
         const bool skinny = c.order == kOrderSkinny;
         if (skinny && (N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
+        if (c.order == kOrderShare4 && (N + c.bn - 1) / c.bn > 65535) continue;       // what its kernel numbers
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;
             if (c.order != kOrderShared && 4 * sp > K / 16) break;

@@ -153,9 +153,22 @@ __device__ __forceinline__ void store1(unsigned char* base, size_t elem_index, f
     }
 }
 
-// x / d as a multiplication, for x d < 2^32; 0 stands for d = 1.
-inline unsigned magic_of(unsigned d) { return d <= 1 ? 0u : (unsigned)((1ull << 32) / d + 1); }
-__device__ __forceinline__ int div_by(int x, unsigned magic) { return magic ? (int)__umulhi((unsigned)x, magic) : x; }
+// x / d for every x of 0 .. 2^31 - 1 as a multiplication and a shift:  with 2^shift the first power of two that is not below d,
+// magic = ceil(2^(31 + shift) / d) is below 2^32 and exceeds 2^(31 + shift) / d by less than 1, so that x magic / 2^(31 + shift) exceeds x / d by
+// less than x / 2^(31 + shift) < 1 / d.
+struct Divisor {
+    unsigned magic = 1u << 31, shift = 0;
+};
+inline Divisor divisor_of(unsigned d) {
+    Divisor v;
+    while ((1ull << v.shift) < d) ++v.shift;
+    if (d > 1) v.magic = (unsigned)(((1ull << (31 + v.shift)) + d - 1) / d);
+    return v;
+}
+// (shift: its low five bits)
+__host__ __device__ __forceinline__ int div_by(int x, unsigned magic, unsigned shift) {
+    return (int)((unsigned)(((unsigned long long)((unsigned)x << 1) * magic) >> 32) >> (shift & 31));
+}
 
 // Workgroup id -> (tile_n, tile_m).  Hardware hands consecutive workgroup ids to
 // the eight XCDs round-robin, and every XCD has its own 4 MiB L2.  xn_parts = 4 or

@@ -14,7 +14,7 @@
 // features a thread, and eight waves with the whole of a K of 1024 in flight.  With four waves, eight features and divisions -> now, weights
 // from memory, smallest tile that gives each CU one workgroup: bf16 17 x 2304 x 768 4.8 -> 3.6 us, 17 x 4096 x 1024 7.8 -> 5.5, 128 x 3072 x 768
 // 5.5 -> 4.6, 128 x 4096 x 1024 7.9 -> 6.4; split operands 17 x 4096 x 1024 11.4 -> 10.3, 64 x 3072 x 1024 13.1 -> 9.8.
-#include "gemm_common.h"
+#include "gemm_skinny_map.h"
 
 namespace cubert {
 namespace {
@@ -55,18 +55,16 @@ struct SkinnyRest {
     unsigned char *Y, *k, *vt;          // QKV: Y is q
     const int* rowmap;
     int S, Sp, heads;
-    unsigned s_magic;                   // divisor S (magic_of)
+    unsigned s_magic, s_shift;          // divisor S
     int v_rowmajor;                     // bf16 QKV: V like k; else [B, heads, 64, Sp]
 };
 
-// Workgroup ids go round the XCDs.  Each of them owns a run of the tiles, all rows of a band of features before the next band, so
-// that a weight row is fetched into one L2 (two at the ends of a run); the K shares of a tile follow each other.
-// An XCD has per_xcd tiles, one more on the first `more`; tiles_m: tiles in a band of features (divisor m_magic).  A wave has `share` K
-// steps, one more for the first `extra` of the kWaves * splits (divisor split_magic) waves of a tile.
+// Workgroup -> tile and part of K: skinny_tile (gemm_skinny_map.h).  A wave has `share` K steps, one more for the first `extra` of the
+// kWaves * splits waves of a tile.
 template <int ELT, int EPI, int NBI, int NBJ, int DEPTH>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsigned char* W, const unsigned char* X, int M, int N, int K,
                                                                      int per_xcd, int tiles_m, unsigned m_magic, unsigned split_magic,
-                                                                     int splits_more, int share_extra, const SkinnyRest p) {
+                                                                     int splits_more, unsigned shifts, int share_extra, const SkinnyRest p) {
     typedef Operand<ELT> Op;
     constexpr int FR = Op::kFrags, THREADS = 64 * kWaves;
     constexpr bool QKV = EPI == kEpiQKV || EPI == kEpiQKVMap;
@@ -80,11 +78,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsig
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    const int splits = splits_more >> 3, more = splits_more & 7, share = share_extra >> 11, extra = share_extra & 2047;
-    const int xcd = blockIdx.x & 7, is = blockIdx.x >> 3, idx0 = div_by(is, split_magic), split = is - idx0 * splits;
-    if (idx0 >= per_xcd + (xcd < more ? 1 : 0)) return;                // the whole workgroup: no barrier has been met
-    const int tile = xcd * per_xcd + (xcd < more ? xcd : more) + idx0, tile_n = div_by(tile, m_magic);
-    const int n0 = tile_n * 32 * NBI, m0 = (tile - tile_n * tiles_m) * 32 * NBJ;
+    const int share = share_extra >> 11, extra = share_extra & 2047;
+    int tile_n, tile_m, split;
+    if (!skinny_tile(blockIdx.x, blockIdx.y, per_xcd, tiles_m, m_magic, split_magic, splits_more, shifts, &tile_n, &tile_m, &split))
+        return;                                                        // the whole workgroup: no barrier has been met
+    const int n0 = tile_n * 32 * NBI, m0 = tile_m * 32 * NBJ;
 
     const int me = kWaves * split + wave;
     const int s0 = me * share + (me < extra ? me : extra), s1 = s0 + share + (me < extra ? 1 : 0);
@@ -226,7 +224,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsig
             if constexpr (QKV) {
                 const int hidden = p.heads * 64;                       // a tile lies in one head: hidden and n0 are multiples of its width
                 const int which = n0 >= 2 * hidden ? 2 : n0 >= hidden ? 1 : 0, head = (n0 - which * hidden) >> 6;
-                const int hn = n & 63, b = div_by(tok[it], p.s_magic), s = tok[it] - b * p.S;
+                const int hn = n & 63, b = div_by(tok[it], p.s_magic, p.s_shift), s = tok[it] - b * p.S;
                 unsigned char* base = which == 2 ? p.vt : which ? p.k : p.Y;
                 if constexpr (ELT == kBF16) {
                     if (which == 2 && !p.v_rowmajor) {
@@ -256,15 +254,15 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
     p.Y = epi == kEpiQKV || epi == kEpiQKVMap ? d.q : d.Y;
     p.k = d.k; p.vt = d.vt; p.rowmap = d.rowmap;
     p.S = d.S; p.Sp = d.Sp; p.heads = d.heads;
-    p.s_magic = magic_of(d.S);
+    const Divisor by_s = divisor_of(d.S);
+    p.s_magic = by_s.magic; p.s_shift = by_s.shift;
     p.v_rowmajor = d.v_rowmajor;
-    const int tiles_m = (d.M + 32 * NBJ - 1) / (32 * NBJ), tiles = (d.N + 32 * NBI - 1) / (32 * NBI) * tiles_m;
-    const int waves = kWaves * d.splits, steps = d.K / Operand<ELT>::kStepK;
-    const unsigned m_magic = magic_of(tiles_m), split_magic = magic_of(d.splits);
-    const int splits_more = d.splits << 3 | tiles % 8, share_extra = steps / waves << 11 | steps % waves;      // (splits < 256)
-    const dim3 grid(8 * ((tiles + 7) / 8) * d.splits), block(64 * kWaves);
+    SkinnyMap map;
+    if (!skinny_map((d.N + 32 * NBI - 1) / (32 * NBI), (d.M + 32 * NBJ - 1) / (32 * NBJ), d.splits, &map)) { set_error("gemm: too many tiles"); return false; }
+    const int waves = kWaves * d.splits, steps = d.K / Operand<ELT>::kStepK, share_extra = steps / waves << 11 | steps % waves;      // (splits < 256)
+    const dim3 grid(map.grid_x, map.grid_y), block(64 * kWaves);
 #define CUBERT_SKINNY(E) hipLaunchKernelGGL((gemm_skinny_kernel<ELT, E, NBI, NBJ, DEPTH>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, \
-                                            tiles / 8, tiles_m, m_magic, split_magic, splits_more, share_extra, p)
+                                            map.per_xcd, map.tiles_m, map.m_magic, map.split_magic, map.splits_more, map.shifts, share_extra, p)
     switch (epi) {
         case kEpiBias: CUBERT_SKINNY(kEpiBias); break;
         case kEpiBiasGelu: CUBERT_SKINNY(kEpiBiasGelu); break;

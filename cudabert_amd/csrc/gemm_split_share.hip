@@ -29,13 +29,14 @@ constexpr int kWaves = 4, kNBJ = 4, kDepth = 2;
 
 constexpr int kGroupM = 8;
 
-// What the operands' addresses take comes as arguments of its own, fourteen words that arrive in registers, with every division done by the host.
-// Workgroup -> tile as in tile_of_block: xn = log2(xn_parts) + 1 or 0, cell = features' tiles << 16 | tokens' tiles of an XCD's cell (xn > 0) or of the
-// grid, run = tiles / 8 << 3 | tiles % 8; divisors kGroupM * features' tiles of the cell and the bands of its last group.
+// What the operands' addresses take comes as arguments of its own, thirteen words that arrive in registers, with every division done by the host.
+// Workgroup -> tile as in tile_of_block: xn (low byte of xn_shifts) = log2(xn_parts) + 1 or 0, cell = features' tiles << 16 | tokens' tiles of an XCD's cell (xn > 0) or of the
+// grid, run = tiles / 8 << 3 | tiles % 8; divisors kGroupM * features' tiles of the cell and the bands of its last group, their shifts
+// in the other bytes of xn_shifts.
 // A wave has share >> 16 steps of 16 k, one more for the first share & 65535 of the kWaves * splits waves of a tile.
 template <int EPI, int NBI>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_share_kernel(
-    const unsigned char* W, const unsigned char* X, int M, int N, int K, unsigned share_extra, int xn, unsigned cell, int run, unsigned group_magic,
+    const unsigned char* W, const unsigned char* X, int M, int N, int K, unsigned share_extra, int xn_shifts, unsigned cell, int run, unsigned group_magic,
     unsigned last_magic, const GemmDev p) {
     constexpr bool F32OUT = EPI == kEpiBias || EPI == kEpiBiasRes;
     // [token block][source wave ^ token block, less one][block of 32 features][quad][lane]
@@ -43,7 +44,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    const int xcd = blockIdx.x & 7, n_count = cell >> 16, m_count = cell & 65535;
+    const int xcd = blockIdx.x & 7, n_count = cell >> 16, m_count = cell & 65535, xn = xn_shifts & 255;
     int t = blockIdx.x >> 3, tile_n = 0, tile_m = 0;
     if (xn) {
         tile_n = (xcd & ((1 << (xn - 1)) - 1)) * n_count;
@@ -51,8 +52,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 
     } else {
         t += xcd * (run >> 3) + (xcd < (run & 7) ? xcd : run & 7);
     }
-    const int group = div_by(t, group_magic), r = t - group * kGroupM * n_count, bands = m_count - group * kGroupM;
-    const int c = bands >= kGroupM ? r / kGroupM : div_by(r, last_magic);
+    const int group = div_by(t, group_magic, xn_shifts >> 8), r = t - group * kGroupM * n_count, bands = m_count - group * kGroupM;
+    const int c = bands >= kGroupM ? r / kGroupM : div_by(r, last_magic, xn_shifts >> 16);
     tile_n += c;
     tile_m += group * kGroupM + r - c * (bands >= kGroupM ? kGroupM : bands);
     const int n0 = tile_n * 32 * NBI, m0 = tile_m * 32 * kNBJ;
@@ -211,11 +212,12 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
     int xn = d.xn_parts == 4 ? 3 : d.xn_parts == 2 ? 2 : 0;
     if (xn && (total % 8 != 0 || d.tiles_n % d.xn_parts != 0 || d.tiles_m % (8 / d.xn_parts) != 0)) xn = 0;
     const int n_count = xn ? d.tiles_n / d.xn_parts : d.tiles_n, m_count = xn ? d.tiles_m / (8 / d.xn_parts) : d.tiles_m;
-    if (n_count > 65535 || m_count > 65535 || steps / waves > 65535 || (double)total * kGroupM * n_count >= 4294967296.0) { set_error("gemm: too many tiles"); return false; }
+    if (n_count > 65535 || m_count > 65535 || steps / waves > 65535 || (long)d.tiles_n * d.tiles_m >= 1L << 24) { set_error("gemm: too many tiles"); return false; }
     const unsigned share = (unsigned)(steps / waves) << 16 | steps % waves, cell = (unsigned)n_count << 16 | m_count;
-    const unsigned group_magic = magic_of(kGroupM * n_count), last_magic = magic_of(m_count % kGroupM);
-#define CUBERT_SHARE(E) hipLaunchKernelGGL((gemm_split_share_kernel<E, NBI>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, share, xn, cell, \
-                                           total / 8 << 3 | total % 8, group_magic, last_magic, d)
+    const Divisor group = divisor_of(kGroupM * n_count), last = divisor_of(m_count % kGroupM);
+    const int xn_shifts = xn | group.shift << 8 | last.shift << 16;
+#define CUBERT_SHARE(E) hipLaunchKernelGGL((gemm_split_share_kernel<E, NBI>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, share, xn_shifts, cell, \
+                                           total / 8 << 3 | total % 8, group.magic, last.magic, d)
     switch (epi) {
         case kEpiBias: CUBERT_SHARE(kEpiBias); break;
         case kEpiBiasGelu: CUBERT_SHARE(kEpiBiasGelu); break;
