@@ -62,30 +62,44 @@ __device__ __forceinline__ int frag_kphase(int units) { return units ? 0x400 : 0
 constexpr int kLnCntFirst = 64;           // first counter word of the workspace (the words before it: flags)
 constexpr int kLnSpinLimit = 1 << 21;     // polls of a band's arrival counter before a workgroup gives up
 
-// GELU in float32:  gelu(x) = x / 2 + a G,  a = |x|,  G = erf(a / sqrt 2) / 2 = 1/2 - e / 2 + e a Q,  e = exp(-a^2 / 2),
-// Q a degree-11 polynomial in 2 a / 5 - 1 fitted (minimax of e a Q) to (1/2 - erfc(a / sqrt 2) / (2 e)) / a on [0, 5] and kept at its value beyond,
-// where e a is below 2e-5 and falls: G is 1/2 there and x / 2 + a G is exactly x or 0.  The halves that cancel near 0 do so before anything is
-// rounded.  24 issue slots a value, no branch; with the library's erff, both of whose branches a wave takes, 4.8 of the 30 us of
-// 1024 x 3072 x 768 were this function (gemm_split_share.hip).  Error against float64 over four million normal inputs of deviation 0.02 /
-// 0.3 / 1 / 2, root mean square relative to that of the results: 3.1e-8 / 3.3e-8 / 3.3e-8 / 3.1e-8, with x / 2 (1 + erff) 3.7e-8 / 4.1e-8 /
-// 3.9e-8 / 3.5e-8; the largest over |x| 1.0e-7 against 1.2e-7.
+// GELU in float32, from e = exp(-x^2 / 2); a = |x|.
+//   a < 1:  x / 2 + x^2 R,        R = erf(a / sqrt 2) / (2 a), a degree-5 polynomial in x^2 (off by less than 4e-10)
+//   else:   max(x, 0) - a e P,    P = erfc(a / sqrt 2) / (2 e), a degree-9 polynomial in a / 2 - 3/2 fitted on [1, 5] for the smallest largest
+//                                 error of a e P (4.6e-9) and kept at its value beyond, where a e P is below 1.5e-6 and falls
+// so that nothing that has been rounded is subtracted from a number of its own size, on either side of 0.  (max(x, 0) as |x| / 2 + x / 2: minus
+// infinity ends as NaN, as in x / 2 (1 + erf).)
+__host__ __device__ __forceinline__ float gelu_with_exp(float x, float e) {
+#pragma clang fp contract(off)
+    const float a = fminf(fabsf(x), 5.0f), s = fmaf(a, 0.5f, -1.5f), xx = x * x;
+    float p = -5.624590558e-04f;
+    p = fmaf(p, s, -1.265096944e-04f);
+    p = fmaf(p, s, -5.884463317e-04f);
+    p = fmaf(p, s, 2.300337190e-03f);
+    p = fmaf(p, s, -3.971423488e-03f);
+    p = fmaf(p, s, 8.816573769e-03f);
+    p = fmaf(p, s, -1.852843165e-02f);
+    p = fmaf(p, s, 3.662370890e-02f);
+    p = fmaf(p, s, -6.879935414e-02f);
+    p = fmaf(p, s, 1.215140596e-01f);
+    float r = -6.753106391e-06f;
+    r = fmaf(r, xx, 1.108878132e-04f);
+    r = fmaf(r, xx, -1.183557441e-03f);
+    r = fmaf(r, xx, 9.971991181e-03f);
+    r = fmaf(r, xx, -6.649008393e-02f);
+    r = fmaf(r, xx, 3.989422619e-01f);
+    const bool small = a < 1.0f;
+    return fmaf(small ? xx : a, small ? r : -(e * p), fmaf(fabsf(x), small ? 0.0f : 0.5f, x * 0.5f));
+}
+// Some 30 issue slots a value, no branch; with the library's erff, both of whose branches a wave takes, some 60: 4.8 of the 30 us of 1024 x 3072 x 768
+// were the function (gemm_split_share.hip).  One form for all x, x / 2 + |x| G with six slots fewer, loses digits for negative x (4.5e-8 on -4 .. -3) and
+// is no faster in short passes, 0.5 % in 16 lines of 512, BERT-base (7 718 us, here 7 759).
+// Error against float64 on the device, root mean square, here / x / 2 (1 + erff):  two million inputs of each interval, -0.01 .. 0 7.7e-11 / 9.1e-11,
+// -0.75 .. -0.625 7.3e-9 / 1.2e-8, -2 .. -1.5 5.8e-9 / 1.9e-8, -4 .. -3 3.3e-9 / 3.0e-8, 0.25 .. 0.375 4.5e-9 / 7.3e-9, 1 .. 1.125 2.0e-8 / 3.1e-8, 3 .. 4
+// 6.9e-8 / 1.1e-7 (no larger in any of the twenty intervals of either sign, nor is the largest error);  normal inputs of deviation 0.02 / 0.3 / 1 / 2,
+// relative to the results' own, 2.5e-8 / 2.8e-8 / 2.7e-8 / 2.5e-8 against 3.7e-8 / 4.1e-8 / 3.9e-8 / 3.5e-8.
 __device__ __forceinline__ float gelu_erf(float x) {
 #pragma clang fp contract(off)
-    const float a = fminf(fabsf(x), 5.0f), s = fmaf(a, 0.4f, -1.0f), e = __builtin_amdgcn_exp2f(x * x * -0.72134752044448170368f);
-    float q = -1.142469118e-03f;
-    q = fmaf(q, s, 5.211298703e-04f);
-    q = fmaf(q, s, 3.688280995e-04f);
-    q = fmaf(q, s, 2.818360692e-03f);
-    q = fmaf(q, s, -5.052679684e-03f);
-    q = fmaf(q, s, 7.229824085e-03f);
-    q = fmaf(q, s, -1.370374672e-02f);
-    q = fmaf(q, s, 2.401246130e-02f);
-    q = fmaf(q, s, -3.978192806e-02f);
-    q = fmaf(q, s, 6.372629851e-02f);
-    q = fmaf(q, s, -9.785424173e-02f);
-    q = fmaf(q, s, 1.434675008e-01f);
-    const float half = fmaf(-0.5f, e, 0.5f);
-    return fmaf(fabsf(x), fmaf(a * e, q, half), x * 0.5f);
+    return gelu_with_exp(x, __builtin_amdgcn_exp2f(x * x * -0.72134752044448170368f));
 }
 
 // GELU for results that are stored as bf16, without transcendentals:
