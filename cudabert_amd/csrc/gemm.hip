@@ -631,6 +631,7 @@ bool launch_split_operands(const GemmParams& p, hipStream_t stream) {
             set_error("gemm: operand exceeds the 2 GiB addressable through one buffer descriptor");
             return false;
         }
+        d.xn_parts = p.xcd_partition > 0 ? p.xcd_partition : 0;
         return launch_gemm_skinny(d, kF32Split, tile, epi, stream);
     }
     const int bn = is_share(tile) ? share_features(tile) : tile == kTile256x128 ? 256 : 128;
@@ -796,6 +797,7 @@ bool launch_gemm(const GemmParams& p, hipStream_t stream) {
             set_error("gemm: the skinny tiles need bf16 operands in the units layout and a GELU result in it, row-major QKV or float32 result");
             return false;
         }
+        d.xn_parts = p.xcd_partition > 0 ? p.xcd_partition : 0;
         return launch_gemm_skinny(d, kBF16, bt, epi == kEpiBiasGeluUnits ? (int)kEpiBiasGelu : epi, stream);
     }
     if (bt == kTile128Hand) {

@@ -258,7 +258,7 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
     p.s_magic = by_s.magic; p.s_shift = by_s.shift;
     p.v_rowmajor = d.v_rowmajor;
     SkinnyMap map;
-    if (!skinny_map((d.N + 32 * NBI - 1) / (32 * NBI), (d.M + 32 * NBJ - 1) / (32 * NBJ), d.splits, &map)) { set_error("gemm: too many tiles"); return false; }
+    if (!skinny_map((d.N + 32 * NBI - 1) / (32 * NBI), (d.M + 32 * NBJ - 1) / (32 * NBJ), d.splits, d.xn_parts, &map)) { set_error("gemm: too many tiles"); return false; }
     const int waves = kWaves * d.splits, steps = d.K / Operand<ELT>::kStepK, share_extra = steps / waves << 11 | steps % waves;      // (splits < 256)
     const dim3 grid(map.grid_x, map.grid_y), block(64 * kWaves);
 #define CUBERT_SKINNY(E) hipLaunchKernelGGL((gemm_skinny_kernel<ELT, E, NBI, NBJ, DEPTH>), grid, block, 0, stream, d.W, d.X, d.M, d.N, d.K, \
@@ -279,7 +279,7 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
 }  // namespace
 
 // elt kBF16 (both operands and a GELU result in the units layout; per-head Q, K, V; float32 results) or kF32Split; tile a
-// skinny one; d.N % 8 == 0.
+// skinny one; d.N % 8 == 0; d.xn_parts 0, 2 or 4 (skinny_map's cells).
 bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int epilogue, hipStream_t stream) {
     const int step = elt == kBF16 ? 32 : 16;
     if (d.K % step != 0 || d.N % 8 != 0 || d.splits < 1 || d.splits > 255 || 4 * d.splits > d.K / step) {

@@ -59,3 +59,25 @@ def test_qkv_rows(lib, tile, B, S, heads):  # noqa: F811
         ref = want[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
         lim = scale[:, i * H:(i + 1) * H].view(B, S, heads, 64).permute(0, 2, 1, 3)
         assert ((t.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + (H / 16 + 6) * U * lim).all()
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N", [(129, 256), (256, 320)])
+@pytest.mark.parametrize("split_operands", [False, True])
+def test_xcd_partitions_give_the_same_bits(lib, tile, M, N, split_operands):  # noqa: F811
+    """Who computes a tile is all that a partition changes; one that does not divide the grid is left out."""
+    K = 256
+    X, W, b = (f32.operands(M, N, K) if split_operands else b16.operands(M, N, K))[:3]
+    if split_operands:
+        xp, wp, elt, flags = f32.split(lib, X.cuda()), f32.split(lib, W.cuda()), f32.SPLIT, 0
+    else:
+        xp, wp, elt, flags = b16.pack(lib, X, True), b16.pack(lib, W, True), 1, 3 | b16.UNITS["X"] | b16.UNITS["W"]
+    bd, out = b.cuda(), []
+    for partition in (-1, 0, 2, 4):
+        Y = torch.full((2, M, N), float("nan"), device="cuda")
+        f32.check(lib.cubert_op_gemm(xp.data_ptr(), wp.data_ptr(), bd.data_ptr(), Y.data_ptr(), M, N, K, K, elt, 0, 0, tile,
+                                     flags | ((partition + 1) << 16) | 2 << 8, None))
+        torch.cuda.synchronize()
+        assert not torch.isnan(Y).any()
+        out.append(Y)
+    assert all(torch.equal(out[0], y) for y in out[1:])
