@@ -93,7 +93,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsig
     const int w_off = Op::lane_offset(n0, K, l32, g), x_off = Op::lane_offset(m0, K, l32, g), stride = Op::block_stride(K);
     u32x4_t wf[DEPTH][NBI][FR], xf[DEPTH][NBJ][FR];
     auto load = [&](int d, int step) {
-        // Loads past the wave's share lie outside the descriptor (bit 31 of the lane offset): no traffic.
+        // Loads past the wave's share lie outside the descriptor (bit 31 of the lane offset): nothing is fetched, but the CU takes as long
+        // over their addresses as over others', hence the depths (launch_depth).
         // They are issued all the same: with a fixed number of loads in flight the compiler waits for exactly the oldest ones.
         const int k = step * Op::kStepBytes, none = step < s1 ? 0 : (int)0x80000000u;
 #pragma unroll
@@ -276,6 +277,16 @@ bool launch_epi(const GemmDev& d, int epi, hipStream_t stream) {
     return true;
 }
 
+// Steps in flight: the fewest of the depths that hold a wave's share, or the last, as many as its 256 registers hold.  With the last for every
+// share, most loads of narrow models were past it: six layers, us, last depth / chosen, hidden 64, float32, 17 rows 206 / 157, 2048 rows 270 / 222;
+// hidden 128 17 rows 213 / 167, bf16 152 / 143; hidden 768 17 rows 253 / 226, bf16 168 / 163; level where a share fills it (hidden 1024, bf16 228 / 228).
+template <int ELT, int NBI, int NBJ, int DEPTH, int... MORE>
+bool launch_depth(const GemmDev& d, int share, int epi, hipStream_t stream) {
+    if constexpr (sizeof...(MORE) > 0)
+        if (share > DEPTH) return launch_depth<ELT, NBI, NBJ, MORE...>(d, share, epi, stream);
+    return launch_epi<ELT, NBI, NBJ, DEPTH>(d, epi, stream);
+}
+
 }  // namespace
 
 // elt kBF16 (both operands and a GELU result in the units layout; per-head Q, K, V; float32 results) or kF32Split; tile a
@@ -286,20 +297,20 @@ bool launch_gemm_skinny(const gemm_detail::GemmDev& d, int elt, int tile, int ep
         set_error("gemm: the skinny kernel needs N a multiple of 8 and at least four K steps per split");
         return false;
     }
-    // (depth: the steps a wave has in flight, as many as its 256 registers hold)
+    const int share = (d.K / step + kWaves * d.splits - 1) / (kWaves * d.splits);
     if (elt == kBF16) {
         switch (tile) {
-            case kTileSkinny11: return launch_epi<kBF16, 1, 1, 4>(d, epilogue, stream);
-            case kTileSkinny21: return launch_epi<kBF16, 2, 1, 4>(d, epilogue, stream);
-            case kTileSkinny12: return launch_epi<kBF16, 1, 2, 4>(d, epilogue, stream);
-            default: return launch_epi<kBF16, 2, 2, 4>(d, epilogue, stream);
+            case kTileSkinny11: return launch_depth<kBF16, 1, 1, 1, 2, 3, 4>(d, share, epilogue, stream);
+            case kTileSkinny21: return launch_depth<kBF16, 2, 1, 1, 2, 3, 4>(d, share, epilogue, stream);
+            case kTileSkinny12: return launch_depth<kBF16, 1, 2, 1, 2, 3, 4>(d, share, epilogue, stream);
+            default: return launch_depth<kBF16, 2, 2, 1, 2, 3, 4>(d, share, epilogue, stream);
         }
     }
     switch (tile) {
-        case kTileSkinny11: return launch_epi<kF32Split, 1, 1, 8>(d, epilogue, stream);
-        case kTileSkinny21: return launch_epi<kF32Split, 2, 1, 5>(d, epilogue, stream);
-        case kTileSkinny12: return launch_epi<kF32Split, 1, 2, 5>(d, epilogue, stream);
-        default: return launch_epi<kF32Split, 2, 2, 3>(d, epilogue, stream);
+        case kTileSkinny11: return launch_depth<kF32Split, 1, 1, 2, 4, 6, 8>(d, share, epilogue, stream);
+        case kTileSkinny21: return launch_depth<kF32Split, 2, 1, 1, 2, 3, 5>(d, share, epilogue, stream);
+        case kTileSkinny12: return launch_depth<kF32Split, 1, 2, 1, 2, 3, 5>(d, share, epilogue, stream);
+        default: return launch_depth<kF32Split, 2, 2, 1, 2, 3>(d, share, epilogue, stream);
     }
 }
 

@@ -81,3 +81,24 @@ def test_xcd_partitions_give_the_same_bits(lib, tile, M, N, split_operands):  # 
         assert not torch.isnan(Y).any()
         out.append(Y)
     assert all(torch.equal(out[0], y) for y in out[1:])
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 9, 13])
+@pytest.mark.parametrize("split_operands", [False, True])
+def test_steps_of_a_wave(lib, tile, steps, split_operands):  # noqa: F811
+    """Every number of K steps that a wave keeps in flight, and more than those; some waves have a step less."""
+    K = 128 * steps - 48 if split_operands else 256 * steps - 64
+    M, N = 40, 72
+    X, W, b = (f32.operands(M, N, K) if split_operands else b16.operands(M, N, K))[:3]
+    want = X.double() @ W.double().t() + b.double()
+    scale = X.double().abs() @ W.double().abs().t() + b.double().abs()
+    if split_operands:
+        xp, wp, elt, flags = f32.split(lib, X.cuda()), f32.split(lib, W.cuda()), f32.SPLIT, 0
+    else:
+        xp, wp, elt, flags = b16.pack(lib, X, True), b16.pack(lib, W, True), 1, 3 | b16.UNITS["X"] | b16.UNITS["W"]
+    bd = b.cuda()
+    Y = torch.full((M, N), float("nan"), device="cuda")
+    f32.check(lib.cubert_op_gemm(xp.data_ptr(), wp.data_ptr(), bd.data_ptr(), Y.data_ptr(), M, N, K, K, elt, 0, 0, tile, flags, None))
+    torch.cuda.synchronize()
+    assert ((Y.double().cpu() - want).abs() <= ((6 if split_operands else 1) * K / 16 + 7) * U * scale).all()
