@@ -407,6 +407,12 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 constexpr int kPlanSmallRows = 6144;
 constexpr int kShareRows = 8192;         // split operands: rows from which no tile whose waves share K is taken (a pass runs in parts there, in one k order)
 constexpr int kMidFirst = 257, kMidLast = 1280;      // bf16: rows from and up to which mid_cost estimates; others: skinny_cost and the table in plan_small
+// ... and the K from which: below, a tile's estimate falls with the workgroups of a CU (the costs are fitted to K of 768 and more).  Passes of six
+// layers, us, by them for every K / from 512 on: hidden 128, 800 to 1280 rows 213 to 230 / 187 to 206, hidden 256, 1280 rows 263 / 241.
+constexpr int kMidK = 512;
+// bf16: rows up to which a skinny tile is chosen (of narrow models: wider ones leave them before).  Hidden 64, us, with / without from 2048 rows on: 2560
+// rows 212 / 215, 3200 223 / 224, 4000 235 / 234, 4800 251 / 246, 6080 269 / 263.
+constexpr int kSkinnyLast = 4096;
 
 namespace {
 constexpr int kSkinnyTiles[] = {kTileSkinny11, kTileSkinny21, kTileSkinny12, kTileSkinny22};
@@ -474,7 +480,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         {kTile256x128Deep, 128, 256, 6.25, 1.33, 0.263, 1.50, 0.62, 0.86, 0.43, false, true},
         {256, 256, 256, 8.00, 3.43, 0.448, 1.15, 0.85, 0.97, 0.11, false, true},
     };
-    const bool mid = M >= kMidFirst && M <= kMidLast;
+    const bool mid = M >= kMidFirst && M <= kMidLast && K >= kMidK;
     GemmPlan best{order == kOrderSkinny ? (int)kTileSkinny12 : 64, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
@@ -500,7 +506,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
     // 128 rows 6.4 / 4.1 against 8.4 / 6.6, 200 rows 8.2 / 5.3 against 8.3 / 6.9, 400 rows 13.4 / 9.2 against 12.0 / 8.6; attn-out 128
     // rows 7.2 / 6.3 against 8.9 / 8.2, 600 rows 10.9 / 10.2 against 12.3 / 11.8.
     for (int tile : kSkinnyTiles) {
-        if (order == kOrderShared) break;
+        if (order == kOrderShared || (order == kOrderAny && M > kSkinnyLast)) break;
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (4 * sp > K / 32 || (sp > min_splits && K / sp < 128)) break;
             const double cost = mid ? mid_cost(M, N, K, tile, skinny_features(tile), skinny_tokens(tile), sp, f32_result, gelu)

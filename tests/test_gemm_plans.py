@@ -42,3 +42,26 @@ def program(tmp_path_factory):
 def test_plans_fit_their_kernels(program, split_operands, hidden, inter):
     bad, share, skinny = map(int, lines(program, split_operands, hidden, inter)[0].split())
     assert bad == 0 and (skinny > 0 or hidden < 128) and (share > 0 or not (split_operands and hidden >= 768))
+
+
+NARROW = r"""
+#include <cstdio>
+#include "kernels.h"
+using namespace cubert;
+int main() {
+    int bad = 0;
+    for (int hidden : {64, 128, 192, 256})
+        for (int M = 1; M < 6144; M += M < 300 ? 7 : 61)
+            for (int s = 0; s < 4; ++s) {
+                const int N = s == 0 ? 3 * hidden : s == 2 ? 4 * hidden : hidden, K = s == 3 ? 4 * hidden : hidden;
+                const GemmPlan p = gemm_plan(M, N, K, kBF16, s % 2 ? 8 : 1, s % 2 == 1, s == 2, true);
+                bad += M <= 1280 ? !is_skinny(p.tile) && p.tile != 64 : M > 4096 && is_skinny(p.tile);
+            }
+    std::printf("%d\n", bad);
+}
+"""
+
+
+def test_narrow_models_take_small_tiles(tmp_path):
+    """bf16, up to hidden 256: tiles of at most 64 x 64 while larger ones would leave most CUs without one, no skinny ones for many rows."""
+    assert lines(compile_program(NARROW, tmp_path)) == ["0"]
