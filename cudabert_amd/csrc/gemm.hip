@@ -405,6 +405,7 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 // measured inside whole forward passes at the power limit) and K is split only where 64 x 64 tiles would not give 512
 // workgroups, which takes fewer output features than any BERT has.
 constexpr int kPlanSmallRows = 6144;
+constexpr int kShareFirst = 257;         // split operands: rows from which a tile whose four waves share K is chosen
 constexpr int kShareRows = 8192;         // split operands: rows from which no tile whose waves share K is taken (a pass runs in parts there, in one k order)
 constexpr int kMidFirst = 257, kMidLast = 1280;      // bf16: rows from and up to which mid_cost estimates; others: skinny_cost and the table in plan_small
 // ... and the K from which: below, a tile's estimate falls with the workgroups of a CU (the costs are fitted to K of 768 and more).  Passes of six
@@ -517,34 +518,37 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
     return best;
 }
 
-// Estimated time (microseconds) of a launch on split operands, w workgroups per CU, of a tile whose four waves share K (one workgroup to a
-// CU, so whole rounds, which last as long as their fetches and products; a round's GELU is not hidden) or of 128 x 128 (two to a CU).
-// out: the result at 4 TB/s; parts: what the consumer reads beside the first part.  Least squares over launches of 160 to 6000 rows of the four
-// linears of BERT-base and BERT-large, 1 to 8 parts, weights from memory, float32 results with the LayerNorm that adds the parts (mean error
-// 6 %; what is chosen by it and skinny_cost is 0.3 % slower on average than the best, 8 % at the worst).
-double share_or_128_cost(int M, int N, int K, int tile, int sp, double w, bool f32_result, bool gelu) {
+// Estimated time (microseconds) of a launch on split operands, w workgroups per CU, on the scale of skinny_cost: of a tile whose four waves share K (one
+// workgroup to a CU, so whole rounds, which last as long as their fetches and products; a round's GELU is not hidden), of 128 x 128 or of 256 x 128
+// (two to a CU).  out: the result at 4 TB/s; parts: what the consumer reads beside the first part.  Least squares over 408 problems of 200 to 8100 rows of
+// the four linears of hidden 256, 384, 512, 768 and 1024, 1 to 8 parts, weights from memory, float32 results with the LayerNorm that adds the parts,
+// the competitive ones weighted most (mean error 6 %; what is chosen by it and skinny_cost is 1.4 % slower on average than the best).  A microsecond on
+// all of them for the weights that a skinny tile finds in the L2s in a pass (l2_touch.h; with none, 1024 rows of BERT-large 985 us for six layers, with two
+// 512 rows 658: 973 and 642 / 660 with one), and 3 % on tiles that share K beyond 4096 rows, where they are chosen too often otherwise.
+double staged_or_share_cost(int M, int N, int K, int tile, int sp, double w, bool f32_result, bool gelu) {
     const double out = (double)M * N * (f32_result ? 4.0 : 6.0) / 4.0e6, parts = (double)M * N * 4.0 * (sp - 1) / 4.0e6, rounds = std::ceil(w);
-    if (tile == 128) {
-        const double g = w > 1.0 ? w : 1.0, steps = K / 16.0 / sp;
-        return 9.44 + g * (0.476 * steps - 5.83 + (gelu ? 2.54 : 0.0)) + (w > 1.0 ? 0.38 * (rounds - g) * steps : 0.0) + 1.51 * out + 3.59 * parts;
+    const double g = w > 1.0 ? w : 1.0, stretch = w > 1.0 ? rounds - g : 0.0;
+    if (is_share(tile)) {
+        const double blocks = share_features(tile) / 32, steps = (K / 16 + 4 * sp - 1) / (4 * sp);
+        const double us = 3.3 + rounds * (steps * (0.391 + 0.299 * blocks) + (0.231 + (gelu ? 0.392 : 0.0)) * blocks) + 1.47 * out + 3.68 * parts;
+        return M > 4096 ? 1.03 * us : us;
     }
-    const double blocks = share_features(tile) / 32, steps = (K / 16 + 4 * sp - 1) / (4 * sp);
-    return 2.75 + rounds * (steps * (0.475 + 0.281 * blocks) + (gelu ? 1.35 : 0.0) * blocks) + 2.38 * out + 4.56 * parts - 0.34 * w;
+    const double steps = K / 16.0 / sp;
+    if (tile == kTile256x128) return 13.39 + g * (1.038 * steps - 8.02 + (gelu ? 3.2 : 0.0)) + 0.603 * stretch * steps + 0.632 * out;
+    return 8.37 + g * (0.478 * steps - 2.6 + (gelu ? 1.22 : 0.0)) + 0.349 * stretch * steps + 0.836 * out + 2.71 * parts;
 }
 
-// float32 operands in the split layout.  Estimated time (microseconds) of a launch from that of a workgroup alone on its CU
-// and w = workgroups / 256, with constants measured on MI355X (cold weights: launches that cycle through 24 matrices, 17 to
-// 1600 rows of the linears of BERT-base and BERT-large, and up to 19600 rows for the large tiles):
-//   128 x 128, 256 x 128: (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly
-//     what the first did, and the hand-out is uneven by half a workgroup; the larger tile wins from about 900 tiles on;
-//   where tiles whose waves share K may be chosen too: skinny_cost, and share_or_128_cost for 128 x 128 as well.  LayerNorm included, us, best
-//   share tile / best of the others: 512 rows, BERT-base 18.8 / 19.7 (QKV), 22.9 / 25.4 (FFN-in), 25.0 / 25.9 (FFN-out); 1024 rows 24.4 / 27.7,
-//   17.3 / 23.2 (attn-out), 31.9 / 35.3, 34.1 / 39.3; 2048 rows, BERT-large 67.1 / 72.3, 31.4 / 42.0, 107.7 / 85.1 (FFN-in stays), 83.4 / 95.3;
-//   6000 rows 186.8 / 172.2, 82.5 / 85.7, 279.7 / 227.8, 232.8 / 251.1.
-// The 128 x 128 constants here are those of its loop before it read fragments a step ahead (gemm_split.hip), which takes less from launches
-// of few workgroups: 1024 x 768 x 768 in 23.6 us for an estimate of 27.8.  Best skinny tile against 128 x 128, us, weights from memory:
-// 128 rows, QKV / FFN-in of BERT-large 13.5 / 14.0 against 33.4 / 34.9; 400 rows 29.2 / 30.4 against 32.6 / 34.8; 600 rows 30.4 / 42.5
-// against 33.2 / 35.3; of BERT-base 600 rows 23.1 / 23.9 against 26.6 / 28.5.
+// float32 operands in the split layout.  Where tiles whose waves share K may be chosen (launches of a pass in one part), skinny_cost and
+// staged_or_share_cost.  Best skinny tile / best share tile / 128 x 128 / 256 x 128, us, LayerNorm included:  BERT-large QKV 256 rows 16.2 / 17.5 / 33.2 / 74.1
+// (share tiles are chosen from kShareFirst rows on), 400 rows 29.0 / 20.4 / 32.9 / 73.9, 1280 rows 59.9 / 45.5 / 43.5 / 74.4, 2048 rows 104.4 / 63.5 / 71.7 /
+// 75.5, 5000 rows - / 152.4 / 141.5 / 139.3;  FFN-in of BERT-base 1408 rows 58.3 / 49.3 / 50.9 / 62.9, of BERT-large 1280 rows 79.8 / 62.4 / 71.4 / 78.0, 2048 rows
+// 142.7 / 94.1 / 80.7 / 85.9;  FFN-out of BERT-base 1024 rows 42.2 / 33.0 / 39.1 / -, 1280 rows 44.0 / 38.2 / 44.3 / -.  (With 256 x 128 on the scale below, which
+// knows no GELU and no result, FFN-in took it from 1280 rows on;
+// passes of six layers, us, before / now: BERT-large 1280 rows 1251 / 1191, 1408 rows 1386 / 1332, BERT-base 1408 rows 980 / 956, 2048 rows 1197 / 1142.)
+// Otherwise the time of a workgroup alone on its CU, stretched by w = workgroups / 256 (cold weights, up to 19600 rows):
+//   (fixed + per_step * 16-k steps) * (w > 1 ? w + 0.5 : 1): a second workgroup on a CU costs nearly what the first did, and the hand-out is uneven by
+//   half a workgroup; 256 x 128 wins from about 900 tiles on.  The constants of 128 x 128 are those of its loop before it read fragments a step
+//   ahead (gemm_split.hip), which takes less from launches of few workgroups.
 GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits, bool f32_result, bool gelu, int order) {
     struct Cand { int tile, bm, bn; double fixed, per_step; int order; };
     static const Cand cands[] = {
@@ -564,17 +568,18 @@ GemmPlan plan_split_operands(int M, int N, int K, int min_splits, int max_splits
         if (order != kOrderAny && order != c.order) continue;
         const bool skinny = c.order == kOrderSkinny;
         if (skinny && (N % 8 != 0 || split_bytes(M, K) >= (1ull << 31) || split_bytes(N, K) >= (1ull << 31))) continue;
-        if (c.order == kOrderShare4 && (N + c.bn - 1) / c.bn > 65535) continue;       // what its kernel numbers
+        if (c.order == kOrderShare4 && ((order == kOrderAny && M < kShareFirst) || (N + c.bn - 1) / c.bn > 65535)) continue;      // (65535: what its kernel numbers)
         for (int sp = min_splits; sp <= max_splits && sp <= 16; sp *= 2) {
             if (sp > min_splits && K / sp < 128) break;
             if (c.order != kOrderShared && 4 * sp > K / 16) break;
+            if (c.tile == kTile256x128 && sp > 1 && order != kOrderShared) break;          // staged_or_share_cost knows it whole only
             double cost;
             if (skinny) {
                 cost = skinny_cost(M, N, K, true, c.tile, sp, f32_result);
             } else {
                 const double w = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * sp / 256.0, g = w > 1.0 ? w + 0.5 : 1.0;
-                if (order != kOrderShared && c.tile != kTile256x128) {
-                    cost = share_or_128_cost(M, N, K, c.tile, sp, w, f32_result, gelu);
+                if (order != kOrderShared) {
+                    cost = staged_or_share_cost(M, N, K, c.tile, sp, w, f32_result, gelu);
                 } else {
                     cost = (c.fixed + c.per_step * (K / 16.0 / sp)) * (w > 4.0 && c.tile == kTile256x128 ? w : g);
                     // every part of a split result is written and read again by the consumer
