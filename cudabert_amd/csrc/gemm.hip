@@ -32,6 +32,7 @@
 //
 // The 256 tile in bf16 has a hand-scheduled twin (gemm_bf16_256.hip); this
 // file is the general kernel (any tile, f32, odd step counts).
+#include <algorithm>
 #include <cmath>
 
 #include "gemm_common.h"
@@ -407,10 +408,16 @@ int gemm_pick_tile(int M, int N, int K, int elt) {
 constexpr int kPlanSmallRows = 6144;
 constexpr int kShareFirst = 257;         // split operands: rows from which a tile whose four waves share K is chosen
 constexpr int kShareRows = 8192;         // split operands: rows from which no tile whose waves share K is taken (a pass runs in parts there, in one k order)
-constexpr int kMidFirst = 257, kMidLast = 1280;      // bf16: rows from and up to which mid_cost estimates; others: skinny_cost and the table in plan_small
-// ... and the K from which: below, a tile's estimate falls with the workgroups of a CU (the costs are fitted to K of 768 and more).  Passes of six
-// layers, us, by them for every K / from 512 on: hidden 128, 800 to 1280 rows 213 to 230 / 187 to 206, hidden 256, 1280 rows 263 / 241.
-constexpr int kMidK = 512;
+// bf16: rows from and up to which mid_cost estimates, the latter for models from hidden 1024 on and for narrower ones; others: skinny_cost and the table in
+// plan_small.  Passes of six layers, us, by those / by mid_cost:  from below, hidden 1024, 257 rows 295 / 296, 270 rows 299 / 284, 384 rows 333 / 314,
+// hidden 640, 288 rows 233 / 235, 400 rows 278 / 263;  to above, hidden 1024, 1408 rows 566 / 542, 1536 rows 581 / 554, 1552 rows 603 / 608, 1800 rows
+// 617 / 630;  hidden 768, 1536 rows 473 / 441, 2048 rows 506 / 478, 2400 rows 544 / 539, 2800 rows 603 / 603;  hidden 512, 2400 rows 439 / 435, 2800 rows
+// 433 / 461.
+constexpr int kMidFirst = 257, kMidLast = 1536, kMidLastNarrow = 2400;
+// ... and the K from which, for float32 results (few features: a CU has one workgroup at most) and for others: below, a tile's estimate falls with the
+// workgroups of a CU (the costs are fitted to K of 768 and more).  Passes of six layers, us, by mid_cost for every K / from these on: hidden 128, 800 to 1280
+// rows 213 to 230 / 187 to 206, hidden 256, 1280 rows 263 / 241; hidden 384, 1280 rows, with 512 for both 277, with 384 for float32 results 269.
+constexpr int kMidK = 512, kMidKF32 = 384;
 // bf16: rows up to which a skinny tile is chosen (of narrow models: wider ones leave them before).  Hidden 64, us, with / without from 2048 rows on: 2560
 // rows 212 / 215, 3200 223 / 224, 4000 235 / 234, 4800 251 / 246, 6080 269 / 263.
 constexpr int kSkinnyLast = 4096;
@@ -434,15 +441,14 @@ double skinny_cost(int M, int N, int K, bool split_operands, int tile, int sp, b
                           : 1.67 + q * (1.08 * fetch + 0.73 * mfma) + 0.70 * weights + 0.135 * blocks + 4.03 * out + 0.02 * (sp - 1);
 }
 
-// The same for kMidFirst to kMidLast rows, the skinny tiles and the others on one scale.  w: workgroups per CU; a tile's time grows with w (1 at
+// The same for a few hundred to some two thousand rows (kMidFirst), the skinny tiles and the others on one scale.  w: workgroups per CU; a tile's time grows with w (1 at
 // least), half-steps of 32 k and with how much of its last round is empty.  The skinny kernel as above, with what the average CU fetches beside
 // the busiest one.  Least squares, then a search for the fewest microseconds lost by the choice, over 300 to 6000 rows of the four linears of
 // BERT-base and BERT-large, every tile with 1 to 8 parts, weights from memory (40 matrices in turn), float32 results with the LayerNorm that
 // adds the parts.  Up to 1280 rows the tile chosen is 0.6 % slower than the best on average (8 % at the worst), with the costs for fewer rows 8 % (39 %).
 // Microseconds, LayerNorm included, their choice -> this one's:  FFN-out of BERT-base 1200 rows 22.0 -> 17.8, of BERT-large 800 rows 27.7 -> 22.1;
 // attn-out of BERT-large 640 rows 12.5 -> 9.0, 1000 rows 12.3 -> 10.7.  Passes, pooled output on the host, 400 / 640 / 1024 / 1280 rows: BERT-base
-// 526 -> 497, 586 -> 559, 696 -> 680, 730 -> 710; BERT-large 1350 -> 1309, 1640 -> 1587, 1858 -> 1818, 2286 -> 2199.  Beyond kMidLast the launches
-// come out the same or, in a pass, slower than the table's choice (1600 rows 2467 -> 2495, 1771 rows 2588 -> 2645).
+// 526 -> 497, 586 -> 559, 696 -> 680, 730 -> 710; BERT-large 1350 -> 1309, 1640 -> 1587, 1858 -> 1818, 2286 -> 2199.
 double mid_cost(int M, int N, int K, int tile, int bn, int bm, int sp, bool f32_result, bool gelu) {
     const double tiles = (double)((N + bn - 1) / bn) * ((M + bm - 1) / bm), w = tiles * sp / 256.0;
     const double out = (double)M * N * (f32_result ? 4.0 : 2.0) / 4.0e6, parts = (double)M * N * 4.0 * (sp - 1) / 4.0e6;
@@ -481,7 +487,7 @@ GemmPlan plan_small(int M, int N, int K, int min_splits, int max_splits, bool f3
         {kTile256x128Deep, 128, 256, 6.25, 1.33, 0.263, 1.50, 0.62, 0.86, 0.43, false, true},
         {256, 256, 256, 8.00, 3.43, 0.448, 1.15, 0.85, 0.97, 0.11, false, true},
     };
-    const bool mid = M >= kMidFirst && M <= kMidLast && K >= kMidK;
+    const bool mid = M >= kMidFirst && M <= (std::min(N, K) < 1024 ? kMidLastNarrow : kMidLast) && K >= (f32_result ? kMidKF32 : kMidK);
     GemmPlan best{order == kOrderSkinny ? (int)kTileSkinny12 : 64, min_splits};
     double best_cost = 1e30;
     for (const Cand& c : cands) {
