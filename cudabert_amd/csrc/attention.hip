@@ -597,9 +597,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_split_kernel(
     const int l32 = lane & 31, g = lane >> 5;
     const int h = blockIdx.x, b = blockIdx.y, q0 = blockIdx.z * 32;
     if ((int)blockIdx.z >= query_blocks) {               // the workgroups after the queries: weights for the next launch
-        const int plane = gridDim.x * gridDim.y, id = h + gridDim.x * b + plane * blockIdx.z, e = id - plane * query_blocks;
-        const int per_xcd = plane * (int)(gridDim.z - query_blocks) / 8;
-        if ((e >> 3) < per_xcd) l2_touch<false>(ahead, id & 7, (e >> 3) * NW + wave, per_xcd * NW, lane);
+        l2_touch<false>(ahead, l2_share_after_planes(h, b, blockIdx.z, gridDim.x, gridDim.y, gridDim.z, query_blocks, NW, wave), lane);
         return;
     }
     const int qlen = cu ? cu[b + 1] - cu[b] : S;

@@ -5,7 +5,9 @@
 // before it leave the memory and most CUs idle, so workgroups added to them touch every line of those weights once, on each XCD the
 // eighth of the features whose tiles the skinny kernel gives it.  (Touched from another XCD a line comes from the Infinity Cache
 // afterwards, which is worth a fifth of that.  The GEMMs themselves as launches that touch gain nothing: their own waves are in the way.)
-// A wave takes one piece of 64 lines: with four a wave the added workgroups outlast the launch.
+// A wave takes a piece of 64 lines, and of weights with more pieces an XCD than 128 (BERT-large FFN-in in float32, 384) up to three one after the other: the
+// workgroups added are 32 an XCD at most.  They are not free: LayerNorm of 128 rows of BERT-large in float32
+// lasts 5.1 us without them and 6.2 with (BERT-large in bf16, 200 rows, 4.2 and 4.9).
 // The description is 16 bytes, since what it adds to the record of arguments is paid by every launch: 48 bytes, 0.18 us.
 #pragma once
 #include "kernels.h"
@@ -25,21 +27,43 @@ __host__ __device__ constexpr size_t l2_offset(int K, int g, int line) {
                  : (size_t)(g >> 3) * (K / 32 * 16384) + (g & 7) * 2048 + (line >> 4) * 16384 + (line & 15) * 128;
 }
 
-#if defined(__HIPCC__)
-// The index'th of `waves` waves on that XCD.
-template <bool SPLIT>
-__device__ __forceinline__ void l2_touch(const WeightsAhead& a, int xcd, int index, int waves, int lane) {
-    const int pieces = l2_pieces<SPLIT>(a.K), lines = l2_lines<SPLIT>(a.K), first = a.groups * xcd / 8, end = a.groups * (xcd + 1) / 8;
-    for (int u = index; u < (end - first) * pieces; u += waves) {
+// Which XCD's weights, and which share of them, an added wave takes: the index'th of `waves`.  Workgroups go round the XCDs in the order of their ids.
+struct L2Share {
+    int xcd, index, waves;
+};
+// Workgroup `block` of a grid of `rows` workgroups and the added ones.
+__host__ __device__ __forceinline__ L2Share l2_share_after_rows(int block, int rows, int grid, int wave) {
+    return {block & 7, ((block - rows) >> 3) * 4 + wave, (grid - rows) / 8 * 4};
+}
+// Workgroup (x, y, z) of a grid of gx x gy x (blocks + added planes); workgroups of `nw` waves.  index >= waves: none (the last few workgroups, where they are
+// no multiple of eight).
+__host__ __device__ __forceinline__ L2Share l2_share_after_planes(int x, int y, int z, int gx, int gy, int gz, int blocks, int nw, int wave) {
+    const int plane = gx * gy, id = x + gx * y + plane * z, e = id - plane * blocks;
+    return {id & 7, (e >> 3) * nw + wave, plane * (gz - blocks) / 8 * nw};
+}
+
+// Offsets that a lane of that wave touches.
+template <bool SPLIT, class Touch>
+__host__ __device__ __forceinline__ void l2_walk(const WeightsAhead& a, const L2Share& s, int lane, Touch touch) {
+    if (s.index >= s.waves) return;
+    const int pieces = l2_pieces<SPLIT>(a.K), lines = l2_lines<SPLIT>(a.K), first = a.groups * s.xcd / 8, end = a.groups * (s.xcd + 1) / 8;
+    for (int u = s.index; u < (end - first) * pieces; u += s.waves) {
         const int rel = u / pieces, g = first + rel, line = (u - rel * pieces) * 64 + lane;
-        unsigned t = 0;
-        if (line < lines) t = *reinterpret_cast<const unsigned*>(static_cast<const unsigned char*>(a.w) + l2_offset<SPLIT>(a.K, g, line));
-        asm volatile("" :: "v"(t));              // a use, or the load would not be there
+        if (line < lines) touch(l2_offset<SPLIT>(a.K, g, line));
     }
+}
+
+#if defined(__HIPCC__)
+template <bool SPLIT>
+__device__ __forceinline__ void l2_touch(const WeightsAhead& a, const L2Share& s, int lane) {
+    l2_walk<SPLIT>(a, s, lane, [&](size_t at) {
+        const unsigned t = *reinterpret_cast<const unsigned*>(static_cast<const unsigned char*>(a.w) + at);
+        asm volatile("" :: "v"(t));              // a use, or the load would not be there
+    });
 }
 #endif
 
-// Workgroups of four waves to add to a launch, a multiple of eight: a piece a wave, or a few.
+// Workgroups of four waves to add to a launch, a multiple of eight.
 template <bool SPLIT>
 int l2_touch_workgroups(const WeightsAhead& a) {
     if (!a.w) return 0;

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void add_layernorm_parts_kernel(float* __restr
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = blockIdx.x;
     if (row >= rows) {                     // the workgroups after the rows: weights for the next launch
-        l2_touch<LAYOUT == kSplit>(ahead, row & 7, ((row - rows) >> 3) * 4 + wave, (int)(gridDim.x - rows) / 8 * 4, lane);
+        l2_touch<LAYOUT == kSplit>(ahead, l2_share_after_rows(row, rows, gridDim.x, wave), lane);
         return;
     }
     float* xrow = x + (size_t)row * H;
