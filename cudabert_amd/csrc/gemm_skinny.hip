@@ -80,7 +80,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_skinny_kernel(const unsig
     const int l32 = lane & 31, g = lane >> 5;
     const int share = share_extra >> 11, extra = share_extra & 2047;
     int tile_n, tile_m, split;
-    if (!skinny_tile(blockIdx.x, blockIdx.y, per_xcd, tiles_m, m_magic, split_magic, splits_more, shifts, &tile_n, &tile_m, &split))
+    if (!skinny_tile(blockIdx.x, blockIdx.y, (int)((unsigned)(N + 32 * NBI - 1) / (32 * NBI)), per_xcd, tiles_m, m_magic, split_magic, splits_more, shifts, &tile_n, &tile_m, &split))
         return;                                                        // the whole workgroup: no barrier has been met
     const int n0 = tile_n * 32 * NBI, m0 = tile_m * 32 * NBJ;
 

@@ -14,7 +14,7 @@ namespace gemm_detail {
 struct SkinnyMap {
     int per_xcd, tiles_m;
     unsigned m_magic, split_magic;      // divisors tiles_m, splits
-    int splits_more;                    // log2(cells) << 16 | splits << 3 | tiles % 8
+    int splits_more;                    // 3 or log2(cells) << 16 | splits << 3 | tiles % 8
     unsigned shifts;                    // of the divisors, tiles_m's in the low byte
     unsigned grid_x, grid_y;
 };
@@ -32,26 +32,23 @@ inline bool skinny_map(int tiles_n, int tiles_m, int splits, int cells, SkinnyMa
     const Divisor dm = divisor_of(tiles_m), ds = divisor_of(splits);
     m->per_xcd = (int)(tiles / 8); m->tiles_m = tiles_m;
     m->m_magic = dm.magic; m->split_magic = ds.magic;
-    m->splits_more = cells / 2 << 16 | splits << 3 | (int)(tiles % 8);      // log2(2) = 1, log2(4) = 2
+    m->splits_more = (cells ? cells / 2 : 3) << 16 | splits << 3 | (int)(tiles % 8);      // log2(2) = 1, log2(4) = 2
     m->shifts = dm.shift | ds.shift << 8;
     m->grid_x = rows > 1 ? kSkinnyGridX : (unsigned)all; m->grid_y = (unsigned)rows;
     return true;
 }
 
 // False: a workgroup without a tile.
-__host__ __device__ __forceinline__ bool skinny_tile(unsigned block_x, unsigned block_y, int per_xcd, int tiles_m, unsigned m_magic, unsigned split_magic,
+__host__ __device__ __forceinline__ bool skinny_tile(unsigned block_x, unsigned block_y, int tiles_n, int per_xcd, int tiles_m, unsigned m_magic, unsigned split_magic,
                                                      int splits_more, unsigned shifts, int* tile_n, int* tile_m, int* split) {
     const int id = (int)(block_x + (block_y << kSkinnyGridXLog2)), splits = (splits_more >> 3) & 255, more = splits_more & 7, lg = splits_more >> 16;
     const int xcd = id & 7, is = id >> 3, idx = div_by(is, split_magic, shifts >> 8);
     if (idx >= per_xcd + (xcd < more ? 1 : 0)) return false;
     *split = is - idx * splits;
-    const int tile = lg ? idx : xcd * per_xcd + (xcd < more ? xcd : more) + idx;
-    *tile_n = div_by(tile, m_magic, shifts);
-    *tile_m = tile - *tile_n * tiles_m;
-    if (lg) {
-        *tile_n += (xcd & ((1 << lg) - 1)) * div_by(per_xcd, m_magic, shifts);
-        *tile_m += (xcd >> lg) * tiles_m;
-    }
+    // Runs: tile / tiles_m and what is left.  Cells: the quotient goes on through all cells, those of the next rows begin at its multiples of tiles_n.
+    const int tile = xcd * per_xcd + (xcd < more ? xcd : more) + idx, q = div_by(tile, m_magic, shifts), rows = xcd >> lg;
+    *tile_n = q - rows * tiles_n;
+    *tile_m = tile - q * tiles_m + rows * tiles_m;
     return true;
 }
 

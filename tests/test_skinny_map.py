@@ -39,7 +39,7 @@ int main(int argc, char** argv) {
     for (unsigned y = 0; y < m.grid_y; ++y)
         for (unsigned x = 0; x < m.grid_x; ++x) {
             int n, t, s;
-            if (!skinny_tile(x, y, m.per_xcd, m.tiles_m, m.m_magic, m.split_magic, m.splits_more, m.shifts, &n, &t, &s)) { ++idle; continue; }
+            if (!skinny_tile(x, y, tiles_n, m.per_xcd, m.tiles_m, m.m_magic, m.split_magic, m.splits_more, m.shifts, &n, &t, &s)) { ++idle; continue; }
             if (n < 0 || n >= tiles_n || t < 0 || t >= tiles_m || s < 0 || s >= splits) { ++outside; continue; }
             if (cells) elsewhere += n / (tiles_n / cells) != (int)(x & 7) % cells || t / (tiles_m * cells / 8) != (int)(x & 7) / cells;
             twice += seen[((size_t)n * tiles_m + t) * splits + s]++;
