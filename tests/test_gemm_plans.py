@@ -89,3 +89,20 @@ def test_float32_tiles_are_compared_on_one_scale(tmp_path):
     """FFN-in of 1024 to 2048 rows: 256 x 128, by launches 5 to 28 % slower than the best there, is not what comes out; nor are tiles that share K in
     fours up to 256 rows."""
     assert lines(compile_program(ONE_SCALE, tmp_path)) == ["0"]
+
+
+LONG = r"""
+#include <cstdio>
+#include "kernels.h"
+using namespace cubert;
+int main() {
+    int staged = 0;
+    for (int M : {513, 521, 544}) staged += !is_skinny(gemm_plan(M, 768, 256, kBF16, 1, false, false, true).tile);
+    std::printf("%d\n", staged);
+}
+"""
+
+
+def test_long_lines_of_a_narrow_model_take_skinny_tiles(tmp_path):
+    """What tests/test_gpu_skinny_tiles.py takes for given of lines just beyond 512 positions."""
+    assert lines(compile_program(LONG, tmp_path)) == ["0"]

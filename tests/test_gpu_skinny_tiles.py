@@ -102,3 +102,43 @@ def test_steps_of_a_wave(lib, tile, steps, split_operands):  # noqa: F811
     f32.check(lib.cubert_op_gemm(xp.data_ptr(), wp.data_ptr(), bd.data_ptr(), Y.data_ptr(), M, N, K, K, elt, 0, 0, tile, flags, None))
     torch.cuda.synchronize()
     assert ((Y.double().cpu() - want).abs() <= ((6 if split_operands else 1) * K / 16 + 7) * U * scale).all()
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K", [(1, 32, 128), (33, 96, 192), (130, 160, 512), (65, 224, 256)])
+def test_gelu_in_both_layouts(lib, tile, M, N, K):  # noqa: F811
+    """Features and rows that end inside a tile and inside a unit; the 32 x 32 tile leaves half of the threads without a result of their own."""
+    b16.test_gelu_result_in_units(lib, tile, M, N, K)
+    f32.test_gelu_result_is_the_next_split_operand(lib, tile, M, N, K)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("B,S,heads", [(1, 1, 1), (3, 45, 2), (2, 129, 3)])
+def test_split_qkv_and_attention(lib, tile, B, S, heads):  # noqa: F811
+    f32.test_qkv_projection_and_attention(lib, B, S, heads, tile)
+
+
+def test_transposed_values(lib, tmp_path, monkeypatch):  # noqa: F811
+    """Lines beyond 512 positions, whose V is stored transposed: a narrow model's QKV takes a skinny tile there (tests/test_gemm_plans.py).  Against the same
+    model with sums over K in one piece, which takes the staged tile: bf16 results that differ by roundings of 2^-8, carried through one layer."""
+    import dataclasses
+    import numpy as np
+    from cudabert_amd import pybert, synth
+    from cudabert_amd import weights as Wt
+    from oracle import bert_oracle as O
+    dims = dataclasses.replace(Wt.BASE, hidden=256, heads=4, inter=1024, layers=1, vocab=500, max_pos=600)
+    d = str(tmp_path)
+    Wt.export_npy_dir(Wt.bf16_representable(Wt.synth_state(dims, seed=3, degenerate=False)), d)
+    npy = Wt.load_npy_dir(d)
+    out = {}
+    for S in (513, 521, 544):
+        ids, seg, mask = synth.make_inputs(1, S, np.full(1, S), vocab=dims.vocab, seed=S, prune=False)
+        seq_ref, _ = O.forward_torch(npy, dims.heads, ids, seg, mask)
+        for split in ("1", "0"):
+            monkeypatch.setenv("CUBERT_SPLIT_K", split)
+            m = pybert.load_model_ex(d, dims.hidden, dims.layers, dims.heads, dims.inter, precision=1, max_batchsize=1, max_seq_length=600)
+            out[split] = pybert.encode(m, ids, seg, mask, want_seq=True)[1]
+            pybert.unload_model(m)
+            assert np.abs(out[split] - seq_ref).max() < 3e-2
+        rms = np.sqrt((seq_ref ** 2).mean())
+        assert np.sqrt(((out["1"] - out["0"]) ** 2).mean()) < 2.0 ** -8 * rms
