@@ -9,12 +9,12 @@
 //
 // Against a tile staged in the LDS this takes a third of a workgroup's work per wave without its barriers, and a tile of 96 features makes one
 // even round of launches that 128 x 128 leaves a quarter or half of the chip idle in: 1024 x 3072 x 768 256 workgroups instead of 192.
-// Microseconds, weights from memory, LayerNorm included, against 128 x 128 with its best split:  1024 rows of BERT-base, QKV 27.7 -> 24.4,
-// attn-out 23.2 -> 17.3, FFN-in 35.3 -> 31.9, FFN-out 39.3 -> 34.1; 512 rows of BERT-large, QKV 33.6 -> 23.9, FFN-in 39.7 -> 29.4.
+// Microseconds, weights from memory, LayerNorm included, against 128 x 128 with its best split:  1024 rows of BERT-base, QKV 28.7 -> 24.0,
+// attn-out 23.2 -> 17.5, FFN-in 31.6 -> 28.3, FFN-out 39.1 -> 33.0; 512 rows of BERT-large, QKV 33.6 -> 23.9.
 // Bound: 1.05 us a step of the 96 x 128 tile (0.96 at the peak rate of the matrix pipe), 0.9 of 64 x 128 and 0.7 of 32 x 128, which their fetches
 // bound (80 to 90 GB/s a CU) where few CUs work; with all of them 1.3 to 1.5 us, the socket being at its power limit (1.6 PFLOP/s of bf16 products).
 // Around the loop (time stamps, 1024 x 3072 x 768): 2.1 us until it begins, 1.1 for its first operands, 1.1 for the exchange, 2.6 for Q, K and V, 1.6
-// for a float32 result, GELU 7.3 with the library's erff and some 4 with gelu_erf; 3.6 between launches.  Without divisions on the device and with what
+// for a float32 result, GELU 7.3 with the library's erff and some 4 with a polynomial of 24 issue slots a value (gelu_erf: 30); 3.6 between launches.  Without divisions on the device and with what
 // addresses take in registers at the start, against tile_of_block and the argument record: passes of 270 to 2048 rows 1.1 to 2.4 % (8 lines of 128,
 // BERT-base, 1665 -> 1626 us).
 // Steps in flight beside the one at work: one; two are 2 % slower.

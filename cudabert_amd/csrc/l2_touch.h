@@ -5,9 +5,9 @@
 // before it leave the memory and most CUs idle, so workgroups added to them touch every line of those weights once, on each XCD the
 // eighth of the features whose tiles the skinny kernel gives it.  (Touched from another XCD a line comes from the Infinity Cache
 // afterwards, which is worth a fifth of that.  The GEMMs themselves as launches that touch gain nothing: their own waves are in the way.)
-// A wave takes a piece of 64 lines, and of weights with more pieces an XCD than 128 (BERT-large FFN-in in float32, 384) up to three one after the other: the
-// workgroups added are 32 an XCD at most.  They are not free: LayerNorm of 128 rows of BERT-large in float32
-// lasts 5.1 us without them and 6.2 with (BERT-large in bf16, 200 rows, 4.2 and 4.9).
+// A wave takes a piece of 64 lines, and of weights with more pieces an XCD than 128 (BERT-large FFN-in in float32, 384) up to three one after
+// the other: the workgroups added are 32 an XCD at most.  Many of them are not free: LayerNorm of 128 rows of BERT-large in float32 lasts 5.1 us
+// without and 6.2 with them, of 17 rows of BERT-base in bf16 3.0 and 2.9.
 // The description is 16 bytes, since what it adds to the record of arguments is paid by every launch: 48 bytes, 0.18 us.
 #pragma once
 #include "kernels.h"
