@@ -409,7 +409,7 @@ constexpr int kPlanSmallRows = 6144;
 constexpr int kShareFirst = 257;         // split operands: rows from which a tile whose four waves share K is chosen
 constexpr int kShareRows = 8192;         // split operands: rows from which no tile whose waves share K is taken (a pass runs in parts there, in one k order)
 // bf16: rows from and up to which mid_cost estimates, the latter for models from hidden 1024 on and for narrower ones; others: skinny_cost and the table in
-// plan_small.  Passes of six layers, us, by those / by mid_cost:  from below, hidden 1024, 257 rows 295 / 296, 270 rows 299 / 284, 384 rows 333 / 314,
+// plan_small.  Passes of six layers, us, by those / by mid_cost:  from below, hidden 1024, 257 rows 295 / 284, 270 rows 299 / 284, 384 rows 333 / 314,
 // hidden 640, 288 rows 233 / 235, 400 rows 278 / 263;  to above, hidden 1024, 1408 rows 566 / 542, 1536 rows 581 / 554, 1552 rows 603 / 608, 1800 rows
 // 617 / 630;  hidden 768, 1536 rows 473 / 441, 2048 rows 506 / 478, 2400 rows 544 / 539, 2800 rows 603 / 603;  hidden 512, 2400 rows 439 / 435, 2800 rows
 // 433 / 461.
@@ -468,8 +468,9 @@ double mid_cost(int M, int N, int K, int tile, int bn, int bm, int sp, bool f32_
     const Tile* t = costs;
     while (t->tile != tile) ++t;
     const double g = w > 1.0 ? w : 1.0, empty = std::ceil(w) - g, hs = K / 32.0 / sp;
-    return t->fixed + g * (t->per_wg + hs * (t->per_hs + (K > 2048 ? t->deep_k : 0.0)) + (gelu ? t->gelu : 0.0)) + empty * (t->empty + t->empty_hs * hs) +
-           t->out * out + t->parts * parts;
+    // (a workgroup more on a CU takes time also at a K below those of the fit)
+    const double one = t->per_wg + hs * (t->per_hs + (K > 2048 ? t->deep_k : 0.0)) + (gelu ? t->gelu : 0.0);
+    return t->fixed + one + (g - 1.0) * std::max(one, 0.01 * hs) + empty * (t->empty + t->empty_hs * hs) + t->out * out + t->parts * parts;
 }
 
 // Best (tile, splits) with min_splits <= splits <= max_splits (powers of two times min_splits), all of one k order (kOrderAny:

@@ -91,8 +91,9 @@ __host__ __device__ __forceinline__ float gelu_with_exp(float x, float e) {
     return fmaf(small ? xx : a, small ? r : -(e * p), fmaf(fabsf(x), small ? 0.0f : 0.5f, x * 0.5f));
 }
 // Some 30 issue slots a value, no branch; with the library's erff, both of whose branches a wave takes, some 60: 4.8 of the 30 us of 1024 x 3072 x 768
-// were the function (gemm_split_share.hip).  One form for all x, x / 2 + |x| G with six slots fewer, loses digits for negative x (4.5e-8 on -4 .. -3) and
-// is no faster in short passes, 0.5 % in 16 lines of 512, BERT-base (7 718 us, here 7 759).
+// were the function (gemm_split_share.hip).  One form for all x, x / 2 + |x| G with six slots fewer, is 0.3 to 1.1 % of a pass faster (twelve layers, 2048
+// rows of BERT-large 3365 us, here 3402; 8000 rows 11 365, here 11 365 to 11 412) but loses digits for negative x: 4.5e-8 on -4 .. -3.  A degree less in
+// either polynomial is further off than erff's form in some interval.
 // Error against float64 on the device, root mean square, here / x / 2 (1 + erff):  two million inputs of each interval, -0.01 .. 0 7.7e-11 / 9.1e-11,
 // -0.75 .. -0.625 7.3e-9 / 1.2e-8, -2 .. -1.5 5.8e-9 / 1.9e-8, -4 .. -3 3.3e-9 / 3.0e-8, 0.25 .. 0.375 4.5e-9 / 7.3e-9, 1 .. 1.125 2.0e-8 / 3.1e-8, 3 .. 4
 // 6.9e-8 / 1.1e-7 (no larger in any of the twenty intervals of either sign, nor is the largest error);  normal inputs of deviation 0.02 / 0.3 / 1 / 2,

@@ -106,3 +106,24 @@ int main() {
 def test_long_lines_of_a_narrow_model_take_skinny_tiles(tmp_path):
     """What tests/test_gpu_skinny_tiles.py takes for given of lines just beyond 512 positions."""
     assert lines(compile_program(LONG, tmp_path)) == ["0"]
+
+
+PARTS = r"""
+#include <cstdio>
+#include "kernels.h"
+using namespace cubert;
+int main() {
+    int most = 0;
+    for (int M = 257; M <= 300; ++M) {
+        const int parts = gemm_plan(M, 1024, 4096, kBF16, 16, true, false, true).splits;
+        most = parts > most ? parts : most;
+    }
+    std::printf("%d\n", most);
+}
+"""
+
+
+def test_parts_cost_workgroups(tmp_path):
+    """FFN-out of BERT-large for some hundred rows: an eighth of K is below what the costs are fitted to, where more workgroups on a CU must not come
+    out as cheaper ones."""
+    assert int(lines(compile_program(PARTS, tmp_path))[0]) <= 4
