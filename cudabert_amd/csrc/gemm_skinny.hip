@@ -21,15 +21,17 @@ namespace {
 
 using namespace gemm_detail;
 
+// (An operand is smaller than 2 GiB, so that its size and offsets in it take 32 bits: the size by 64 bits was a dozen instructions of a wave's way to
+// its first load.)
 template <int ELT>
 struct Operand;
 // float32 split: a step is 16 k; per block of 32 rows three fragments, one per plane
 template <>
 struct Operand<kF32Split> {
     static constexpr int kFrags = 3, kStepK = 16;
-    static __host__ __device__ size_t bytes(int rows, int K) { return split_bytes(rows, K); }
-    static __device__ int lane_offset(int row0, int K, int l32, int g) { return (row0 >> 5) * (K / 16) * 3072 + (l32 + 32 * g) * 16; }
-    static __device__ int block_stride(int K) { return K / 16 * 3072; }      // 32 rows further
+    static __device__ unsigned bytes(int rows, int K) { return ((unsigned)(rows + 31) >> 5) * (K >> 4) * 3072; }      // split_bytes
+    static __device__ int lane_offset(int row0, int K, int l32, int g) { return (row0 >> 5) * (K >> 4) * 3072 + (l32 + 32 * g) * 16; }
+    static __device__ int block_stride(int K) { return (K >> 4) * 3072; }    // 32 rows further
     static constexpr int kStepBytes = 3072;
     static __device__ int frag_offset(int lane_off, int f) { return lane_off + f * 1024; }
 };
@@ -37,9 +39,9 @@ struct Operand<kF32Split> {
 template <>
 struct Operand<kBF16> {
     static constexpr int kFrags = 2, kStepK = 32;
-    static __host__ __device__ size_t bytes(int rows, int K) { return packed_bytes(rows, (size_t)K * 2); }
+    static __device__ unsigned bytes(int rows, int K) { return ((unsigned)(rows + 255) >> 8) * (K >> 5) * 16384; }    // packed_bytes
     static __device__ int lane_offset(int row0, int K, int l32, int g) {
-        return (row0 >> 8) * (K / 32) * 16384 + (row0 & 255) * 64 + (l32 + 32 * g) * 16;
+        return (row0 >> 8) * (K >> 5) * 16384 + (row0 & 255) * 64 + (l32 + 32 * g) * 16;
     }
     static __device__ int block_stride(int) { return 2048; }                 // 32 rows further in the same 256-row block
     static constexpr int kStepBytes = 16384;

@@ -35,17 +35,16 @@ struct L2Share {
 __host__ __device__ __forceinline__ L2Share l2_share_after_rows(int block, int rows, int grid, int wave) {
     return {block & 7, ((block - rows) >> 3) * 4 + wave, (grid - rows) / 8 * 4};
 }
-// Workgroup (x, y, z) of a grid of gx x gy x (blocks + added planes); workgroups of `nw` waves.  index >= waves: none (the last few workgroups, where they are
-// no multiple of eight).
+// Workgroup (x, y, z) of a grid of gx x gy x (blocks + added planes); workgroups of `nw` waves.  The last few, where they are no multiple of eight, take
+// nothing (an index past all pieces).
 __host__ __device__ __forceinline__ L2Share l2_share_after_planes(int x, int y, int z, int gx, int gy, int gz, int blocks, int nw, int wave) {
-    const int plane = gx * gy, id = x + gx * y + plane * z, e = id - plane * blocks;
-    return {id & 7, (e >> 3) * nw + wave, plane * (gz - blocks) / 8 * nw};
+    const int plane = gx * gy, id = x + gx * y + plane * z, e = id - plane * blocks, per_xcd = plane * (gz - blocks) / 8;
+    return {id & 7, (e >> 3) < per_xcd ? (e >> 3) * nw + wave : 1 << 30, per_xcd * nw};
 }
 
 // Offsets that a lane of that wave touches.
 template <bool SPLIT, class Touch>
 __host__ __device__ __forceinline__ void l2_walk(const WeightsAhead& a, const L2Share& s, int lane, Touch touch) {
-    if (s.index >= s.waves) return;
     const int pieces = l2_pieces<SPLIT>(a.K), lines = l2_lines<SPLIT>(a.K), first = a.groups * s.xcd / 8, end = a.groups * (s.xcd + 1) / 8;
     for (int u = s.index; u < (end - first) * pieces; u += s.waves) {
         const int rel = u / pieces, g = first + rel, line = (u - rel * pieces) * 64 + lane;
