@@ -125,8 +125,8 @@ def two_layers(tmp_path_factory):
 
 @pytest.mark.parametrize("B,S", [(1, 1), (1, 17), (1, 64), (1, 65), (1, 128), (1, 129), (1, 256), (1, 257), (2, 129)])
 def test_rows_at_which_the_model_changes_layout_and_tile(two_layers, B, S):
-    """The units layout and the skinny tiles end at 128 rows; eager and replayed pass against the float32 oracle at the bf16
-    mode's tolerance, 3e-2."""
+    """Row counts at the edges of 32- and 256-row blocks and at the line where the plan changes its costs (257); eager and replayed pass against the float32
+    oracle at the bf16 mode's tolerance, 3e-2."""
     from cudabert_amd import pybert, synth
     from oracle import bert_oracle as O
     m, npy, dims = two_layers
